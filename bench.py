@@ -442,7 +442,7 @@ def main():
         "levels": es * samples // 4 + 4 * samples // 16,
         "final": 4 * samples // 4 + es * 3 * samples // 4 + samples,
     }
-    kernel_name = {"blocks": "sgn_ht_rows", "levels": "sgn_idwt_level", "final": "sgn_final"}[dom]
+    kernel_name = {"blocks": "sgn_ht_magsgn", "levels": "sgn_idwt_level", "final": "sgn_final"}[dom]
     traffic = None
     tpath = os.path.join(ROOT, "profiles", "hbm_traffic_4096x256_rgb8.json")
     if args.tiles == 4096 and os.path.exists(tpath):

@@ -270,10 +270,9 @@ int sgn_j2k_plan_decode_stage(sgn_hip_session *session, sgn_j2k_plan *plan, int 
 
 /* ---- autotuning of the HT lane kernel ------------------------------------
  * No counterpart in the reference (its CPU decoder has no launch shapes):
- * the lane kernel comes in variants of work-group size, quad pairs decoded
- * between LDS refills, one-shot grid versus persistent waves pulling chunks
- * of 64, 128 or 256 code-blocks from a device work counter, and the
- * cooperative one-block-per-wave kernel. */
+ * the cleanup of a plan's code-blocks runs as three kernels (stuffing removal,
+ * the serial symbol chain with 64 or 32 lanes of a wave in use, magnitudes) or
+ * as the cooperative one-block-per-wave kernel. */
 int sgn_ht_lane_variant_count(void);
 const char *sgn_ht_lane_variant_name(int variant);
 int sgn_j2k_plan_set_lane_variant(sgn_j2k_plan *plan, int variant);

@@ -4,8 +4,8 @@
 //   passes (cleanup, SigProp, MagRef).  The symbol table, sigma map and the
 //   block itself live in LDS; lane 0 walks the serial bit streams, then the
 //   whole wave converts and stores the block with coalesced writes.  The
-//   cleanup-only blocks of at most 64x64 samples (every block of the lossless
-//   batches) take the lane kernel in ht_rows.hip instead.
+//   blocks of at most 64x64 samples (every block of the lossless batches) take
+//   the kernels in ht_split.hip instead.
 //
 // Restates crates/signinum-j2k-native/src/j2c/ht_block_decode.rs (decode_impl
 // :1563-1680 and the phases it calls) and produces coefficient_to_i32

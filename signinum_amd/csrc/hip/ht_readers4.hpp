@@ -9,8 +9,8 @@
 // in it, byte by byte otherwise; the delivered bit sequence is the same.
 //
 // Words come from a source object with `uint64_t word(uint32_t addr) const`
-// returning the aligned 8 bytes at byte address addr of the arena (an LDS
-// ring in the lane kernel).  The including file provides __device__ and
+// returning the aligned 8 bytes at byte address addr of the arena (staged in
+// LDS in the cooperative kernel).  The including file provides __device__ and
 // __forceinline__.
 #pragma once
 #include <stdint.h>

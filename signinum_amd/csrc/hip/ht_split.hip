@@ -1,0 +1,853 @@
+// HT cleanup decode in three kernels, each with the shape of its own work:
+//
+//   sgn_ht_clean    sixteen lanes per code-block: removes the bit stuffing of
+//                   the VLC stream, eight bytes a lane, into a plain bit string
+//                   in the block's workspace;
+//   sgn_ht_symbols  one block per lane (L of a wave's 64 lanes in use): the
+//                   serial MEL / VLC / UVLC chain, reading plain bits, writing
+//                   16 bits per quad into the workspace;
+//   sgn_ht_magsgn   sixteen lanes per block, a quad pair each: magnitudes and
+//                   signs of a quad row at once, each quad's place in the
+//                   MagSgn stream a prefix sum of the quads' bit counts.
+//
+// The steps are those of crates/signinum-j2k-native/src/j2c/ht_block_decode.rs
+// (decode_cleanup_symbols :1056-1204, decode_magnitude_sign_phase :1435-1560);
+// only the order in which independent work happens differs: the chain never
+// needs a magnitude (its contexts are significance bits alone), so all symbols
+// of a block come first.
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "../host/plan_types.h"
+#include "ht_common.hpp"
+#include "ht_readers4.hpp"
+#include "ht_refine.hpp"
+
+namespace sgn {
+
+constexpr int kSplitWaves = 4;  // waves per work-group of the three kernels
+
+// A block's part of its group's workspace.
+struct HtWork {
+    uint4 *head, *vlc, *mel, *sym;
+};
+__device__ __forceinline__ HtWork ht_work(uint4 *work, const HtGroup *groups, uint32_t i) {
+    const HtGroup g = groups[i / kHtGroup];
+    HtWork w;
+    w.head = work + g.base + i % kHtGroup;
+    w.vlc = w.head + kHtGroup;
+    w.mel = w.vlc + size_t(kHtGroup) * g.vlc_units;
+    w.sym = w.mel + kHtGroup * kHtMelUnits + i % kHtGroup;  // two units a block
+    return w;
+}
+
+// Header of a block's workspace.
+struct HtHead {
+    uint32_t vlc_last;  // last 16-byte unit of the VLC string (all zeros)
+    uint32_t scup;      // length of the MEL + VLC segment; 0: nothing to decode
+    uint32_t bad;       // malformed
+    uint32_t pad;
+};
+
+// Decode tables of the symbol kernel, fields where the chain uses them.
+// Context entries (index: 7 stream bits, then the context): bits 0-2 codeword
+// length, 8 u-offset, 9-11 the context that the quad gives its right neighbour
+// (first row: sigma_0 | sigma_1, sigma_2, sigma_3; other rows: bit 9 sigma_2 |
+// sigma_3, bits 10-11 come from the row above), 16-23 two bits per sample (0
+// insignificant, 1 significant, 2 exponent known to be 0, 3 to be 1), 30
+// sigma_3, 31 sigma_1.  u-offset entries (index: 6 stream bits, the quads'
+// u-offset flags): bits 0-4 prefix length plus 2, 5-9 suffix length, 10-14 the
+// first quad's part of it, 16-20 both lengths; then the same number of words
+// with the prefixes' values in bytes 1 and 3.
+struct HtSplitTables {
+    uint32_t first[1024], other[1024];
+    uint32_t ufirst[2 * 320], uother[2 * 256];
+};
+
+// From the tables of T.814 (length, u_off, rho, e_1, e_k; prefix and suffix).
+inline void ht_split_tables(const uint16_t *vlc0, const uint16_t *vlc1, const uint16_t *u0,
+                            const uint16_t *u1, HtSplitTables &T) {
+    auto entry = [](uint32_t t, bool first) {
+        uint32_t code = 0;
+        for (uint32_t s = 0; s < 4; ++s) {
+            const uint32_t sig = (t >> (4 + s)) & 1u, e1 = (t >> (8 + s)) & 1u,
+                           ek = (t >> (12 + s)) & 1u;
+            code |= (sig ? 1u + ek + (ek & e1) : 0u) << (2 * s);
+        }
+        const uint32_t r0 = (t >> 4) & 1u, r1 = (t >> 5) & 1u, r2 = (t >> 6) & 1u, r3 = (t >> 7) & 1u;
+        const uint32_t right = first ? (r0 | r1) | r2 << 1 | r3 << 2 : r2 | r3;
+        return (t & 7u) | ((t >> 3) & 1u) << 8 | right << 9 | code << 16 | r3 << 30 | r1 << 31;
+    };
+    for (uint32_t k = 0; k < 1024; ++k) {
+        T.first[k] = entry(vlc0[k], true);
+        // context bits: left, (sigma_3 of the quad above or sigma_1 of the one
+        // after it), (sigma_1 of the quad above or sigma_3 of the one before)
+        const uint32_t left = (k >> 7) & 1u, after = (k >> 8) & 1u, before = (k >> 9) & 1u;
+        T.other[k] = entry(vlc1[(k & 0x7Fu) | before << 7 | left << 8 | after << 9], false);
+    }
+    auto uentry = [](uint32_t e, uint32_t add, uint32_t &word, uint32_t &base) {
+        const uint32_t lp = e & 7u, ls = (e >> 3) & 0xFu, n0 = (e >> 7) & 7u;
+        word = (lp + 2) | ls << 5 | n0 << 10 | (lp + ls) << 16;
+        base = (((e >> 10) & 7u) + add) << 8 | ((e >> 13) + add) << 24;
+    };
+    for (uint32_t k = 0; k < 320; ++k) uentry(u0[k], 1, T.ufirst[k], T.ufirst[320 + k]);
+    for (uint32_t k = 0; k < 256; ++k) uentry(u1[k], 0, T.uother[k], T.uother[256 + k]);
+}
+
+// The clean and magnitude kernels give a block one DPP row (16 lanes), so that
+// neighbours, prefix sums and broadcasts inside a block are single VALU
+// operations that never cross into the next block.
+constexpr uint32_t kSplitLanes = 16;
+constexpr uint32_t kSplitBlocks = kSplitWaves * 64 / kSplitLanes;  // per work-group
+
+// Value of another lane of the row (CTRL), 0 past the row's ends.
+template <int CTRL>
+__device__ __forceinline__ uint32_t row_dpp(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+}
+
+// Inclusive prefix sum over each row.  Called by all lanes.
+__device__ __forceinline__ uint32_t row_scan(uint32_t v) {
+    v += row_dpp<0x111>(v);  // row_shr:1
+    v += row_dpp<0x112>(v);  // row_shr:2
+    v += row_dpp<0x114>(v);  // row_shr:4
+    v += row_dpp<0x118>(v);  // row_shr:8
+    return v;
+}
+
+// The value that the row's last lane holds (row_newbcast:15).
+__device__ __forceinline__ uint32_t row_last(uint32_t v) { return row_dpp<0x15F>(v); }
+
+// Orders the LDS accesses of one wave for the compiler; the LDS unit executes
+// a wave's instructions in order, so nothing is waited for.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// ---- stuffing removal ------------------------------------------------------
+
+constexpr uint32_t kCleanRing = 64;  // dwords of a block's ring: a partly filled unit and a round's 33
+
+// The VLC string of one block per row: two zero bits, the 3 or 4 bits of the
+// segment's second last byte, and from there it runs backward from the byte before; a byte
+// whose low 7 bits are ones after a byte > 0x8F carries 7 bits, and is ORed in
+// whole, as the byte-wise reader does (ht_block_decode.rs:931-999); zeros
+// follow it.  Two dependent trips to memory per block bound it (the first
+// bytes are asked for beside the length field); a round takes 128 bytes, eight
+// a lane, through a ring of words in LDS that whole 16-byte units leave.
+__global__ void __launch_bounds__(kSplitWaves * 64)
+sgn_ht_clean(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restrict__ arena,
+             const HtGroup *__restrict__ groups, uint4 *__restrict__ work) {
+    __shared__ __attribute__((aligned(16))) uint32_t s_buf[kSplitBlocks][kCleanRing];
+    const uint32_t row = threadIdx.x / kSplitLanes, q = threadIdx.x % kSplitLanes;
+    uint32_t *buf = s_buf[row];
+    const uint32_t i = blockIdx.x * kSplitBlocks + row;
+    const bool valid = i < n;
+    CbJob j{};
+    if (valid) j = jobs[i];
+    const bool coded = valid && !(j.flags & kCbZero) && j.lcup >= 2;
+    const uint32_t lcup = coded ? j.lcup : 0, seg1 = j.src + lcup;
+    // the four bytes e - 3 .. e (e: arena address), the last in the top byte
+    auto load4 = [&](uint32_t e) -> uint32_t {
+        uint32_t x;
+        if (e >= 3) {
+            __builtin_memcpy(&x, arena + e - 3, 4);
+            return x;
+        }
+        __builtin_memcpy(&x, arena, 4);
+        return x << (8 * (3 - e));
+    };
+    // this lane's eight bytes of a round, k0 bytes into the stream
+    uint32_t hi = 0, lo = 0;
+    auto fetch = [&](uint32_t k0, uint32_t len) {
+        hi = lo = 0;
+        if (k0 < len) hi = load4(seg1 - 3 - k0);
+        if (k0 + 4 < len) lo = load4(seg1 - 3 - k0 - 4);
+    };
+    uint32_t b0 = 0, top = 0;
+    if (coded) {
+        b0 = arena[seg1 - 2];
+        top = arena[seg1 - 1];
+    }
+    // (bytes past a shorter segment are dropped below)
+    fetch(8 * q, lcup > 2 ? lcup - 2 : 0);
+    uint32_t scup = (top << 4) + (b0 & 0x0F);
+    uint32_t bad = 0;
+    if (valid && !(j.flags & kCbZero))
+        bad = lcup < 2 || j.zblk >= 30 || scup < 2 || scup > lcup || scup > 4079;
+    if (!coded || bad) scup = 0;
+    const HtWork w = ht_work(work, groups, valid ? i : 0);
+    // the first MEL bytes, as they are
+    if (q < kHtMelUnits && scup > 16 * q) {
+        uint4 v;
+        __builtin_memcpy(&v, arena + (seg1 - scup) + 16 * q, 16);
+        w.mel[kHtGroup * q] = v;
+    }
+    const uint32_t len = scup ? scup - 2 : 0;
+    const uint32_t units = (6 + 8 * len + 127) >> 7;  // 16-byte units that hold stream bits
+    const uint32_t first = b0 >> 4;
+    uint32_t fill = 6u - ((first & 7u) == 7u ? 1u : 0u);  // two bits in front
+    uint32_t carry = b0 | 0x0Fu;  // the byte before this round's
+    if (q < 4) buf[q] = q == 0 ? first << 2 : 0u;
+    uint4 *d = w.vlc;
+    uint32_t done = 0;  // units written
+
+    // one dword of stream bytes (the first in bits 0..7), `g`: bit 7 of a byte
+    // set where it is above 0x8F, `pg`: the same of the dword before
+    auto pack = [](uint32_t d, uint32_t g, uint32_t pg, uint32_t &bits) -> uint32_t {
+        const uint32_t f = ((d & 0x7F7F7F7Fu) + 0x01010101u) & __builtin_amdgcn_alignbit(g, pg, 24) &
+                           0x80808080u;
+        const uint32_t o1 = 8u - ((f >> 7) & 1u), o2 = o1 + 8u - ((f >> 15) & 1u),
+                       o3 = o2 + 8u - ((f >> 23) & 1u);
+        bits = o3 + 8u - (f >> 31);
+        return (d & 0xFFu) | (((d >> 8) & 0xFFu) << o1) | (((d >> 16) & 0xFFu) << o2) |
+               ((d >> 24) << o3);
+    };
+    auto above = [](uint32_t d) {  // bit 7 of every byte above 0x8F
+        return ((d & 0x7F7F7F7Fu) + 0x70707070u) & d & 0x80808080u;
+    };
+    for (uint32_t at = 0; __any(at < len); at += 128) {
+        const uint32_t k0 = at + 8 * q;
+        uint32_t d0 = __builtin_bswap32(hi), d1 = __builtin_bswap32(lo);
+        if (k0 + 4 > len) d0 &= k0 < len ? 0xFFFFFFFFu >> (8 * (4 - (len - k0))) : 0u;
+        if (k0 + 8 > len) d1 &= k0 + 4 < len ? 0xFFFFFFFFu >> (8 * (8 - (len - k0))) : 0u;
+        fetch(k0 + 128, len);
+        const uint32_t g0 = above(d0), g1 = above(d1);
+        uint32_t pg = row_dpp<0x111>(g1);
+        if (q == 0) pg = carry > 0x8Fu ? 0x80000000u : 0u;
+        carry = row_last(d1 >> 24);
+        uint32_t n0, n1;
+        const uint32_t v0 = pack(d0, g0, pg, n0), v1 = pack(d1, g1, g0, n1);
+        const uint32_t incl = row_scan(n0 + n1), tot = row_last(incl);
+        if (at < len) {
+            const uint32_t z = (fill >> 5) + 1 + q;
+            buf[z & (kCleanRing - 1)] = 0;
+            buf[(z + 16) & (kCleanRing - 1)] = 0;
+        }
+        wave_lds_fence();
+        if (at < len) {
+            // the lane's 50 to 64 bits: three words at most
+            const uint64_t v = (uint64_t)v0 | ((uint64_t)v1 << n0);
+            const uint32_t pos = fill + incl - (n0 + n1), wi = pos >> 5, sh = pos & 31u;
+            const uint64_t a = v << sh;
+            const uint32_t x2 = sh ? (uint32_t)(v >> 32) >> (32u - sh) : 0u;
+            if ((uint32_t)a) atomicOr(&buf[wi & (kCleanRing - 1)], (uint32_t)a);
+            if ((uint32_t)(a >> 32))
+                atomicOr(&buf[(wi + 1) & (kCleanRing - 1)], (uint32_t)(a >> 32));
+            if (x2) atomicOr(&buf[(wi + 2) & (kCleanRing - 1)], x2);
+            fill += tot;
+        }
+        wave_lds_fence();
+        // whole units (at most 9 a round; the padding of the last round's
+        // bytes may reach past the string's last unit)
+        const uint32_t full = min(fill >> 7, units), u = done + q;
+        if (at < len && u < full) d[kHtGroup * u] = *reinterpret_cast<uint4 *>(&buf[4 * u & (kCleanRing - 1)]);
+        done = at < len ? full : done;
+    }
+    if (scup) {
+        // the partly filled unit, then zeros (seven-bit bytes leave the string
+        // short of `units`)
+        const uint32_t last = fill >> 5;
+        for (uint32_t u = done + q; u <= units; u += kSplitLanes) {
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (u < units) {
+                const uint32_t *x = &buf[4 * u & (kCleanRing - 1)];
+                v.x = 4 * u <= last ? x[0] : 0u;
+                v.y = 4 * u + 1 <= last ? x[1] : 0u;
+                v.z = 4 * u + 2 <= last ? x[2] : 0u;
+                v.w = 4 * u + 3 <= last ? x[3] : 0u;
+            }
+            d[kHtGroup * u] = v;
+        }
+    }
+    if (valid && q == 0) *reinterpret_cast<HtHead *>(w.head) = HtHead{units, scup, bad, 0};
+}
+
+// ---- MEL / VLC / UVLC chain --------------------------------------------------
+
+// MEL events as a bit queue: bit n is the outcome of the n-th quad (or, in the
+// first row, u-offset pair) from here that asks the MEL decoder.  A run symbol
+// (ht_block_decode.rs:860-929) adds its zeros and, if the run ended early, a
+// one; so the chain takes one bit per question instead of counting runs down.
+struct MelQueue {
+    uint64_t buf;   // undecoded MEL bits, next in bit 63
+    uint64_t ev;    // events, next in bit 0
+    uint32_t bits;  // valid bits of buf
+    uint32_t n;     // valid events
+    uint32_t k;     // run-length state, 0..12
+    uint32_t next;  // four stream bytes, loaded ahead
+    int32_t left;   // stream bytes from `next` on
+    uint32_t at;    // their arena address
+    uint32_t idx;   // their dword index in the string
+    uint32_t ff;    // the byte before them was 0xFF
+    const uint4 *copy;  // the string's first units in the workspace
+};
+
+// The four bytes at `at` (from the workspace as far as its copy goes).
+__device__ __forceinline__ void mel_queue_load(MelQueue &m, const uint8_t *arena) {
+    const uint8_t *p = m.idx < 4 * kHtMelUnits
+                           ? reinterpret_cast<const uint8_t *>(m.copy + kHtGroup * (m.idx >> 2)) +
+                                 4 * (m.idx & 3u)
+                           : arena + m.at;
+    __builtin_memcpy(&m.next, p, 4);
+}
+
+// Appends the four bytes loaded ahead (MSB-first, 7 bits after 0xFF, the
+// segment's last byte ORed with 0x0F, 0xFF past it) and asks for the next
+// (past the segment for bytes inside it, which are not used).
+__device__ __forceinline__ void mel_queue_bytes(MelQueue &m, const uint8_t *arena) {
+    uint32_t w = m.next;
+    if (m.left <= 4) {
+        if (m.left > 0) w |= 0x0Fu << (8 * (m.left - 1));
+        if (m.left < 4) w |= 0xFFFFFFFFu << (8 * max(m.left, 0));
+    }
+    m.left -= 4;
+    m.at += m.left > 0 ? 4u : 0u;
+    m.idx += m.left > 0 ? 1u : 0u;
+    mel_queue_load(m, arena);
+    uint32_t v = 0, n = 0;
+#pragma unroll
+    for (uint32_t t = 0; t < 4; ++t) {
+        const uint32_t b = (w >> (8 * t)) & 0xFFu;
+        const uint32_t nb = 8u - m.ff;
+        v = (v << nb) | (b & (0xFFu >> m.ff));
+        n += nb;
+        m.ff = b == 0xFFu ? 1u : 0u;
+    }
+    m.buf |= (uint64_t)v << (64u - m.bits - n);
+    m.bits += n;
+}
+
+// Decodes run symbols until every lane of the wave that is `on` holds `need`
+// (at most 32) events; lanes with room and bits join in.  Sixteen events take
+// 41 bits at most when they start from the longest runs, so the buffer (over 32
+// bits at a segment's start) hardly ever has to wait for its next bytes here.
+__device__ __forceinline__ void mel_queue_fill(MelQueue &m, uint32_t need, bool on,
+                                               const uint8_t *arena) {
+    // E for k = 0..12, four bits each
+    constexpr uint64_t kExp = 0x5433222111000ull;
+    while (__any(on && m.n < need)) {
+        if (on && (m.n < need || (m.n < 32u && m.bits >= 6u))) {
+            if (m.bits < 6u) mel_queue_bytes(m, arena);
+            const uint32_t e = (uint32_t)(kExp >> (4u * m.k)) & 0xFu;
+            const uint32_t hi = (uint32_t)(m.buf >> 32), one = hi >> 31;
+            // run length bits of an early end (none for E = 0)
+            const uint32_t v = __builtin_amdgcn_ubfe(hi, 31u - e, e);
+            const uint32_t used = one ? 1u : 1u + e;
+            m.buf <<= used;
+            m.bits -= used;
+            m.k = one ? min(m.k + 1u, 12u) : max(m.k, 1u) - 1u;
+            m.n += one ? 1u << e : v + 1u;
+            m.ev |= (uint64_t)(one ^ 1u) << (m.n - 1u);
+        }
+    }
+}
+
+// Symbols of the blocks jobs[0 .. n): lane l < L of wave k takes block k * L +
+// l.  Fewer lanes a wave spread few blocks over more waves (every SIMD gets
+// some).  The VLC string is staged through a ring of four 16-byte units per
+// lane in LDS, two units loaded ahead in registers, so that no read of the
+// chain waits for memory.  Everything else of a lane's state is in
+// registers: the significance that contexts need is two bits per quad of the
+// row above, as one bit string with the left neighbours' bits beside it.
+//
+// The chain is bound by latency when waves are few (four dependent LDS reads a
+// pair: the stream window, two context tables, the u-offset table) and by VALU
+// issue when they are many, so a pair is straight-line code of few operations:
+// the tables (HtSplitTables) hold every field where it is used, a quad past the
+// block's edge is a quad whose table entry is masked to zero, and the MEL
+// question is arithmetic on 0/1 words.
+//
+// TIMED (the decode-cost model's samples, with L = 1): each wave records the
+// shader-clock cycles of its block's chain.
+template <int L, bool TIMED = false>
+__global__ void __launch_bounds__(kSplitWaves * 64)
+sgn_ht_symbols(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restrict__ arena,
+               const HtGroup *__restrict__ groups, uint4 *__restrict__ work,
+               const HtSplitTables *__restrict__ tables, uint64_t *__restrict__ cycles) {
+    __shared__ __attribute__((aligned(16))) HtSplitTables s_t;
+    // the ring's 16 dwords, and the first again: two adjacent ones can be read
+    // from any place
+    __shared__ uint32_t s_ring[kSplitWaves][17][L];
+    for (uint32_t t = threadIdx.x; t < sizeof(HtSplitTables) / 16; t += kSplitWaves * 64)
+        reinterpret_cast<uint4 *>(&s_t)[t] = reinterpret_cast<const uint4 *>(tables)[t];
+    __syncthreads();
+    const uint64_t began = TIMED ? clock64() : 0;
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const uint32_t i = (blockIdx.x * kSplitWaves + wv) * L + lane;
+    const bool valid = lane < (uint32_t)L && i < n;
+    uint32_t(*ring)[L] = s_ring[wv];
+    const uint32_t rl = lane < (uint32_t)L ? lane : 0u;  // idle lanes read, never write
+
+    uint32_t width = 0, height = 0;
+    const HtWork w = ht_work(work, groups, valid ? i : 0);
+    HtHead hd{0, 0, 0, 0};
+    uint32_t seg1 = 0;
+    if (valid) {
+        const CbJob j = jobs[i];
+        width = j.w;
+        height = j.h;
+        seg1 = j.src + j.lcup;
+        if (!(j.flags & kCbZero)) hd = *reinterpret_cast<const HtHead *>(w.head);
+    }
+    const bool on = hd.scup != 0;
+    const uint32_t nq = (width + 1) >> 1, npairs = (width + 3) >> 2;
+    const uint32_t nrows = on ? (height + 1) >> 1 : 0, nseg = (npairs + 7) >> 3;
+    auto vlc = [&](uint32_t u) -> uint4 { return w.vlc[kHtGroup * min(u, hd.vlc_last)]; };
+    uint4 *sym = w.sym;
+
+    MelQueue mel{0, 0, 0, 0, 0, 0, (int32_t)hd.scup - 1, seg1 - hd.scup, 0, 0, w.mel};
+    uint4 pend0 = make_uint4(0, 0, 0, 0), pend1 = pend0;
+    uint32_t res = 4;  // unit that pend0 holds (pend1 the next): those below are or were in the ring
+    auto put = [&](uint32_t unit, const uint4 &v) {
+        const uint32_t s = (unit & 3u) * 4u;
+        ring[s + 0][rl] = v.x;
+        ring[s + 1][rl] = v.y;
+        ring[s + 2][rl] = v.z;
+        ring[s + 3][rl] = v.w;
+        ring[s ? s : 16u][rl] = v.x;
+    };
+    if (on) {
+        mel_queue_load(mel, arena);
+        uint4 u[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) u[k] = vlc(k);
+        pend0 = vlc(4);
+        pend1 = vlc(5);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) put(k, u[k]);
+        mel_queue_bytes(mel, arena);
+    }
+    // next bit of the VLC string less two (the string starts at bit 2): the
+    // window's next bit is bit 2, a table's byte offset
+    uint32_t pos = 0;
+    uint32_t x0 = 0, x1 = 0;    // contexts from the row above, two bits per quad, first quad on top
+    uint32_t sig0 = 0;          // this row's sigma_1, sigma_3 bits of its first 16 quads
+    uint32_t t1 = 0;            // table entry of the quad to the left
+    uint32_t row = 0, seg = 0;
+
+    const uint8_t *ctx0 = reinterpret_cast<const uint8_t *>(s_t.first);
+    const uint8_t *ctx1 = reinterpret_cast<const uint8_t *>(s_t.other);
+
+    while (__any(row < nrows)) {
+        const bool run = row < nrows;
+        const bool first = row == 0;
+        // events of up to 16 quads and, in the first row, 8 u-offset pairs
+        mel_queue_fill(mel, first ? 24u : 16u, run, arena);
+        const uint32_t ev = (uint32_t)mel.ev;
+        uint32_t used = 0, acc = 0;
+        uint32_t out[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        const uint32_t pa = 8 * seg;
+        const uint32_t pairs = run ? npairs - pa : 0;           // from here to the row's end
+        const uint32_t quads = run ? min(nq - 2 * pa, 16u) : 0;
+        const uint32_t exist = (1u << quads) - 1u;              // bit per quad
+        // one pair: FIRST rows take contexts from the left alone and may ask
+        // MEL for the u-offsets; later rows add the row above
+        uint32_t x = (seg ? x1 : x0) | (quads < 16u ? 0xFFFFFFFFu >> (2u * quads) : 0u);
+        auto pair = [&](auto is_first, uint32_t p) {
+            constexpr bool kFirst = decltype(is_first)::value;
+            const uint32_t k = (pos >> 5) & 15u;
+            uint32_t win = __builtin_amdgcn_alignbit(ring[k + 1][rl], ring[k][rl], pos & 31u);
+            uint32_t t0, len = 0;
+#pragma unroll
+            for (uint32_t q = 2 * p; q < 2 * p + 2; ++q) {
+                // context: table offset bits 9-11
+                uint32_t c;
+                if constexpr (kFirst) {
+                    c = t1 & 0xE00u;
+                } else {
+                    const uint32_t above = q < 10 ? x >> (20 - 2 * q) : x << (2 * q - 20);
+                    c = (above & 0xC00u) | (t1 & 0x200u);
+                }
+                uint32_t t = *reinterpret_cast<const uint32_t *>((kFirst ? ctx0 : ctx1) +
+                                                                 ((win & 0x1FCu) | c));
+                // a quad without context asks MEL; its 0 makes the entry 0
+                uint32_t ask = (c - 1u) >> 31;
+                if constexpr (kFirst) ask &= exist >> q;
+                const uint32_t drop = ask & ~(ev >> used);
+                used += ask;
+                t &= (drop - 1u) & (uint32_t)__builtin_amdgcn_sbfe((int)exist, q, 1);
+                win >>= t & 7u;
+                len += t & 7u;
+                acc = __builtin_amdgcn_alignbit(acc, t, 30);
+                if (q & 1)
+                    t1 = t;
+                else
+                    t0 = t1 = t;
+            }
+            uint32_t mode = (t0 & 0x100u) | ((t1 & 0x100u) << 1);
+            if constexpr (kFirst) {
+                const uint32_t both = (mode >> 8) & (mode >> 9);
+                mode += ((ev >> used) & both) << 8;
+                used += both;
+            }
+            const uint32_t *ut = (kFirst ? s_t.ufirst : s_t.uother) + (((win & 0xFCu) | mode) >> 2);
+            const uint32_t e = ut[0], base = ut[kFirst ? 320 : 256];
+            const uint32_t sfx = __builtin_amdgcn_ubfe(win, e & 31u, (e >> 5) & 31u);
+            const uint32_t n0 = (e >> 10) & 31u;
+            const uint32_t low = __builtin_amdgcn_ubfe(sfx, 0, n0), high = sfx >> n0;
+            out[p] = ((t0 >> 16) & 0xFFu) | (t1 & 0xFF0000u) | (base + (low << 8) + (high << 24));
+            pos += len + (e >> 16);
+        };
+        if (__any(run && first)) {
+            // the wave's other lanes (blocks of other heights start their rows
+            // together, so there are none but idle ones) sit this out
+            if (first) {
+#pragma unroll
+                for (uint32_t p = 0; p < 8; ++p) {
+                    if (p < pairs) pair(std::true_type{}, p);
+                    else acc <<= 4;
+                }
+            }
+        }
+        if (run && !first) {
+#pragma unroll
+            for (uint32_t p = 0; p < 8; ++p) {
+                if (p && p % 2 == 0 && !__any(p < pairs)) {
+                    acc <<= 4 * (8 - p);
+                    break;
+                }
+                pair(std::false_type{}, p);
+            }
+        }
+        mel.ev >>= used;
+        mel.n -= used;
+        // What was loaded a segment ago goes into the ring (eight pairs take at
+        // most 240 bits: two units fill it again) and the MEL buffer, and the
+        // next loads go out; all before this segment's stores, whose
+        // completion the next wait for a load would include.
+        if (run && res < (pos >> 7) + 4u) {
+            put(res, pend0);
+            ++res;
+            if (res < (pos >> 7) + 4u) {
+                put(res, pend1);
+                ++res;
+            }
+            pend0 = vlc(res);
+            pend1 = vlc(res + 1);
+        }
+        if (run && mel.bits <= 32u) mel_queue_bytes(mel, arena);
+        if (run) {
+            sym[0] = make_uint4(out[0], out[1], out[2], out[3]);
+            sym[1] = make_uint4(out[4], out[5], out[6], out[7]);
+            sym += 2 * kHtGroup;
+        }
+        if (seg + 1 < nseg) {
+            sig0 = acc;
+            ++seg;
+        } else {
+            // contexts of the next row: sigma_1 of the quad or sigma_3 of the
+            // one before, sigma_3 of the quad or sigma_1 of the one after; in
+            // the bit string s1 s3 s1 s3 ... each bit joins its neighbour on
+            // the other quad's side
+            const uint32_t lo = seg ? sig0 : acc, hi = seg ? acc : 0u;
+            x0 = lo | ((lo >> 1) & 0xAAAAAAAAu) |
+                 (__builtin_amdgcn_alignbit(lo, hi, 31) & 0x55555555u);
+            x1 = hi | (__builtin_amdgcn_alignbit(lo, hi, 1) & 0xAAAAAAAAu) |
+                 ((hi << 1) & 0x55555555u);
+            t1 = 0;
+            seg = 0;
+            ++row;
+        }
+    }
+    if constexpr (TIMED) {
+        if (valid && lane == 0) cycles[i] = clock64() - began;
+    }
+}
+
+// ---- magnitudes and signs ------------------------------------------------------
+
+constexpr uint32_t kMagRing = 256;  // dwords of a block's unstuffed MagSgn ring (a power of two)
+
+using s16x2 = int16_t __attribute__((ext_vector_type(2)));
+
+// One block per DPP row, a quad pair (eight samples) per lane.  A quad row
+// takes at most 32 quads * 4 samples * 31 bits = 496 bytes of the 1024-byte
+// ring, which is topped up 128 bytes at a time, eight bytes a lane, from words
+// loaded a round ahead.  Sample rows leave as whole 128-byte (int16) lines.
+// Bound by VALU issue.
+template <typename C>
+__global__ void __launch_bounds__(kSplitWaves * 64)
+sgn_ht_magsgn(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restrict__ arena,
+              C *__restrict__ coef, const HtGroup *__restrict__ groups, uint4 *__restrict__ work,
+              uint8_t *__restrict__ status) {
+    // one dword more than the ring: a copy of the first, so that two adjacent
+    // dwords can be read at any place
+    __shared__ uint32_t s_ring[kSplitBlocks][kMagRing + 1];
+    // per symbol code: byte s of .x is 0xFF where sample s is significant, of
+    // .y 1 where its exponent is known, of .z that exponent bit
+    __shared__ uint4 s_code[256];
+    {
+        const uint32_t t = threadIdx.x;
+        uint32_t sig = 0, known = 0, bit = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t c = (t >> (2 * k)) & 3u;
+            sig |= (c ? 0xFFu : 0u) << (8 * k);
+            known |= (c >> 1) << (8 * k);
+            bit |= (c == 3 ? 1u : 0u) << (8 * k);
+        }
+        s_code[t] = make_uint4(sig, known, bit, 0);
+    }
+    __syncthreads();
+    const uint32_t row = threadIdx.x / kSplitLanes, q = threadIdx.x % kSplitLanes;
+    uint32_t *ring = s_ring[row];
+    const uint32_t i = blockIdx.x * kSplitBlocks + row;
+    const bool valid = i < n;
+    CbJob j{};
+    if (valid) j = jobs[i];
+    const uint32_t w = j.w, h = j.h, stride = j.stride;
+    HtHead hd{0, 0, 0, 0};
+    const HtWork ws = ht_work(work, groups, valid ? i : 0);
+    if (valid && !(j.flags & kCbZero)) hd = *reinterpret_cast<const HtHead *>(ws.head);
+    const bool on = hd.scup != 0;
+    const uint32_t nrows = (h + 1) >> 1;
+    // pair q of a row: dword q % 8 of the row's chunk q / 8
+    const uint32_t *sym = reinterpret_cast<const uint32_t *>(ws.sym) +
+                          (q >> 3) * (8 * kHtGroup) + (q & 7u);
+    const uint32_t spitch = ((w + 31) >> 5) * (8 * kHtGroup);  // dwords per symbol row
+    // columns of this lane (4 q .. 4 q + 3) inside the block
+    const uint32_t cols = 4 * q < w ? min(w - 4 * q, 4u) : 0u;
+    // the samples of its two quads, two bits each
+    const uint32_t mask = !on || !cols ? 0u
+                          : cols >= 4  ? 0xFFFFu
+                          : cols == 3  ? 0x0FFFu
+                          : cols == 2  ? 0x00FFu
+                                       : 0x000Fu;
+    const uint32_t p = 30 - j.zblk, mmsbp2 = j.zblk + 2u;
+    const uint32_t shift = j.kmax >= 31 ? 0u : 31u - j.kmax;
+    const bool vec = ((j.dst | stride) & 3u) == 0 && cols == 4;
+    C *out = coef + j.dst + 4 * q;
+
+    // MagSgn bytes [next, end): forward, a byte after 0xFF carries 7 bits and
+    // is ORed in whole, 0xFF past the end (ht_block_decode.rs:881-929).  `raw`
+    // holds the eight bytes at `next`, whatever lies there.
+    const uint32_t end = on ? j.src + j.lcup - hd.scup : 0;
+    uint32_t next = (on ? j.src : 0) + 8 * q;
+    uint2 raw = make_uint2(0, 0);
+    if (next < end) __builtin_memcpy(&raw, arena + next, 8);
+    uint32_t fill = 0, prev = 0, pos = 0;
+    if (q == 0) ring[0] = ring[kMagRing] = 0;
+    uint32_t bad = hd.bad;
+    uint32_t e1 = 0, e3 = 0, e5 = 0, e7 = 0;  // exponents of the bottom samples of the row above
+    uint32_t s_next = mask && nrows ? *sym : 0u;
+    uint32_t rows_max = (uint32_t)__builtin_amdgcn_readlane((int)nrows, 0);
+#pragma unroll
+    for (int k = 16; k < 64; k += 16)
+        rows_max = max(rows_max, (uint32_t)__builtin_amdgcn_readlane((int)nrows, k));
+    for (uint32_t r = 0; r < rows_max; ++r) {
+        const bool live = r < nrows;
+        const uint32_t s = s_next;
+        if (mask && r + 1 < nrows) s_next = *(sym += spitch);
+        uint32_t uq0 = (s >> 8) & 0xFFu, uq1 = s >> 24;
+        if (r) {
+            // exponent bound of the row above, over the quad and the samples
+            // beside it, for quads with more than one significant sample
+            const uint32_t l = row_dpp<0x111>(e7), t = row_dpp<0x101>(e1);
+            const uint32_t mid = max(e3, e5);
+            const uint32_t m0 = max(max(max(e1, mid), l), 1u), m1 = max(max(max(e7, mid), t), 1u);
+            const uint32_t nz = (s | (s >> 1)) & 0x00550055u;
+            const uint32_t z0 = nz & 0xFFu, z1 = nz >> 16;
+            uq0 += (z0 & (z0 - 1u)) ? m0 : 1u;
+            uq1 += (z1 & (z1 - 1u)) ? m1 : 1u;
+        }
+        const bool over = live && ((mask && uq0 > mmsbp2) || ((mask >> 8) && uq1 > mmsbp2));
+        const uint64_t ov = __ballot(over) >> (threadIdx.x & 48u);
+        if ((uint32_t)ov & 0xFFFFu) bad = 1;
+        const uint32_t code0 = live && !bad ? s & mask & 0xFFu : 0u;
+        const uint32_t code1 = live && !bad ? (s >> 16) & (mask >> 8) : 0u;
+        // bits per sample, a byte each: U_q, one less where the exponent is known
+        const uint4 g0 = s_code[code0], g1 = s_code[code1];
+        const uint32_t b0 = (g0.x & (uq0 * 0x01010101u)) - g0.y;
+        const uint32_t b1 = (g1.x & (uq1 * 0x01010101u)) - g1.y;
+        // running sums, a byte each (at most 124)
+        uint32_t a0 = b0 + (b0 << 8), a1 = b1 + (b1 << 8);
+        a0 += a0 << 16;
+        a1 += a1 << 16;
+        const uint32_t t0 = a0 >> 24, tot = t0 + (a1 >> 24);
+        const uint32_t incl = row_scan(tot);
+        const uint32_t at = pos + incl - tot;
+        pos += row_last(incl);
+        // every bit this row reads, and the sign bit that a sample without
+        // magnitude bits takes from the position after the last one
+        const uint32_t need = on ? pos + 1 : 0;
+        if (__any(fill < need)) {
+            do {
+                const bool act = fill < need;
+                uint32_t d0 = raw.x, d1 = raw.y;
+                const int32_t over8 = (int32_t)(next + 8 - end);  // bytes past the end
+                if (over8 > 0) {
+                    d1 |= over8 >= 4 ? 0xFFFFFFFFu : 0xFFFFFFFFu << (32 - 8 * over8);
+                    if (over8 > 4) d0 |= over8 >= 8 ? 0xFFFFFFFFu : 0xFFFFFFFFu << (64 - 8 * over8);
+                }
+                if (act) {
+                    next += 128;
+                    if (next < end) __builtin_memcpy(&raw, arena + next, 8);
+                }
+                // bit 7 of every byte that is 0xFF, and of every byte after one
+                auto ff = [](uint32_t d) {
+                    return ((d & 0x7F7F7F7Fu) + 0x01010101u) & d & 0x80808080u;
+                };
+                const uint32_t f0 = ff(d0), f1 = ff(d1);
+                uint32_t pf = row_dpp<0x111>(f1);
+                if (q == 0) pf = prev;
+                const uint32_t s0 = __builtin_amdgcn_alignbit(f0, pf, 24) >> 7,
+                               s1 = __builtin_amdgcn_alignbit(f1, f0, 24) >> 7;
+                // the bytes of a dword moved down by the seven-bit bytes
+                // before them (running counts, a byte each)
+                auto pack = [](uint32_t d, uint32_t s, uint32_t &bits) {
+                    uint32_t c = s + (s << 8);
+                    c += c << 16;
+                    bits = 32u - (c >> 24);
+                    return (d & 0xFFu) | ((d & 0xFF00u) >> (c & 31u)) |
+                           ((d & 0xFF0000u) >> ((c >> 8) & 31u)) |
+                           ((d & 0xFF000000u) >> ((c >> 16) & 31u));
+                };
+                uint32_t n0, n1;
+                const uint32_t v0 = pack(d0, s0, n0), v1 = pack(d1, s1, n1);
+                const uint32_t sc = row_scan(n0 + n1), bits = row_last(sc), last = row_last(f1);
+                const uint32_t wz = (fill >> 5) + 1 + q;
+                if (act) {
+                    // the words past the partly filled one that this round reaches
+                    ring[wz & (kMagRing - 1)] = 0;
+                    ring[(wz + 16) & (kMagRing - 1)] = 0;
+                }
+                wave_lds_fence();
+                if (act) {
+                    const uint32_t b = fill + sc - (n0 + n1), sh = b & 31u, wa = b >> 5;
+                    const uint64_t v = (uint64_t)v0 | ((uint64_t)v1 << n0);
+                    const uint64_t x = v << sh;
+                    const uint32_t y = (uint32_t)(v >> 32) >> 1 >> (31u - sh);
+                    atomicOr(&ring[wa & (kMagRing - 1)], (uint32_t)x);
+                    atomicOr(&ring[(wa + 1) & (kMagRing - 1)], (uint32_t)(x >> 32));
+                    atomicOr(&ring[(wa + 2) & (kMagRing - 1)], y);
+                    fill += bits;
+                    prev = last;
+                }
+                wave_lds_fence();
+            } while (__any(fill < need));
+            ring[kMagRing] = ring[0];
+            wave_lds_fence();
+        }
+        // stream bits at the row's position plus off
+        auto window = [&](uint32_t off) -> uint32_t {
+            const uint32_t b = at + off, wi = (b >> 5) & (kMagRing - 1);
+            return __builtin_amdgcn_alignbit(ring[wi + 1], ring[wi], b & 31u);
+        };
+        auto offset = [&](uint32_t k) -> uint32_t {  // of sample k in the lane's bits
+            return k == 0   ? 0u
+                   : k < 4  ? (a0 >> (8 * (k - 1))) & 0xFFu
+                   : k == 4 ? t0
+                            : t0 + ((a1 >> (8 * (k - 5))) & 0xFFu);
+        };
+        uint32_t bits[8];
+        if constexpr (sizeof(C) == 2) {
+            // K <= 15: U_q is at most 17, two samples come from one window
+#pragma unroll
+            for (uint32_t k = 0; k < 8; k += 2) {
+                bits[k] = window(offset(k));
+                bits[k + 1] = bits[k] >> (((k < 4 ? b0 : b1) >> (8 * (k & 3u))) & 31u);
+            }
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) bits[k] = window(offset(k));
+        }
+        uint32_t vn[8], mag[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) {
+            const uint32_t m = ((k < 4 ? b0 : b1) >> (8 * (k & 3u))) & 31u;
+            const uint32_t e = ((k < 4 ? g0.z : g1.z) >> (8 * (k & 3u))) & 0xFFu;
+            // an insignificant sample has no bits: v is 1, its exponent 0
+            vn[k] = __builtin_amdgcn_ubfe(bits[k], 0, m) | (e << m) | 1u;
+            mag[k] = __builtin_amdgcn_ubfe((vn[k] + 2) << (p - 1), shift, 31u - shift);
+        }
+        e1 = 31u - __builtin_clz(vn[1]);
+        e3 = 31u - __builtin_clz(vn[3]);
+        e5 = 31u - __builtin_clz(vn[5]);
+        e7 = 31u - __builtin_clz(vn[7]);
+        // rows y and y + 1: signs applied, insignificant samples 0
+        uint32_t o0[sizeof(C)], o1[sizeof(C)];
+        if constexpr (sizeof(C) == 2) {
+            // two samples a dword
+            auto pair = [&](uint32_t k, uint32_t sig) -> uint32_t {
+                const s16x2 m = __builtin_bit_cast(s16x2, mag[k] | (mag[k + 2] << 16));
+                const s16x2 neg = __builtin_bit_cast(
+                    s16x2, __builtin_amdgcn_perm(bits[k + 2], bits[k], 0x05040100u) & 0x00010001u);
+                const s16x2 x = (m ^ -neg) + neg;
+                return __builtin_bit_cast(uint32_t, x) &
+                       __builtin_amdgcn_perm(0u, sig, k & 1u ? 0x03030101u : 0x02020000u);
+            };
+            o0[0] = pair(0, g0.x);
+            o0[1] = pair(4, g1.x);
+            o1[0] = pair(1, g0.x);
+            o1[1] = pair(5, g1.x);
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) {
+                const uint32_t sgn = (uint32_t)((int32_t)(bits[k] << 31) >> 31);
+                const uint32_t sig =
+                    (uint32_t)((int32_t)((k < 4 ? g0.x : g1.x) << (31 - 8 * (k & 3u))) >> 31);
+                (k & 1u ? o1 : o0)[k >> 1] = ((mag[k] ^ sgn) - sgn) & sig;
+            }
+        }
+        if (live && cols) {
+            const bool second = 2 * r + 1 < h;
+            if (vec) {
+                if constexpr (sizeof(C) == 2) {
+                    *reinterpret_cast<uint2 *>(out) = make_uint2(o0[0], o0[1]);
+                    if (second) *reinterpret_cast<uint2 *>(out + stride) = make_uint2(o1[0], o1[1]);
+                } else {
+                    *reinterpret_cast<uint4 *>(out) = make_uint4(o0[0], o0[1], o0[2], o0[3]);
+                    if (second)
+                        *reinterpret_cast<uint4 *>(out + stride) =
+                            make_uint4(o1[0], o1[1], o1[2], o1[3]);
+                }
+            } else {
+                constexpr uint32_t kPer = 4 / sizeof(C);  // samples a dword
+#pragma unroll
+                for (uint32_t c = 0; c < 4; ++c) {
+                    if (c >= cols) break;
+                    const uint32_t sh = 16 * (c % kPer);
+                    out[c] = (C)(int32_t)(o0[c / kPer] >> sh);
+                    if (second) out[stride + c] = (C)(int32_t)(o1[c / kPer] >> sh);
+                }
+            }
+            out += 2 * stride;
+        }
+    }
+    if (bad) {  // a malformed block reads as zeros
+        C *o = coef + j.dst + 4 * q;
+        for (uint32_t y = 0; y < h; ++y, o += stride)
+            for (uint32_t c = 0; c < cols; ++c) o[c] = 0;
+    }
+    if (valid && q == 0) status[i] = bad ? kCbBad : kCbOk;
+}
+
+// ---- refinement passes ---------------------------------------------------------
+
+// SigProp / MagRef passes of the code-blocks jobs[0 .. n) (each with more
+// than one pass, at most 64x64), one block per lane, after the
+// cleanup kernels wrote their samples.  A block whose cleanup failed holds zeros or
+// partial samples; the passes keep to its rectangle and its refinement
+// segment whatever the samples, and its status already reports it.
+template <typename C>
+__global__ void __launch_bounds__(256)
+sgn_ht_refine(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restrict__ arena,
+              C *__restrict__ coef) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const CbJob j = jobs[i];
+    // pass count rules of decode_impl (ht_block_decode.rs:1578-1592); more
+    // than three passes never reach this kernel
+    if ((j.flags & kCbZero) || j.passes < 2 || j.passes > 3 || j.lref == 0 || j.zblk >= 29 ||
+        j.lcup < 2 || j.w > 64 || j.h > 64)
+        return;
+    const uint32_t shift = j.kmax >= 31 ? 0u : 31u - j.kmax;
+    rows_refine<C>(coef + j.dst, j.w, j.h, j.stride, ((j.dst | j.stride) & 3u) == 0, arena,
+                   j.src + j.lcup, j.lref, j.passes, (j.flags & kCbStripeCausal) != 0,
+                   30u - j.zblk, shift);
+}
+
+}  // namespace sgn

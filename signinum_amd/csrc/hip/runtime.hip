@@ -30,7 +30,7 @@
 #include "../host/sgn_api.hpp"
 #include "ht_decode.hip"
 #include "ht_coop.hip"
-#include "ht_rows.hip"
+#include "ht_split.hip"
 #include "idwt.hip"
 #include "t1_classic.hip"
 #include "packets.hpp"
@@ -74,11 +74,9 @@ struct sgn_hip_session {
     int device = 0;
     hipStream_t stream = nullptr;
     uint16_t *d_tables = nullptr;
+    HtSplitTables *d_split = nullptr;
     uint64_t dispatches = 0;
     int cus = 0;                    // compute units of the device
-    // per lane-kernel variant and sample type (2 v + narrow): resident
-    // work-groups (0: unknown)
-    std::vector<uint32_t> resident;
     uint32_t classic_resident[4][3] = {};  // resident work-groups per classic kernel (shape, lanes)
     // pipelined batch decode: host-to-device copies run on copy_stream
     // while the previous chunk decodes on `stream`; two staging slots
@@ -90,29 +88,45 @@ struct sgn_hip_session {
 
 namespace {
 
-// Lane-kernel variants the autotuner chooses from: work-group shape, quad
-// pairs per segment (and MagSgn ring slots), and one-shot grid versus
-// persistent waves pulling 64-block chunks from a device work counter.
-// refine: the list holds blocks with SigProp / MagRef passes (the lane
-// kernel handles them in any case; the cooperative one needs its refining
-// instance)
-using RowsLaunch = void (*)(hipStream_t, uint32_t, const CbJob *, uint32_t, const uint8_t *,
-                            void *, const uint16_t *, uint8_t *, uint32_t *, bool);
+// Kernels of the lane list that the autotuner chooses from: the split cleanup
+// (ht_split.hip) with 64 or 32 lanes a wave in its symbol kernel, or one
+// code-block per wave in one kernel.
+using SymbolsLaunch = void (*)(hipStream_t, const CbJob *, uint32_t, const uint8_t *,
+                               const HtGroup *, uint4 *, const HtSplitTables *);
 
-template <int W, int S, int M, int VS, int LS, bool PERSIST, typename C, int MINW, int CHUNK>
-void rows_launch(hipStream_t st, uint32_t grid, const CbJob *jobs, uint32_t n,
-                 const uint8_t *arena, void *coef, const uint16_t *tables, uint8_t *status,
-                 uint32_t *queue, bool) {
-    hipLaunchKernelGGL((sgn_ht_rows<W, S, M, VS, LS, PERSIST, C, MINW, CHUNK>), dim3(grid),
-                       dim3(W * 64), 0, st, jobs, n, arena, static_cast<C *>(coef), tables, status,
-                       queue);
+template <int L>
+void symbols_launch(hipStream_t st, const CbJob *jobs, uint32_t n, const uint8_t *arena,
+                    const HtGroup *groups, uint4 *work, const HtSplitTables *tables) {
+    constexpr uint32_t per_group = L * kSplitWaves;
+    hipLaunchKernelGGL(sgn_ht_symbols<L>, dim3((n + per_group - 1) / per_group),
+                       dim3(kSplitWaves * 64), 0, st, jobs, n, arena, groups, work, tables,
+                       static_cast<uint64_t *>(nullptr));
 }
 
-// The cooperative kernel as a lane-list variant: one code-block per wave,
-// one wave per work-group (the grid is the block count).
+struct RowsVariant {
+    const char *name;
+    SymbolsLaunch symbols;  // null: the cooperative kernel
+};
+const RowsVariant kRowsVariants[] = {
+    {"split-l64", symbols_launch<64>},
+    {"split-l32", symbols_launch<32>},
+    {"wave-coop", nullptr},
+};
+constexpr int kRowsVariantCount = int(sizeof(kRowsVariants) / sizeof(kRowsVariants[0]));
+constexpr int kSplit64Variant = 0, kSplit32Variant = 1, kCoopVariant = 2;
+// Lane-list size from which a plan nobody autotuned uses all lanes of the
+// symbol kernel's waves: 64 lanes then give each of the 1024 SIMDs two waves.
+// Measured (clean + symbols + magnitudes, us): 307,200 blocks 1124 with 64
+// lanes, 1218 with 32; 28,800 blocks 258 and 252; 1,800 blocks 210 and 212;
+// 210 blocks 206 and 199 (16, 8, 4, 2 and 1 lanes are slower or within 2%
+// everywhere).
+constexpr size_t kSplit64Blocks = 131072;
+
+// The cooperative kernel: one code-block per wave, one wave per work-group.
+// refine: the list holds blocks with SigProp / MagRef passes
 template <typename C>
-void coop_launch(hipStream_t st, uint32_t, const CbJob *jobs, uint32_t n, const uint8_t *arena,
-                 void *coef, const uint16_t *tables, uint8_t *status, uint32_t *, bool refine) {
+void coop_launch(hipStream_t st, const CbJob *jobs, uint32_t n, const uint8_t *arena, void *coef,
+                 const uint16_t *tables, uint8_t *status, bool refine) {
     if (refine)
         hipLaunchKernelGGL((sgn_ht_coop<64, true, C>), dim3(n), dim3(64), 0, st, jobs, n, arena,
                            static_cast<C *>(coef), tables, status, 0u);
@@ -120,54 +134,6 @@ void coop_launch(hipStream_t st, uint32_t, const CbJob *jobs, uint32_t n, const 
         hipLaunchKernelGGL((sgn_ht_coop<64, false, C>), dim3(n), dim3(64), 0, st, jobs, n, arena,
                            static_cast<C *>(coef), tables, status, 0u);
 }
-
-// launch[0] / kernel[0]: int32 samples; [1]: int16 samples (narrow plans)
-struct RowsVariant {
-    const char *name;
-    int waves;
-    bool persist;
-    RowsLaunch launch[2];
-    const void *kernel[2];
-    bool coop = false;  // one code-block per wave (grid = block count)
-};
-
-// MINW: waves per SIMD the register allocation must allow (1: no bound);
-// CHUNK: code-blocks a persistent wave takes per work-counter grab
-#define SGN_ROWS_VARIANT(name, W, S, M, VS, LS, Q, MINW, CHUNK)                              \
-    {name,                                                                                 \
-     W,                                                                                    \
-     Q,                                                                                    \
-     {rows_launch<W, S, M, VS, LS, Q, int32_t, MINW, CHUNK>,                               \
-      rows_launch<W, S, M, VS, LS, Q, int16_t, MINW, CHUNK>},                              \
-     {reinterpret_cast<const void *>(sgn_ht_rows<W, S, M, VS, LS, Q, int32_t, MINW, CHUNK>), \
-      reinterpret_cast<const void *>(sgn_ht_rows<W, S, M, VS, LS, Q, int16_t, MINW, CHUNK>)}}
-
-// name: waves per work-group, quad pairs per segment, small rings (3 work-
-// groups per CU instead of 2), persistent queue and its chunk
-const RowsVariant kRowsVariants[] = {
-    SGN_ROWS_VARIANT("w4-seg8", 4, 8, 8, 4, 2, false, 1, 64),
-    SGN_ROWS_VARIANT("w4-seg8-queue", 4, 8, 8, 4, 2, true, 1, 64),
-    SGN_ROWS_VARIANT("w4-seg4-queue", 4, 4, 4, 4, 2, true, 1, 64),
-    SGN_ROWS_VARIANT("w4-seg4-small-queue", 4, 4, 4, 2, 1, true, 1, 64),
-    SGN_ROWS_VARIANT("w2-seg16-queue", 2, 16, 16, 4, 2, true, 1, 64),
-    SGN_ROWS_VARIANT("w1-seg8-queue", 1, 8, 8, 4, 2, true, 1, 64),
-    {"wave-coop",
-     1,
-     false,
-     {coop_launch<int32_t>, coop_launch<int16_t>},
-     {reinterpret_cast<const void *>(sgn_ht_coop<64, false, int32_t>),
-      reinterpret_cast<const void *>(sgn_ht_coop<64, false, int16_t>)},
-     true},
-    SGN_ROWS_VARIANT("w4-seg4-small-queue128", 4, 4, 4, 2, 1, true, 1, 128),
-    SGN_ROWS_VARIANT("w4-seg4-small-queue256", 4, 4, 4, 2, 1, true, 1, 256),
-};
-#undef SGN_ROWS_VARIANT
-constexpr int kRowsVariantCount = int(sizeof(kRowsVariants) / sizeof(kRowsVariants[0]));
-// variant of a plan nobody autotuned: w4-seg4-small-queue, the autotuner's
-// choice on every batch measured (small rings, three work-groups per CU)
-constexpr int kDefaultLaneVariant = 3;
-// the cooperative kernel (one code-block per wave)
-constexpr int kCoopVariant = 6;
 
 // Work-group shapes of the synthesis-level launches the autotuner chooses
 // from: the 64x64-block kernel (four or two waves per block) and whether
@@ -211,12 +177,6 @@ int classic_shape(uint32_t w) {
 uint32_t classic_lanes(int v, int opt) {
     return v == 3 ? uint32_t(ClassicW1024::kLanes) : kClassicLaneCount[opt];
 }
-// Lane-list size up to which plans start with the cooperative kernel.  On
-// 256x256 RGB tiles (75 code-blocks each) it took 0.28 against 1.41 ms for
-// 16 tiles and 1.21 against 1.61 ms for 256 tiles (19,200 blocks); the lane
-// kernel wins once its waves fill the device.
-constexpr size_t kCoopMaxBlocks = 24576;
-
 }  // namespace
 
 namespace {
@@ -230,6 +190,25 @@ bool lane_eligible(const CbJob &j) {
 }
 
 bool lane_refines(const CbJob &j) { return !(j.flags & kCbZero) && j.passes > 1; }
+
+// Workspace layout of a lane list (in its order); returns the units it takes.
+// unknown: the blocks' lengths are known on the device only (device packets),
+// the longest are reserved.
+uint64_t layout_groups(const std::vector<CbJob> &list, bool unknown, std::vector<HtGroup> &groups) {
+    uint64_t units = 0;
+    groups.clear();
+    for (size_t a = 0; a < list.size(); a += kHtGroup) {
+        uint32_t v = 0, y = 0;
+        for (size_t k = a; k < std::min(a + kHtGroup, list.size()); ++k) {
+            const CbJob &j = list[k];
+            v = std::max(v, ht_vlc_units(unknown ? 0xFFFFu : j.lcup));
+            y = std::max(y, ht_sym_units(j.w, j.h));
+        }
+        groups.push_back({static_cast<uint32_t>(units), v});
+        units += uint64_t(kHtGroup) * (1 + v + kHtMelUnits + y);
+    }
+    return units;
+}
 
 struct LevelRange {
     uint8_t rev, depth;
@@ -368,7 +347,14 @@ struct sgn_j2k_plan {
     uint32_t *d_lv_block_job[2] = {nullptr, nullptr}, *d_fin_block_job[2] = {nullptr, nullptr};
     uint32_t *d_fin_redo = nullptr;  // 5/3 final blocks left to the int32-plane pass
     uint8_t *d_status_lane = nullptr, *d_status_wave = nullptr;
-    uint32_t *d_queue = nullptr;  // work counter of the persistent lane kernel
+    uint32_t *d_queue = nullptr;  // count of d_fin_redo
+    // workspace of the split cleanup kernels, laid out for the lane list's
+    // order: a new order may need more than the plan's block holds (d_work_own)
+    std::vector<HtGroup> groups;
+    uint64_t work_units = 0, work_cap = 0;  // 16-byte units in use and allocated
+    HtGroup *d_groups = nullptr;
+    uint4 *d_work = nullptr;  // absent when the plan is carved from memory too small for it
+    void *d_work_own = nullptr;
     // packet headers parsed on the device (tiles planned with device
     // packets): tables, tag-tree and length scratch, per-tile status; the
     // lane list then keeps the per-tile order (its jobs are filled on the
@@ -406,7 +392,7 @@ struct sgn_j2k_plan {
     std::vector<std::pair<uint32_t, uint32_t>> tile_store;  // (first, count)
     StoreJob *d_store = nullptr;
     uint32_t *d_store_block_job = nullptr;
-    int lane_variant = kDefaultLaneVariant;  // index into kRowsVariants
+    int lane_variant = kSplit64Variant;  // index into kRowsVariants
     int dwt_shape = 0;                       // index into kDwtShapes
     hipGraphExec_t graph_exec = nullptr;
     hipGraph_t graph = nullptr;
@@ -420,6 +406,7 @@ struct sgn_j2k_plan {
     ~sgn_j2k_plan() {
         if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
         if (graph) (void)hipGraphDestroy(graph);
+        if (d_work_own) (void)hipFree(d_work_own);
         if (d_block && !borrowed) {
             if (blocks)
                 blocks->put(d_block);
@@ -848,6 +835,11 @@ Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
         sort_by_cost(P.cb_lane_plain, P.cb_lane);
         P.lane_refined = !P.cb_refine.empty();
     }
+    P.work_units = layout_groups(P.cb_lane, P.device_packets, P.groups);
+    if (P.work_units >= (1ull << 32)) {
+        set_last_error("batch too large for 32-bit plan offsets; split it");
+        return kErrArg;
+    }
     std::stable_sort(P.cb_refine.begin(), P.cb_refine.end(), [](const CbJob &a, const CbJob &b) {
         return uint32_t(a.lref) + a.lcup > uint32_t(b.lref) + b.lcup;
     });
@@ -866,10 +858,7 @@ Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
             P.classic_begin[v + 1] = e;
         }
     }
-    // kernel of a plan nobody autotuned: below kCoopMaxBlocks code-blocks the
-    // lane kernel cannot fill the device (each wave takes 64 blocks) and its
-    // time is one block's serial decode, so one block per wave finishes first
-    P.lane_variant = P.cb_lane.size() <= kCoopMaxBlocks ? kCoopVariant : kDefaultLaneVariant;
+    P.lane_variant = P.cb_lane.size() >= kSplit64Blocks ? kSplit64Variant : kSplit32Variant;
     // synthesis levels grouped by (transform, depth), tiles in order: the
     // levels of each depth counted, then placed tile by tile
     const uint32_t D = P.depth_max;
@@ -1032,7 +1021,7 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
     const uint64_t o_sto = take(bytes_of(P.store)), o_sbj = take(bytes_of(P.store_block_job));
     const uint64_t o_pkt = take(bytes_of(P.pk_tiles)), o_pkp = take(bytes_of(P.pk_parts));
     const uint64_t o_pkk = take(bytes_of(P.pk_pkts)), o_pkb = take(bytes_of(P.pk_bands));
-    const uint64_t o_pkc = take(bytes_of(P.pk_cbs));
+    const uint64_t o_pkc = take(bytes_of(P.pk_cbs)), o_grp = take(bytes_of(P.groups));
     const uint64_t host_bytes = off;
     const uint64_t o_pkn = take(P.pk_nodes * 2 * sizeof(uint32_t));
     const uint64_t o_pkl = take(P.pk_cbs.size() * sizeof(uint32_t)), o_pks = take(P.pk_tiles.size());
@@ -1063,6 +1052,11 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
     }
     const uint64_t o_crows = take(crows_bytes);
     const uint64_t o_queue = take(16), o_coef = take(P.coef_elems * sizeof(uint32_t));
+    // the workspace last: a plan carved from fixed memory does without when
+    // it does not fit (the cooperative kernel needs none)
+    const uint64_t no_work = off, o_work = take(P.work_units * sizeof(uint4));
+    const bool has_work = P.work_units != 0 && !(fixed && off > fixed_cap);
+    if (!has_work) off = no_work;
     P.device_bytes = off;
     if (fixed) {
         if (off > fixed_cap) {
@@ -1103,6 +1097,7 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
         HIP_TRY(put_dev(o_pkk, P.pk_pkts));
         HIP_TRY(put_dev(o_pkb, P.pk_bands));
         HIP_TRY(put_dev(o_pkc, P.pk_cbs));
+        HIP_TRY(put_dev(o_grp, P.groups));
         HIP_TRY(hipStreamSynchronize(copy));
         P.t_stage = 0;
         P.t_copy = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() -
@@ -1167,6 +1162,7 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
         put(o_pkk, P.pk_pkts);
         put(o_pkb, P.pk_bands);
         put(o_pkc, P.pk_cbs);
+        put(o_grp, P.groups);
         const auto t1 = std::chrono::steady_clock::now();
         uint8_t *d = static_cast<uint8_t *>(P.d_block);
         // direct runs first, then the staged range: consecutive staged runs and
@@ -1243,6 +1239,9 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
     at(o_crows, P.d_crows, crows_bytes != 0);
     at(o_queue, P.d_queue, true);
     at(o_coef, P.d_coef, P.coef_elems != 0);
+    at(o_grp, P.d_groups, !P.groups.empty());
+    at(o_work, P.d_work, has_work);
+    P.work_cap = has_work ? P.work_units : 0;
     return kOk;
 }
 
@@ -1254,27 +1253,6 @@ uint32_t group_blocks(const std::vector<LevelJob> &v, uint32_t a, uint32_t b) {
 uint32_t final_blocks(const std::vector<FinalJob> &v, uint32_t a, uint32_t b) {
     if (a >= b) return 0;
     return v[b - 1].block_base + uint32_t(v[b - 1].nbx) * v[b - 1].nby - v[a].block_base;
-}
-
-// Enqueue helpers; each returns the number of kernel launches issued.
-// Work-groups of variant v that the device holds at once.
-uint32_t resident_groups(sgn_hip_session *s, int v, bool narrow) {
-    if (s->resident.empty()) s->resident.assign(2 * kRowsVariantCount, 0);
-    const int slot = 2 * v + (narrow ? 1 : 0);
-    if (!s->resident[slot]) {
-        int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu, kRowsVariants[v].kernel[narrow ? 1 : 0], kRowsVariants[v].waves * 64,
-                0) != hipSuccess ||
-            per_cu < 1)
-            per_cu = 1;
-        if (!s->cus && (hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount,
-                                              s->device) != hipSuccess ||
-                        s->cus < 1))
-            s->cus = 1;
-        s->resident[slot] = uint32_t(per_cu) * uint32_t(s->cus);
-    }
-    return s->resident[slot];
 }
 
 uint32_t session_cus(sgn_hip_session *s) {
@@ -1298,29 +1276,35 @@ uint32_t classic_resident(sgn_hip_session *s, int v, int opt) {
     return s->classic_resident[v][opt];
 }
 
-// Clears the plan's device counters (word 0: lane work counter, word 1:
-// final redo count) with a kernel, never a memset node (graph capture).
-uint32_t clear_counters(sgn_hip_session *s, sgn_j2k_plan &P, uint32_t words) {
-    hipLaunchKernelGGL(sgn_fill_bytes, dim3(1), dim3(64), 0, s->stream,
-                       reinterpret_cast<uint8_t *>(P.d_queue), size_t(4) * words, size_t(words), 0u);
-    return 1;
-}
-
-// clear: reset the work counter first (false: the caller already did)
+// Enqueue helpers; each returns the number of kernel launches issued.
 uint32_t launch_lane_variant(sgn_hip_session *s, sgn_j2k_plan &P, int v, const CbJob *d_jobs,
-                             uint32_t count, uint8_t *status, bool clear = true) {
+                             uint32_t count, uint8_t *status) {
     if (!count) return 0;
-    const RowsVariant &rv = kRowsVariants[v];
-    const uint32_t per_group = rv.coop ? 1u : 64u * uint32_t(rv.waves);
-    uint32_t grid = (count + per_group - 1) / per_group;
-    uint32_t k = 1;
-    if (rv.persist) {
-        if (clear) k += clear_counters(s, P, 1);
-        grid = std::min(grid, resident_groups(s, v, P.narrow));
+    // The split kernels need their workspace, which is laid out for the
+    // ordered list.
+    const SymbolsLaunch symbols =
+        P.d_work && d_jobs == P.d_cb_lane ? kRowsVariants[v].symbols : nullptr;
+    if (!symbols) {
+        if (P.narrow)
+            coop_launch<int16_t>(s->stream, d_jobs, count, P.d_arena, P.d_coef, s->d_tables, status,
+                                 P.lane_refined);
+        else
+            coop_launch<int32_t>(s->stream, d_jobs, count, P.d_arena, P.d_coef, s->d_tables, status,
+                                 P.lane_refined);
+        return 1;
     }
-    rv.launch[P.narrow ? 1 : 0](s->stream, grid, d_jobs, count, P.d_arena, P.d_coef, s->d_tables,
-                                status, P.d_queue, P.lane_refined);
-    if (!rv.coop && d_jobs == P.d_cb_lane && (!P.cb_refine.empty() || P.device_packets)) {
+    uint32_t k = 3;
+    const dim3 g((count + kSplitBlocks - 1) / kSplitBlocks), b(kSplitWaves * 64);
+    hipLaunchKernelGGL(sgn_ht_clean, g, b, 0, s->stream, d_jobs, count, P.d_arena, P.d_groups,
+                       P.d_work);
+    symbols(s->stream, d_jobs, count, P.d_arena, P.d_groups, P.d_work, s->d_split);
+    if (P.narrow)
+        hipLaunchKernelGGL(sgn_ht_magsgn<int16_t>, g, b, 0, s->stream, d_jobs, count, P.d_arena,
+                           reinterpret_cast<int16_t *>(P.d_coef), P.d_groups, P.d_work, status);
+    else
+        hipLaunchKernelGGL(sgn_ht_magsgn<int32_t>, g, b, 0, s->stream, d_jobs, count, P.d_arena,
+                           reinterpret_cast<int32_t *>(P.d_coef), P.d_groups, P.d_work, status);
+    if (!P.cb_refine.empty() || P.device_packets) {
         // refinement passes of the batch's lane blocks, after their cleanup
         // (with device packets the pass counts are known on the device only:
         // the kernel walks the whole lane list and skips the other blocks)
@@ -1338,9 +1322,9 @@ uint32_t launch_lane_variant(sgn_hip_session *s, sgn_j2k_plan &P, int v, const C
     return k;
 }
 
-uint32_t launch_lane(sgn_hip_session *s, sgn_j2k_plan &P, const CbJob *d_jobs, uint32_t count,
-                     uint8_t *status, bool clear = true) {
-    return launch_lane_variant(s, P, P.lane_variant, d_jobs, count, status, clear);
+uint32_t launch_lane(sgn_hip_session *s, sgn_j2k_plan &P) {
+    return launch_lane_variant(s, P, P.lane_variant, P.d_cb_lane,
+                               static_cast<uint32_t>(P.cb_lane.size()), P.d_status_lane);
 }
 
 uint32_t launch_wave(sgn_hip_session *s, sgn_j2k_plan &P, const CbJob *d_jobs, uint32_t count,
@@ -1400,22 +1384,18 @@ uint32_t launch_levels(sgn_hip_session *s, sgn_j2k_plan &P, int rev, uint32_t a,
     return 1;
 }
 
-uint32_t launch_finals(sgn_hip_session *s, sgn_j2k_plan &P, int rev, uint32_t a, uint32_t b,
-                       bool clear = true) {
+uint32_t launch_finals(sgn_hip_session *s, sgn_j2k_plan &P, int rev, uint32_t a, uint32_t b) {
     const uint32_t blocks = final_blocks(P.fin[rev], a, b);
     if (!blocks) return 0;
     const uint32_t off = P.fin[rev][a].block_base;
     if (rev) {
         // int16-plane pass over every block, then the int32-plane pass over
-        // the blocks it listed (word 1 of the work-counter area counts them;
-        // cleared by a kernel, graph-safe)
-        uint32_t *redo_n = P.d_queue + 1;
-        uint32_t k = 2;
-        if (clear) {
-            hipLaunchKernelGGL(sgn_fill_bytes, dim3(1), dim3(64), 0, s->stream,
-                               reinterpret_cast<uint8_t *>(redo_n), size_t(4), size_t(1), 0u);
-            ++k;
-        }
+        // the blocks it listed (d_queue counts them; cleared by a kernel,
+        // graph-safe)
+        uint32_t *redo_n = P.d_queue;
+        const uint32_t k = 3;
+        hipLaunchKernelGGL(sgn_fill_bytes, dim3(1), dim3(64), 0, s->stream,
+                           reinterpret_cast<uint8_t *>(redo_n), size_t(4), size_t(1), 0u);
         hipLaunchKernelGGL(sgn_final_rev16, dim3(blocks), dim3(kIdwtThreads), 0, s->stream,
                            P.d_fin[1], uint32_t(P.fin[1].size()), off, P.d_fin_block_job[1],
                            P.d_final_lv, P.d_coef, P.d_fin_redo, redo_n);
@@ -1459,17 +1439,15 @@ uint32_t launch_packets(sgn_hip_session *s, sgn_j2k_plan &P) {
 }
 
 uint32_t enqueue_batched(sgn_hip_session *s, sgn_j2k_plan &P) {
-    uint32_t k = clear_counters(s, P, 2);  // one node for both counters
-    k += launch_packets(s, P);
+    uint32_t k = launch_packets(s, P);
     k += launch_classic(s, P);
-    k += launch_lane(s, P, P.d_cb_lane, static_cast<uint32_t>(P.cb_lane.size()), P.d_status_lane,
-                     false);
+    k += launch_lane(s, P);
     k += launch_wave(s, P, P.d_cb_wave, static_cast<uint32_t>(P.cb_wave.size()), P.d_status_wave);
     for (uint32_t d = 1; d <= P.depth_max; ++d)
         for (int rev = 0; rev < 2; ++rev)
             k += launch_levels(s, P, rev, P.lv_group[rev][d - 1], P.lv_group[rev][d]);
     for (int rev = 0; rev < 2; ++rev)
-        k += launch_finals(s, P, rev, 0, static_cast<uint32_t>(P.fin[rev].size()), false);
+        k += launch_finals(s, P, rev, 0, static_cast<uint32_t>(P.fin[rev].size()));
     k += launch_stores(s, P, 0, static_cast<uint32_t>(P.store.size()));
     return k;
 }
@@ -1481,8 +1459,7 @@ uint32_t enqueue_plain(sgn_hip_session *s, sgn_j2k_plan &P) {
     k += launch_classic(s, P);
     for (size_t t = 0; t < P.ntiles; ++t) {
         const uint32_t a0 = P.lane_plain_begin[t], a1 = P.lane_plain_begin[t + 1];
-        // one tile's code-blocks: the cooperative kernel (a tile has far
-        // fewer blocks than the lane kernel needs to fill the device)
+        // one tile's code-blocks: the cooperative kernel (one launch a tile)
         k += launch_lane_variant(s, P, kCoopVariant, P.d_cb_lane_plain + a0, a1 - a0,
                                  P.d_status_lane + a0);
         const uint32_t b0 = P.wave_begin[t], b1 = P.wave_begin[t + 1];
@@ -1640,7 +1617,7 @@ class OnStream {
 
 // Tiles per chunk of a pipelined batch decode (SGN_PIPELINE_TILES
 // overrides; 0 or a value >= n decodes the batch as one plan).  768 tiles
-// of 256x256 RGB: chunks large enough for the lane kernel (57600
+// of 256x256 RGB: chunks large enough to fill the device (57600
 // code-blocks), small enough that the first parse and the last decode,
 // which nothing overlaps, stay short.
 size_t pipeline_tiles() {
@@ -1805,6 +1782,10 @@ int sgn_hip_session_create(int device, sgn_hip_session **out) {
     std::memcpy(tab.data() + 2368, T.uvlc1, 512);
     HIP_TRY(hipMalloc(&s->d_tables, tab.size() * 2));
     HIP_TRY(hipMemcpy(s->d_tables, tab.data(), tab.size() * 2, hipMemcpyHostToDevice));
+    const auto split = std::make_unique<HtSplitTables>();
+    ht_split_tables(T.vlc0, T.vlc1, T.uvlc0, T.uvlc1, *split);
+    HIP_TRY(hipMalloc(&s->d_split, sizeof(HtSplitTables)));
+    HIP_TRY(hipMemcpy(s->d_split, split.get(), sizeof(HtSplitTables), hipMemcpyHostToDevice));
     {
         void *scr = nullptr;
         const Status st = noalloc_scratch(device, &scr);
@@ -1829,6 +1810,7 @@ void sgn_hip_session_destroy(sgn_hip_session *s) {
     }
     delete s->blocks;
     if (s->d_tables) (void)hipFree(s->d_tables);
+    if (s->d_split) (void)hipFree(s->d_split);
     delete s;
 }
 
@@ -2148,8 +2130,7 @@ int sgn_j2k_plan_decode_stage(sgn_hip_session *s, sgn_j2k_plan *P, int stage) {
     if (stage == SGN_STAGE_BLOCKS) {
         k += launch_packets(s, *P);
         k += launch_classic(s, *P);
-        k += launch_lane(s, *P, P->d_cb_lane, static_cast<uint32_t>(P->cb_lane.size()),
-                         P->d_status_lane);
+        k += launch_lane(s, *P);
         k += launch_wave(s, *P, P->d_cb_wave, static_cast<uint32_t>(P->cb_wave.size()),
                          P->d_status_wave);
     } else if (stage == SGN_STAGE_LEVELS) {
@@ -2439,9 +2420,8 @@ static int hook_blocks(sgn_hip_session *s, const uint8_t *data, size_t data_len,
     }
     // a hook call is one sub-band or a few: the cooperative kernel
     if (!lane.empty())
-        kRowsVariants[kCoopVariant].launch[0](s->stream, uint32_t(lane.size()), d_lane,
-                                              uint32_t(lane.size()), d_data, d_out, s->d_tables,
-                                              d_st, nullptr, refined);
+        coop_launch<int32_t>(s->stream, d_lane, uint32_t(lane.size()), d_data, d_out, s->d_tables,
+                             d_st, refined);
     if (!wave.empty())
         hipLaunchKernelGGL((sgn_ht_coop<1024, true, int32_t>), dim3(wave.size()), dim3(64), 0,
                            s->stream, d_wave, uint32_t(wave.size()), d_data,
@@ -2895,28 +2875,27 @@ int sgn_j2k_plan_time_code_blocks(sgn_hip_session *s, sgn_j2k_plan *P, size_t st
         if (!(P->cb_lane[i].flags & kCbZero)) pick.push_back(i);
     *count = pick.size();
     if (pick.empty()) return SGN_OK;
-    // wave k: lane 0 holds sample k, lanes 1..63 an empty block
-    CbJob empty{};
-    empty.flags = kCbZero;
-    std::vector<CbJob> jobs(pick.size() * 64, empty);
-    for (size_t k = 0; k < pick.size(); ++k) jobs[k * 64] = P->cb_lane[pick[k]];
+    std::vector<CbJob> jobs(pick.size());
+    for (size_t k = 0; k < pick.size(); ++k) jobs[k] = P->cb_lane[pick[k]];
+    std::vector<HtGroup> groups;
+    const uint64_t units = layout_groups(jobs, false, groups);
     DevBuf<CbJob> djobs;
-    DevBuf<uint8_t> dst;
+    DevBuf<HtGroup> dgroups;
+    DevBuf<uint4> dwork;
     DevBuf<uint64_t> dcyc;
     Status st;
-    if ((st = djobs.upload(jobs.data(), jobs.size())) || (st = dst.alloc(jobs.size())) ||
+    if ((st = djobs.upload(jobs.data(), jobs.size())) ||
+        (st = dgroups.upload(groups.data(), groups.size())) || (st = dwork.alloc(units)) ||
         (st = dcyc.alloc(pick.size())))
         return st;
-    const uint32_t waves = uint32_t(pick.size());
-    if (P->narrow)
-        hipLaunchKernelGGL(sgn_ht_rows_timed<int16_t>, dim3((waves + 3) / 4), dim3(256), 0,
-                           s->stream, djobs.p, uint32_t(jobs.size()), P->d_arena,
-                           reinterpret_cast<int16_t *>(P->d_coef), s->d_tables, dst.p, dcyc.p);
-    else
-        hipLaunchKernelGGL(sgn_ht_rows_timed<int32_t>, dim3((waves + 3) / 4), dim3(256), 0,
-                           s->stream, djobs.p, uint32_t(jobs.size()), P->d_arena,
-                           reinterpret_cast<int32_t *>(P->d_coef), s->d_tables, dst.p, dcyc.p);
-    s->dispatches++;
+    const uint32_t n = uint32_t(pick.size());
+    hipLaunchKernelGGL(sgn_ht_clean, dim3((n + kSplitBlocks - 1) / kSplitBlocks),
+                       dim3(kSplitWaves * 64), 0, s->stream, djobs.p, n, P->d_arena, dgroups.p,
+                       dwork.p);
+    hipLaunchKernelGGL((sgn_ht_symbols<1, true>), dim3((n + kSplitWaves - 1) / kSplitWaves),
+                       dim3(kSplitWaves * 64), 0, s->stream, djobs.p, n, P->d_arena, dgroups.p,
+                       dwork.p, s->d_split, dcyc.p);
+    s->dispatches += 2;
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s->stream));
     std::vector<uint64_t> cyc(pick.size());
@@ -2986,9 +2965,28 @@ int sgn_j2k_plan_order_code_blocks(sgn_hip_session *s, sgn_j2k_plan *P, int orde
     std::vector<CbJob> w(v.size());
     for (size_t i = 0; i < idx.size(); ++i) w[i] = v[idx[i]];
     v.swap(w);
+    std::vector<HtGroup> groups;
+    const uint64_t units = layout_groups(v, false, groups);
+    if (units >= (1ull << 32)) {
+        set_last_error("batch too large for 32-bit plan offsets; split it");
+        return SGN_E_ARG;
+    }
     HIP_TRY(hipStreamSynchronize(s->stream));
-    if (!v.empty())
+    if (P->d_work && units > P->work_cap) {
+        void *own = nullptr;
+        HIP_TRY(hipMalloc(&own, units * sizeof(uint4)));
+        if (P->d_work_own) (void)hipFree(P->d_work_own);
+        P->d_work_own = own;
+        P->d_work = static_cast<uint4 *>(own);
+        P->work_cap = units;
+    }
+    P->work_units = units;
+    if (!v.empty()) {
         HIP_TRY(hipMemcpy(P->d_cb_lane, v.data(), v.size() * sizeof(CbJob), hipMemcpyHostToDevice));
+        HIP_TRY(hipMemcpy(P->d_groups, groups.data(), groups.size() * sizeof(HtGroup),
+                          hipMemcpyHostToDevice));
+    }
+    P->groups.swap(groups);
     P->cb_lane.swap(v);
     drop_graph(*P);
     return SGN_OK;

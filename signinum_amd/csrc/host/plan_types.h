@@ -21,6 +21,26 @@ struct CbJob {
 };
 static_assert(sizeof(CbJob) == 32, "CbJob layout");
 
+// Workspace of 64 consecutive lane-list code-blocks between the kernels of
+// their cleanup decode, in 16-byte units; unit u of block b of the group is at
+// base + part + 64 u + b, so that the lanes of a wave (one block each, all at
+// much the same place) share cache lines.  Parts: a header per block; the VLC
+// strings (a segment's MEL and VLC bytes are at most 4079; a few bits in front
+// and a zero unit come on top); the first MEL bytes; the quad symbols, eight
+// pairs of a row in two adjacent units.
+struct HtGroup {
+    uint32_t base;
+    uint32_t vlc_units;  // per block: the most that any block of the group takes
+};
+constexpr uint32_t kHtGroup = 64;
+constexpr uint32_t kHtMelUnits = 8;
+constexpr inline uint32_t ht_vlc_units(uint32_t lcup) {
+    return ((lcup < 4096 ? lcup : 4096) + 15) / 16 + 2;
+}
+constexpr inline uint32_t ht_sym_units(uint32_t w, uint32_t h) {
+    return (h + 1) / 2 * ((w + 31) / 32) * 2;
+}
+
 // flags: bit 0 stripe-causal, bit 1 decodes to zero, bits 2-3 sub-band
 // (0 LL, 1 HL, 2 LH, 3 HH; a feature of the decode-cost model)
 enum : uint8_t { kCbStripeCausal = 1, kCbZero = 2, kCbBandShift = 2 };
