@@ -248,6 +248,14 @@ typedef struct {
  * Synchronous. */
 int sgn_j2k_decode_tiles_region_device(sgn_hip_session *session, const sgn_tile_req *reqs,
                                        size_t n, size_t *first_fail);
+/* decode_tiles_into / decode_tiles_region_scaled_into (crates/signinum-j2k/src/
+ * batch.rs:110-195): as above with dst, pitch and capacity naming host arrays,
+ * every request decoded in one batch (`mode` as for sgn_j2k_plan_decode; a
+ * batched call of many whole tiles is pipelined) and written to its array.  If
+ * an array is too small nothing is decoded: SGN_E_BUFFER with *first_fail
+ * SIZE_MAX.  Synchronous. */
+int sgn_j2k_decode_reqs_into(sgn_hip_session *session, const sgn_tile_req *reqs, size_t n, int mode,
+                             size_t *first_fail);
 /* As sgn_j2k_plan_create, with format, scale and region per tile. */
 int sgn_j2k_plan_create_mixed(sgn_hip_session *session, const sgn_tile_req *reqs, size_t n,
                               sgn_j2k_plan **out, int32_t *tile_status);

@@ -731,6 +731,26 @@ def decode_tiles_to_device(session, inputs, fmt, scale=Downscale.NONE, mode=MODE
     return surfaces
 
 
+def _decode_reqs_into(session, keep, arrays, strides, fmt, scales, rois, mode):
+    """One batch from host codestreams to host arrays.  False, with nothing
+    decoded, if an array is not one the library can write to."""
+    n = len(keep)
+    reqs = (_lib.TileReq * max(1, n))()
+    for i, (k, a, stride, scale, roi) in enumerate(zip(keep, arrays, strides, scales, rois)):
+        if not (a.flags["C_CONTIGUOUS"] and a.flags["WRITEABLE"]) or stride < 0:
+            return False
+        reqs[i] = _lib.TileReq(k.ctypes.data, k.size, a.ctypes.data, int(stride), a.nbytes, int(fmt),
+                               int(scale), 0 if roi is None else 1,
+                               *((0, 0, 0, 0) if roi is None else (int(v) for v in roi)))
+    ff = ctypes.c_size_t(0)
+    rc = _lib.load().sgn_j2k_decode_reqs_into(session.handle, reqs, n, int(mode), ctypes.byref(ff))
+    if rc == _lib.SGN_E_BUFFER and ff.value == ctypes.c_size_t(-1).value:
+        return False
+    if rc != _lib.SGN_OK:
+        raise TileBatchError(ff.value, _ERRORS.get(rc, J2kError)(rc, _lib.last_error()))
+    return True
+
+
 def decode_tiles_region_scaled_into(jobs, fmt, session=None):
     """decode_tiles_region_scaled_into (crates/signinum-j2k/src/batch.rs:
     151-195): jobs are (input_bytes, out_array, stride, roi, scale) with roi
@@ -749,6 +769,12 @@ def decode_tiles_region_scaled_into(jobs, fmt, session=None):
                 dims.append(region_dims(keep[-1], roi, scale)[2:])
             except J2kError as e:
                 raise TileBatchError(i, e)
+        if _decode_reqs_into(session, keep, [np.asarray(j[1]) for j in jobs], [j[2] for j in jobs],
+                             fmt, [Downscale(j[4]) for j in jobs], [j[3] for j in jobs],
+                             MODE_BATCHED):
+            return
+        # an array that cannot take its region: the regions before it are
+        # still written
         surfs = _alloc_surfaces(session, dims, [fmt] * len(jobs))
         n = len(jobs)
         reqs = (_lib.TileReq * max(1, n))()
@@ -776,6 +802,14 @@ def decode_tiles_into(jobs, fmt, session=None, scale=Downscale.NONE, mode=MODE_B
     if own:
         session = HipSession()
     try:
+        fmt = PixelFormat(fmt)
+        scale = Downscale(scale)
+        keep = [np.frombuffer(bytes(j[0]), np.uint8) for j in jobs]
+        if _decode_reqs_into(session, keep, [np.asarray(j[1]) for j in jobs], [j[2] for j in jobs],
+                             fmt, [scale] * len(keep), [None] * len(keep), mode):
+            return
+        # an array that cannot take its tile: the tiles before it are still
+        # written
         surfs = decode_tiles_to_device(session, [j[0] for j in jobs], fmt, scale, mode)
         for (inp, out, stride), s in zip(jobs, surfs):
             s.download_into(out, stride)

@@ -160,6 +160,8 @@ SIGNATURES = {
     "sgn_j2k_decode_tiles_region_device": (ctypes.c_int, [ctypes.c_void_p,
                                                           ctypes.POINTER(TileReq), c_size_t,
                                                           ctypes.POINTER(c_size_t)]),
+    "sgn_j2k_decode_reqs_into": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(TileReq), c_size_t,
+                                                ctypes.c_int, ctypes.POINTER(c_size_t)]),
     "sgn_dicom_extract_frames": (ctypes.c_int, [ctypes.c_void_p, c_size_t, c_size_t,
                                                 ctypes.c_void_p, c_size_t,
                                                 ctypes.POINTER(c_size_t),

@@ -83,7 +83,8 @@ struct sgn_hip_session {
     hipStream_t copy_stream = nullptr;
     hipStream_t aux_stream = nullptr;  // second decode stream: chunks alternate
     PinnedSlot slot[2];
-    DeviceBlocks *blocks = nullptr;  // device blocks of pipelined chunk plans, reused
+    PinnedSlot down[2], stat;        // downloads to host arrays (two chunks), block status words
+    DeviceBlocks *blocks = nullptr;  // device blocks of the plans of one call, reused
 };
 
 namespace {
@@ -959,10 +960,10 @@ bool host_pinned(const void *p) {
     return e == hipSuccess && a.type == hipMemoryTypeHost;
 }
 
-// Reserves `bytes` of the session's pinned staging slot k, after the copies
-// out of its previous contents have finished.
-Status slot_reserve(sgn_hip_session *s, int k, size_t bytes, uint8_t **out) {
-    PinnedSlot &sl = s->slot[k];
+// Reserves `bytes` of a pinned staging slot (grown to at least `least`), after
+// the copies out of its previous contents have finished.
+Status slot_reserve(PinnedSlot &sl, size_t bytes, uint8_t **out,
+                    size_t least = size_t(16) << 20) {
     if (sl.pending) {
         HIP_TRY(hipEventSynchronize(sl.done));
         sl.pending = false;
@@ -972,7 +973,7 @@ Status slot_reserve(sgn_hip_session *s, int k, size_t bytes, uint8_t **out) {
         if (sl.p) HIP_TRY(hipHostFree(sl.p));
         sl.p = nullptr;
         sl.cap = 0;
-        const size_t cap = (std::max<size_t>(bytes, size_t(16) << 20) + (size_t(2) << 20) - 1) &
+        const size_t cap = (std::max<size_t>(bytes, least) + (size_t(2) << 20) - 1) &
                            ~((size_t(2) << 20) - 1);
         HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&sl.p), cap, hipHostMallocDefault));
         sl.cap = cap;
@@ -1117,7 +1118,7 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
         // bytes of direct runs are left unfilled there and never copied
         uint8_t *h = nullptr;
         {
-            const Status st = slot_reserve(s, slot, host_bytes, &h);
+            const Status st = slot_reserve(s->slot[slot], host_bytes, &h);
             if (st) return st;
         }
         // staged codestream bytes, copied by the worker pool in 1 MB pieces
@@ -1499,45 +1500,57 @@ Status decode_plan(sgn_hip_session *s, sgn_j2k_plan &P, int mode) {
     return kOk;
 }
 
-// First failing tile from the per-block status words (after a sync).
-Status check_status(sgn_j2k_plan &P, int mode, size_t *first_fail) {
+// First failing tile from the per-block status words, which follow the decode
+// into pinned memory: status_fetch enqueues the copy, status_check reads it
+// once the stream has got there.
+Status status_fetch(sgn_hip_session *s, sgn_j2k_plan &P) {
+    const size_t np = P.pk_tiles.size(), nl = P.cb_lane.size(), nw = P.cb_wave.size();
+    uint8_t *h = nullptr;
+    const Status st = slot_reserve(s->stat, np + nl + nw, &h, 1);
+    if (st) return st;
+    if (np) HIP_TRY(hipMemcpyAsync(h, P.d_pk_status, np, hipMemcpyDeviceToHost, s->stream));
+    if (nl) HIP_TRY(hipMemcpyAsync(h + np, P.d_status_lane, nl, hipMemcpyDeviceToHost, s->stream));
+    if (nw)
+        HIP_TRY(hipMemcpyAsync(h + np + nl, P.d_status_wave, nw, hipMemcpyDeviceToHost, s->stream));
+    return kOk;
+}
+
+Status status_check(sgn_j2k_plan &P, const uint8_t *h, int mode, size_t *first_fail) {
     size_t bad = SIZE_MAX;
-    if (!P.pk_tiles.empty()) {
-        std::vector<uint8_t> h(P.pk_tiles.size());
-        HIP_TRY(hipMemcpy(h.data(), P.d_pk_status, h.size(), hipMemcpyDeviceToHost));
-        for (size_t k = 0; k < h.size(); ++k)
-            if (h[k]) {
-                // the tile of this packet table: its first job's tile
-                const PktTile &t = P.pk_tiles[k];
-                for (uint32_t c = 0; c < t.ncbs; ++c) {
-                    const uint32_t job = P.pk_cbs[t.cb0 + c].job;
-                    if (job == kPktNoJob) continue;
-                    const CbJob &j = (job & kPktWave) ? P.cb_wave[job & ~kPktWave]
-                                                      : P.cb_lane_plain[job];
-                    bad = std::min<size_t>(bad, j.tile);
-                    break;
-                }
+    for (size_t k = 0; k < P.pk_tiles.size(); ++k, ++h)
+        if (*h) {
+            // the tile of this packet table: its first job's tile
+            const PktTile &t = P.pk_tiles[k];
+            for (uint32_t c = 0; c < t.ncbs; ++c) {
+                const uint32_t job = P.pk_cbs[t.cb0 + c].job;
+                if (job == kPktNoJob) continue;
+                const CbJob &j =
+                    (job & kPktWave) ? P.cb_wave[job & ~kPktWave] : P.cb_lane_plain[job];
+                bad = std::min<size_t>(bad, j.tile);
+                break;
             }
-    }
-    if (!P.cb_lane.empty()) {
-        std::vector<uint8_t> h(P.cb_lane.size());
-        HIP_TRY(hipMemcpy(h.data(), P.d_status_lane, h.size(), hipMemcpyDeviceToHost));
-        const std::vector<CbJob> &jobs = mode == SGN_MODE_PLAIN ? P.cb_lane_plain : P.cb_lane;
-        for (size_t k = 0; k < h.size(); ++k)
-            if (h[k]) bad = std::min<size_t>(bad, jobs[k].tile);
-    }
-    if (!P.cb_wave.empty()) {
-        std::vector<uint8_t> h(P.cb_wave.size());
-        HIP_TRY(hipMemcpy(h.data(), P.d_status_wave, h.size(), hipMemcpyDeviceToHost));
-        for (size_t k = 0; k < h.size(); ++k)
-            if (h[k]) bad = std::min<size_t>(bad, P.cb_wave[k].tile);
-    }
+        }
+    const std::vector<CbJob> &jobs = mode == SGN_MODE_PLAIN ? P.cb_lane_plain : P.cb_lane;
+    for (size_t k = 0; k < P.cb_lane.size(); ++k, ++h)
+        if (*h) bad = std::min<size_t>(bad, jobs[k].tile);
+    for (size_t k = 0; k < P.cb_wave.size(); ++k, ++h)
+        if (*h) bad = std::min<size_t>(bad, P.cb_wave[k].tile);
     if (bad != SIZE_MAX) {
         if (first_fail) *first_fail = bad;
         set_last_error("code-block decode failure in tile " + std::to_string(bad));
         return kErrBlock;
     }
     return kOk;
+}
+
+// The same after a sync, without pinned memory.
+Status check_status(sgn_j2k_plan &P, int mode, size_t *first_fail) {
+    const size_t np = P.pk_tiles.size(), nl = P.cb_lane.size(), nw = P.cb_wave.size();
+    std::vector<uint8_t> h(np + nl + nw);
+    if (np) HIP_TRY(hipMemcpy(h.data(), P.d_pk_status, np, hipMemcpyDeviceToHost));
+    if (nl) HIP_TRY(hipMemcpy(h.data() + np, P.d_status_lane, nl, hipMemcpyDeviceToHost));
+    if (nw) HIP_TRY(hipMemcpy(h.data() + np + nl, P.d_status_wave, nw, hipMemcpyDeviceToHost));
+    return status_check(P, h.data(), mode, first_fail);
 }
 
 void drop_graph(sgn_j2k_plan &P) {
@@ -1549,7 +1562,7 @@ void drop_graph(sgn_j2k_plan &P) {
 
 Status make_plan(sgn_hip_session *s, const sgn_tile_req *jobs, size_t n,
                  std::unique_ptr<sgn_j2k_plan> &out, int32_t *tile_status,
-                 DeviceBlocks *blocks = nullptr) {
+                 DeviceBlocks *blocks = nullptr, bool sync = true) {
     if (!s || (!jobs && n)) {
         set_last_error("null session or jobs");
         return kErrArg;
@@ -1559,8 +1572,11 @@ Status make_plan(sgn_hip_session *s, const sgn_tile_req *jobs, size_t n,
     P->blocks = blocks;
     Status st = build_plan(jobs, n, *P, tile_status);
     if (st) return st;
-    st = upload_plan(s, jobs, *P, s->stream, 0, true);
-    if (st) return st;
+    st = upload_plan(s, jobs, *P, s->stream, 0, sync);
+    if (st) {
+        (void)hipStreamSynchronize(s->stream);  // before the block goes back
+        return st;
+    }
     out = std::move(P);
     return kOk;
 }
@@ -1729,6 +1745,162 @@ Status decode_pipelined(sgn_hip_session *s, const sgn_tile_req *reqs, size_t n, 
     return kOk;
 }
 
+// Waits for the session's streams when a scope ends: declared after a plan (or
+// a device block) that goes back to the session's cache, so that nothing
+// enqueued still uses it then, whatever way the scope is left.
+struct StreamDone {
+    sgn_hip_session *s;
+    ~StreamDone() {
+        for (hipStream_t q : {s->copy_stream, s->aux_stream, s->stream})
+            (void)hipStreamSynchronize(q);
+    }
+};
+
+struct CachedBlock {
+    DeviceBlocks *blocks;
+    void *p = nullptr;
+    ~CachedBlock() { blocks->put(p); }
+};
+
+// One batch decoded synchronously as one plan; `after` enqueues work behind the
+// decode (and is not called if that failed).
+template <class F>
+Status decode_once(sgn_hip_session *s, const sgn_tile_req *reqs, size_t n, int mode,
+                   size_t *first_fail, F after) {
+    std::vector<int32_t> ts(n, 0);
+    std::unique_ptr<sgn_j2k_plan> P;
+    Status st = make_plan(s, reqs, n, P, ts.data(), s->blocks, false);
+    if (st) {
+        if (first_fail)
+            for (size_t i = 0; i < n; ++i)
+                if (ts[i]) {
+                    *first_fail = i;
+                    break;
+                }
+        return st;
+    }
+    StreamDone done{s};
+    if ((st = decode_plan(s, *P, mode)) || (st = status_fetch(s, *P)) || (st = after())) return st;
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    return status_check(*P, s->stat.p, mode, first_fail);
+}
+
+// An image in a call's device block (rows without gaps) and its host array.
+struct HostImage {
+    uint8_t *dst;
+    size_t stride, off, row, rows;
+};
+
+// Device images to host arrays.  The bytes travel in pinned chunks, one copied
+// by the DMA engine while the worker pool writes the previous one to its
+// arrays; a pitched copy straight to pageable memory took 1.6 ms for the 192 KB
+// of a 256x256 tile, this way takes about 25 us.
+class HostWriter {
+  public:
+    HostWriter(sgn_hip_session *s, const uint8_t *dev, std::vector<HostImage> images)
+        : s_(s), dev_(dev) {
+        // chunks of whole rows, consecutive in the device block
+        for (const HostImage &im : images) {
+            if (!im.row || !im.rows) continue;
+            const size_t most = std::max<size_t>(1, kChunk / im.row);
+            for (size_t y = 0; y < im.rows; y += most) {
+                const size_t k = std::min(most, im.rows - y);
+                const size_t a = im.off + y * im.row, e = a + k * im.row;
+                if (chunks_.empty() || e - chunks_.back().a > kChunk) chunks_.push_back({a, e, {}});
+                Chunk &c = chunks_.back();
+                c.e = e;
+                // pieces the pool copies, about 256 KB each
+                const size_t step = std::max<size_t>(1, (size_t(256) << 10) / im.row);
+                for (size_t z = 0; z < k; z += step)
+                    c.pieces.push_back({im.dst + (y + z) * im.stride, im.stride,
+                                        a + z * im.row - c.a, im.row, std::min(step, k - z)});
+            }
+        }
+    }
+    // Enqueues the first chunk's copy behind what the stream holds.
+    Status start() { return chunks_.empty() ? kOk : fetch(0); }
+    Status finish() {
+        for (size_t k = 0; k < chunks_.size(); ++k) {
+            if (k + 1 < chunks_.size()) {
+                const Status st = fetch(k + 1);
+                if (st) return st;
+            }
+            PinnedSlot &sl = s_->down[k & 1];
+            HIP_TRY(hipEventSynchronize(sl.done));
+            sl.pending = false;
+            const std::vector<HostImage> &ps = chunks_[k].pieces;
+            WorkerPool::get().run(ps.size(), [&](size_t i) {
+                const HostImage &q = ps[i];
+                const uint8_t *src = sl.p + q.off;
+                if (q.stride == q.row) {
+                    std::memcpy(q.dst, src, q.row * q.rows);
+                } else {
+                    for (size_t y = 0; y < q.rows; ++y)
+                        std::memcpy(q.dst + y * q.stride, src + y * q.row, q.row);
+                }
+            });
+        }
+        return kOk;
+    }
+
+  private:
+    struct Chunk {
+        size_t a, e;
+        std::vector<HostImage> pieces;
+    };
+    static constexpr size_t kChunk = size_t(8) << 20;
+    Status fetch(size_t k) {
+        PinnedSlot &sl = s_->down[k & 1];
+        uint8_t *h = nullptr;
+        const size_t len = chunks_[k].e - chunks_[k].a;
+        const Status st = slot_reserve(sl, len, &h, 1);
+        if (st) return st;
+        HIP_TRY(hipMemcpyAsync(h, dev_ + chunks_[k].a, len, hipMemcpyDeviceToHost, s_->stream));
+        HIP_TRY(hipEventRecord(sl.done, s_->stream));
+        sl.pending = true;
+        return kOk;
+    }
+    sgn_hip_session *s_;
+    const uint8_t *dev_;
+    std::vector<Chunk> chunks_;
+};
+
+// Decodes requests whose dst / pitch are host arrays of images[i].row bytes by
+// images[i].rows.  chunk: decode in pipelined chunks of so many tiles (0: one
+// plan).
+Status decode_to_host(sgn_hip_session *s, const sgn_tile_req *reqs, size_t n,
+                      std::vector<HostImage> images, int mode, size_t chunk, size_t *first_fail) {
+    HIP_TRY(hipSetDevice(s->device));
+    std::vector<sgn_tile_req> dev(reqs, reqs + n);
+    size_t total = 0;
+    for (size_t i = 0; i < n; ++i) {
+        images[i].off = total;
+        total = (total + images[i].row * images[i].rows + 255) & ~size_t(255);
+    }
+    CachedBlock out{s->blocks};
+    if (s->blocks->get(std::max<size_t>(1, total), &out.p) != hipSuccess) {
+        out.p = nullptr;
+        set_last_error("hipMalloc failed for the output (" + std::to_string(total) + " bytes)");
+        return kErrDevice;
+    }
+    StreamDone done{s};
+    for (size_t i = 0; i < n; ++i) {
+        dev[i].dst = static_cast<uint8_t *>(out.p) + images[i].off;
+        dev[i].pitch = images[i].row;
+        dev[i].capacity = images[i].row * images[i].rows;
+    }
+    HostWriter w(s, static_cast<const uint8_t *>(out.p), std::move(images));
+    Status st;
+    if (chunk) {
+        std::vector<int32_t> ts(n, 0);
+        st = decode_pipelined(s, dev.data(), n, chunk, ts.data(), first_fail);
+        if (!st) st = w.start();
+    } else {
+        st = decode_once(s, dev.data(), n, mode, first_fail, [&] { return w.start(); });
+    }
+    return st ? st : w.finish();
+}
+
 // Uniform-format batch as per-tile requests.
 std::vector<sgn_tile_req> as_requests(const sgn_tile_job *jobs, size_t n, int fmt, uint32_t den) {
     std::vector<sgn_tile_req> r(n);
@@ -1804,9 +1976,9 @@ void sgn_hip_session_destroy(sgn_hip_session *s) {
             (void)hipStreamSynchronize(st);
             (void)hipStreamDestroy(st);
         }
-    for (PinnedSlot &sl : s->slot) {
-        if (sl.p) (void)hipHostFree(sl.p);
-        if (sl.done) (void)hipEventDestroy(sl.done);
+    for (PinnedSlot *sl : {&s->slot[0], &s->slot[1], &s->down[0], &s->down[1], &s->stat}) {
+        if (sl->p) (void)hipHostFree(sl->p);
+        if (sl->done) (void)hipEventDestroy(sl->done);
     }
     delete s->blocks;
     if (s->d_tables) (void)hipFree(s->d_tables);
@@ -1885,13 +2057,21 @@ int sgn_device_upload(sgn_hip_session *s, void *dev, const void *host, size_t by
 
 int sgn_device_download_2d(sgn_hip_session *s, void *host, size_t host_stride, const void *dev,
                            size_t dev_pitch, size_t row_bytes, size_t rows) {
+    API_GUARD_BEGIN
     if (!s || !host || !dev) return SGN_E_ARG;
     if (!rows || !row_bytes) return SGN_OK;
     HIP_TRY(hipSetDevice(s->device));
+    if (dev_pitch == row_bytes && host_stride >= row_bytes) {
+        HostWriter w(s, static_cast<const uint8_t *>(dev),
+                     {{static_cast<uint8_t *>(host), host_stride, 0, row_bytes, rows}});
+        const Status st = w.start();
+        return st ? st : w.finish();
+    }
     HIP_TRY(hipMemcpy2DAsync(host, host_stride, dev, dev_pitch, row_bytes, rows,
                              hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipStreamSynchronize(s->stream));
     return SGN_OK;
+    API_GUARD_END
 }
 
 int sgn_host_alloc(size_t bytes, void **out) {
@@ -2182,26 +2362,13 @@ int sgn_j2k_decode_tiles_device(sgn_hip_session *s, const sgn_tile_job *jobs, si
                                 uint32_t den, int mode, size_t *first_fail) {
     API_GUARD_BEGIN
     if (!s || (!jobs && n)) return SGN_E_ARG;
-    std::vector<int32_t> ts(n, 0);
-    std::unique_ptr<sgn_j2k_plan> P;
     const std::vector<sgn_tile_req> reqs = as_requests(jobs, n, fmt, den);
     const size_t chunk = pipeline_tiles();
-    if (mode == SGN_MODE_BATCHED && chunk && n > chunk)
+    if (mode == SGN_MODE_BATCHED && chunk && n > chunk) {
+        std::vector<int32_t> ts(n, 0);
         return decode_pipelined(s, reqs.data(), n, chunk, ts.data(), first_fail);
-    Status st = make_plan(s, reqs.data(), n, P, ts.data());
-    if (st) {
-        if (first_fail)
-            for (size_t i = 0; i < n; ++i)
-                if (ts[i]) {
-                    *first_fail = i;
-                    break;
-                }
-        return st;
     }
-    st = decode_plan(s, *P, mode);
-    if (st) return st;
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    return check_status(*P, mode, first_fail);
+    return decode_once(s, reqs.data(), n, mode, first_fail, [] { return kOk; });
     API_GUARD_END
 }
 
@@ -2248,22 +2415,43 @@ int sgn_j2k_decode_tiles_region_device(sgn_hip_session *s, const sgn_tile_req *r
                                        size_t *first_fail) {
     API_GUARD_BEGIN
     if (!s || (!reqs && n)) return SGN_E_ARG;
-    std::vector<int32_t> ts(n, 0);
-    std::unique_ptr<sgn_j2k_plan> P;
-    Status st = make_plan(s, reqs, n, P, ts.data());
-    if (st) {
-        if (first_fail)
-            for (size_t i = 0; i < n; ++i)
-                if (ts[i]) {
-                    *first_fail = i;
-                    break;
-                }
-        return st;
+    return decode_once(s, reqs, n, SGN_MODE_BATCHED, first_fail, [] { return kOk; });
+    API_GUARD_END
+}
+
+int sgn_j2k_decode_reqs_into(sgn_hip_session *s, const sgn_tile_req *reqs, size_t n, int mode,
+                             size_t *first_fail) {
+    API_GUARD_BEGIN
+    if (!s || (!reqs && n)) return SGN_E_ARG;
+    std::vector<HostImage> images(n);
+    bool regions = false, usable = true;
+    for (size_t i = 0; i < n; ++i) {
+        const sgn_tile_req &q = reqs[i];
+        static const uint32_t kPixelBytes[5] = {1, 3, 4, 2, 6};
+        if (q.fmt < 0 || q.fmt > 4) return SGN_E_ARG;
+        uint32_t x, y, w, h;
+        const int rc = q.has_roi ? sgn_j2k_region_dims(q.bytes, q.len, q.denominator, q.roi_x, q.roi_y,
+                                                       q.roi_w, q.roi_h, &x, &y, &w, &h)
+                                 : sgn_j2k_scaled_dims(q.bytes, q.len, q.denominator, &w, &h);
+        if (rc) {
+            if (first_fail) *first_fail = i;
+            return rc;
+        }
+        regions |= q.has_roi != 0;
+        const size_t row = size_t(w) * kPixelBytes[q.fmt];
+        images[i] = {static_cast<uint8_t *>(q.dst), q.pitch, 0, row, h};
+        if (row && h && (!q.dst || q.pitch < row || q.capacity < q.pitch * (h - 1) + row))
+            usable = false;
     }
-    st = decode_plan(s, *P, SGN_MODE_BATCHED);
-    if (st) return st;
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    return check_status(*P, SGN_MODE_BATCHED, first_fail);
+    if (!usable) {
+        if (first_fail) *first_fail = SIZE_MAX;
+        set_last_error("output buffer too small");
+        return SGN_E_BUFFER;
+    }
+    if (!n) return SGN_OK;
+    const size_t chunk = pipeline_tiles();
+    const bool pipelined = !regions && mode == SGN_MODE_BATCHED && chunk && n > chunk;
+    return decode_to_host(s, reqs, n, std::move(images), mode, pipelined ? chunk : 0, first_fail);
     API_GUARD_END
 }
 
@@ -2296,17 +2484,9 @@ int sgn_j2k_decode_region_into(sgn_hip_session *s, const uint8_t *bytes, size_t 
         return SGN_E_BUFFER;
     }
     if (!rw || !rh) return SGN_OK;
-    HIP_TRY(hipSetDevice(s->device));
-    void *d = nullptr;
-    HIP_TRY(hipMalloc(&d, row * rh));
-    int rc = sgn_j2k_decode_region_device(s, bytes, len, fmt, den, x, y, w, h, d, row, row * rh);
-    if (rc == SGN_OK &&
-        hipMemcpy2D(out, stride, d, row, row, rh, hipMemcpyDeviceToHost) != hipSuccess) {
-        set_last_error("download failed");
-        rc = SGN_E_DEVICE;
-    }
-    (void)hipFree(d);
-    return rc;
+    const sgn_tile_req r{bytes, len, out, stride, out_len, fmt, den, 1u, x, y, w, h};
+    size_t ff = 0;
+    return decode_to_host(s, &r, 1, {{out, stride, 0, row, rh}}, SGN_MODE_BATCHED, 0, &ff);
     API_GUARD_END
 }
 
@@ -2334,20 +2514,10 @@ int sgn_j2k_decode_into(sgn_hip_session *s, const uint8_t *bytes, size_t len, in
         set_last_error("output buffer too small");
         return SGN_E_BUFFER;
     }
-    HIP_TRY(hipSetDevice(s->device));
-    void *d = nullptr;
-    const size_t bytes_dev = std::max<size_t>(1, og.row_bytes * og.height);
-    HIP_TRY(hipMalloc(&d, bytes_dev));
-    int rc = sgn_j2k_decode_device(s, bytes, len, fmt, den, d, og.row_bytes, bytes_dev);
-    if (rc == SGN_OK && og.height) {
-        if (hipMemcpy2D(out, stride, d, og.row_bytes, og.row_bytes, og.height,
-                        hipMemcpyDeviceToHost) != hipSuccess) {
-            set_last_error("download failed");
-            rc = SGN_E_DEVICE;
-        }
-    }
-    (void)hipFree(d);
-    return rc;
+    const sgn_tile_req r{bytes, len, out, stride, out_len, fmt, den};
+    size_t ff = 0;
+    return decode_to_host(s, &r, 1, {{out, stride, 0, og.row_bytes, og.height}}, SGN_MODE_BATCHED, 0,
+                          &ff);
     API_GUARD_END
 }
 
