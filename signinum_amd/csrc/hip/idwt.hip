@@ -1122,15 +1122,15 @@ sgn_final_rev(const FinalJob *jobs, uint32_t njobs, uint32_t block_offset,
                               block_job, lv, coef, nullptr, nullptr);
 }
 
-// 5/3 final stage with int16 component planes.  *redo_n must be zero at
-// launch; blocks with a sample outside the int16 range are listed in `redo`
+// 5/3 final stage with int16 component planes, of the blocks in `list` (null:
+// the launch's own numbers).  *redo_n must be zero at launch; blocks with a sample outside the int16 range are listed in `redo`
 // (capacity: the launch's block count) for sgn_final_rev_redo.
 extern "C" __global__ void __launch_bounds__(kIdwtThreads)
-sgn_final_rev16(const FinalJob *jobs, uint32_t njobs, uint32_t block_offset,
-                const uint32_t *block_job, const LevelJob *lv, const uint32_t *coef,
-                uint32_t *redo, uint32_t *redo_n) {
-    final_body<true, int16_t>(jobs, njobs, xcd_remap(blockIdx.x, gridDim.x) + block_offset,
-                              block_job, lv, coef, redo, redo_n);
+sgn_final_rev16(const FinalJob *jobs, uint32_t njobs, const uint32_t *list,
+                uint32_t block_offset, const uint32_t *block_job, const LevelJob *lv,
+                const uint32_t *coef, uint32_t *redo, uint32_t *redo_n) {
+    const uint32_t i = xcd_remap(blockIdx.x, gridDim.x) + block_offset;
+    final_body<true, int16_t>(jobs, njobs, list ? list[i] : i, block_job, lv, coef, redo, redo_n);
 }
 
 // The blocks sgn_final_rev16 listed, with int32 planes; a fixed grid walks

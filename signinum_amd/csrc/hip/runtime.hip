@@ -32,6 +32,7 @@
 #include "ht_coop.hip"
 #include "ht_split.hip"
 #include "idwt.hip"
+#include "final_rgb8.hip"
 #include "t1_classic.hip"
 #include "packets.hpp"
 #include "cost_model.hip"
@@ -312,6 +313,8 @@ struct sgn_j2k_plan {
     std::vector<FinalJob> fin[2];
     // work-group (64x64 output block) -> index of its job in lv[rev] / fin[rev]
     std::vector<uint32_t> lv_block_job[2], fin_block_job[2];
+    // 5/3 final blocks of tiles that sgn_final_rgb8 decodes, and the others
+    std::vector<uint32_t> fin_rgb8, fin_rest;
     std::vector<std::pair<uint8_t, uint32_t>> tile_final_first;  // (rev, first index)
     std::vector<uint32_t> tile_final_count;
     std::vector<uint32_t> tile_width, tile_height;
@@ -346,6 +349,7 @@ struct sgn_j2k_plan {
     LevelJob *d_final_lv = nullptr;
     FinalJob *d_fin[2] = {nullptr, nullptr};
     uint32_t *d_lv_block_job[2] = {nullptr, nullptr}, *d_fin_block_job[2] = {nullptr, nullptr};
+    uint32_t *d_fin_rgb8 = nullptr, *d_fin_rest = nullptr;
     uint32_t *d_fin_redo = nullptr;  // 5/3 final blocks left to the int32-plane pass
     uint8_t *d_status_lane = nullptr, *d_status_wave = nullptr;
     uint32_t *d_queue = nullptr;  // count of d_fin_redo
@@ -583,6 +587,28 @@ void parse_batch(const sgn_tile_req *reqs, size_t n, ParsedBatch &B, int32_t *ti
     }
     B.t_parse = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0)
                     .count();
+}
+
+// Whether sgn_final_rgb8 takes a 5/3 final job (besides its bit-planes): whole
+// 8-bit RGB tiles under RCT whose components share an even origin, with int16
+// high-pass bands on 16-byte boundaries.
+bool rgb8_final(const FinalJob &fj, const std::vector<LevelJob> &lv) {
+    if (!fj.reversible || fj.ncomp != 3 || !fj.mct || !fj.same8 || fj.fmt != SGN_RGB8 || fj.cx0 ||
+        fj.cy0 || fj.cx1 != fj.width || fj.cy1 != fj.height)
+        return false;
+    const LevelJob &a = lv[fj.level[0]];
+    if ((a.x0 | a.y0) & 1u || a.x1 - a.x0 < 8 || a.y1 - a.y0 < 8) return false;
+    for (int c = 0; c < 3; ++c) {
+        const LevelJob &l = lv[fj.level[c]];
+        if (l.x0 != a.x0 || l.y0 != a.y0 || l.x1 != a.x1 || l.y1 != a.y1 || !l.levels ||
+            !l.reversible || l.lift53 || (l.narrow & 0xEu) != 0xEu)
+            return false;
+        for (int b = 0; b < 4; ++b) {
+            const int sh = ((l.narrow >> b) & 1u) ? 1 : 2;
+            if (((uint64_t(l.band[b]) << sh) | (uint64_t(l.bw[b]) << sh)) & 15u) return false;
+        }
+    }
+    return true;
 }
 
 // Merges the parsed tiles into the batch tables.  pool: fill the code-block
@@ -918,6 +944,21 @@ Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
             P.tile_final_count[i]++;
         }
     }
+    // blocks of the 16-bit RGB final stage
+    {
+        P.fin_rgb8.clear();
+        P.fin_rest.clear();
+        for (size_t i = 0, k = 0; i < n; ++i)
+            for (size_t f = 0; f < lps[i].finals.size(); ++f) {
+                if (!lps[i].finals[f].reversible) continue;
+                const FinalJob &fj = P.fin[1][k++];
+                std::vector<uint32_t> &to =
+                    P.narrow && lps[i].max_k <= 11 && rgb8_final(fj, P.final_lv) ? P.fin_rgb8
+                                                                                 : P.fin_rest;
+                for (uint32_t b = 0; b < uint32_t(fj.nbx) * fj.nby; ++b)
+                    to.push_back(fj.block_base + b);
+            }
+    }
     // block -> job tables: one load per work-group instead of a search
     for (int rev = 0; rev < 2; ++rev) {
         P.lv_block_job[rev].clear();
@@ -1023,6 +1064,7 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
     const uint64_t o_pkt = take(bytes_of(P.pk_tiles)), o_pkp = take(bytes_of(P.pk_parts));
     const uint64_t o_pkk = take(bytes_of(P.pk_pkts)), o_pkb = take(bytes_of(P.pk_bands));
     const uint64_t o_pkc = take(bytes_of(P.pk_cbs)), o_grp = take(bytes_of(P.groups));
+    const uint64_t o_frg = take(bytes_of(P.fin_rgb8)), o_frs = take(bytes_of(P.fin_rest));
     const uint64_t host_bytes = off;
     const uint64_t o_pkn = take(P.pk_nodes * 2 * sizeof(uint32_t));
     const uint64_t o_pkl = take(P.pk_cbs.size() * sizeof(uint32_t)), o_pks = take(P.pk_tiles.size());
@@ -1099,6 +1141,8 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
         HIP_TRY(put_dev(o_pkb, P.pk_bands));
         HIP_TRY(put_dev(o_pkc, P.pk_cbs));
         HIP_TRY(put_dev(o_grp, P.groups));
+        HIP_TRY(put_dev(o_frg, P.fin_rgb8));
+        HIP_TRY(put_dev(o_frs, P.fin_rest));
         HIP_TRY(hipStreamSynchronize(copy));
         P.t_stage = 0;
         P.t_copy = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() -
@@ -1164,6 +1208,8 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
         put(o_pkb, P.pk_bands);
         put(o_pkc, P.pk_cbs);
         put(o_grp, P.groups);
+        put(o_frg, P.fin_rgb8);
+        put(o_frs, P.fin_rest);
         const auto t1 = std::chrono::steady_clock::now();
         uint8_t *d = static_cast<uint8_t *>(P.d_block);
         // direct runs first, then the staged range: consecutive staged runs and
@@ -1241,6 +1287,8 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
     at(o_queue, P.d_queue, true);
     at(o_coef, P.d_coef, P.coef_elems != 0);
     at(o_grp, P.d_groups, !P.groups.empty());
+    at(o_frg, P.d_fin_rgb8, !P.fin_rgb8.empty());
+    at(o_frs, P.d_fin_rest, !P.fin_rest.empty());
     at(o_work, P.d_work, has_work);
     P.work_cap = has_work ? P.work_units : 0;
     return kOk;
@@ -1394,12 +1442,27 @@ uint32_t launch_finals(sgn_hip_session *s, sgn_j2k_plan &P, int rev, uint32_t a,
         // the blocks it listed (d_queue counts them; cleared by a kernel,
         // graph-safe)
         uint32_t *redo_n = P.d_queue;
-        const uint32_t k = 3;
+        uint32_t k = 3;
         hipLaunchKernelGGL(sgn_fill_bytes, dim3(1), dim3(64), 0, s->stream,
                            reinterpret_cast<uint8_t *>(redo_n), size_t(4), size_t(1), 0u);
-        hipLaunchKernelGGL(sgn_final_rev16, dim3(blocks), dim3(kIdwtThreads), 0, s->stream,
-                           P.d_fin[1], uint32_t(P.fin[1].size()), off, P.d_fin_block_job[1],
-                           P.d_final_lv, P.d_coef, P.d_fin_redo, redo_n);
+        uint32_t rest = blocks;
+        const uint32_t *list = nullptr;
+        if (blocks == P.fin_block_job[1].size()) {  // the whole plan: by kernel
+            if (!P.fin_rgb8.empty()) {
+                hipLaunchKernelGGL(sgn_final_rgb8, dim3(P.fin_rgb8.size()), dim3(kIdwtThreads), 0,
+                                   s->stream, P.d_fin[1], P.d_fin_rgb8, P.d_fin_block_job[1],
+                                   P.d_final_lv, P.d_coef, P.d_fin_redo, redo_n);
+                ++k;
+            }
+            rest = static_cast<uint32_t>(P.fin_rest.size());
+            list = P.d_fin_rest;
+        }
+        if (rest)
+            hipLaunchKernelGGL(sgn_final_rev16, dim3(rest), dim3(kIdwtThreads), 0, s->stream,
+                               P.d_fin[1], uint32_t(P.fin[1].size()), list, off,
+                               P.d_fin_block_job[1], P.d_final_lv, P.d_coef, P.d_fin_redo, redo_n);
+        else
+            --k;
         const uint32_t cus = s->cus ? uint32_t(s->cus) : 256u;
         hipLaunchKernelGGL(sgn_final_rev_redo, dim3(std::min(blocks, 2 * cus)), dim3(kIdwtThreads),
                            0, s->stream, P.d_fin[1], uint32_t(P.fin[1].size()),
