@@ -130,6 +130,91 @@ __device__ __forceinline__ void wave_lds_fence() {
 
 constexpr uint32_t kCleanRing = 64;  // dwords of a block's ring: a partly filled unit and a round's 33
 
+// A plain bit string that a row of lanes writes to a block's interleaved
+// units, 128 bytes of stream a round, through a ring of words in LDS that whole
+// units leave.  Every byte is ORed in at its place.
+struct PlainString {
+    uint32_t *buf;  // kCleanRing words, 16-byte aligned
+    uint32_t q;     // lane of the row
+    uint4 *d;       // unit 0
+    uint32_t units, fill, done;
+
+    __device__ __forceinline__ PlainString(uint32_t *b, uint32_t lane, uint4 *out, uint32_t n,
+                                           uint32_t head, uint32_t bits)
+        : buf(b), q(lane), d(out), units(n), fill(bits), done(0) {
+        if (q < 4) buf[q] = q == 0 ? head : 0u;
+    }
+    // This lane's n0 and n1 next bits (25 to 32 each; a value may reach one bit
+    // past its count).  Called by all lanes; rows that are not `act` sit out.
+    __device__ __forceinline__ void round(bool act, uint32_t v0, uint32_t n0, uint32_t v1,
+                                          uint32_t n1) {
+        const uint32_t incl = row_scan(n0 + n1), tot = row_last(incl);
+        if (act) {
+            const uint32_t z = (fill >> 5) + 1 + q;
+            buf[z & (kCleanRing - 1)] = 0;
+            buf[(z + 16) & (kCleanRing - 1)] = 0;
+        }
+        wave_lds_fence();
+        if (act) {
+            // the lane's 50 to 64 bits: three words at most
+            const uint64_t v = (uint64_t)v0 | ((uint64_t)v1 << n0);
+            const uint32_t pos = fill + incl - (n0 + n1), wi = pos >> 5, sh = pos & 31u;
+            const uint64_t a = v << sh;
+            const uint32_t x2 = sh ? (uint32_t)(v >> 32) >> (32u - sh) : 0u;
+            if ((uint32_t)a) atomicOr(&buf[wi & (kCleanRing - 1)], (uint32_t)a);
+            if ((uint32_t)(a >> 32))
+                atomicOr(&buf[(wi + 1) & (kCleanRing - 1)], (uint32_t)(a >> 32));
+            if (x2) atomicOr(&buf[(wi + 2) & (kCleanRing - 1)], x2);
+            fill += tot;
+        }
+        wave_lds_fence();
+        // whole units (at most 9 a round; the padding of the last round's
+        // bytes may reach past the string's last unit)
+        const uint32_t full = min(fill >> 7, units), u = done + q;
+        if (act && u < full)
+            d[kHtGroup * u] = *reinterpret_cast<uint4 *>(&buf[4 * u & (kCleanRing - 1)]);
+        done = act ? full : done;
+    }
+    // The partly filled unit, then zeros up to and with unit `units`
+    // (seven-bit bytes leave the string short of it).
+    __device__ __forceinline__ void finish() {
+        const uint32_t last = fill >> 5;
+        for (uint32_t u = done + q; u <= units; u += kSplitLanes) {
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (u < units) {
+                const uint32_t *x = &buf[4 * u & (kCleanRing - 1)];
+                v.x = 4 * u <= last ? x[0] : 0u;
+                v.y = 4 * u + 1 <= last ? x[1] : 0u;
+                v.z = 4 * u + 2 <= last ? x[2] : 0u;
+                v.w = 4 * u + 3 <= last ? x[3] : 0u;
+            }
+            d[kHtGroup * u] = v;
+        }
+    }
+};
+
+// Stream bytes that carry 7 bits (bit 0 of each byte of s) close up: the
+// dword's bits from bit 0, and their count.
+__device__ __forceinline__ uint32_t close_up(uint32_t d, uint32_t s, uint32_t &bits) {
+    // running counts, a byte each
+    uint32_t c = s + (s << 8);
+    c += c << 16;
+    bits = 32u - (c >> 24);
+    return (d & 0xFFu) | ((d & 0xFF00u) >> (c & 31u)) | ((d & 0xFF0000u) >> ((c >> 8) & 31u)) |
+           ((d & 0xFF000000u) >> ((c >> 16) & 31u));
+}
+// Bit 7 of every byte of d that is 0xFF.
+__device__ __forceinline__ uint32_t bytes_ff(uint32_t d) {
+    return ((d & 0x7F7F7F7Fu) + 0x01010101u) & d & 0x80808080u;
+}
+// Bit 7 of every byte above 0x8F, and of every byte whose low 7 bits are ones.
+__device__ __forceinline__ uint32_t bytes_above(uint32_t d) {
+    return ((d & 0x7F7F7F7Fu) + 0x70707070u) & d & 0x80808080u;
+}
+__device__ __forceinline__ uint32_t bytes_7f(uint32_t d) {
+    return ((d & 0x7F7F7F7Fu) + 0x01010101u) & 0x80808080u;
+}
+
 // The VLC string of one block per row: two zero bits, the 3 or 4 bits of the
 // segment's second last byte, and from there it runs backward from the byte before; a byte
 // whose low 7 bits are ones after a byte > 0x8F carries 7 bits, and is ORed in
@@ -188,80 +273,28 @@ sgn_ht_clean(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restri
     const uint32_t len = scup ? scup - 2 : 0;
     const uint32_t units = (6 + 8 * len + 127) >> 7;  // 16-byte units that hold stream bits
     const uint32_t first = b0 >> 4;
-    uint32_t fill = 6u - ((first & 7u) == 7u ? 1u : 0u);  // two bits in front
+    // two bits in front
+    PlainString str(buf, q, w.vlc, units, first << 2, 6u - ((first & 7u) == 7u ? 1u : 0u));
     uint32_t carry = b0 | 0x0Fu;  // the byte before this round's
-    if (q < 4) buf[q] = q == 0 ? first << 2 : 0u;
-    uint4 *d = w.vlc;
-    uint32_t done = 0;  // units written
 
-    // one dword of stream bytes (the first in bits 0..7), `g`: bit 7 of a byte
-    // set where it is above 0x8F, `pg`: the same of the dword before
-    auto pack = [](uint32_t d, uint32_t g, uint32_t pg, uint32_t &bits) -> uint32_t {
-        const uint32_t f = ((d & 0x7F7F7F7Fu) + 0x01010101u) & __builtin_amdgcn_alignbit(g, pg, 24) &
-                           0x80808080u;
-        const uint32_t o1 = 8u - ((f >> 7) & 1u), o2 = o1 + 8u - ((f >> 15) & 1u),
-                       o3 = o2 + 8u - ((f >> 23) & 1u);
-        bits = o3 + 8u - (f >> 31);
-        return (d & 0xFFu) | (((d >> 8) & 0xFFu) << o1) | (((d >> 16) & 0xFFu) << o2) |
-               ((d >> 24) << o3);
-    };
-    auto above = [](uint32_t d) {  // bit 7 of every byte above 0x8F
-        return ((d & 0x7F7F7F7Fu) + 0x70707070u) & d & 0x80808080u;
-    };
     for (uint32_t at = 0; __any(at < len); at += 128) {
         const uint32_t k0 = at + 8 * q;
         uint32_t d0 = __builtin_bswap32(hi), d1 = __builtin_bswap32(lo);
         if (k0 + 4 > len) d0 &= k0 < len ? 0xFFFFFFFFu >> (8 * (4 - (len - k0))) : 0u;
         if (k0 + 8 > len) d1 &= k0 + 4 < len ? 0xFFFFFFFFu >> (8 * (8 - (len - k0))) : 0u;
         fetch(k0 + 128, len);
-        const uint32_t g0 = above(d0), g1 = above(d1);
+        const uint32_t g0 = bytes_above(d0), g1 = bytes_above(d1);
         uint32_t pg = row_dpp<0x111>(g1);
         if (q == 0) pg = carry > 0x8Fu ? 0x80000000u : 0u;
         carry = row_last(d1 >> 24);
         uint32_t n0, n1;
-        const uint32_t v0 = pack(d0, g0, pg, n0), v1 = pack(d1, g1, g0, n1);
-        const uint32_t incl = row_scan(n0 + n1), tot = row_last(incl);
-        if (at < len) {
-            const uint32_t z = (fill >> 5) + 1 + q;
-            buf[z & (kCleanRing - 1)] = 0;
-            buf[(z + 16) & (kCleanRing - 1)] = 0;
-        }
-        wave_lds_fence();
-        if (at < len) {
-            // the lane's 50 to 64 bits: three words at most
-            const uint64_t v = (uint64_t)v0 | ((uint64_t)v1 << n0);
-            const uint32_t pos = fill + incl - (n0 + n1), wi = pos >> 5, sh = pos & 31u;
-            const uint64_t a = v << sh;
-            const uint32_t x2 = sh ? (uint32_t)(v >> 32) >> (32u - sh) : 0u;
-            if ((uint32_t)a) atomicOr(&buf[wi & (kCleanRing - 1)], (uint32_t)a);
-            if ((uint32_t)(a >> 32))
-                atomicOr(&buf[(wi + 1) & (kCleanRing - 1)], (uint32_t)(a >> 32));
-            if (x2) atomicOr(&buf[(wi + 2) & (kCleanRing - 1)], x2);
-            fill += tot;
-        }
-        wave_lds_fence();
-        // whole units (at most 9 a round; the padding of the last round's
-        // bytes may reach past the string's last unit)
-        const uint32_t full = min(fill >> 7, units), u = done + q;
-        if (at < len && u < full) d[kHtGroup * u] = *reinterpret_cast<uint4 *>(&buf[4 * u & (kCleanRing - 1)]);
-        done = at < len ? full : done;
+        const uint32_t v0 =
+            close_up(d0, (bytes_7f(d0) & __builtin_amdgcn_alignbit(g0, pg, 24)) >> 7, n0);
+        const uint32_t v1 =
+            close_up(d1, (bytes_7f(d1) & __builtin_amdgcn_alignbit(g1, g0, 24)) >> 7, n1);
+        str.round(at < len, v0, n0, v1, n1);
     }
-    if (scup) {
-        // the partly filled unit, then zeros (seven-bit bytes leave the string
-        // short of `units`)
-        const uint32_t last = fill >> 5;
-        for (uint32_t u = done + q; u <= units; u += kSplitLanes) {
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (u < units) {
-                const uint32_t *x = &buf[4 * u & (kCleanRing - 1)];
-                v.x = 4 * u <= last ? x[0] : 0u;
-                v.y = 4 * u + 1 <= last ? x[1] : 0u;
-                v.z = 4 * u + 2 <= last ? x[2] : 0u;
-                v.w = 4 * u + 3 <= last ? x[3] : 0u;
-            }
-            d[kHtGroup * u] = v;
-        }
-    }
+    if (scup) str.finish();
     if (valid && q == 0) *reinterpret_cast<HtHead *>(w.head) = HtHead{units, scup, bad, 0};
 }
 
@@ -686,27 +719,13 @@ sgn_ht_magsgn(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restr
                     next += 128;
                     if (next < end) __builtin_memcpy(&raw, arena + next, 8);
                 }
-                // bit 7 of every byte that is 0xFF, and of every byte after one
-                auto ff = [](uint32_t d) {
-                    return ((d & 0x7F7F7F7Fu) + 0x01010101u) & d & 0x80808080u;
-                };
-                const uint32_t f0 = ff(d0), f1 = ff(d1);
+                // bytes that are 0xFF, and those after one
+                const uint32_t f0 = bytes_ff(d0), f1 = bytes_ff(d1);
                 uint32_t pf = row_dpp<0x111>(f1);
                 if (q == 0) pf = prev;
-                const uint32_t s0 = __builtin_amdgcn_alignbit(f0, pf, 24) >> 7,
-                               s1 = __builtin_amdgcn_alignbit(f1, f0, 24) >> 7;
-                // the bytes of a dword moved down by the seven-bit bytes
-                // before them (running counts, a byte each)
-                auto pack = [](uint32_t d, uint32_t s, uint32_t &bits) {
-                    uint32_t c = s + (s << 8);
-                    c += c << 16;
-                    bits = 32u - (c >> 24);
-                    return (d & 0xFFu) | ((d & 0xFF00u) >> (c & 31u)) |
-                           ((d & 0xFF0000u) >> ((c >> 8) & 31u)) |
-                           ((d & 0xFF000000u) >> ((c >> 16) & 31u));
-                };
                 uint32_t n0, n1;
-                const uint32_t v0 = pack(d0, s0, n0), v1 = pack(d1, s1, n1);
+                const uint32_t v0 = close_up(d0, __builtin_amdgcn_alignbit(f0, pf, 24) >> 7, n0);
+                const uint32_t v1 = close_up(d1, __builtin_amdgcn_alignbit(f1, f0, 24) >> 7, n1);
                 const uint32_t sc = row_scan(n0 + n1), bits = row_last(sc), last = row_last(f1);
                 const uint32_t wz = (fill >> 5) + 1 + q;
                 if (act) {
@@ -826,9 +845,346 @@ sgn_ht_magsgn(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restr
 }
 
 // ---- refinement passes ---------------------------------------------------------
+//
+// SigProp (ht_block_decode.rs:1254-1374) is a serial chain per block, over
+// significance alone; what it finds and the MagRef bits are then applied to all
+// samples in parallel.  After the cleanup a sample is significant exactly when
+// it is nonzero (ht_refine.hpp).  Three kernels as for the cleanup; one lane
+// per block doing everything, samples included, took 1290 us for 512 tiles of
+// 256x256 with both passes in every block; prepare 69, chain 123 and apply 121
+// us do the same (the two parallel ones move 200 and 400 MB of samples in rows
+// of up to 128 bytes, the chain issues about 12 instructions a sample).
 
-// SigProp / MagRef passes of the code-blocks jobs[0 .. n) (each with more
-// than one pass, at most 64x64), one block per lane, after the
+// A refined block's part of its group's workspace; pass count rules of
+// decode_impl (:1578-1592).
+struct RefWork {
+    uint4 *cs, *out, *sp;
+};
+__device__ __forceinline__ RefWork ref_work(uint4 *work, const RefGroup *groups, uint32_t i) {
+    const RefGroup g = groups[i / kHtGroup];
+    RefWork w;
+    w.cs = work + g.base + i % kHtGroup;
+    w.out = w.cs + size_t(kHtGroup) * 2 * g.stripes;
+    w.sp = w.out + size_t(kHtGroup) * 4 * g.stripes;
+    return w;
+}
+__device__ __forceinline__ bool ref_runs(const CbJob &j) {
+    return !(j.flags & kCbZero) && j.passes >= 2 && j.passes <= 3 && j.lref != 0 && j.zblk < 29 &&
+           j.lcup >= 2 && j.w <= 64 && j.h <= 64;
+}
+
+// Significance of the cleanup (16 bits per group of 4x4 samples, bit 4 column +
+// row; two groups a dword) and the plain SigProp bits: LSB-first, 7 bits after
+// 0xFF, zeros past the end.  One block per DPP row, a group a lane.
+template <typename C>
+__global__ void __launch_bounds__(kSplitWaves * 64)
+sgn_ht_refine_prep(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restrict__ arena,
+                   const C *__restrict__ coef, const RefGroup *__restrict__ groups,
+                   uint4 *__restrict__ work) {
+    __shared__ __attribute__((aligned(16))) uint32_t s_buf[kSplitBlocks][kCleanRing];
+    const uint32_t row = threadIdx.x / kSplitLanes, q = threadIdx.x % kSplitLanes;
+    const uint32_t i = blockIdx.x * kSplitBlocks + row;
+    CbJob j{};
+    if (i < n) j = jobs[i];
+    const bool on = i < n && ref_runs(j);
+    const RefWork w = ref_work(work, groups, i < n ? i : 0);
+    // SigProp bytes, eight a lane
+    const uint32_t len = on ? min((uint32_t)j.lref, kRefSpBytes) : 0;
+    const uint8_t *src = arena + j.src + j.lcup;
+    PlainString str(s_buf[row], q, w.sp, (8 * len + 127) >> 7, 0, 0);
+    uint32_t prev = 0;
+    for (uint32_t at = 0; __any(at < len); at += 128) {
+        const uint32_t k = at + 8 * q;
+        uint2 d = make_uint2(0, 0);
+        if (k < len) {
+            __builtin_memcpy(&d, src + k, 8);
+            const uint32_t have = (uint32_t)j.lref - k;  // the rest are not of the segment
+            if (have < 8) d.y &= have > 4 ? 0xFFFFFFFFu >> (8 * (8 - have)) : 0u;
+            if (have < 4) d.x &= 0xFFFFFFFFu >> (8 * (4 - have));
+        }
+        const uint32_t f0 = bytes_ff(d.x), f1 = bytes_ff(d.y);
+        uint32_t pf = row_dpp<0x111>(f1);
+        if (q == 0) pf = prev;
+        prev = row_last(f1);
+        uint32_t n0, n1;
+        const uint32_t v0 = close_up(d.x, __builtin_amdgcn_alignbit(f0, pf, 24) >> 7, n0);
+        const uint32_t v1 = close_up(d.y, __builtin_amdgcn_alignbit(f1, f0, 24) >> 7, n1);
+        str.round(at < len, v0, n0, v1, n1);
+    }
+    if (on) str.finish();
+    // significance
+    const bool vec = ((j.dst | j.stride) & 3u) == 0;
+    const C *out = coef + j.dst;
+    const uint32_t stripes = on ? (j.h + 3u) >> 2 : 0;
+    uint16_t *cs = reinterpret_cast<uint16_t *>(w.cs + kHtGroup * (q >> 3)) + (q & 7u);
+    for (uint32_t s = 0; s < stripes; ++s) {
+        int32_t v[4][4];
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r)
+            refine_load<C>(v[r], out, 4 * s + r, 4 * q, j.w, j.h, j.stride, vec);
+        cs[s * (kHtGroup * 16)] = (uint16_t)group_sig(v);
+    }
+}
+
+// SigProp of one block per lane: per group the samples that become
+// significant and the 16 stream bits that their signs start.  The bits come
+// through an LDS ring as in sgn_ht_symbols: four groups take at most 128.
+// Full waves, unlike the symbol chain: every lane issues the same instructions
+// for every group, so half-filled waves gain nothing at 38000 blocks (125
+// against 124 us) and lose at 150000 (341 against 200 us).
+__global__ void __launch_bounds__(kSplitWaves * 64)
+sgn_ht_sigprop(const CbJob *__restrict__ jobs, uint32_t n, const RefGroup *__restrict__ groups,
+               uint4 *__restrict__ work) {
+    __shared__ uint32_t s_ring[kSplitWaves][17][64];
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const uint32_t i = blockIdx.x * kSplitWaves * 64 + threadIdx.x;
+    const bool valid = i < n;
+    uint32_t(*ring)[64] = s_ring[wv];
+    CbJob j{};
+    if (valid) j = jobs[i];
+    const bool on = valid && ref_runs(j);
+    if (!on) j.w = j.h = 0;
+    const RefWork w = ref_work(work, groups, valid ? i : 0);
+    const uint32_t width = j.w, height = j.h, stripes = (height + 3u) >> 2;
+    const uint32_t groups_x = (width + 3u) >> 2;
+    const bool causal = (j.flags & kCbStripeCausal) != 0;
+    const uint32_t last = (8 * min((uint32_t)j.lref, kRefSpBytes) + 127) >> 7;  // zeros from here
+    auto unit = [&](uint32_t u) -> uint4 { return w.sp[kHtGroup * min(u, last)]; };
+    auto put = [&](uint32_t u, const uint4 &v) {
+        const uint32_t s = (u & 3u) * 4u;
+        ring[s + 0][lane] = v.x;
+        ring[s + 1][lane] = v.y;
+        ring[s + 2][lane] = v.z;
+        ring[s + 3][lane] = v.w;
+        ring[s ? s : 16u][lane] = v.x;
+    };
+    uint4 pend = make_uint4(0, 0, 0, 0);
+    uint32_t res = 4, pos = 0;
+    uint32_t cur[9], nxt[9], bot[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) cur[k] = nxt[k] = bot[k] = 0;
+    auto load_cs = [&](uint32_t s, uint32_t (&c)[9]) {
+        const uint4 a = w.cs[kHtGroup * (2 * s)], b = w.cs[kHtGroup * (2 * s + 1)];
+        c[0] = a.x, c[1] = a.y, c[2] = a.z, c[3] = a.w;
+        c[4] = b.x, c[5] = b.y, c[6] = b.z, c[7] = b.w;
+    };
+    if (on) {
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) put(k, unit(k));
+        pend = unit(4);
+        load_cs(0, nxt);
+    }
+    for (uint32_t s = 0; __any(s < stripes); ++s) {
+        const bool run = s < stripes;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) cur[k] = nxt[k];
+        if (s + 1 < stripes) {
+            load_cs(s + 1, nxt);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) nxt[k] = 0;
+        }
+        const uint32_t rows = run ? min(4u, height - 4 * s) : 0;
+        const uint32_t pattern = 0x1111u * ((1u << rows) - 1u);
+        uint32_t prev = 0, found[16];
+        uint32_t nbot[8];
+#pragma unroll
+        for (uint32_t g = 0; g < 16; ++g) {
+            found[g] = 0;
+            if ((g & 1u) == 0) nbot[g >> 1] = 0;
+            if (!__any(run && g < groups_x)) continue;
+            if ((g & 3u) == 0 && run && res < (pos >> 7) + 4u) {
+                put(res, pend);
+                ++res;
+                pend = unit(res);
+            }
+            // this group's 16 bits and the next one's
+            auto pair = [&](const uint32_t (&c)[9]) -> uint32_t {
+                return g & 1u ? __builtin_amdgcn_alignbit(c[(g >> 1) + 1], c[g >> 1], 16)
+                              : c[g >> 1];
+            };
+            const uint32_t cs = pair(cur), csa = cs & 0xFFFFu;
+            // the row above as the reference's prev_row_sig holds it (see
+            // rows_refine in ht_refine.hpp), the row below, and the column before
+            uint32_t u = (((g ? cs : bot[0]) >> 3) & 0x1111u) | ((pair(bot) >> 3) & 0x11110000u);
+            if (!causal) u |= (pair(nxt) & 0x11111111u) << 3;
+            uint32_t mbr = cs | ((cs & 0x77777777u) << 1) | ((cs & 0xEEEEEEEEu) >> 1) | u;
+            mbr |= (mbr << 4) | (mbr >> 4) | (prev >> 12);
+            const uint32_t past = 4 * g + 4 > width ? 4 * g + 4 - width : 0u;  // columns past the block
+            const uint32_t inv = run && past < 4 ? ~csa & (pattern >> (4 * past)) : 0u;
+            uint32_t cand = mbr & inv, nsig = 0;
+            const uint32_t k = (pos >> 5) & 15u;
+            uint32_t bits = __builtin_amdgcn_alignbit(ring[k + 1][lane], ring[k][lane], pos & 31u);
+            // All 16 places in order, without a branch: a member takes a bit,
+            // and a one makes the insignificant samples below and in the next
+            // column members too.  A loop over the members alone runs as often
+            // as the fullest group of the wave needs and took 2.9 times as long
+            // (356 against 123 us for 512 tiles of 256x256, two passes in
+            // every block).
+            if (__any(cand)) {
+#pragma unroll
+                for (uint32_t at = 0; at < 16; ++at) {
+                    const uint32_t r = at & 3u, is = (cand >> at) & 1u, hit = bits & is;
+                    const uint32_t nb = (((2u << r) & 0xFu) | ((((7u << r) >> 1) & 0xFu) << 4))
+                                        << (at & ~3u);
+                    cand |= (0u - hit) & (inv & nb);
+                    nsig |= hit << at;
+                    bits >>= is;
+                }
+            }
+            found[g] = nsig | (bits << 16);
+            pos += (uint32_t)__builtin_popcount(cand) + (uint32_t)__builtin_popcount(nsig);
+            const uint32_t comb = nsig | cs;
+            nbot[g >> 1] |= (comb & 0xFFFFu) << (16 * (g & 1u));
+            const uint32_t np = comb | ((comb & 0x7777u) << 1) | ((comb & 0xEEEEu) >> 1);
+            prev = (np | u) & 0xF000u;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) bot[k] = nbot[k];
+        if (run) {
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k)
+                if (4 * k < groups_x)
+                    w.out[kHtGroup * (4 * s + k)] = make_uint4(found[4 * k], found[4 * k + 1],
+                                                               found[4 * k + 2], found[4 * k + 3]);
+        }
+    }
+}
+
+// What SigProp found and the MagRef bits (:1377-1432), applied to the samples:
+// one block per DPP row, a group a lane.  A sample that SigProp found gets the
+// word 3 << (p - 2); MagRef exchanges bit p - 1 of a sample that the cleanup
+// found for its bit and sets the midpoint 1 << (p - 2).  MagRef bits run
+// backward from the segment's last byte with the VLC stuffing rule, zeros past
+// its start, one per such sample in stripe-column order: a group's place is a
+// row scan of the groups' counts (a stripe takes at most 256 bits).
+template <typename C>
+__global__ void __launch_bounds__(kSplitWaves * 64)
+sgn_ht_refine_apply(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restrict__ arena,
+                    C *__restrict__ coef, const RefGroup *__restrict__ groups,
+                    uint4 *__restrict__ work) {
+    constexpr uint32_t kRing = 64;  // dwords: a stripe's 256 bits and a round's 1024 (a power of two)
+    __shared__ uint32_t s_ring[kSplitBlocks][kRing + 1];  // and a copy of the first
+    const uint32_t row = threadIdx.x / kSplitLanes, q = threadIdx.x % kSplitLanes;
+    uint32_t *ring = s_ring[row];
+    const uint32_t i = blockIdx.x * kSplitBlocks + row;
+    CbJob j{};
+    if (i < n) j = jobs[i];
+    const bool on = i < n && ref_runs(j);
+    if (!on) j.w = j.h = 0;
+    const RefWork w = ref_work(work, groups, i < n ? i : 0);
+    const bool mag = on && j.passes > 2;
+    const uint32_t p = 30u - j.zblk, shift = j.kmax >= 31 ? 0u : 31u - j.kmax;
+    const int32_t vnew = on ? (int32_t)((3u << (p - 2)) >> shift) : 0;
+    const uint32_t ref0 = on ? ((1u << (p - 1)) | (1u << (p - 2))) >> shift : 0u;  // MagRef bit 0
+    const uint32_t ref1 = on ? (1u << (p - 2)) >> shift : 0u;                      // MagRef bit 1
+    const bool vec = ((j.dst | j.stride) & 3u) == 0;
+    C *out = coef + j.dst;
+    const uint32_t stripes = (j.h + 3u) >> 2;
+    const uint32_t len = mag ? j.lref : 0, end = j.src + j.lcup + j.lref;
+    uint32_t next = 8 * q, carry = 0x80000000u;  // the first byte counts as after one > 0x8F
+    uint2 raw = make_uint2(0, 0);
+    // bytes next .. next + 7 of the backward stream, the first in bits 0..7
+    auto fetch = [&]() {
+        raw = make_uint2(0, 0);
+        if (next < len) {
+            uint64_t x;
+            const uint32_t e = end - next;  // one past the first
+            if (e >= 8) {
+                __builtin_memcpy(&x, arena + e - 8, 8);
+            } else {
+                __builtin_memcpy(&x, arena, 8);
+                x <<= 8 * (8 - e);
+            }
+            raw.x = __builtin_bswap32((uint32_t)(x >> 32));
+            raw.y = __builtin_bswap32((uint32_t)x);
+            const uint32_t have = len - next;
+            if (have < 8) raw.y &= have > 4 ? 0xFFFFFFFFu >> (8 * (8 - have)) : 0u;
+            if (have < 4) raw.x &= 0xFFFFFFFFu >> (8 * (4 - have));
+        }
+    };
+    fetch();
+    uint32_t fill = 0, pos = 0;
+    if (q == 0) ring[0] = ring[kRing] = 0;
+    const uint32_t *found = reinterpret_cast<const uint32_t *>(w.out + kHtGroup * (q >> 2)) + (q & 3u);
+    for (uint32_t s = 0; __any(s < stripes); ++s) {
+        const bool run = s < stripes && 4 * q < j.w;
+        int32_t v[4][4];
+        uint32_t f = 0;
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[r][c] = 0;
+        if (run) {
+            f = found[s * (kHtGroup * 16)];
+#pragma unroll
+            for (uint32_t r = 0; r < 4; ++r)
+                refine_load<C>(v[r], out, 4 * s + r, 4 * q, j.w, j.h, j.stride, vec);
+        }
+        const uint32_t cs = group_sig(v);
+        const uint32_t cnt = mag ? (uint32_t)__builtin_popcount(cs) : 0u;
+        const uint32_t incl = row_scan(cnt);
+        const uint32_t at = pos + incl - cnt;
+        pos += row_last(incl);
+        while (__any(fill < pos)) {
+            const bool act = fill < pos;
+            const uint32_t g0 = bytes_above(raw.x), g1 = bytes_above(raw.y);
+            uint32_t pg = row_dpp<0x111>(g1);
+            if (q == 0) pg = carry;
+            const uint32_t last = row_last(g1);
+            uint32_t n0, n1;
+            const uint32_t v0 =
+                close_up(raw.x, (bytes_7f(raw.x) & __builtin_amdgcn_alignbit(g0, pg, 24)) >> 7, n0);
+            const uint32_t v1 =
+                close_up(raw.y, (bytes_7f(raw.y) & __builtin_amdgcn_alignbit(g1, g0, 24)) >> 7, n1);
+            const uint32_t sc = row_scan(n0 + n1), bits = row_last(sc);
+            if (act) {
+                next += 128;
+                fetch();
+                const uint32_t z = (fill >> 5) + 1 + q;
+                ring[z & (kRing - 1)] = 0;
+                ring[(z + 16) & (kRing - 1)] = 0;
+            }
+            wave_lds_fence();
+            if (act) {
+                const uint32_t b = fill + sc - (n0 + n1), sh = b & 31u, wa = b >> 5;
+                const uint64_t x = (uint64_t)v0 | ((uint64_t)v1 << n0), y = x << sh;
+                atomicOr(&ring[wa & (kRing - 1)], (uint32_t)y);
+                atomicOr(&ring[(wa + 1) & (kRing - 1)], (uint32_t)(y >> 32));
+                atomicOr(&ring[(wa + 2) & (kRing - 1)], (uint32_t)(x >> 32) >> 1 >> (31u - sh));
+                fill += bits;
+                carry = last;
+            }
+            wave_lds_fence();
+            ring[kRing] = ring[0];
+            wave_lds_fence();
+        }
+        if (!run) continue;
+        const uint32_t wi = (at >> 5) & (kRing - 1);
+        uint32_t mw = __builtin_amdgcn_alignbit(ring[wi + 1], ring[wi], at & 31u);
+        uint32_t nsig = f & 0xFFFFu, sg = f >> 16;
+        const uint32_t refine = mag ? cs : 0u;
+#pragma unroll
+        for (uint32_t k = 0; k < 16; ++k) {
+            int32_t &x = v[k & 3][k >> 2];
+            const uint32_t hit = (refine >> k) & 1u, nw = (nsig >> k) & 1u;
+            const uint32_t m = (uint32_t)(x < 0 ? -x : x) ^ ((mw & 1u) ? ref1 : ref0);
+            const int32_t changed = x < 0 ? -(int32_t)m : (int32_t)m;
+            x = hit ? changed : nw ? ((sg & 1u) ? -vnew : vnew) : x;
+            mw >>= hit;
+            sg >>= nw;
+        }
+        if (refine | nsig) {
+#pragma unroll
+            for (uint32_t r = 0; r < 4; ++r)
+                refine_store<C>(v[r], out, 4 * s + r, 4 * q, j.w, j.h, j.stride, vec);
+        }
+    }
+}
+
+// The same of plans whose packet headers are parsed on the device (the host
+// knows neither which blocks are refined nor their lengths): all passes of the
+// code-blocks jobs[0 .. n), one block per lane, after the
 // cleanup kernels wrote their samples.  A block whose cleanup failed holds zeros or
 // partial samples; the passes keep to its rectangle and its refinement
 // segment whatever the samples, and its status already reports it.

@@ -212,6 +212,22 @@ uint64_t layout_groups(const std::vector<CbJob> &list, bool unknown, std::vector
     return units;
 }
 
+// The same of the refined blocks' list.
+uint64_t layout_refine(const std::vector<CbJob> &list, std::vector<RefGroup> &groups) {
+    uint64_t units = 0;
+    groups.clear();
+    for (size_t a = 0; a < list.size(); a += kHtGroup) {
+        uint32_t sp = 0, ns = 0;
+        for (size_t k = a; k < std::min(a + kHtGroup, list.size()); ++k) {
+            sp = std::max(sp, ref_sp_units(list[k].lref));
+            ns = std::max(ns, (list[k].h + 3u) / 4u);
+        }
+        groups.push_back({static_cast<uint32_t>(units), ns, sp});
+        units += uint64_t(kHtGroup) * (6 * ns + sp);
+    }
+    return units;
+}
+
 struct LevelRange {
     uint8_t rev, depth;
     uint32_t start, count;
@@ -360,6 +376,10 @@ struct sgn_j2k_plan {
     HtGroup *d_groups = nullptr;
     uint4 *d_work = nullptr;  // absent when the plan is carved from memory too small for it
     void *d_work_own = nullptr;
+    std::vector<RefGroup> ref_groups;  // of cb_refine
+    uint64_t ref_units = 0;
+    RefGroup *d_ref_groups = nullptr;
+    uint4 *d_ref_work = nullptr;
     // packet headers parsed on the device (tiles planned with device
     // packets): tables, tag-tree and length scratch, per-tile status; the
     // lane list then keeps the per-tile order (its jobs are filled on the
@@ -870,6 +890,11 @@ Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
     std::stable_sort(P.cb_refine.begin(), P.cb_refine.end(), [](const CbJob &a, const CbJob &b) {
         return uint32_t(a.lref) + a.lcup > uint32_t(b.lref) + b.lcup;
     });
+    P.ref_units = layout_refine(P.cb_refine, P.ref_groups);
+    if (P.ref_units >= (1ull << 32)) {
+        set_last_error("batch too large for 32-bit plan offsets; split it");
+        return kErrArg;
+    }
     // classic blocks: by kernel shape, costliest first within each
     {
         auto shape = [](const ClassicJob &j) { return classic_shape(j.w); };
@@ -1065,6 +1090,7 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
     const uint64_t o_pkk = take(bytes_of(P.pk_pkts)), o_pkb = take(bytes_of(P.pk_bands));
     const uint64_t o_pkc = take(bytes_of(P.pk_cbs)), o_grp = take(bytes_of(P.groups));
     const uint64_t o_frg = take(bytes_of(P.fin_rgb8)), o_frs = take(bytes_of(P.fin_rest));
+    const uint64_t o_rgr = take(bytes_of(P.ref_groups));
     const uint64_t host_bytes = off;
     const uint64_t o_pkn = take(P.pk_nodes * 2 * sizeof(uint32_t));
     const uint64_t o_pkl = take(P.pk_cbs.size() * sizeof(uint32_t)), o_pks = take(P.pk_tiles.size());
@@ -1095,9 +1121,10 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
     }
     const uint64_t o_crows = take(crows_bytes);
     const uint64_t o_queue = take(16), o_coef = take(P.coef_elems * sizeof(uint32_t));
-    // the workspace last: a plan carved from fixed memory does without when
-    // it does not fit (the cooperative kernel needs none)
+    // the workspaces last: a plan carved from fixed memory does without when
+    // they do not fit (the cooperative kernel needs none)
     const uint64_t no_work = off, o_work = take(P.work_units * sizeof(uint4));
+    const uint64_t o_rwork = take(P.ref_units * sizeof(uint4));
     const bool has_work = P.work_units != 0 && !(fixed && off > fixed_cap);
     if (!has_work) off = no_work;
     P.device_bytes = off;
@@ -1143,6 +1170,7 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
         HIP_TRY(put_dev(o_grp, P.groups));
         HIP_TRY(put_dev(o_frg, P.fin_rgb8));
         HIP_TRY(put_dev(o_frs, P.fin_rest));
+        HIP_TRY(put_dev(o_rgr, P.ref_groups));
         HIP_TRY(hipStreamSynchronize(copy));
         P.t_stage = 0;
         P.t_copy = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() -
@@ -1210,6 +1238,7 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
         put(o_grp, P.groups);
         put(o_frg, P.fin_rgb8);
         put(o_frs, P.fin_rest);
+        put(o_rgr, P.ref_groups);
         const auto t1 = std::chrono::steady_clock::now();
         uint8_t *d = static_cast<uint8_t *>(P.d_block);
         // direct runs first, then the staged range: consecutive staged runs and
@@ -1290,6 +1319,8 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
     at(o_frg, P.d_fin_rgb8, !P.fin_rgb8.empty());
     at(o_frs, P.d_fin_rest, !P.fin_rest.empty());
     at(o_work, P.d_work, has_work);
+    at(o_rgr, P.d_ref_groups, !P.ref_groups.empty());
+    at(o_rwork, P.d_ref_work, has_work && P.ref_units != 0);
     P.work_cap = has_work ? P.work_units : 0;
     return kOk;
 }
@@ -1325,6 +1356,21 @@ uint32_t classic_resident(sgn_hip_session *s, int v, int opt) {
     return s->classic_resident[v][opt];
 }
 
+// Refinement passes of the lane list's blocks, after their cleanup (three
+// launches).
+template <typename C>
+void launch_refine(sgn_hip_session *s, sgn_j2k_plan &P) {
+    const uint32_t n = static_cast<uint32_t>(P.cb_refine.size());
+    C *coef = reinterpret_cast<C *>(P.d_coef);
+    const dim3 g((n + kSplitBlocks - 1) / kSplitBlocks), b(kSplitWaves * 64);
+    hipLaunchKernelGGL(sgn_ht_refine_prep<C>, g, b, 0, s->stream, P.d_cb_refine, n, P.d_arena,
+                       static_cast<const C *>(coef), P.d_ref_groups, P.d_ref_work);
+    hipLaunchKernelGGL(sgn_ht_sigprop, dim3((n + 64 * kSplitWaves - 1) / (64 * kSplitWaves)), b, 0,
+                       s->stream, P.d_cb_refine, n, P.d_ref_groups, P.d_ref_work);
+    hipLaunchKernelGGL(sgn_ht_refine_apply<C>, g, b, 0, s->stream, P.d_cb_refine, n, P.d_arena, coef,
+                       P.d_ref_groups, P.d_ref_work);
+}
+
 // Enqueue helpers; each returns the number of kernel launches issued.
 uint32_t launch_lane_variant(sgn_hip_session *s, sgn_j2k_plan &P, int v, const CbJob *d_jobs,
                              uint32_t count, uint8_t *status) {
@@ -1353,20 +1399,23 @@ uint32_t launch_lane_variant(sgn_hip_session *s, sgn_j2k_plan &P, int v, const C
     else
         hipLaunchKernelGGL(sgn_ht_magsgn<int32_t>, g, b, 0, s->stream, d_jobs, count, P.d_arena,
                            reinterpret_cast<int32_t *>(P.d_coef), P.d_groups, P.d_work, status);
-    if (!P.cb_refine.empty() || P.device_packets) {
-        // refinement passes of the batch's lane blocks, after their cleanup
-        // (with device packets the pass counts are known on the device only:
-        // the kernel walks the whole lane list and skips the other blocks)
-        const CbJob *rj = P.device_packets ? P.d_cb_lane : P.d_cb_refine;
-        const uint32_t nr = static_cast<uint32_t>(P.device_packets ? P.cb_lane.size()
-                                                                   : P.cb_refine.size());
+    if (P.device_packets) {
+        // the pass counts are known on the device only: the kernel walks the
+        // whole lane list and skips the other blocks
+        const dim3 gr((count + 255) / 256), br(256);
         if (P.narrow)
-            hipLaunchKernelGGL((sgn_ht_refine<int16_t>), dim3((nr + 255) / 256), dim3(256), 0,
-                               s->stream, rj, nr, P.d_arena, reinterpret_cast<int16_t *>(P.d_coef));
+            hipLaunchKernelGGL((sgn_ht_refine<int16_t>), gr, br, 0, s->stream, d_jobs, count,
+                               P.d_arena, reinterpret_cast<int16_t *>(P.d_coef));
         else
-            hipLaunchKernelGGL((sgn_ht_refine<int32_t>), dim3((nr + 255) / 256), dim3(256), 0,
-                               s->stream, rj, nr, P.d_arena, reinterpret_cast<int32_t *>(P.d_coef));
+            hipLaunchKernelGGL((sgn_ht_refine<int32_t>), gr, br, 0, s->stream, d_jobs, count,
+                               P.d_arena, reinterpret_cast<int32_t *>(P.d_coef));
         ++k;
+    } else if (!P.cb_refine.empty()) {
+        if (P.narrow)
+            launch_refine<int16_t>(s, P);
+        else
+            launch_refine<int32_t>(s, P);
+        k += 3;
     }
     return k;
 }

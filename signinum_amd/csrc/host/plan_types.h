@@ -41,6 +41,20 @@ constexpr inline uint32_t ht_sym_units(uint32_t w, uint32_t h) {
     return (h + 1) / 2 * ((w + 31) / 32) * 2;
 }
 
+// Workspace of 64 consecutive refined code-blocks between the kernels of their
+// SigProp / MagRef passes, laid out as HtGroup's: the cleanup's significance
+// (two units a stripe), what SigProp found (four units a stripe), and the plain
+// SigProp bits (at most two bits a sample: 1024 bytes, 1170 of stuffed ones).
+struct RefGroup {
+    uint32_t base;
+    uint32_t stripes;   // the most stripes of any block of the group
+    uint32_t sp_units;  // units of a block's SigProp bits
+};
+constexpr uint32_t kRefSpBytes = 1184;
+constexpr inline uint32_t ref_sp_units(uint32_t lref) {
+    return ((lref < kRefSpBytes ? lref : kRefSpBytes) + 15) / 16 + 2;
+}
+
 // flags: bit 0 stripe-causal, bit 1 decodes to zero, bits 2-3 sub-band
 // (0 LL, 1 HL, 2 LH, 3 HH; a feature of the decode-cost model)
 enum : uint8_t { kCbStripeCausal = 1, kCbZero = 2, kCbBandShift = 2 };
