@@ -1115,13 +1115,6 @@ __device__ __forceinline__ void final_body(const FinalJob *jobs, uint32_t njobs,
     }
 }
 
-extern "C" __global__ void __launch_bounds__(kIdwtThreads)
-sgn_final_rev(const FinalJob *jobs, uint32_t njobs, uint32_t block_offset,
-              const uint32_t *block_job, const LevelJob *lv, const uint32_t *coef) {
-    final_body<true, int32_t>(jobs, njobs, xcd_remap(blockIdx.x, gridDim.x) + block_offset,
-                              block_job, lv, coef, nullptr, nullptr);
-}
-
 // 5/3 final stage with int16 component planes, of the blocks in `list` (null:
 // the launch's own numbers).  *redo_n must be zero at launch; blocks with a sample outside the int16 range are listed in `redo`
 // (capacity: the launch's block count) for sgn_final_rev_redo.
@@ -1145,10 +1138,11 @@ sgn_final_rev_redo(const FinalJob *jobs, uint32_t njobs, const uint32_t *block_j
 }
 
 extern "C" __global__ void __launch_bounds__(kIdwtThreads)
-sgn_final_irr(const FinalJob *jobs, uint32_t njobs, uint32_t block_offset,
+sgn_final_irr(const FinalJob *jobs, uint32_t njobs, const uint32_t *list, uint32_t block_offset,
               const uint32_t *block_job, const LevelJob *lv, const uint32_t *coef) {
-    final_body<false, float>(jobs, njobs, xcd_remap(blockIdx.x, gridDim.x) + block_offset,
-                             block_job, lv, coef, nullptr, nullptr);
+    const uint32_t i = list ? list[xcd_remap(blockIdx.x, gridDim.x)]
+                            : xcd_remap(blockIdx.x, gridDim.x) + block_offset;
+    final_body<false, float>(jobs, njobs, i, block_job, lv, coef, nullptr, nullptr);
 }
 
 // Byte fill used instead of memset nodes (safe under graph capture).

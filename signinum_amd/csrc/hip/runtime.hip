@@ -33,6 +33,7 @@
 #include "ht_split.hip"
 #include "idwt.hip"
 #include "final_rgb8.hip"
+#include "synth_rows.hip"
 #include "t1_classic.hip"
 #include "packets.hpp"
 #include "cost_model.hip"
@@ -329,8 +330,9 @@ struct sgn_j2k_plan {
     std::vector<FinalJob> fin[2];
     // work-group (64x64 output block) -> index of its job in lv[rev] / fin[rev]
     std::vector<uint32_t> lv_block_job[2], fin_block_job[2];
-    // 5/3 final blocks of tiles that sgn_final_rgb8 decodes, and the others
-    std::vector<uint32_t> fin_rgb8, fin_rest;
+    // [rev] final blocks of tiles that sgn_final_rgb8 / sgn_final_ict8 decode,
+    // and the others
+    std::vector<uint32_t> fin_rgb8[2], fin_rest[2];
     std::vector<std::pair<uint8_t, uint32_t>> tile_final_first;  // (rev, first index)
     std::vector<uint32_t> tile_final_count;
     std::vector<uint32_t> tile_width, tile_height;
@@ -365,7 +367,7 @@ struct sgn_j2k_plan {
     LevelJob *d_final_lv = nullptr;
     FinalJob *d_fin[2] = {nullptr, nullptr};
     uint32_t *d_lv_block_job[2] = {nullptr, nullptr}, *d_fin_block_job[2] = {nullptr, nullptr};
-    uint32_t *d_fin_rgb8 = nullptr, *d_fin_rest = nullptr;
+    uint32_t *d_fin_rgb8[2] = {}, *d_fin_rest[2] = {};
     uint32_t *d_fin_redo = nullptr;  // 5/3 final blocks left to the int32-plane pass
     uint8_t *d_status_lane = nullptr, *d_status_wave = nullptr;
     uint32_t *d_queue = nullptr;  // count of d_fin_redo
@@ -609,24 +611,36 @@ void parse_batch(const sgn_tile_req *reqs, size_t n, ParsedBatch &B, int32_t *ti
                     .count();
 }
 
-// Whether sgn_final_rgb8 takes a 5/3 final job (besides its bit-planes): whole
-// 8-bit RGB tiles under RCT whose components share an even origin, with int16
-// high-pass bands on 16-byte boundaries.
+// Whether the register kernels (final_rgb8.hip, synth_rows.hip) can synthesise a
+// level: an even origin, sides of at least 8, high-pass bands of one integer
+// type, rows on 16-byte boundaries.
+bool rows_level(const LevelJob &l) {
+    const uint32_t hi = l.narrow & 0xEu;
+    if ((l.x0 | l.y0) & 1u || l.x1 - l.x0 < 8 || l.y1 - l.y0 < 8 || !l.levels || l.lift53 ||
+        (hi != 0xEu && hi != 0) || (l.float_in & 0xEu))
+        return false;
+    for (int b = 0; b < 4; ++b) {
+        const int sh = ((l.narrow >> b) & 1u) ? 1 : 2;
+        if (((uint64_t(l.band[b]) << sh) | (uint64_t(l.bw[b]) << sh)) & 15u) return false;
+    }
+    return true;
+}
+
+// Whether a final job is one of sgn_final_rgb8 (5/3 and RCT; its bit-planes
+// aside) or sgn_final_ict8 (9/7 and ICT, two levels or more): a whole 8-bit RGB
+// tile whose components are such levels of one rectangle, with int16 high-pass
+// bands.
 bool rgb8_final(const FinalJob &fj, const std::vector<LevelJob> &lv) {
-    if (!fj.reversible || fj.ncomp != 3 || !fj.mct || !fj.same8 || fj.fmt != SGN_RGB8 || fj.cx0 ||
-        fj.cy0 || fj.cx1 != fj.width || fj.cy1 != fj.height)
+    if (fj.ncomp != 3 || !fj.mct || !fj.same8 || fj.fmt != SGN_RGB8 || fj.cx0 || fj.cy0 ||
+        fj.cx1 != fj.width || fj.cy1 != fj.height || (!fj.reversible && fj.rct_f32))
         return false;
     const LevelJob &a = lv[fj.level[0]];
-    if ((a.x0 | a.y0) & 1u || a.x1 - a.x0 < 8 || a.y1 - a.y0 < 8) return false;
     for (int c = 0; c < 3; ++c) {
         const LevelJob &l = lv[fj.level[c]];
-        if (l.x0 != a.x0 || l.y0 != a.y0 || l.x1 != a.x1 || l.y1 != a.y1 || !l.levels ||
-            !l.reversible || l.lift53 || (l.narrow & 0xEu) != 0xEu)
+        if (l.x0 != a.x0 || l.y0 != a.y0 || l.x1 != a.x1 || l.y1 != a.y1 ||
+            l.reversible != fj.reversible || !rows_level(l) || !(l.narrow & 2u) ||
+            (!fj.reversible && !(l.float_in & 1u)))
             return false;
-        for (int b = 0; b < 4; ++b) {
-            const int sh = ((l.narrow >> b) & 1u) ? 1 : 2;
-            if (((uint64_t(l.band[b]) << sh) | (uint64_t(l.bw[b]) << sh)) & 15u) return false;
-        }
     }
     return true;
 }
@@ -969,17 +983,17 @@ Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
             P.tile_final_count[i]++;
         }
     }
-    // blocks of the 16-bit RGB final stage
-    {
-        P.fin_rgb8.clear();
-        P.fin_rest.clear();
+    // blocks of the 8-bit RGB final stages
+    for (int rev = 0; rev < 2; ++rev) {
+        P.fin_rgb8[rev].clear();
+        P.fin_rest[rev].clear();
         for (size_t i = 0, k = 0; i < n; ++i)
             for (size_t f = 0; f < lps[i].finals.size(); ++f) {
-                if (!lps[i].finals[f].reversible) continue;
-                const FinalJob &fj = P.fin[1][k++];
+                if ((lps[i].finals[f].reversible != 0) != (rev != 0)) continue;
+                const FinalJob &fj = P.fin[rev][k++];
+                const bool fits = rev ? P.narrow && lps[i].max_k <= 11 : true;
                 std::vector<uint32_t> &to =
-                    P.narrow && lps[i].max_k <= 11 && rgb8_final(fj, P.final_lv) ? P.fin_rgb8
-                                                                                 : P.fin_rest;
+                    fits && rgb8_final(fj, P.final_lv) ? P.fin_rgb8[rev] : P.fin_rest[rev];
                 for (uint32_t b = 0; b < uint32_t(fj.nbx) * fj.nby; ++b)
                     to.push_back(fj.block_base + b);
             }
@@ -1089,7 +1103,8 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
     const uint64_t o_pkt = take(bytes_of(P.pk_tiles)), o_pkp = take(bytes_of(P.pk_parts));
     const uint64_t o_pkk = take(bytes_of(P.pk_pkts)), o_pkb = take(bytes_of(P.pk_bands));
     const uint64_t o_pkc = take(bytes_of(P.pk_cbs)), o_grp = take(bytes_of(P.groups));
-    const uint64_t o_frg = take(bytes_of(P.fin_rgb8)), o_frs = take(bytes_of(P.fin_rest));
+    const uint64_t o_frg[2] = {take(bytes_of(P.fin_rgb8[0])), take(bytes_of(P.fin_rgb8[1]))};
+    const uint64_t o_frs[2] = {take(bytes_of(P.fin_rest[0])), take(bytes_of(P.fin_rest[1]))};
     const uint64_t o_rgr = take(bytes_of(P.ref_groups));
     const uint64_t host_bytes = off;
     const uint64_t o_pkn = take(P.pk_nodes * 2 * sizeof(uint32_t));
@@ -1168,8 +1183,10 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
         HIP_TRY(put_dev(o_pkb, P.pk_bands));
         HIP_TRY(put_dev(o_pkc, P.pk_cbs));
         HIP_TRY(put_dev(o_grp, P.groups));
-        HIP_TRY(put_dev(o_frg, P.fin_rgb8));
-        HIP_TRY(put_dev(o_frs, P.fin_rest));
+        for (int r = 0; r < 2; ++r) {
+            HIP_TRY(put_dev(o_frg[r], P.fin_rgb8[r]));
+            HIP_TRY(put_dev(o_frs[r], P.fin_rest[r]));
+        }
         HIP_TRY(put_dev(o_rgr, P.ref_groups));
         HIP_TRY(hipStreamSynchronize(copy));
         P.t_stage = 0;
@@ -1236,8 +1253,10 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
         put(o_pkb, P.pk_bands);
         put(o_pkc, P.pk_cbs);
         put(o_grp, P.groups);
-        put(o_frg, P.fin_rgb8);
-        put(o_frs, P.fin_rest);
+        for (int r = 0; r < 2; ++r) {
+            put(o_frg[r], P.fin_rgb8[r]);
+            put(o_frs[r], P.fin_rest[r]);
+        }
         put(o_rgr, P.ref_groups);
         const auto t1 = std::chrono::steady_clock::now();
         uint8_t *d = static_cast<uint8_t *>(P.d_block);
@@ -1316,8 +1335,10 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
     at(o_queue, P.d_queue, true);
     at(o_coef, P.d_coef, P.coef_elems != 0);
     at(o_grp, P.d_groups, !P.groups.empty());
-    at(o_frg, P.d_fin_rgb8, !P.fin_rgb8.empty());
-    at(o_frs, P.d_fin_rest, !P.fin_rest.empty());
+    for (int r = 0; r < 2; ++r) {
+        at(o_frg[r], P.d_fin_rgb8[r], !P.fin_rgb8[r].empty());
+        at(o_frs[r], P.d_fin_rest[r], !P.fin_rest[r].empty());
+    }
     at(o_work, P.d_work, has_work);
     at(o_rgr, P.d_ref_groups, !P.ref_groups.empty());
     at(o_rwork, P.d_ref_work, has_work && P.ref_units != 0);
@@ -1486,44 +1507,51 @@ uint32_t launch_finals(sgn_hip_session *s, sgn_j2k_plan &P, int rev, uint32_t a,
     const uint32_t blocks = final_blocks(P.fin[rev], a, b);
     if (!blocks) return 0;
     const uint32_t off = P.fin[rev][a].block_base;
-    if (rev) {
-        // int16-plane pass over every block, then the int32-plane pass over
-        // the blocks it listed (d_queue counts them; cleared by a kernel,
-        // graph-safe)
-        uint32_t *redo_n = P.d_queue;
-        uint32_t k = 3;
-        hipLaunchKernelGGL(sgn_fill_bytes, dim3(1), dim3(64), 0, s->stream,
-                           reinterpret_cast<uint8_t *>(redo_n), size_t(4), size_t(1), 0u);
-        uint32_t rest = blocks;
-        const uint32_t *list = nullptr;
-        if (blocks == P.fin_block_job[1].size()) {  // the whole plan: by kernel
-            if (!P.fin_rgb8.empty()) {
-                hipLaunchKernelGGL(sgn_final_rgb8, dim3(P.fin_rgb8.size()), dim3(kIdwtThreads), 0,
-                                   s->stream, P.d_fin[1], P.d_fin_rgb8, P.d_fin_block_job[1],
-                                   P.d_final_lv, P.d_coef, P.d_fin_redo, redo_n);
-                ++k;
-            }
-            rest = static_cast<uint32_t>(P.fin_rest.size());
-            list = P.d_fin_rest;
+    const uint32_t njobs = static_cast<uint32_t>(P.fin[rev].size());
+    // a launch of the whole plan goes by kernel
+    const bool whole = blocks == P.fin_block_job[rev].size();
+    const uint32_t rgb8 = whole ? static_cast<uint32_t>(P.fin_rgb8[rev].size()) : 0;
+    const uint32_t rest = blocks - rgb8;
+    const uint32_t *list = whole ? P.d_fin_rest[rev] : nullptr;
+    uint32_t k = 0;
+    if (!rev) {
+        if (rgb8) {
+            hipLaunchKernelGGL(sgn_final_ict8, dim3(rgb8), dim3(kIctThreads), 0, s->stream,
+                               P.d_fin[0], P.d_fin_rgb8[0], P.d_fin_block_job[0], P.d_final_lv,
+                               P.d_coef);
+            ++k;
         }
-        if (rest)
-            hipLaunchKernelGGL(sgn_final_rev16, dim3(rest), dim3(kIdwtThreads), 0, s->stream,
-                               P.d_fin[1], uint32_t(P.fin[1].size()), list, off,
-                               P.d_fin_block_job[1], P.d_final_lv, P.d_coef, P.d_fin_redo, redo_n);
-        else
-            --k;
-        const uint32_t cus = s->cus ? uint32_t(s->cus) : 256u;
-        hipLaunchKernelGGL(sgn_final_rev_redo, dim3(std::min(blocks, 2 * cus)), dim3(kIdwtThreads),
-                           0, s->stream, P.d_fin[1], uint32_t(P.fin[1].size()),
-                           P.d_fin_block_job[1], P.d_final_lv, P.d_coef,
-                           static_cast<const uint32_t *>(P.d_fin_redo),
-                           static_cast<const uint32_t *>(redo_n));
+        if (rest) {
+            hipLaunchKernelGGL(sgn_final_irr, dim3(rest), dim3(kIdwtThreads), 0, s->stream,
+                               P.d_fin[0], njobs, list, off, P.d_fin_block_job[0], P.d_final_lv,
+                               P.d_coef);
+            ++k;
+        }
         return k;
     }
-    hipLaunchKernelGGL(sgn_final_irr, dim3(blocks), dim3(kIdwtThreads), 0, s->stream,
-                       P.d_fin[0], uint32_t(P.fin[0].size()), off, P.d_fin_block_job[0],
-                       P.d_final_lv, P.d_coef);
-    return 1;
+    // int16-plane pass over every block, then the int32-plane pass over the
+    // blocks it listed (d_queue counts them; cleared by a kernel, graph-safe)
+    uint32_t *redo_n = P.d_queue;
+    hipLaunchKernelGGL(sgn_fill_bytes, dim3(1), dim3(64), 0, s->stream,
+                       reinterpret_cast<uint8_t *>(redo_n), size_t(4), size_t(1), 0u);
+    if (rgb8) {
+        hipLaunchKernelGGL(sgn_final_rgb8, dim3(rgb8), dim3(kIdwtThreads), 0, s->stream,
+                           P.d_fin[1], P.d_fin_rgb8[1], P.d_fin_block_job[1], P.d_final_lv,
+                           P.d_coef, P.d_fin_redo, redo_n);
+        ++k;
+    }
+    if (rest) {
+        hipLaunchKernelGGL(sgn_final_rev16, dim3(rest), dim3(kIdwtThreads), 0, s->stream,
+                           P.d_fin[1], njobs, list, off, P.d_fin_block_job[1], P.d_final_lv,
+                           P.d_coef, P.d_fin_redo, redo_n);
+        ++k;
+    }
+    const uint32_t cus = s->cus ? uint32_t(s->cus) : 256u;
+    hipLaunchKernelGGL(sgn_final_rev_redo, dim3(std::min(blocks, 2 * cus)), dim3(kIdwtThreads), 0,
+                       s->stream, P.d_fin[1], njobs, P.d_fin_block_job[1], P.d_final_lv, P.d_coef,
+                       static_cast<const uint32_t *>(P.d_fin_redo),
+                       static_cast<const uint32_t *>(redo_n));
+    return k + 2;
 }
 
 // Store jobs [a, b) (sub-sampled components): one work-group per 64x64
