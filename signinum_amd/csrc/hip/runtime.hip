@@ -35,6 +35,7 @@
 #include "final_rgb8.hip"
 #include "synth_rows.hip"
 #include "t1_classic.hip"
+#include "t1_rows.hip"
 #include "packets.hpp"
 #include "cost_model.hip"
 
@@ -79,7 +80,7 @@ struct sgn_hip_session {
     HtSplitTables *d_split = nullptr;
     uint64_t dispatches = 0;
     int cus = 0;                    // compute units of the device
-    uint32_t classic_resident[4][3] = {};  // resident work-groups per classic kernel (shape, lanes)
+    uint32_t classic_resident[5][8] = {};  // resident work-groups per classic kernel (shape, lanes)
     // pipelined batch decode: host-to-device copies run on copy_stream
     // while the previous chunk decodes on `stream`; two staging slots
     hipStream_t copy_stream = nullptr;
@@ -157,28 +158,72 @@ const DwtShape kDwtShapes[] = {
 };
 constexpr int kDwtShapeCount = int(sizeof(kDwtShapes) / sizeof(kDwtShapes[0]));
 
-// Classic code-block kernels by block width (32, 64, 256, 1024) and active
-// lanes per wave (64, 32, 16; the 1024-wide shape always takes 16).
+// Classic code-block kernels by block size (groups of 8x4 samples, without and
+// with a stripe above and below: a 32x32 block has 32 and 40, a 64x64 one 128
+// and 144, a 1024x4 one 128 and 384, a 4x1024 one 256 and 258), by whether the
+// style has raw segments, and by lanes per wave.
 using ClassicKernel = void (*)(const ClassicJob *, uint32_t, const uint8_t *, const ClassicSeg *,
-                               int32_t *, uint32_t *);
-constexpr int kClassicLaneOpts = 3;
-constexpr uint32_t kClassicLaneCount[kClassicLaneOpts] = {64, 32, 16};
-const ClassicKernel kClassicKernels[4][kClassicLaneOpts] = {
-    {sgn_t1_classic<ClassicW32<64>>, sgn_t1_classic<ClassicW32<32>>,
-     sgn_t1_classic<ClassicW32<16>>},
-    {sgn_t1_classic<ClassicW64<64>>, sgn_t1_classic<ClassicW64<32>>,
-     sgn_t1_classic<ClassicW64<16>>},
-    {sgn_t1_classic<ClassicW256<64>>, sgn_t1_classic<ClassicW256<32>>,
-     sgn_t1_classic<ClassicW256<16>>},
-    {sgn_t1_classic<ClassicW1024>, sgn_t1_classic<ClassicW1024>, sgn_t1_classic<ClassicW1024>}};
-int classic_shape(uint32_t w) {
-    return w <= uint32_t(ClassicW32<64>::kMaxW) ? 0
-           : w <= uint32_t(ClassicW64<64>::kMaxW) ? 1
-           : w <= uint32_t(ClassicW256<64>::kMaxW) ? 2
-                                                    : 3;
+                               int32_t *, uint32_t *, uint32_t, uint32_t *);
+constexpr int kClassicShapes = 5;
+constexpr int kClassicLaneOpts = 4;
+template <int LANES>
+using ClassicSmall = ClassicShape<32, 40, LANES, false>;
+template <int LANES, bool RAW>
+using ClassicUsual = ClassicShape<128, 144, LANES, RAW>;
+template <int LANES, bool RAW>
+using ClassicLong = ClassicShape<256, 384, LANES, RAW>;
+// Lanes per wave, and the most blocks per CU of a list that takes them: more
+// lanes decode more blocks at once, fewer wait less for each other.  32x32
+// blocks (210 a tile of 256x256): 16 tiles take 4.7, 5.3, 6.4 and 9.1 ms with
+// one, two, four and sixteen lanes, 64 tiles 9.1, 5.6, 6.2 and 9.0, 128 tiles
+// 17.7, 10.3, 6.5 and 9.1, 256 tiles 34.7, 20.1, 12.2 and 8.6.  64x64 blocks (75
+// a tile): up to 64 tiles 17.8 ms with one (the longest chain) and 22 with
+// three, 256 tiles 35.6 and 21.3.  Lists past the last line go to sgn_t1_rows,
+// whose header has the figures.
+struct ClassicChoice {
+    ClassicKernel kernel;
+    uint32_t lanes, per_cu;
+};
+const ClassicChoice kClassicKernels[kClassicShapes][kClassicLaneOpts] = {
+    {{sgn_t1_classic<ClassicSmall<1>>, 1, 16},
+     {sgn_t1_classic<ClassicSmall<2>>, 2, 64},
+     {sgn_t1_classic<ClassicSmall<4>>, 4, 128},
+     {sgn_t1_classic<ClassicSmall<16>>, 16, 384}},
+    {{sgn_t1_classic<ClassicUsual<1, false>>, 1, 32},
+     {sgn_t1_classic<ClassicUsual<3, false>>, 3, 192}},
+    {{sgn_t1_classic<ClassicLong<1, false>>, 1, 32},
+     {sgn_t1_classic<ClassicLong<3, false>>, 3, 64}},
+    {{sgn_t1_classic<ClassicUsual<1, true>>, 1, 32},
+     {sgn_t1_classic<ClassicUsual<3, true>>, 3, 192}},
+    {{sgn_t1_classic<ClassicLong<1, true>>, 1, 32},
+     {sgn_t1_classic<ClassicLong<3, true>>, 3, 64}}};
+// ... and of the row kernels by block width.
+using ClassicRowsKernel = void (*)(const ClassicJob *, uint32_t, const uint8_t *,
+                                   const ClassicSeg *, int32_t *, uint32_t *);
+struct ClassicRowsChoice {
+    ClassicRowsKernel kernel;
+    uint32_t lanes, max_w;
+};
+const ClassicRowsChoice kClassicRows[4] = {{rows::sgn_t1_rows<rows::W32>, 64, 32},
+                                           {rows::sgn_t1_rows<rows::W64>, 32, 64},
+                                           {rows::sgn_t1_rows<rows::W256>, 32, 256},
+                                           {rows::sgn_t1_rows<rows::W1024>, 16, 1024}};
+// Kernel options of a list: kClassicLaneOpts of its shape, then the row kernels.
+const void *classic_kernel(int v, int opt) {
+    return opt < kClassicLaneOpts
+               ? reinterpret_cast<const void *>(kClassicKernels[v][opt].kernel)
+               : reinterpret_cast<const void *>(kClassicRows[opt - kClassicLaneOpts].kernel);
 }
 uint32_t classic_lanes(int v, int opt) {
-    return v == 3 ? uint32_t(ClassicW1024::kLanes) : kClassicLaneCount[opt];
+    return opt < kClassicLaneOpts ? kClassicKernels[v][opt].lanes
+                                  : kClassicRows[opt - kClassicLaneOpts].lanes;
+}
+// `small`: small blocks have a list of their own.
+int classic_shape(const ClassicJob &j, bool small) {
+    const uint32_t g = classic_groups(j.w, j.h), p = classic_padded(j.w, j.h);
+    const bool raw = (j.style & kCbsBypass) != 0;
+    if (g <= 32 && p <= 40 && !raw && small) return 0;
+    return (g <= 128 && p <= 144 ? 1 : 2) + (raw ? 2 : 0);
 }
 }  // namespace
 
@@ -370,7 +415,7 @@ struct sgn_j2k_plan {
     uint32_t *d_fin_rgb8[2] = {}, *d_fin_rest[2] = {};
     uint32_t *d_fin_redo = nullptr;  // 5/3 final blocks left to the int32-plane pass
     uint8_t *d_status_lane = nullptr, *d_status_wave = nullptr;
-    uint32_t *d_queue = nullptr;  // count of d_fin_redo
+    uint32_t *d_queue = nullptr;  // count of d_fin_redo; from word 4 on, classic blocks taken per shape
     // workspace of the split cleanup kernels, laid out for the lane list's
     // order: a new order may need more than the plan's block holds (d_work_own)
     std::vector<HtGroup> groups;
@@ -404,10 +449,11 @@ struct sgn_j2k_plan {
     // [classic_begin[v], classic_begin[v + 1])), costliest first; their
     // segment table; bytes of blocks joined from several packets
     std::vector<ClassicJob> classic;
-    uint32_t classic_begin[5] = {0, 0, 0, 0, 0};
-    uint32_t classic_grid[4] = {0, 0, 0, 0};  // work-groups launched per shape
-    int classic_opt[4] = {0, 0, 0, 0};        // lane option per shape (kClassicLaneCount)
-    uint32_t *d_crows = nullptr;              // the lanes' row stores
+    uint32_t classic_begin[6] = {};
+    uint32_t classic_grid[5] = {};  // work-groups launched per shape
+    int classic_opt[5] = {};        // kernel option per shape (classic_kernel)
+    uint32_t classic_mag[5] = {};   // dwords of a lane's magnitude bits or row store
+    uint32_t *d_crows = nullptr;              // the lanes' magnitude bits or row stores
     std::vector<ClassicSeg> cseg;
     std::vector<uint8_t> joined;
     ClassicJob *d_classic = nullptr;
@@ -719,7 +765,7 @@ Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
         const bool allow = !(env && env[0] == '0');
         bool classic = false;
         for (const LocalPlan &lp : lps) classic |= !lp.classic.empty();
-        // classic blocks OR magnitude bits into int32 samples
+        // classic blocks leave int32 samples
         P.narrow = allow && !classic && kmax <= 15 && 2 * coef < (1ull << 32);
     }
     // code-block jobs: each tile's slice of the three lists from prefix sums
@@ -911,14 +957,23 @@ Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
     }
     // classic blocks: by kernel shape, costliest first within each
     {
-        auto shape = [](const ClassicJob &j) { return classic_shape(j.w); };
+        // small blocks go with the usual ones (one launch) unless they are most
+        // of the list: 64 tiles in 64x64 blocks take 17.8 ms so, 22.0 apart
+        size_t n_small = 0, n_usual = 0;
+        for (const ClassicJob &j : P.classic) {
+            const int v = classic_shape(j, true);
+            n_small += v == 0;
+            n_usual += v == 1;
+        }
+        const bool small = n_small > 4 * n_usual;
+        auto shape = [&](const ClassicJob &j) { return classic_shape(j, small); };
         std::stable_sort(P.classic.begin(), P.classic.end(),
                          [&](const ClassicJob &a, const ClassicJob &b) {
                              const int sa = shape(a), sb = shape(b);
                              return sa != sb ? sa < sb : a.cost > b.cost;
                          });
         P.classic_begin[0] = 0;
-        for (int v = 0; v < 4; ++v) {
+        for (int v = 0; v < kClassicShapes; ++v) {
             uint32_t e = P.classic_begin[v];
             while (e < P.classic.size() && shape(P.classic[e]) == v) ++e;
             P.classic_begin[v + 1] = e;
@@ -1111,31 +1166,51 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
     const uint64_t o_pkl = take(P.pk_cbs.size() * sizeof(uint32_t)), o_pks = take(P.pk_tiles.size());
     const uint64_t o_stl = take(P.cb_lane.size()), o_stw = take(P.cb_wave.size());
     const uint64_t o_ff = take(P.fin_block_job[1].size() * sizeof(uint32_t));
+    // classic kernels by the length of each list (SGN_CLASSIC_LANES forces a
+    // lane count of the shape, or with 32 the row kernels)
     uint64_t crows_bytes = 0;
-    // active lanes per classic wave: the most that still give every SIMD two
-    // waves, else the fewest (SGN_CLASSIC_LANES=64, 32 or 16 forces a count)
     const char *lanes_env = std::getenv("SGN_CLASSIC_LANES");
     const uint32_t forced = lanes_env ? uint32_t(std::atoi(lanes_env)) : 0u;
-    for (int v = 0; v < 4; ++v) {
+    for (int v = 0; v < kClassicShapes; ++v) {
         const uint32_t n = P.classic_begin[v + 1] - P.classic_begin[v];
-        int opt = kClassicLaneOpts - 1;
-        for (int o = 0; o < kClassicLaneOpts; ++o) {
-            const bool fits = forced ? kClassicLaneCount[o] == forced
-                                     : uint64_t(n) >= uint64_t(kClassicLaneCount[o]) * 8u *
-                                                          uint64_t(session_cus(s));
-            if (fits) {
-                opt = o;
-                break;
-            }
+        P.classic_grid[v] = 0;
+        if (!n) continue;
+        uint32_t mag = 0, width = 0;
+        for (uint32_t k = P.classic_begin[v]; k < P.classic_begin[v + 1]; ++k) {
+            const ClassicJob &j = P.classic[k];
+            mag = std::max(mag, classic_mag_dwords(j.planes, classic_groups(j.w, j.h)));
+            width = std::max<uint32_t>(width, j.w);
         }
-        P.classic_opt[v] = opt;
+        int opt = 0;
+        auto ends = [&](int o) { return o >= kClassicLaneOpts || !kClassicKernels[v][o].kernel; };
+        while (!ends(opt) && n > kClassicKernels[v][opt].per_cu * session_cus(s)) ++opt;
+        bool by_rows = ends(opt) || forced == 32;
+        for (int o = 0; !ends(o); ++o)
+            if (kClassicKernels[v][o].lanes == forced) {
+                opt = o;
+                by_rows = false;
+            }
+        // in fixed memory the lanes' magnitude bits keep to 3 KB a block (a
+        // row store's size)
+        const uint64_t budget = std::max<uint64_t>(n, 16) * rows::kStateDwords * 4;
+        if (fixed && !by_rows && uint64_t(classic_lanes(v, opt)) * mag * 4 > budget) opt = 0;
+        if (by_rows) {
+            opt = kClassicLaneOpts;
+            while (kClassicRows[opt - kClassicLaneOpts].max_w < width) ++opt;
+            mag = rows::kStateDwords;
+        }
         const uint32_t lanes = classic_lanes(v, opt);
-        P.classic_grid[v] = n ? std::min((n + lanes - 1) / lanes, classic_resident(s, v, opt)) : 0;
-        crows_bytes = std::max<uint64_t>(crows_bytes, uint64_t(P.classic_grid[v]) * lanes *
-                                                          kClassicStateDwords * sizeof(uint32_t));
+        const uint64_t group_bytes = uint64_t(lanes) * mag * 4;
+        uint64_t grid = std::min((n + lanes - 1) / lanes, classic_resident(s, v, opt));
+        if (fixed && !by_rows && group_bytes)
+            grid = std::min(grid, std::max<uint64_t>(budget / group_bytes, 1));
+        P.classic_opt[v] = opt;
+        P.classic_mag[v] = mag;
+        P.classic_grid[v] = static_cast<uint32_t>(grid);
+        crows_bytes = std::max(crows_bytes, grid * group_bytes);
     }
     const uint64_t o_crows = take(crows_bytes);
-    const uint64_t o_queue = take(16), o_coef = take(P.coef_elems * sizeof(uint32_t));
+    const uint64_t o_queue = take(64), o_coef = take(P.coef_elems * sizeof(uint32_t));
     // the workspaces last: a plan carved from fixed memory does without when
     // they do not fit (the cooperative kernel needs none)
     const uint64_t no_work = off, o_work = take(P.work_units * sizeof(uint4));
@@ -1368,7 +1443,7 @@ uint32_t classic_resident(sgn_hip_session *s, int v, int opt) {
     if (!s->classic_resident[v][opt]) {
         int per_cu = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu, reinterpret_cast<const void *>(kClassicKernels[v][opt]), 64, 0) !=
+                &per_cu, classic_kernel(v, opt), 64, 0) !=
                 hipSuccess ||
             per_cu < 1)
             per_cu = 1;
@@ -1460,20 +1535,29 @@ uint32_t launch_wave(sgn_hip_session *s, sgn_j2k_plan &P, const CbJob *d_jobs, u
     return 1;
 }
 
-// Every classic code-block of the plan: one launch per kernel shape (one
-// block per lane; the grid at most the resident work-groups, which then
-// walk the block groups).
+// Every classic code-block of the plan: one launch per kernel shape, the grid
+// at most the resident work-groups, whose lanes then take the blocks left from a
+// counter (cleared by a kernel, graph-safe).
 uint32_t launch_classic(sgn_hip_session *s, sgn_j2k_plan &P) {
-    uint32_t k = 0;
-    for (int v = 0; v < 4; ++v) {
+    if (P.classic.empty()) return 0;
+    uint32_t k = 1;
+    hipLaunchKernelGGL(sgn_fill_bytes, dim3(1), dim3(64), 0, s->stream,
+                       reinterpret_cast<uint8_t *>(P.d_queue + 4), size_t(32), size_t(8), 0u);
+    for (int v = 0; v < kClassicShapes; ++v) {
         const uint32_t a = P.classic_begin[v], b = P.classic_begin[v + 1];
         if (a >= b || !P.classic_grid[v]) continue;
         const uint32_t n = b - a;
         const ClassicJob *jobs = P.d_classic + a;
         int32_t *coef = reinterpret_cast<int32_t *>(P.d_coef);
-        hipLaunchKernelGGL(kClassicKernels[v][P.classic_opt[v]], dim3(P.classic_grid[v]), dim3(64),
-                           0, s->stream,
-                           jobs, n, P.d_arena, P.d_cseg, coef, P.d_crows);
+        const int opt = P.classic_opt[v];
+        const dim3 g(P.classic_grid[v]), t(64);
+        if (opt < kClassicLaneOpts)
+            hipLaunchKernelGGL(kClassicKernels[v][opt].kernel, g, t, 0, s->stream, jobs, n,
+                               P.d_arena, P.d_cseg, coef, P.d_crows, P.classic_mag[v],
+                               P.d_queue + 4 + v);
+        else
+            hipLaunchKernelGGL(kClassicRows[opt - kClassicLaneOpts].kernel, g, t, 0, s->stream, jobs,
+                               n, P.d_arena, P.d_cseg, coef, P.d_crows);
         ++k;
     }
     return k;

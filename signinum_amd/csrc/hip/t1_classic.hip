@@ -6,23 +6,29 @@
 //   crates/signinum-j2k-native/src/j2c/bitplane.rs:90-317, 903-1116,
 //   1228-1370 and arithmetic_decoder.rs:42-250, 329-386.
 //
-// Decomposition: one code-block per lane.  The MQ decoder is one serial
-// chain per block (every decision updates the interval and the context
-// the next decision reads), so the parallelism is across blocks.  A block's
-// coding state is one 16-bit word per stripe column (4 samples:
-// significance, sign, visited-in-this-bit-plane and refined-before bits),
-// kept in a row store in HBM (one row of w + 2 words per stripe, zero
-// columns at both ends).  A pass walks the stripes with three rows in LDS
-// (the stripe above, this one, the one below: a ring, the row below loaded
-// when a stripe starts and the current row written back when it ends), so
-// a lane needs a few hundred bytes of LDS and several work-groups share a
-// CU; within a stripe the 3x3 words around the current column sit in
-// registers (three LDS loads per column step, one store).  Magnitude bits
-// go to the block's int32 coefficients in HBM by atomic OR (no read in the
-// decode chain); the block is zeroed first and the signs are applied in a
-// final sweep.  Each context state is its packed Qe-table entry plus the
-// MPS bit, so the common decision (MPS, no renormalisation) is one LDS
-// read.
+// Decomposition: one code-block per lane, a few lanes of each wave.  The MQ
+// decoder is one serial chain per block (every decision updates the interval
+// and the context the next decision reads), so the parallelism is across
+// blocks, and the time is that of the longest chain.  The lanes of a wave run
+// one loop whose turn is one decision of each, whatever its pass and kind, as
+// straight-line code: a walk over the samples in step would make all lanes wait
+// at every sample that any of them decides.
+//
+// A lane works on a group of eight stripe columns at a time.  Its masks are
+// 64-bit strings with six bits a column (the row above, the stripe's four rows,
+// the row below) and, where neighbours are needed, a column on either side; the
+// pending samples of the pass are a mask as well, whose lowest bit is the next
+// one in coding order, and a sample's neighbourhood is a shift of the
+// significance string, looked up in a table.  The state of all groups stays in
+// LDS (32 bytes a group), magnitude bits leave as one dword per group and pass,
+// and the whole wave turns them into samples when its blocks are done.
+//
+// What bounds it: a turn is about 100 VALU and 50 scalar operations and three
+// dependent LDS reads, 475 ns alone on a SIMD, and a 64x64 block of noise takes
+// 37,500 of them; with many blocks the VALU.  256 tiles of 256x256 (19,200
+// blocks) take 21 ms.  Sixteen lanes walking samples in step, with stripe rows
+// fetched from memory and magnitude bits ORed into it one by one, took 50 ms
+// (and 8.5 ms more for the 32-wide blocks in a launch of their own).
 #include <hip/hip_runtime.h>
 
 #include "../host/plan_types.h"
@@ -30,7 +36,7 @@
 namespace sgn {
 
 // Table C.2: Qe << 16 | index after an MPS << 8 | index after an LPS << 1 |
-// MPS switch.
+// MPS switch (the kernel's table, of both MPS values: see sgn_t1_classic).
 __constant__ uint32_t kMqTable[47] = {
     0x56010103u, 0x3401020Cu, 0x18010312u, 0x0AC10418u, 0x0521053Au, 0x02212642u, 0x5601070Du,
     0x5401081Cu, 0x4801091Cu, 0x38010A1Cu, 0x30010B22u, 0x24010C24u, 0x1C010D28u, 0x16011D2Au,
@@ -43,33 +49,6 @@ __constant__ uint32_t kMqTable[47] = {
 
 constexpr int kClassicContexts = 19;
 constexpr int kCxRunLength = 17, kCxUniform = 18;
-constexpr uint32_t kMpsBit = 1u << 15;  // MPS bit of a context word (bits 14-15 of an entry are 0)
-
-// Dwords of one stripe row of a block w wide: w + 2 words, padded to even.
-__host__ __device__ inline uint32_t classic_row_dwords(uint32_t w) { return (w + 3) >> 1; }
-// Dwords of a block's row store: one row per stripe.
-__host__ __device__ inline uint32_t classic_state_dwords(uint32_t w, uint32_t h) {
-    return classic_row_dwords(w) * ((h + 3) >> 2);
-}
-// Row-store dwords reserved per lane: the largest block of any shape
-// (4 x 1024: 3 x 256 dwords).
-constexpr uint32_t kClassicStateDwords = 768;
-
-// Kernel shapes: dwords of one LDS ring row (blocks up to kMaxW wide) and
-// the active lanes of the 64-thread work-group.  64 lanes fill a wave; with
-// fewer, a batch with few blocks spreads them over more waves (every SIMD
-// gets some, and a SIMD's waves hide each other's LDS and memory waits).
-template <int ROWDW, int LANES, int MAXW>
-struct ClassicShape {
-    static constexpr int kRowDw = ROWDW, kLanes = LANES, kMaxW = MAXW;
-};
-template <int LANES>
-using ClassicW32 = ClassicShape<17, LANES, 32>;
-template <int LANES>
-using ClassicW64 = ClassicShape<33, LANES, 64>;
-template <int LANES>
-using ClassicW256 = ClassicShape<129, LANES, 256>;
-using ClassicW1024 = ClassicShape<513, 16, 1024>;
 
 // Reads of one codeword segment: absolute arena positions [p, end), bytes
 // past `end` read as 0xFF (the MQ decoder's fill, arithmetic_decoder.rs:
@@ -101,66 +80,6 @@ struct SegBytes {
         const uint32_t w = rel < 4 ? w0 : w1;
         const uint32_t b = (w >> ((rel & 3u) * 8u)) & 0xFFu;
         return p < end ? b : 0xFFu;
-    }
-};
-
-// MQ decoder, register C kept inverted (ITU-T T.88 Annex G conventions).
-struct Mq {
-    uint32_t c, a, ct, p;
-    SegBytes in;
-
-    __device__ void bytein() {
-        const uint32_t b = in.at(p);
-        const uint32_t b1 = in.at(p + 1);
-        if (b == 0xFFu) {
-            if (b1 > 0x8Fu) {
-                ct = 8;  // a marker or the end: 1 bits from here on
-            } else {
-                ++p;
-                c += 0xFE00u - (b1 << 9);
-                ct = 7;
-            }
-        } else {
-            ++p;
-            c += 0xFF00u - (b1 << 8);
-            ct = 8;
-        }
-    }
-    __device__ void init(const uint8_t *arena, uint32_t start, uint32_t len) {
-        in.start(arena, start, start + len);
-        p = start;
-        c = (in.at(p) ^ 0xFFu) << 16;
-        bytein();
-        c <<= 7;
-        ct -= 7;
-        a = 0x8000u;
-    }
-    // decision with context word *cx (its Qe-table entry | MPS bit)
-    __device__ uint32_t decode(uint32_t *cx, const uint32_t *qtab) {
-        const uint32_t e = *cx;
-        const uint32_t qe = e >> 16;
-        uint32_t mps = (e >> 15) & 1u;
-        a -= qe;
-        if ((c >> 16) < a && (a & 0x8000u)) return mps;
-        const bool lps = (c >> 16) >= a;
-        if (lps) c -= a << 16;
-        // conditional exchange (C.3.2): the decision is the LPS, and the
-        // state moves on the LPS side, exactly when (a < qe) differs from
-        // the sub-interval the code value fell in
-        const bool took_lps = (a < qe) != lps;
-        const uint32_t d = took_lps ? 1u - mps : mps;
-        if (lps) a = qe;
-        if (took_lps && (e & 1u)) mps ^= 1u;
-        const uint32_t next = took_lps ? (e >> 1) & 0x7Fu : (e >> 8) & 0x3Fu;
-        *cx = qtab[next] | (mps << 15);
-        do {
-            if (ct == 0) bytein();
-            const uint32_t sh = min(ct, uint32_t(__builtin_clz(a) - 16));
-            a <<= sh;
-            c <<= sh;
-            ct -= sh;
-        } while (!(a & 0x8000u));
-        return d;
     }
 };
 
@@ -215,283 +134,479 @@ __device__ inline uint32_t zc_label(uint32_t h, uint32_t v, uint32_t d, bool swa
     return d >= 2 ? 2 : d;
 }
 
-// Stripe-column word bits: significance rows 0-3, sign (negative) 4-7,
-// visited in this bit-plane's significance pass 8-11, refined before 12-15.
-constexpr uint32_t kSig = 0, kNeg = 4, kVisit = 8, kRef = 12;
+// Masks of a group of eight columns: column c at bits 6 c .. 6 c + 5, bit 0 of
+// them the row above the stripe, bits 1-4 its rows, bit 5 the row below.
+// `Wide` strings have one more column in front and behind.
+constexpr uint64_t kRow0 = 0x0000041041041041ull;  // bit 0 of each column
+constexpr uint64_t kRows = kRow0 * 0x1Eull;        // the stripe's rows
+constexpr uint32_t kGroupCols = 8;
 
-// Six-entry column vector of one flag: the row above the stripe (bit 0),
-// the stripe's rows (1-4), the row below (5).
-__device__ inline uint32_t col6(uint32_t up, uint32_t mid, uint32_t dn, uint32_t f) {
-    return ((up >> (f + 3)) & 1u) | (((mid >> f) & 0xFu) << 1) | (((dn >> f) & 1u) << 5);
+// Decision tables (bytes): the context of a sample by its neighbourhood index
+// (zero coding in LL/LH, HL and HH bands; magnitude refinement, with the
+// refined-before bit at 512), then sign coding (context | flip << 5) by sign
+// index.
+constexpr uint32_t kNbRun = 384, kNbUniform = 385, kNbEntries = 388, kNbRefined = 512;
+constexpr uint32_t kTabMr = 3 * kNbEntries, kTabSign = kTabMr + 1024;
+constexpr uint32_t kTabBytes = kTabSign + 1024;
+
+// Neighbourhood index of the 15-bit window whose bit 7 is the sample (left
+// column bits 0-2, own 6 and 8, right 12-14): right bits move to 3-5.
+__device__ __forceinline__ uint32_t nb_index(uint32_t t) {
+    return (t & 0x147u) | ((t >> 9) & 0x38u);
+}
+// Sign index: horizontal and vertical neighbours' significance (bits 1, 4, 6,
+// 8) and sign (one above each).
+__device__ __forceinline__ uint32_t sign_part(uint32_t t) {
+    return (t & 0x142u) | ((t >> 9) & 0x10u);
+}
+
+__device__ inline uint8_t classic_table(uint32_t k) {
+    if (k >= kTabSign) {
+        // Table D.3
+        const uint32_t i = k - kTabSign;
+        auto contrib = [&](uint32_t b) -> int {
+            return (i >> b) & 1u ? ((i >> (b + 1)) & 1u ? -1 : 1) : 0;
+        };
+        const int hs = contrib(1) + contrib(4), vs = contrib(6) + contrib(8);
+        const int H = hs > 0 ? 1 : hs < 0 ? -1 : 0, V = vs > 0 ? 1 : vs < 0 ? -1 : 0;
+        if (H == 0) return uint8_t(V == 0 ? 9 : V < 0 ? 10 | 32 : 10);
+        return uint8_t((12 + H * V) | (H < 0 ? 32 : 0));
+    }
+    if (k >= kTabMr) return k - kTabMr >= kNbRefined ? 16 : k > kTabMr ? 15 : 14;
+    const uint32_t tab = k / kNbEntries, i = k % kNbEntries;
+    if (i == kNbRun) return kCxRunLength;
+    if (i >= kNbUniform) return kCxUniform;
+    const uint32_t h = ((i >> 1) & 1u) + ((i >> 4) & 1u), v = ((i >> 6) & 1u) + ((i >> 8) & 1u);
+    const uint32_t d = (i & 1u) + ((i >> 2) & 1u) + ((i >> 3) & 1u) + ((i >> 5) & 1u);
+    return uint8_t(zc_label(h, v, d, tab == 1, tab == 2));
+}
+
+// The MQ decoder: C inverted (ITU-T T.88 Annex G conventions), A in the upper
+// half, the last byte read, and the next ones in two dwords (the second is
+// fetched a dword ahead of its use).  Bytes from `end` on read as 0xFF
+// (arithmetic_decoder.rs:250-270).
+struct Mq {
+    uint32_t c, a, ct, last;
+    uint32_t w0, w1, left, pos, end;  // left: bytes in w0; pos: arena offset of w1
+    const uint8_t *arena;
+
+    __device__ __forceinline__ uint32_t masked(uint32_t w, uint32_t at) const {
+        const int have = (int)(end - at);
+        return have >= 4 ? w : have <= 0 ? 0xFFFFFFFFu : w | (0xFFFFFFFFu << (8 * have));
+    }
+    __device__ __forceinline__ void bytein() {
+        const uint32_t b1 = w0 & 0xFFu;
+        const bool ff = last == 0xFFu, stop = ff && b1 > 0x8Fu;  // a marker or the end: 1 bits
+        c += stop ? 0u : ff ? 0xFE00u - (b1 << 9) : 0xFF00u - (b1 << 8);
+        ct = ff && !stop ? 7u : 8u;
+        if (!stop) {
+            last = b1;
+            w0 >>= 8;
+            if (--left == 0) {
+                w0 = masked(w1, pos);
+                left = 4;
+                pos += 4;
+                w1 = *reinterpret_cast<const uint32_t *>(arena + pos);
+            }
+        }
+    }
+    __device__ void init(const uint8_t *ar, uint32_t start, uint32_t len) {
+        arena = ar;
+        end = start + len;
+        const uint32_t a0 = start & ~3u;
+        const uint32_t *q = reinterpret_cast<const uint32_t *>(ar + a0);
+        w0 = masked(q[0], a0) >> (8 * (start & 3u));
+        left = 4 - (start & 3u);
+        w1 = q[1];
+        pos = a0 + 4;
+        last = w0 & 0xFFu;
+        c = (last ^ 0xFFu) << 16;
+        w0 >>= 8;
+        if (--left == 0) {
+            w0 = masked(w1, pos);
+            left = 4;
+            pos += 4;
+            w1 = *reinterpret_cast<const uint32_t *>(ar + pos);
+        }
+        bytein();
+        c <<= 7;
+        ct -= 7;
+        a = 0x80000000u;
+    }
+    // Decision with the context word *cx: a table entry (Qe << 16 | entry after
+    // an MPS << 8 | entry after an LPS << 1 | MPS).
+    __device__ __forceinline__ uint32_t decode(uint32_t *cx, const uint32_t *qtab) {
+        const uint32_t e = *cx, qe = e & 0xFFFF0000u;
+        a -= qe;
+        const bool lps = c >= a;
+        // conditional exchange (C.3.2): the decision is the LPS, and the state
+        // moves on the LPS side, exactly when (a < qe) differs from the
+        // sub-interval the code value fell in
+        const bool took_lps = (a < qe) != lps;
+        c -= lps ? a : 0u;
+        a = lps ? qe : a;
+        if (!(a & 0x80000000u)) {
+            const uint32_t ne = qtab[took_lps ? (e >> 1) & 0x7Fu : (e >> 8) & 0x7Fu];
+            uint32_t n = (uint32_t)__builtin_clz(a), sh = min(n, ct);
+            a <<= n;
+            c <<= sh;
+            ct -= sh;
+            for (n -= sh; n; n -= sh) {
+                bytein();
+                sh = min(n, ct);
+                c <<= sh;
+                ct -= sh;
+            }
+            *cx = ne;
+        }
+        return (e & 1u) ^ (took_lps ? 1u : 0u);
+    }
+};
+
+// Groups a lane keeps in LDS (significance and sign have a stripe of zeros
+// above and below), the lanes in use, and whether segments may be raw.
+template <int GROUPS, int PADDED, int LANES, bool RAW>
+struct ClassicShape {
+    static constexpr bool kRaw = RAW;
+    static constexpr uint32_t kGroups = GROUPS, kPadded = PADDED, kLanes = LANES;
+    static constexpr uint32_t kWords = 2 * (GROUPS + PADDED) * LANES;
+};
+__host__ __device__ inline uint32_t classic_groups(uint32_t w, uint32_t h) {
+    return ((w + kGroupCols - 1) / kGroupCols) * ((h + 3) >> 2);
+}
+__host__ __device__ inline uint32_t classic_padded(uint32_t w, uint32_t h) {
+    return ((w + kGroupCols - 1) / kGroupCols) * (((h + 3) >> 2) + 2);
+}
+// Dwords of a lane's magnitude bits: per bit-plane and group one of the
+// significance passes and one of the refinement.
+__host__ __device__ inline uint32_t classic_mag_dwords(uint32_t planes, uint32_t groups) {
+    return 2 * planes * groups;
+}
+
+// The stripe's rows of a group's mask: four bits a column.
+__device__ __forceinline__ uint32_t group_nibbles(uint64_t m) {
+    const uint32_t lo = (uint32_t)m, hi = (uint32_t)(m >> 32);
+    uint32_t n = (lo >> 1) & 0xFu;
+    n |= ((lo >> 7) & 0xFu) << 4;
+    n |= ((lo >> 13) & 0xFu) << 8;
+    n |= ((lo >> 19) & 0xFu) << 12;
+    n |= ((lo >> 25) & 0xFu) << 16;
+    n |= (__builtin_amdgcn_alignbit(hi, lo, 31) & 0xFu) << 20;
+    n |= ((hi >> 5) & 0xFu) << 24;
+    return n | (((hi >> 11) & 0xFu) << 28);
 }
 
 template <class G>
 struct ClassicLane {
-    uint32_t *ring;     // this lane's three LDS rows (lane-interleaved dwords: stride kLanes)
-    uint32_t *cx;       // this lane's 19 context words (stride kLanes)
-    uint32_t *rows;     // this lane's row store in HBM (ndw dwords per stripe)
+    // LDS: the groups' masks (significance, sign, visited in this bit-plane's
+    // significance pass, refined before) and the 19 contexts, lanes interleaved
+    uint64_t *sig, *neg, *vis, *ref;
+    uint32_t *cx;
     const uint32_t *qtab;
-    int32_t *coef;
-    uint32_t dst, stride, w, h, ns, ndw, band;
-    bool causal, raw;
-    uint32_t bit;
+    const uint8_t *tab, *arena;
+    uint32_t *mag;  // this lane's magnitude bits
+    const ClassicSeg *segs;
+    uint32_t src, len, ns, ng, band, style, planes, nseg, seg, passes;
     Mq mq;
     RawBits rb;
+    bool raw;
+    uint32_t p, p_end, kind, base;  // pass, end of its segment, pass kind, decision table
+    uint32_t s, g;                  // stripe, group
+    uint32_t mode;                  // 0 next sample, 1 its sign, 2 and 3 the run's uniform bits
+    uint32_t run;
+    // Strings of the group, a column in front and behind: significance; signs
+    // (refinement: refined before); pending, visited and admitted samples;
+    // magnitude bits.  next_*: the next group's first two.
+    uint64_t E, N, cand, visited, valid, bits, next_e, next_n;
+    uint64_t last_rows, last_cols, below;  // rows of the last stripe, columns of the last group
 
-    __device__ uint16_t *word_at(uint32_t slot, uint32_t x1) {
-        return reinterpret_cast<uint16_t *>(ring + (slot * G::kRowDw + (x1 >> 1)) * G::kLanes) +
-               (x1 & 1u);
-    }
-    __device__ uint32_t word(uint32_t slot, uint32_t x1) { return *word_at(slot, x1); }
-    __device__ uint32_t &ctx(uint32_t label) { return cx[label * G::kLanes]; }
-
-    // ring slot of stripe s (-1 .. ns)
-    __device__ static uint32_t slot_of(int s) { return uint32_t(s + 3) % 3u; }
-    __device__ void load_row(int s) {
-        uint32_t *r = ring + slot_of(s) * G::kRowDw * G::kLanes;
-        if (s < 0 || uint32_t(s) >= ns) {
-            for (uint32_t k = 0; k < ndw; ++k) r[k * G::kLanes] = 0;
-            return;
-        }
-        const uint32_t *src = rows + uint32_t(s) * ndw;
-        uint32_t k = 0;
-        for (; k + 8 <= ndw; k += 8) {
-            uint32_t v[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) v[q] = src[k + q];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) r[(k + q) * G::kLanes] = v[q];
-        }
-        for (; k < ndw; ++k) r[k * G::kLanes] = src[k];
-    }
-    __device__ void store_row(int s) {
-        const uint32_t *r = ring + slot_of(s) * G::kRowDw * G::kLanes;
-        uint32_t *d = rows + uint32_t(s) * ndw;
-        for (uint32_t k = 0; k < ndw; ++k) d[k] = r[k * G::kLanes];
-    }
-
+    __device__ __forceinline__ uint32_t &ctx(uint32_t k) { return cx[k * G::kLanes]; }
     __device__ void reset_contexts() {
         const uint32_t z = qtab[0];
         for (int k = 0; k < kClassicContexts; ++k) ctx(k) = z;
-        ctx(0) = qtab[4];
-        ctx(kCxRunLength) = qtab[3];
-        ctx(kCxUniform) = qtab[46];
+        ctx(0) = qtab[8];
+        ctx(kCxRunLength) = qtab[6];
+        ctx(kCxUniform) = qtab[92];
     }
-    __device__ uint32_t decide(uint32_t label) {
-        return raw ? rb.get() : mq.decode(&ctx(label), qtab);
+    // The block's state before its first pass; false when there is none.
+    __device__ bool start(const ClassicJob &j) {
+        segs += j.seg;
+        src = j.src;
+        len = j.len;
+        ns = (j.h + 3u) >> 2;
+        ng = (j.w + kGroupCols - 1) / kGroupCols;
+        band = j.band;
+        style = j.style;
+        planes = j.planes;
+        passes = j.passes;
+        nseg = j.nseg;
+        below = (style & kCbsCausal) ? 0 : kRow0 << 5;
+        last_cols = (1ull << (6 * (j.w - kGroupCols * (ng - 1)))) - 1;
+        const uint32_t rows = j.h - 4 * (ns - 1);
+        last_rows = 0;
+        for (uint32_t r = 0; r < rows; ++r) last_rows |= kRow0 << (r + 1);
+        seg = p = mode = run = 0;
+        cand = visited = valid = bits = 0;
+        reset_contexts();
+        if (!open_segment()) return false;
+        begin_pass();
+        enter_group();
+        return true;
     }
-    __device__ void set_mag(uint32_t x, uint32_t y) {
-        atomicOr(reinterpret_cast<unsigned int *>(coef + dst + y * stride + x), 1u << bit);
-    }
-
-    // Sign of the sample at row r (column vectors of significance and sign
-    // of the left, centre and right columns), Table D.3.
-    __device__ uint32_t decode_sign(uint32_t sL, uint32_t sC, uint32_t sR, uint32_t nL, uint32_t nC,
-                                    uint32_t nR, uint32_t r) {
-        auto contrib = [](uint32_t sv, uint32_t nv, uint32_t at) -> int {
-            return ((sv >> at) & 1u) ? (((nv >> at) & 1u) ? -1 : 1) : 0;
-        };
-        const int hs = contrib(sL, nL, r + 1) + contrib(sR, nR, r + 1);
-        const int vs = contrib(sC, nC, r) + contrib(sC, nC, r + 2);
-        const int H = hs > 0 ? 1 : (hs < 0 ? -1 : 0), V = vs > 0 ? 1 : (vs < 0 ? -1 : 0);
-        uint32_t label, flip;
-        if (H == 0) {
-            label = V == 0 ? 9u : 10u;
-            flip = V < 0;
-        } else {
-            label = uint32_t(12 + H * V);
-            flip = H < 0;
-        }
-        const uint32_t s = decide(label);
-        return raw ? s : (s ^ flip);  // a raw sign bit is the sign itself
-    }
-
-    // One coding pass over the block.  KIND 0 cleanup (also clears the
-    // visited bits once a stripe is done), 1 significance propagation,
-    // 2 magnitude refinement.
-    template <int KIND>
-    __device__ void pass() {
-        const bool diag = band == 3, swap = band == 1;
-        load_row(-1);
-        load_row(0);
-        for (uint32_t s = 0; s < ns; ++s) {
-            load_row(int(s) + 1);
-            const uint32_t su = slot_of(int(s) - 1), sm = slot_of(int(s)), sd = slot_of(int(s) + 1);
-            const uint32_t rows4 = min(4u, h - 4 * s);
-            const uint32_t y0 = 4 * s;
-            // words of the previous (L), current (C) and next (R) column in
-            // the stripes above, this and below
-            uint32_t uL = 0, mL = 0, dL = 0;
-            uint32_t uC = word(su, 1), mC = word(sm, 1), dC = word(sd, 1);
-            for (uint32_t x = 0; x < w; ++x) {
-                const uint32_t uR = word(su, x + 2), mR = word(sm, x + 2), dR = word(sd, x + 2);
-                const uint32_t dnL = causal ? 0u : dL, dnC = causal ? 0u : dC, dnR = causal ? 0u : dR;
-                const uint32_t sL = col6(uL, mL, dnL, kSig), sR = col6(uR, mR, dnR, kSig);
-                const uint32_t before = mC;
-                uint32_t r = 0;
-                if (KIND == 0 && rows4 == 4 && ((mC >> kSig) & 0xFu) == 0 &&
-                    ((mC >> kVisit) & 0xFu) == 0 && sL == 0 && sR == 0 &&
-                    col6(uC, 0, dnC, kSig) == 0) {
-                    // run-length mode (D.3.4)
-                    if (!decide(kCxRunLength)) {
-                        r = 4;
-                    } else {
-                        r = decide(kCxUniform) << 1;
-                        r |= decide(kCxUniform);
-                        set_mag(x, y0 + r);
-                        const uint32_t sC = col6(uC, mC, dnC, kSig);
-                        const uint32_t neg = decode_sign(sL, sC, sR, col6(uL, mL, dnL, kNeg),
-                                                         col6(uC, mC, dnC, kNeg),
-                                                         col6(uR, mR, dnR, kNeg), r);
-                        mC |= (1u << (kSig + r)) | (neg << (kNeg + r));
-                        ++r;
-                    }
-                }
-                for (; r < rows4; ++r) {
-                    const uint32_t sC = col6(uC, mC, dnC, kSig);
-                    const uint32_t sig = (mC >> (kSig + r)) & 1u, vis = (mC >> (kVisit + r)) & 1u;
-                    const uint32_t hc = ((sL >> (r + 1)) & 1u) + ((sR >> (r + 1)) & 1u);
-                    const uint32_t vc = ((sC >> r) & 1u) + ((sC >> (r + 2)) & 1u);
-                    const uint32_t dc = ((sL >> r) & 1u) + ((sL >> (r + 2)) & 1u) +
-                                        ((sR >> r) & 1u) + ((sR >> (r + 2)) & 1u);
-                    if (KIND == 2) {
-                        if (!sig || vis) continue;
-                        const uint32_t label =
-                            ((mC >> (kRef + r)) & 1u) ? 16u : (hc + vc + dc ? 15u : 14u);
-                        if (decide(label)) set_mag(x, y0 + r);
-                        mC |= 1u << (kRef + r);
-                        continue;
-                    }
-                    if (sig) continue;
-                    if (KIND == 1) {
-                        if (hc + vc + dc == 0) continue;
-                        mC |= 1u << (kVisit + r);
-                    } else if (vis) {
-                        continue;
-                    }
-                    if (!decide(zc_label(hc, vc, dc, swap, diag))) continue;
-                    set_mag(x, y0 + r);
-                    const uint32_t neg =
-                        decode_sign(sL, sC, sR, col6(uL, mL, dnL, kNeg), col6(uC, mC, dnC, kNeg),
-                                    col6(uR, mR, dnR, kNeg), r);
-                    mC |= (1u << (kSig + r)) | (neg << (kNeg + r));
-                }
-                // the word as the next column sees it; the visited bits end
-                // with the cleanup pass (only this sample reads them)
-                if (mC != before) *word_at(sm, x + 1) = uint16_t(mC);
-                uL = uC;
-                mL = mC;
-                dL = dC;
-                uC = uR;
-                mC = mR;
-                dC = dR;
-            }
-            if (KIND == 0)
-                for (uint32_t k = 0; k < ndw; ++k) ring[(sm * G::kRowDw + k) * G::kLanes] &= ~0x0F000F00u;
-            store_row(int(s));
-        }
-    }
-
-    // passes [p0, p1) of one segment (bitplane.rs:206-317)
-    __device__ void run(uint32_t planes, uint32_t p0, uint32_t p1, uint32_t style) {
-        for (uint32_t p = p0; p < p1; ++p) {
-            bit = planes - 1 - (p + 2) / 3;
-            const uint32_t kind = p % 3;
-            // the previous pass's row stores land before this pass reads them
-            __threadfence();
-            if (kind == 0) {
-                pass<0>();
-                if (style & kCbsSegSym)  // four UNIFORM symbols, not checked (non-strict)
-                    for (int k = 0; k < 4; ++k) (void)decide(kCxUniform);
-            } else if (kind == 1) {
-                pass<1>();
+    // Opens the next segment with passes; false at the end of the data.
+    __device__ bool open_segment() {
+        const uint32_t maxp = 1 + 3 * (planes - 1);
+        while (seg < max(nseg, 1u)) {
+            if (nseg == 0) {
+                raw = false;
+                p_end = min(passes, maxp);
+                mq.init(arena, src, len);
             } else {
-                pass<2>();
+                const ClassicSeg sg = segs[seg];
+                raw = G::kRaw && sg.raw;
+                p_end = min(uint32_t(sg.end), maxp);
+                if (raw)
+                    rb.init(arena, src + sg.off, sg.len);
+                else
+                    mq.init(arena, src + sg.off, sg.len);
             }
-            if (style & kCbsReset) reset_contexts();
+            ++seg;
+            if (p < p_end) return true;
         }
+        return false;
+    }
+
+    // Mask m of padded group k with the rows above and below.
+    __device__ __forceinline__ uint64_t around(const uint64_t *m, uint32_t k) const {
+        const uint64_t own = m[(k + ng) * G::kLanes], up = m[k * G::kLanes];
+        const uint64_t dn = m[(k + 2 * ng) * G::kLanes];
+        return own | ((up >> 4) & kRow0) | ((dn << 4) & below);
+    }
+    __device__ __forceinline__ void begin_stripe() {
+        g = 0;
+        next_e = around(sig, s * ng);
+        next_n = around(neg, s * ng);
+        E = N = 0;  // no column before the first
+    }
+    __device__ __forceinline__ void begin_pass() {
+        kind = p % 3;
+        base = kind == 2 ? kTabMr : band == 1 ? kNbEntries : band == 3 ? 2 * kNbEntries : 0u;
+        s = 0;
+        begin_stripe();
+    }
+    __device__ __forceinline__ uint32_t decide(uint32_t k) {
+        if (G::kRaw && raw) return rb.get();
+        return mq.decode(&ctx(k), qtab);
+    }
+
+    // Takes group g of the stripe.
+    __device__ __forceinline__ void enter_group() {
+        const uint32_t k = s * ng + g;
+        const bool last = g + 1 == ng;
+        const uint64_t le = (E >> 48) & 0x3Fu, ln = (N >> 48) & 0x3Fu;
+        const uint64_t seen = vis[k * G::kLanes] << 6, refined = ref[k * G::kLanes] << 6;
+        E = (next_e << 6) | le;
+        N = (next_n << 6) | ln;
+        next_e = next_n = 0;
+        if (!last) {
+            next_e = around(sig, k + 1);
+            next_n = around(neg, k + 1);
+        }
+        E |= next_e << 54;
+        N |= next_n << 54;
+        N = kind == 2 ? refined : N;
+        valid = ((s + 1 == ns ? last_rows : kRows) & (last ? last_cols : ~0ull)) << 6;
+        const uint64_t a = E | (E << 1) | (E >> 1), near = a | (a << 6) | (a >> 6);
+        visited = kind == 1 ? 0 : seen;
+        cand = (kind == 2 ? E : kind == 1 ? near & ~E : ~E) & valid & ~visited;
+        bits = kind == 0 ? E & visited : 0;  // the cleanup adds to what the first pass found
+    }
+
+    // The group is done: keeps its masks and takes the next one.  False at the
+    // end of the block.
+    __device__ __forceinline__ bool advance() {
+        const uint32_t k = s * ng + g;
+        if (kind == 2) {
+            ref[k * G::kLanes] = (E >> 6) & kRows & ~(visited >> 6);
+        } else {
+            sig[(k + ng) * G::kLanes] = (E >> 6) & kRows;
+            neg[(k + ng) * G::kLanes] = (N >> 6) & kRows;
+            vis[k * G::kLanes] = kind ? visited >> 6 : 0;
+        }
+        const uint32_t slot = (p + 2) / 3 * 2 + (kind == 2 ? 1 : 0);
+        mag[slot * (ns * ng) + k] = group_nibbles(bits >> 6);
+        if (++g == ng) {
+            if (++s == ns) {
+                if (kind == 0 && (style & kCbsSegSym))  // four symbols, not checked (non-strict)
+#pragma unroll 1
+                    for (int q = 0; q < 4; ++q) (void)decide(kCxUniform);
+                if (style & kCbsReset) reset_contexts();
+                if (++p >= p_end && !open_segment()) return false;
+                begin_pass();
+            } else {
+                begin_stripe();
+            }
+        }
+        enter_group();
+        return true;
+    }
+
+    // One decision of the next pending sample.
+    __device__ __forceinline__ void decision() {
+        const uint32_t lo = (uint32_t)cand, hi = (uint32_t)(cand >> 32);
+        const uint32_t q = lo ? (uint32_t)__builtin_ctz(lo) : 32u + (uint32_t)__builtin_ctz(hi);
+        const uint64_t one = 1ull << q;
+        const uint32_t t = (uint32_t)(E >> (q - 7)), tn = (uint32_t)(N >> (q - 7));
+        const bool sign = mode == 1;
+        uint32_t at = base + (nb_index(t) | ((tn << 2) & kNbRefined));
+        bool runs = false;
+        if (mode != 0 || kind == 0) {
+            // run-length mode (D.3.4): a whole column pending in the cleanup
+            // pass, nothing significant in it or beside it
+            runs = mode == 0 && (t & 0x3FFFFu) == 0 && ((uint32_t)(cand >> q) & 0xFu) == 0xFu &&
+                   (one & (kRow0 << 7)) != 0;
+            at = runs ? base + kNbRun : at;
+            at = mode >= 2 ? base + kNbUniform : at;
+            at = sign ? kTabSign + (sign_part(t) | (sign_part(tn) << 1)) : at;
+        }
+        const uint32_t entry = tab[at];
+        uint32_t d = decide(entry & 31u);
+        if (!(G::kRaw && raw)) d ^= entry >> 5;  // a raw sign bit is the sign itself
+        // a significant sample stays pending for its sign
+        const bool found = mode == 0 && kind != 2 && d;
+        uint64_t settled = found ? 0 : one;
+        uint32_t next = found ? 1 : 0;
+        if (runs || mode >= 2) {
+            if (runs) {
+                settled = d ? 0 : one * 15u;
+                next = d ? 2 : 0;
+            } else if (mode == 2) {
+                settled = 0;
+                next = 3;
+                run = d << 1;
+            } else {
+                settled = (one << (run | d)) - one;
+                next = 1;
+            }
+        }
+        cand &= ~settled;
+        visited |= kind == 1 ? one : 0;
+        bits |= sign || (kind == 2 && d) ? one : 0;
+        if (sign) {
+            E |= one;
+            N |= d ? one : 0;
+            // samples further on that it makes members
+            if (kind == 1) cand |= (0xE2ull << q) & valid & ~E;
+        }
+        mode = next;
     }
 };
 
+// Magnitude bits and signs of block j to samples, a group per lane of the wave.
 template <class G>
-__device__ void classic_block(const ClassicJob &j, const uint8_t *arena, const ClassicSeg *segs,
-                              int32_t *coef, uint32_t *ring, uint32_t *cx, uint32_t *rows,
-                              const uint32_t *qtab) {
-    const uint32_t w = j.w, h = j.h;
-    // zero the block's coefficients (magnitude bits arrive by OR)
-    for (uint32_t y = 0; y < h; ++y) {
-        int32_t *row = coef + j.dst + y * j.stride;
-        for (uint32_t x = 0; x < w; ++x) row[x] = 0;
-    }
-    if (!j.planes || !j.passes) return;
-    ClassicLane<G> L;
-    L.ring = ring;
-    L.cx = cx;
-    L.rows = rows;
-    L.qtab = qtab;
-    L.coef = coef;
-    L.dst = j.dst;
-    L.stride = j.stride;
-    L.w = w;
-    L.h = h;
-    L.ns = (h + 3) >> 2;
-    L.ndw = classic_row_dwords(w);
-    L.band = j.band;
-    L.causal = (j.style & kCbsCausal) != 0;
-    L.raw = false;
-    for (uint32_t k = 0; k < L.ns * L.ndw; ++k) rows[k] = 0;
-    L.reset_contexts();
-    const uint32_t maxp = 1 + 3 * (uint32_t(j.planes) - 1);
-    if (j.nseg == 0) {
-        L.mq.init(arena, j.src, j.len);
-        L.run(j.planes, 0, min(uint32_t(j.passes), maxp), j.style);
-    } else {
-        for (uint32_t q = 0; q < j.nseg; ++q) {
-            const ClassicSeg sg = segs[j.seg + q];
-            L.raw = sg.raw != 0;
-            if (L.raw)
-                L.rb.init(arena, j.src + sg.off, sg.len);
-            else
-                L.mq.init(arena, j.src + sg.off, sg.len);
-            L.run(j.planes, sg.start, min(uint32_t(sg.end), maxp), j.style);
+__device__ void classic_samples(const ClassicJob &j, uint32_t passes, const uint32_t *mag,
+                                const uint64_t *neg, int32_t *coef) {
+    const uint32_t ng = (j.w + kGroupCols - 1) / kGroupCols, groups = ng * ((j.h + 3u) >> 2);
+    for (uint32_t k = threadIdx.x; k < groups; k += 64) {
+        uint32_t v[32];
+#pragma unroll
+        for (int q = 0; q < 32; ++q) v[q] = 0;
+        for (uint32_t pl = 0; pl < j.planes; ++pl) {
+            if ((pl ? 3 * pl - 2 : 0) >= passes) break;
+            uint32_t m = mag[2 * pl * groups + k];
+            if (pl && 3 * pl - 1 < passes) m |= mag[(2 * pl + 1) * groups + k];
+            const uint32_t bit = j.planes - 1 - pl;
+#pragma unroll
+            for (int q = 0; q < 32; ++q) v[q] |= ((m >> q) & 1u) << bit;
         }
-    }
-    // signs: the magnitudes' OR results and the last row stores must be
-    // visible to this lane's loads
-    __threadfence();
-    for (uint32_t y = 0; y < h; ++y) {
-        const uint32_t *srow = rows + (y >> 2) * L.ndw;
-        const uint32_t r = y & 3u;
-        int32_t *row = coef + j.dst + y * j.stride;
-        for (uint32_t x = 0; x < w; ++x) {
-            const uint32_t wd = (srow[(x + 1) >> 1] >> (((x + 1) & 1u) * 16u)) & 0xFFFFu;
-            if ((wd >> (kNeg + r)) & 1u) row[x] = -row[x];
+        const uint32_t nb = group_nibbles(neg[(ng + k) * G::kLanes]);
+        const uint32_t x0 = (k % ng) * kGroupCols, y0 = (k / ng) * 4;
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+            if (y0 + r >= j.h) break;
+            int32_t *row = coef + j.dst + (y0 + r) * j.stride + x0;
+#pragma unroll
+            for (uint32_t c = 0; c < kGroupCols; ++c) {
+                const int32_t m = (int32_t)v[4 * c + r];
+                if (x0 + c < j.w) row[c] = (nb >> (4 * c + r)) & 1u ? -m : m;
+            }
         }
     }
 }
 
-// One code-block per lane; a grid of at most the resident work-groups
-// walks the job groups (one group of kLanes blocks per work-group turn),
-// each lane keeping its row store at rows + (blockIdx.x * kLanes + lane) *
-// kClassicStateDwords.
+// One wave per work-group, kLanes of its lanes decoding a block each; a lane
+// whose block is done takes the next of the list (*queue, zero at launch, counts
+// those taken after the first gridDim.x * kLanes).  Each lane keeps its
+// magnitude bits at mag + (blockIdx.x * kLanes + lane) * mag_dwords.
 template <class G>
 __global__ void __launch_bounds__(64)
 sgn_t1_classic(const ClassicJob *__restrict__ jobs, uint32_t n, const uint8_t *__restrict__ arena,
                const ClassicSeg *__restrict__ segs, int32_t *__restrict__ coef,
-               uint32_t *__restrict__ rows) {
-    __shared__ uint32_t ring[3 * G::kRowDw * G::kLanes];
-    __shared__ uint32_t cx[kClassicContexts * G::kLanes];
-    __shared__ uint32_t qtab[48];
+               uint32_t *__restrict__ mag, uint32_t mag_dwords, uint32_t *queue) {
+    __shared__ uint64_t s_mask[G::kWords];  // significance, sign (padded), visited, refined
+    __shared__ uint32_t s_cx[kClassicContexts * G::kLanes];
+    __shared__ uint32_t s_qtab[94];
+    __shared__ uint8_t s_tab[kTabBytes];
     const uint32_t lane = threadIdx.x;
-    if (lane < 47) qtab[lane] = kMqTable[lane];
-    __syncthreads();
-    if (lane >= uint32_t(G::kLanes)) return;
-    uint32_t *my_rows = rows + (size_t(blockIdx.x) * G::kLanes + lane) * kClassicStateDwords;
-    for (uint32_t g = blockIdx.x; g * G::kLanes < n; g += gridDim.x) {
-        const uint32_t i = g * G::kLanes + lane;
-        if (i >= n) break;
-        const ClassicJob j = jobs[i];
-        classic_block<G>(j, arena, segs, coef, ring + lane, cx + lane, my_rows, qtab);
+    for (uint32_t k = lane; k < 94; k += 64) {
+        // entry 2 i + m: state i with MPS m
+        const uint32_t e = kMqTable[k >> 1], m = k & 1u;
+        const uint32_t nm = ((e >> 8) & 0x3Fu) * 2 + m;
+        const uint32_t nl = ((e >> 1) & 0x7Fu) * 2 + ((e & 1u) ? 1u - m : m);
+        s_qtab[k] = (e & 0xFFFF0000u) | (nm << 8) | (nl << 1) | m;
+    }
+    for (uint32_t k = lane; k < kTabBytes; k += 64) s_tab[k] = classic_table(k);
+    const uint32_t me = min(lane, G::kLanes - 1), taken = gridDim.x * G::kLanes;
+    uint32_t *const wave_mag = mag + size_t(blockIdx.x) * G::kLanes * mag_dwords;
+    ClassicLane<G> L;
+    L.sig = s_mask + me;
+    L.neg = L.sig + G::kPadded * G::kLanes;
+    L.vis = L.neg + G::kPadded * G::kLanes;
+    L.ref = L.vis + G::kGroups * G::kLanes;
+    L.cx = s_cx + me;
+    L.qtab = s_qtab;
+    L.tab = s_tab;
+    L.arena = arena;
+    L.mag = wave_mag + size_t(me) * mag_dwords;
+    uint32_t job = lane < G::kLanes ? blockIdx.x * G::kLanes + lane : n;
+    bool fresh = job < n, alive = false;
+    // every turn ends a block of some lane, so at most n turns
+    while (__any(alive || fresh)) {
+        for (uint64_t m = __ballot(fresh); m; m &= m - 1) {
+            const uint32_t b = (uint32_t)__builtin_ctzll(m);
+            for (uint32_t k = lane; k < G::kWords / G::kLanes; k += 64)
+                s_mask[k * G::kLanes + b] = 0;
+        }
+        __syncthreads();
+        bool ended = false;
+        if (fresh) {
+            const ClassicJob j = jobs[job];
+            L.segs = segs;
+            L.p = 0;
+            alive = j.planes && j.passes && L.start(j);
+            ended = !alive;
+            fresh = false;
+        }
+        do {
+            if (alive && L.cand == 0) {
+                alive = L.advance();
+                ended = !alive;
+            }
+            if (alive && L.cand != 0) L.decision();
+        } while (!__any(ended));
+        __syncthreads();
+        for (uint64_t m = __ballot(ended); m; m &= m - 1) {
+            const uint32_t b = (uint32_t)__builtin_ctzll(m);
+            const uint32_t i = (uint32_t)__builtin_amdgcn_readlane((int)job, (int)b);
+            const uint32_t passes = (uint32_t)__builtin_amdgcn_readlane((int)L.p, (int)b);
+            classic_samples<G>(jobs[i], passes, wave_mag + size_t(b) * mag_dwords,
+                               s_mask + G::kPadded * G::kLanes + b, coef);
+        }
+        __syncthreads();
+        if (ended) {
+            job = taken + atomicAdd(queue, 1u);
+            fresh = job < n;
+        }
     }
 }
 
