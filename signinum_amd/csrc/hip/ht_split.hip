@@ -386,12 +386,15 @@ __device__ __forceinline__ void mel_queue_fill(MelQueue &m, uint32_t need, bool 
 // registers: the significance that contexts need is two bits per quad of the
 // row above, as one bit string with the left neighbours' bits beside it.
 //
-// The chain is bound by latency when waves are few (four dependent LDS reads a
-// pair: the stream window, two context tables, the u-offset table) and by VALU
-// issue when they are many, so a pair is straight-line code of few operations:
-// the tables (HtSplitTables) hold every field where it is used, a quad past the
-// block's edge is a quad whose table entry is masked to zero, and the MEL
-// question is arithmetic on 0/1 words.
+// The chain is bound by latency when waves are few (three dependent LDS reads a
+// pair: two context tables and the u-offset table; the stream window is kept in
+// registers, its next dword read a pair ahead) and by VALU issue when they are
+// many, so a pair is straight-line code of about 60 operations: the tables
+// (HtSplitTables) hold every field where it is used, a quad past the block's edge
+// is a quad whose table entry is masked to zero (whole segments go without), and
+// the MEL question is arithmetic on 0/1 words.  One 512x512 RGB tile takes 165
+// us, half of it VALU issue and a third LDS waits; with the window read in the
+// chain 171.
 //
 // TIMED (the decode-cost model's samples, with L = 1): each wave records the
 // shader-clock cycles of its block's chain.
@@ -401,9 +404,7 @@ sgn_ht_symbols(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__rest
                const HtGroup *__restrict__ groups, uint4 *__restrict__ work,
                const HtSplitTables *__restrict__ tables, uint64_t *__restrict__ cycles) {
     __shared__ __attribute__((aligned(16))) HtSplitTables s_t;
-    // the ring's 16 dwords, and the first again: two adjacent ones can be read
-    // from any place
-    __shared__ uint32_t s_ring[kSplitWaves][17][L];
+    __shared__ uint32_t s_ring[kSplitWaves][16][L];
     for (uint32_t t = threadIdx.x; t < sizeof(HtSplitTables) / 16; t += kSplitWaves * 64)
         reinterpret_cast<uint4 *>(&s_t)[t] = reinterpret_cast<const uint4 *>(tables)[t];
     __syncthreads();
@@ -426,6 +427,7 @@ sgn_ht_symbols(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__rest
         if (!(j.flags & kCbZero)) hd = *reinterpret_cast<const HtHead *>(w.head);
     }
     const bool on = hd.scup != 0;
+    uint32_t d0 = 0, d1 = 0;  // the string's dwords at pos
     const uint32_t nq = (width + 1) >> 1, npairs = (width + 3) >> 2;
     const uint32_t nrows = on ? (height + 1) >> 1 : 0, nseg = (npairs + 7) >> 3;
     auto vlc = [&](uint32_t u) -> uint4 { return w.vlc[kHtGroup * min(u, hd.vlc_last)]; };
@@ -440,7 +442,6 @@ sgn_ht_symbols(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__rest
         ring[s + 1][rl] = v.y;
         ring[s + 2][rl] = v.z;
         ring[s + 3][rl] = v.w;
-        ring[s ? s : 16u][rl] = v.x;
     };
     if (on) {
         mel_queue_load(mel, arena);
@@ -451,6 +452,8 @@ sgn_ht_symbols(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__rest
         pend1 = vlc(5);
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) put(k, u[k]);
+        d0 = u[0].x;
+        d1 = u[0].y;
         mel_queue_bytes(mel, arena);
     }
     // next bit of the VLC string less two (the string starts at bit 2): the
@@ -469,8 +472,10 @@ sgn_ht_symbols(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__rest
         const bool first = row == 0;
         // events of up to 16 quads and, in the first row, 8 u-offset pairs
         mel_queue_fill(mel, first ? 24u : 16u, run, arena);
-        const uint32_t ev = (uint32_t)mel.ev;
-        uint32_t used = 0, acc = 0;
+        // events leave at bit 0; a one above the 24 that a segment may take
+        // says at the end how many did
+        uint32_t ev = ((uint32_t)mel.ev & 0xFFFFFFu) | 0x80000000u;
+        uint32_t acc = 0;
         uint32_t out[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         const uint32_t pa = 8 * seg;
         const uint32_t pairs = run ? npairs - pa : 0;           // from here to the row's end
@@ -479,11 +484,13 @@ sgn_ht_symbols(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__rest
         // one pair: FIRST rows take contexts from the left alone and may ask
         // MEL for the u-offsets; later rows add the row above
         uint32_t x = (seg ? x1 : x0) | (quads < 16u ? 0xFFFFFFFFu >> (2u * quads) : 0u);
-        auto pair = [&](auto is_first, uint32_t p) {
-            constexpr bool kFirst = decltype(is_first)::value;
-            const uint32_t k = (pos >> 5) & 15u;
-            uint32_t win = __builtin_amdgcn_alignbit(ring[k + 1][rl], ring[k][rl], pos & 31u);
-            uint32_t t0, len = 0;
+        auto pair = [&](auto is_first, auto is_full, uint32_t p) {
+            constexpr bool kFirst = decltype(is_first)::value, kFull = decltype(is_full)::value;
+            // a pair takes at most 30 bits, so the next one starts in the first
+            // or the second dword: the third is read here, off the chain
+            const uint32_t d2 = ring[((pos >> 5) + 2u) & 15u][rl];
+            uint32_t win = __builtin_amdgcn_alignbit(d1, d0, pos);
+            uint32_t t0;
 #pragma unroll
             for (uint32_t q = 2 * p; q < 2 * p + 2; ++q) {
                 // context: table offset bits 9-11
@@ -499,11 +506,11 @@ sgn_ht_symbols(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__rest
                 // a quad without context asks MEL; its 0 makes the entry 0
                 uint32_t ask = (c - 1u) >> 31;
                 if constexpr (kFirst) ask &= exist >> q;
-                const uint32_t drop = ask & ~(ev >> used);
-                used += ask;
-                t &= (drop - 1u) & (uint32_t)__builtin_amdgcn_sbfe((int)exist, q, 1);
-                win >>= t & 7u;
-                len += t & 7u;
+                const uint32_t drop = ask & ~ev;
+                ev >>= ask;
+                t &= drop - 1u;
+                if constexpr (!kFull) t &= (uint32_t)__builtin_amdgcn_sbfe((int)exist, q, 1);
+                win >>= t & 31u;  // bits 3 to 7 are 0
                 acc = __builtin_amdgcn_alignbit(acc, t, 30);
                 if (q & 1)
                     t1 = t;
@@ -513,16 +520,21 @@ sgn_ht_symbols(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__rest
             uint32_t mode = (t0 & 0x100u) | ((t1 & 0x100u) << 1);
             if constexpr (kFirst) {
                 const uint32_t both = (mode >> 8) & (mode >> 9);
-                mode += ((ev >> used) & both) << 8;
-                used += both;
+                mode += (ev & both) << 8;
+                ev >>= both;
             }
             const uint32_t *ut = (kFirst ? s_t.ufirst : s_t.uother) + (((win & 0xFCu) | mode) >> 2);
             const uint32_t e = ut[0], base = ut[kFirst ? 320 : 256];
-            const uint32_t sfx = __builtin_amdgcn_ubfe(win, e & 31u, (e >> 5) & 31u);
-            const uint32_t n0 = (e >> 10) & 31u;
-            const uint32_t low = __builtin_amdgcn_ubfe(sfx, 0, n0), high = sfx >> n0;
-            out[p] = ((t0 >> 16) & 0xFFu) | (t1 & 0xFF0000u) | (base + (low << 8) + (high << 24));
-            pos += len + (e >> 16);
+            // (field operands count modulo 32)
+            const uint32_t sfx = __builtin_amdgcn_ubfe(win, e, e >> 5);
+            const uint32_t n0 = e >> 10;
+            const uint32_t low = __builtin_amdgcn_ubfe(sfx, 0, n0), high = sfx >> (n0 & 31u);
+            out[p] = __builtin_amdgcn_perm(t1, t0, 0x0C060C02u) + (base + (low << 8) + (high << 24));
+            const uint32_t was = pos;
+            pos += ((t0 + t1) & 0xFFu) + (e >> 16);
+            const bool next = ((was ^ pos) & 32u) != 0;
+            d0 = next ? d1 : d0;
+            d1 = next ? d2 : d1;
         };
         if (__any(run && first)) {
             // the wave's other lanes (blocks of other heights start their rows
@@ -530,21 +542,28 @@ sgn_ht_symbols(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__rest
             if (first) {
 #pragma unroll
                 for (uint32_t p = 0; p < 8; ++p) {
-                    if (p < pairs) pair(std::true_type{}, p);
+                    if (p < pairs) pair(std::true_type{}, std::false_type{}, p);
                     else acc <<= 4;
                 }
             }
         }
-        if (run && !first) {
+        if (!__any(run && (first || quads < 16u))) {
+            // whole segments: no quad to mask
+            if (run) {
+#pragma unroll
+                for (uint32_t p = 0; p < 8; ++p) pair(std::false_type{}, std::true_type{}, p);
+            }
+        } else if (run && !first) {
 #pragma unroll
             for (uint32_t p = 0; p < 8; ++p) {
                 if (p && p % 2 == 0 && !__any(p < pairs)) {
                     acc <<= 4 * (8 - p);
                     break;
                 }
-                pair(std::false_type{}, p);
+                pair(std::false_type{}, std::false_type{}, p);
             }
         }
+        const uint32_t used = (uint32_t)__builtin_clz(ev);
         mel.ev >>= used;
         mel.n -= used;
         // What was loaded a segment ago goes into the ring (eight pairs take at
