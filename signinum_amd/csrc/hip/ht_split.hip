@@ -221,10 +221,12 @@ __device__ __forceinline__ uint32_t bytes_7f(uint32_t d) {
 // whole, as the byte-wise reader does (ht_block_decode.rs:931-999); zeros
 // follow it.  Two dependent trips to memory per block bound it (the first
 // bytes are asked for beside the length field); a round takes 128 bytes, eight
-// a lane, through a ring of words in LDS that whole 16-byte units leave.
+// a lane, through a ring of words in LDS that whole 16-byte units leave.  *clear
+// (null: none) is a counter of a later launch, set to 0.
 __global__ void __launch_bounds__(kSplitWaves * 64)
 sgn_ht_clean(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restrict__ arena,
-             const HtGroup *__restrict__ groups, uint4 *__restrict__ work) {
+             const HtGroup *__restrict__ groups, uint4 *__restrict__ work, uint32_t *clear) {
+    if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
     __shared__ __attribute__((aligned(16))) uint32_t s_buf[kSplitBlocks][kCleanRing];
     const uint32_t row = threadIdx.x / kSplitLanes, q = threadIdx.x % kSplitLanes;
     uint32_t *buf = s_buf[row];

@@ -772,22 +772,16 @@ __device__ __forceinline__ const J *job_of(const J *jobs, uint32_t njobs,
     return jobs + (block_job ? block_job[blk] : find_job(jobs, njobs, blk));
 }
 
-// One output block of one level.  G = Small serves launches whose levels
-// are all at most 32x32 (one block each; the plan's block tables count
-// 64x64 blocks, which are then the same single block).
-template <bool REV, class G = Big>
-__device__ __forceinline__ void level_body(const LevelJob *jobs, uint32_t njobs, uint32_t block_offset,
-                                           const uint32_t *block_job, uint32_t *coef) {
+// One output block of one level: block `local` of job lj.
+template <bool REV, class G>
+__device__ __forceinline__ void level_block(const LevelJob *lj, uint32_t local, uint32_t *coef) {
     constexpr int kBlk = G::kBlk;
     constexpr int N = Win<REV, G>::N;
     __shared__ typename Sample<REV>::T win_lds[Win<REV, G>::kWords];
     typename Sample<REV>::T *const win = win_lds + Win<REV, G>::X0;
     __shared__ uint32_t rows[2 * N];
-    const uint32_t blk = xcd_remap(blockIdx.x, gridDim.x) + block_offset;
-    const LevelJob *lj = job_of(jobs, njobs, block_job, blk);
     __shared__ BandLds sb;
     const LevelView L = level_view(lj, coef, &sb);
-    const uint32_t local = blk - lj->block_base;
     const uint32_t nbx = lj->nbx, out = lj->out;
     const int bx = (int)(lj->bx0 + local % nbx), by = (int)(lj->by0 + local / nbx);
     int bw, bh;
@@ -796,6 +790,42 @@ __device__ __forceinline__ void level_body(const LevelJob *jobs, uint32_t njobs,
     const SinkGlobal<REV> sink{coef, out + (uint32_t)(by * kBlk) * opitch + (uint32_t)(bx * kBlk),
                                opitch, bh_blk};
     synth_block<REV, SinkGlobal<REV>, G>(L, coef, bx, by, win, rows, sink, bw, bh);
+}
+
+// One output block of one level of a launch.  G = Small serves launches whose
+// levels are all at most 32x32 (one block each; the plan's block tables count
+// 64x64 blocks, which are then the same single block).
+template <bool REV, class G = Big>
+__device__ __forceinline__ void level_body(const LevelJob *jobs, uint32_t njobs, uint32_t block_offset,
+                                           const uint32_t *block_job, uint32_t *coef) {
+    const uint32_t blk = xcd_remap(blockIdx.x, gridDim.x) + block_offset;
+    const LevelJob *lj = job_of(jobs, njobs, block_job, blk);
+    level_block<REV, G>(lj, blk - lj->block_base, coef);
+}
+
+// The lowest levels of tile-components, one block each, one after the other in
+// one work-group per component: job first[d] + blockIdx.x is its d-th, whose
+// low-pass band the one before wrote.  A launch of its own takes a level of few
+// components about 6 us, most of it the launch and the loads' latency.
+struct LevelChain {
+    uint32_t first[8];
+    uint32_t levels;
+};
+template <bool REV>
+__device__ __forceinline__ void chain_body(const LevelJob *jobs, const LevelChain &c, uint32_t *coef) {
+    const uint32_t j = xcd_remap(blockIdx.x, gridDim.x);
+    for (uint32_t d = 0; d < c.levels; ++d) {
+        level_block<REV, Big>(jobs + c.first[d] + j, 0, coef);
+        __syncthreads();  // the level's samples are the next one's low-pass band
+    }
+}
+extern "C" __global__ void __launch_bounds__(kIdwtThreads)
+sgn_idwt_chain_rev(const LevelJob *jobs, LevelChain c, uint32_t *coef) {
+    chain_body<true>(jobs, c, coef);
+}
+extern "C" __global__ void __launch_bounds__(kIdwtThreads)
+sgn_idwt_chain_irr(const LevelJob *jobs, LevelChain c, uint32_t *coef) {
+    chain_body<false>(jobs, c, coef);
 }
 
 extern "C" __global__ void __launch_bounds__(kIdwtThreads)

@@ -370,6 +370,7 @@ struct sgn_j2k_plan {
     std::vector<uint32_t> lane_plain_begin, wave_begin;  // per tile, size ntiles+1
     std::vector<LevelJob> lv[2];                          // [rev] sorted by (depth, tile)
     std::vector<uint32_t> lv_group[2];                    // start index of each depth, size D+1
+    LevelChain chain[2] = {};                             // the depths that go in one launch
     std::vector<std::vector<LevelRange>> tile_levels;     // per tile
     std::vector<LevelJob> final_lv;
     std::vector<FinalJob> fin[2];
@@ -655,6 +656,37 @@ void parse_batch(const sgn_tile_req *reqs, size_t n, ParsedBatch &B, int32_t *ti
     }
     B.t_parse = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0)
                     .count();
+}
+
+// The first depths of a transform that sgn_idwt_chain can take: the same number
+// of levels each, one block a level, each reading what its namesake of the depth
+// before wrote.
+LevelChain level_chain(const std::vector<LevelJob> &lv, const std::vector<uint32_t> &group,
+                       uint32_t depths) {
+    LevelChain c{};
+    // Two components a CU: up to there the launches cost more than the waiting
+    // inside them.  Tiles of 256x256 (three components, three chained levels): 1,
+    // 24 and 128 tiles take 201, 244 and 261 us so and 205, 250 and 265 with a
+    // launch a level; 384 tiles 395 and 389, 4096 2199 and 2107.
+    constexpr uint32_t kChainMax = 512;
+    if (depths < 2 || group.size() < 2) return c;
+    const uint32_t n = group[1] - group[0];
+    if (!n || n > kChainMax) return c;
+    for (uint32_t d = 0; d < depths && d < 8; ++d) {
+        const uint32_t a = group[d];
+        if (group[d + 1] - a != n) break;
+        bool fits = true;
+        for (uint32_t j = 0; j < n && fits; ++j) {
+            const LevelJob &l = lv[a + j];
+            fits = l.nbx == 1 && l.nby == 1 &&
+                   (!d || (!(l.narrow & 1u) && l.band[0] == lv[group[d - 1] + j].out));
+        }
+        if (!fits) break;
+        c.first[d] = a;
+        c.levels = d + 1;
+    }
+    if (c.levels < 2) c.levels = 0;
+    return c;
 }
 
 // Whether the register kernels (final_rgb8.hip, synth_rows.hip) can synthesise a
@@ -1038,6 +1070,8 @@ Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
             P.tile_final_count[i]++;
         }
     }
+    for (int rev = 0; rev < 2; ++rev)
+        P.chain[rev] = level_chain(P.lv[rev], P.lv_group[rev], P.depth_max);
     // blocks of the 8-bit RGB final stages
     for (int rev = 0; rev < 2; ++rev) {
         P.fin_rgb8[rev].clear();
@@ -1468,8 +1502,9 @@ void launch_refine(sgn_hip_session *s, sgn_j2k_plan &P) {
 }
 
 // Enqueue helpers; each returns the number of kernel launches issued.
+// `clear`: the split kernels set *clear to 0 and it becomes null.
 uint32_t launch_lane_variant(sgn_hip_session *s, sgn_j2k_plan &P, int v, const CbJob *d_jobs,
-                             uint32_t count, uint8_t *status) {
+                             uint32_t count, uint8_t *status, uint32_t **clear = nullptr) {
     if (!count) return 0;
     // The split kernels need their workspace, which is laid out for the
     // ordered list.
@@ -1487,7 +1522,8 @@ uint32_t launch_lane_variant(sgn_hip_session *s, sgn_j2k_plan &P, int v, const C
     uint32_t k = 3;
     const dim3 g((count + kSplitBlocks - 1) / kSplitBlocks), b(kSplitWaves * 64);
     hipLaunchKernelGGL(sgn_ht_clean, g, b, 0, s->stream, d_jobs, count, P.d_arena, P.d_groups,
-                       P.d_work);
+                       P.d_work, clear ? *clear : nullptr);
+    if (clear) *clear = nullptr;
     symbols(s->stream, d_jobs, count, P.d_arena, P.d_groups, P.d_work, s->d_split);
     if (P.narrow)
         hipLaunchKernelGGL(sgn_ht_magsgn<int16_t>, g, b, 0, s->stream, d_jobs, count, P.d_arena,
@@ -1516,9 +1552,9 @@ uint32_t launch_lane_variant(sgn_hip_session *s, sgn_j2k_plan &P, int v, const C
     return k;
 }
 
-uint32_t launch_lane(sgn_hip_session *s, sgn_j2k_plan &P) {
+uint32_t launch_lane(sgn_hip_session *s, sgn_j2k_plan &P, uint32_t **clear = nullptr) {
     return launch_lane_variant(s, P, P.lane_variant, P.d_cb_lane,
-                               static_cast<uint32_t>(P.cb_lane.size()), P.d_status_lane);
+                               static_cast<uint32_t>(P.cb_lane.size()), P.d_status_lane, clear);
 }
 
 uint32_t launch_wave(sgn_hip_session *s, sgn_j2k_plan &P, const CbJob *d_jobs, uint32_t count,
@@ -1587,7 +1623,29 @@ uint32_t launch_levels(sgn_hip_session *s, sgn_j2k_plan &P, int rev, uint32_t a,
     return 1;
 }
 
-uint32_t launch_finals(sgn_hip_session *s, sgn_j2k_plan &P, int rev, uint32_t a, uint32_t b) {
+// Every level of the plan below the last: the chained ones, then a launch per
+// depth.
+uint32_t launch_all_levels(sgn_hip_session *s, sgn_j2k_plan &P) {
+    uint32_t k = 0;
+    for (int rev = 0; rev < 2; ++rev) {
+        uint32_t d = 1;
+        const LevelChain &c = P.chain[rev];
+        if (c.levels) {
+            const auto kernel = rev ? sgn_idwt_chain_rev : sgn_idwt_chain_irr;
+            hipLaunchKernelGGL(kernel, dim3(P.lv_group[rev][1] - P.lv_group[rev][0]),
+                               dim3(kIdwtThreads), 0, s->stream, P.d_lv[rev], c, P.d_coef);
+            d += c.levels;
+            ++k;
+        }
+        for (; d <= P.depth_max; ++d)
+            k += launch_levels(s, P, rev, P.lv_group[rev][d - 1], P.lv_group[rev][d]);
+    }
+    return k;
+}
+
+// `clear`: the redo count if it is still to be cleared, else null.
+uint32_t launch_finals(sgn_hip_session *s, sgn_j2k_plan &P, int rev, uint32_t a, uint32_t b,
+                       uint32_t *clear) {
     const uint32_t blocks = final_blocks(P.fin[rev], a, b);
     if (!blocks) return 0;
     const uint32_t off = P.fin[rev][a].block_base;
@@ -1614,10 +1672,14 @@ uint32_t launch_finals(sgn_hip_session *s, sgn_j2k_plan &P, int rev, uint32_t a,
         return k;
     }
     // int16-plane pass over every block, then the int32-plane pass over the
-    // blocks it listed (d_queue counts them; cleared by a kernel, graph-safe)
+    // blocks it listed (d_queue counts them; cleared by a kernel, graph-safe: an
+    // earlier one of the decode or a launch of its own, about 4 us)
     uint32_t *redo_n = P.d_queue;
-    hipLaunchKernelGGL(sgn_fill_bytes, dim3(1), dim3(64), 0, s->stream,
-                       reinterpret_cast<uint8_t *>(redo_n), size_t(4), size_t(1), 0u);
+    if (clear) {
+        hipLaunchKernelGGL(sgn_fill_bytes, dim3(1), dim3(64), 0, s->stream,
+                           reinterpret_cast<uint8_t *>(clear), size_t(4), size_t(1), 0u);
+        ++k;
+    }
     if (rgb8) {
         hipLaunchKernelGGL(sgn_final_rgb8, dim3(rgb8), dim3(kIdwtThreads), 0, s->stream,
                            P.d_fin[1], P.d_fin_rgb8[1], P.d_fin_block_job[1], P.d_final_lv,
@@ -1635,7 +1697,7 @@ uint32_t launch_finals(sgn_hip_session *s, sgn_j2k_plan &P, int rev, uint32_t a,
                        s->stream, P.d_fin[1], njobs, P.d_fin_block_job[1], P.d_final_lv, P.d_coef,
                        static_cast<const uint32_t *>(P.d_fin_redo),
                        static_cast<const uint32_t *>(redo_n));
-    return k + 2;
+    return k + 1;
 }
 
 // Store jobs [a, b) (sub-sampled components): one work-group per 64x64
@@ -1666,13 +1728,12 @@ uint32_t launch_packets(sgn_hip_session *s, sgn_j2k_plan &P) {
 uint32_t enqueue_batched(sgn_hip_session *s, sgn_j2k_plan &P) {
     uint32_t k = launch_packets(s, P);
     k += launch_classic(s, P);
-    k += launch_lane(s, P);
+    uint32_t *clear = P.d_queue;
+    k += launch_lane(s, P, &clear);
     k += launch_wave(s, P, P.d_cb_wave, static_cast<uint32_t>(P.cb_wave.size()), P.d_status_wave);
-    for (uint32_t d = 1; d <= P.depth_max; ++d)
-        for (int rev = 0; rev < 2; ++rev)
-            k += launch_levels(s, P, rev, P.lv_group[rev][d - 1], P.lv_group[rev][d]);
+    k += launch_all_levels(s, P);
     for (int rev = 0; rev < 2; ++rev)
-        k += launch_finals(s, P, rev, 0, static_cast<uint32_t>(P.fin[rev].size()));
+        k += launch_finals(s, P, rev, 0, static_cast<uint32_t>(P.fin[rev].size()), clear);
     k += launch_stores(s, P, 0, static_cast<uint32_t>(P.store.size()));
     return k;
 }
@@ -1693,7 +1754,8 @@ uint32_t enqueue_plain(sgn_hip_session *s, sgn_j2k_plan &P) {
             k += launch_levels(s, P, rg.rev, rg.start, rg.start + rg.count);
         if (P.tile_final_count[t]) {
             const auto ff = P.tile_final_first[t];
-            k += launch_finals(s, P, ff.first, ff.second, ff.second + P.tile_final_count[t]);
+            k += launch_finals(s, P, ff.first, ff.second, ff.second + P.tile_final_count[t],
+                               P.d_queue);
         }
         k += launch_stores(s, P, P.tile_store[t].first,
                            P.tile_store[t].first + P.tile_store[t].second);
@@ -2538,12 +2600,11 @@ int sgn_j2k_plan_decode_stage(sgn_hip_session *s, sgn_j2k_plan *P, int stage) {
         k += launch_wave(s, *P, P->d_cb_wave, static_cast<uint32_t>(P->cb_wave.size()),
                          P->d_status_wave);
     } else if (stage == SGN_STAGE_LEVELS) {
-        for (uint32_t d = 1; d <= P->depth_max; ++d)
-            for (int rev = 0; rev < 2; ++rev)
-                k += launch_levels(s, *P, rev, P->lv_group[rev][d - 1], P->lv_group[rev][d]);
+        k += launch_all_levels(s, *P);
     } else if (stage == SGN_STAGE_FINAL) {
         for (int rev = 0; rev < 2; ++rev)
-            k += launch_finals(s, *P, rev, 0, static_cast<uint32_t>(P->fin[rev].size()));
+            k += launch_finals(s, *P, rev, 0, static_cast<uint32_t>(P->fin[rev].size()),
+                               P->d_queue);
         k += launch_stores(s, *P, 0, static_cast<uint32_t>(P->store.size()));
     } else {
         set_last_error("unknown stage");
@@ -3285,7 +3346,7 @@ int sgn_j2k_plan_time_code_blocks(sgn_hip_session *s, sgn_j2k_plan *P, size_t st
     const uint32_t n = uint32_t(pick.size());
     hipLaunchKernelGGL(sgn_ht_clean, dim3((n + kSplitBlocks - 1) / kSplitBlocks),
                        dim3(kSplitWaves * 64), 0, s->stream, djobs.p, n, P->d_arena, dgroups.p,
-                       dwork.p);
+                       dwork.p, static_cast<uint32_t *>(nullptr));
     hipLaunchKernelGGL((sgn_ht_symbols<1, true>), dim3((n + kSplitWaves - 1) / kSplitWaves),
                        dim3(kSplitWaves * 64), 0, s->stream, djobs.p, n, P->d_arena, dgroups.p,
                        dwork.p, s->d_split, dcyc.p);
