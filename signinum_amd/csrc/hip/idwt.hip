@@ -538,12 +538,13 @@ __device__ __forceinline__ void fetch_chunks(const LevelView &L, int bx, int by,
     const int wl = (L.w + 1) >> 1, wh = L.w >> 1;  // low- and high-pass columns
     const int tid = threadIdx.x;
     uint32_t raw[kPer][2][4];
+    constexpr int kNone = -X0 - 1;  // no item (the first row's first chunk is at -X0)
     int dst[kPer];
     uint32_t slot[kPer];  // bit b: band slot of the item's bands, for the conversion
 #pragma unroll
     for (int it = 0; it < kPer; ++it) {
         const int i = tid + it * kIdwtThreads;
-        dst[it] = -1;
+        dst[it] = kNone;
         if (i >= kItems) continue;
         const int t = i >> 1;
         const int yy = t % N, k = 2 * (t / N) + (i & 1);
@@ -577,7 +578,7 @@ __device__ __forceinline__ void fetch_chunks(const LevelView &L, int bx, int by,
     }
 #pragma unroll
     for (int it = 0; it < kPer; ++it) {
-        if (dst[it] < 0) continue;
+        if (dst[it] == kNone) continue;
         T *d = win + dst[it];
 #pragma unroll
         for (int xp = 0; xp < 2; ++xp) {
