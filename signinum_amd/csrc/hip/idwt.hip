@@ -415,7 +415,10 @@ struct WinFetch {
                   "pass-0 rows stay inside the window");
     uint32_t raw0[kRows0];
     uint32_t raw1[kRows1];
-    uint32_t y1m0, y1m1;  // bit k: row k of the pass read the row-parity-1 slots
+    // bit k: row k of the pass read the row-parity-1 slots
+    uint64_t y1m0;  // up to 36 rows with two waves a block
+    uint32_t y1m1;
+    static_assert(kRows0 <= 64 && kRows1 <= 32, "a bit per row");
 };
 
 // Column `xx` of the window: its parity and, for row parity 0 and 1, the
@@ -478,11 +481,11 @@ __device__ __forceinline__ void fetch_window(const LevelView &L, int bx, int by,
         uint32_t rr[F::kRows0];
 #pragma unroll
         for (int k = 0; k < F::kRows0; ++k) rr[k] = rows[2 * (y0 + F::kGroups * k) + c.xp];
-        uint32_t m = 0;
+        uint64_t m = 0;
 #pragma unroll
         for (int k = 0; k < F::kRows0; ++k) {
             f.raw0[k] = window_word(L, c, rr[k], colok && y0 + F::kGroups * k < nh);
-            m |= (rr[k] & 1u) << k;
+            m |= (uint64_t)(rr[k] & 1u) << k;
         }
         f.y1m0 = m;
     }
