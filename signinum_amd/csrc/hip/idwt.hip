@@ -807,31 +807,6 @@ __device__ __forceinline__ void level_body(const LevelJob *jobs, uint32_t njobs,
     level_block<REV, G>(lj, blk - lj->block_base, coef);
 }
 
-// The lowest levels of tile-components, one block each, one after the other in
-// one work-group per component: job first[d] + blockIdx.x is its d-th, whose
-// low-pass band the one before wrote.  A launch of its own takes a level of few
-// components about 6 us, most of it the launch and the loads' latency.
-struct LevelChain {
-    uint32_t first[8];
-    uint32_t levels;
-};
-template <bool REV>
-__device__ __forceinline__ void chain_body(const LevelJob *jobs, const LevelChain &c, uint32_t *coef) {
-    const uint32_t j = xcd_remap(blockIdx.x, gridDim.x);
-    for (uint32_t d = 0; d < c.levels; ++d) {
-        level_block<REV, Big>(jobs + c.first[d] + j, 0, coef);
-        __syncthreads();  // the level's samples are the next one's low-pass band
-    }
-}
-extern "C" __global__ void __launch_bounds__(kIdwtThreads)
-sgn_idwt_chain_rev(const LevelJob *jobs, LevelChain c, uint32_t *coef) {
-    chain_body<true>(jobs, c, coef);
-}
-extern "C" __global__ void __launch_bounds__(kIdwtThreads)
-sgn_idwt_chain_irr(const LevelJob *jobs, LevelChain c, uint32_t *coef) {
-    chain_body<false>(jobs, c, coef);
-}
-
 extern "C" __global__ void __launch_bounds__(kIdwtThreads)
 sgn_idwt_level_rev(const LevelJob *jobs, uint32_t njobs, uint32_t block_offset,
                    const uint32_t *block_job, uint32_t *coef) {

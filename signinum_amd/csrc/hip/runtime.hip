@@ -140,7 +140,8 @@ void coop_launch(hipStream_t st, const CbJob *jobs, uint32_t n, const uint8_t *a
 }
 
 // Work-group shapes of the synthesis-level launches the autotuner chooses
-// from: the 64x64-block kernel (four or two waves per block) and whether
+// from: the 64x64-block kernel (four or two waves per block; with four, the
+// register kernel of synth_rows.hip where it can) and whether
 // launches whose levels are all at most 32x32 take the one-wave 32x32
 // kernel instead.  Every shape computes the same blocks.
 using LevelKernel = void (*)(const LevelJob *, uint32_t, uint32_t, const uint32_t *, uint32_t *);
@@ -371,6 +372,8 @@ struct sgn_j2k_plan {
     std::vector<LevelJob> lv[2];                          // [rev] sorted by (depth, tile)
     std::vector<uint32_t> lv_group[2];                    // start index of each depth, size D+1
     LevelChain chain[2] = {};                             // the depths that go in one launch
+    // [rev][j]: how many of the first j jobs the register kernels cannot take
+    std::vector<uint32_t> lv_general[2];
     std::vector<std::vector<LevelRange>> tile_levels;     // per tile
     std::vector<LevelJob> final_lv;
     std::vector<FinalJob> fin[2];
@@ -658,37 +661,6 @@ void parse_batch(const sgn_tile_req *reqs, size_t n, ParsedBatch &B, int32_t *ti
                     .count();
 }
 
-// The first depths of a transform that sgn_idwt_chain can take: the same number
-// of levels each, one block a level, each reading what its namesake of the depth
-// before wrote.
-LevelChain level_chain(const std::vector<LevelJob> &lv, const std::vector<uint32_t> &group,
-                       uint32_t depths) {
-    LevelChain c{};
-    // Two components a CU: up to there the launches cost more than the waiting
-    // inside them.  Tiles of 256x256 (three components, three chained levels): 1,
-    // 24 and 128 tiles take 201, 244 and 261 us so and 205, 250 and 265 with a
-    // launch a level; 384 tiles 395 and 389, 4096 2199 and 2107.
-    constexpr uint32_t kChainMax = 512;
-    if (depths < 2 || group.size() < 2) return c;
-    const uint32_t n = group[1] - group[0];
-    if (!n || n > kChainMax) return c;
-    for (uint32_t d = 0; d < depths && d < 8; ++d) {
-        const uint32_t a = group[d];
-        if (group[d + 1] - a != n) break;
-        bool fits = true;
-        for (uint32_t j = 0; j < n && fits; ++j) {
-            const LevelJob &l = lv[a + j];
-            fits = l.nbx == 1 && l.nby == 1 &&
-                   (!d || (!(l.narrow & 1u) && l.band[0] == lv[group[d - 1] + j].out));
-        }
-        if (!fits) break;
-        c.first[d] = a;
-        c.levels = d + 1;
-    }
-    if (c.levels < 2) c.levels = 0;
-    return c;
-}
-
 // Whether the register kernels (final_rgb8.hip, synth_rows.hip) can synthesise a
 // level: an even origin, sides of at least 8, high-pass bands of one integer
 // type, rows on 16-byte boundaries.
@@ -702,6 +674,39 @@ bool rows_level(const LevelJob &l) {
         if (((uint64_t(l.band[b]) << sh) | (uint64_t(l.bw[b]) << sh)) & 15u) return false;
     }
     return true;
+}
+
+// The first depths of a transform that sgn_idwt_chain can take: the same number
+// of levels each, one block a level, each reading what its namesake of the depth
+// before wrote.
+LevelChain level_chain(const std::vector<LevelJob> &lv, const std::vector<uint32_t> &group,
+                       uint32_t depths) {
+    LevelChain c{};
+    // Two components a CU: up to there the launches cost more than the waiting
+    // inside them.  Tiles of 256x256 (three components, three chained levels): 1,
+    // 24 and 128 tiles take 192, 234 and 251 us so, 6 to 9 more with a launch a
+    // level; 384 tiles lose 6 us by it and 4096 tiles 90.
+    constexpr uint32_t kChainMax = 512;
+    if (depths < 2 || group.size() < 2) return c;
+    const uint32_t n = group[1] - group[0];
+    if (!n || n > kChainMax) return c;
+    for (uint32_t d = 0; d < depths && d < 8; ++d) {
+        const uint32_t a = group[d];
+        if (group[d + 1] - a != n) break;
+        bool fits = true, general = false;
+        for (uint32_t j = 0; j < n && fits; ++j) {
+            const LevelJob &l = lv[a + j];
+            general |= !rows_level(l);
+            fits = l.nbx == 1 && l.nby == 1 &&
+                   (!d || (!(l.narrow & 1u) && l.band[0] == lv[group[d - 1] + j].out));
+        }
+        if (!fits) break;
+        c.first[d] = a;
+        c.general |= (general ? 1u : 0u) << d;
+        c.levels = d + 1;
+    }
+    if (c.levels < 2) c.levels = 0;
+    return c;
 }
 
 // Whether a final job is one of sgn_final_rgb8 (5/3 and RCT; its bit-planes
@@ -1070,8 +1075,13 @@ Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
             P.tile_final_count[i]++;
         }
     }
-    for (int rev = 0; rev < 2; ++rev)
+    for (int rev = 0; rev < 2; ++rev) {
         P.chain[rev] = level_chain(P.lv[rev], P.lv_group[rev], P.depth_max);
+        std::vector<uint32_t> &g = P.lv_general[rev];
+        g.assign(P.lv[rev].size() + 1, 0);
+        for (size_t k = 0; k < P.lv[rev].size(); ++k)
+            g[k + 1] = g[k] + (rows_level(P.lv[rev][k]) ? 0 : 1);
+    }
     // blocks of the 8-bit RGB final stages
     for (int rev = 0; rev < 2; ++rev) {
         P.fin_rgb8[rev].clear();
@@ -1615,8 +1625,12 @@ uint32_t launch_levels(sgn_hip_session *s, sgn_j2k_plan &P, int rev, uint32_t a,
     // levels of at most 32x32 take the one-wave kernel where the shape says
     // so (same block count: each is one block for either kernel)
     const bool small = g.small && small_levels(P.lv[rev], a, b);
-    const auto kernel = small ? (rev ? sgn_idwt_level_rev_small : sgn_idwt_level_irr_small)
-                              : g.kernel[rev];
+    // the four-wave shapes lift in registers where every level allows it
+    const bool rows = !small && g.threads == uint32_t(kIdwtThreads) &&
+                      P.lv_general[rev][a] == P.lv_general[rev][b];
+    const auto kernel = small  ? (rev ? sgn_idwt_level_rev_small : sgn_idwt_level_irr_small)
+                        : rows ? (rev ? sgn_idwt_rows_rev : sgn_idwt_rows_irr)
+                               : g.kernel[rev];
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(small ? Small::kThreads : g.threads), 0,
                        s->stream, P.d_lv[rev], uint32_t(P.lv[rev].size()), off,
                        P.d_lv_block_job[rev], P.d_coef);

@@ -293,6 +293,116 @@ __device__ __forceinline__ void col_lift(const typename Sample<REV>::T *tile, in
     }
 }
 
+// One 64x64 block of a level below the last into the coefficient arena: 256
+// threads, the rows past the 32nd pair by the first wave.
+template <bool REV, bool HI16, bool LL16, bool LLF>
+__device__ __forceinline__ void level_rows(const LevelJob *lj, uint32_t local, uint32_t *coef,
+                                           typename Sample<REV>::T *tile) {
+    using R = RowTile<REV>;
+    const RowBands b = row_bands<HI16, LL16>(lj, coef);
+    const uint32_t nbx = lj->nbx;
+    const int ox = (int)(lj->bx0 + local % nbx) * kBlk, oy = (int)(lj->by0 + local / nbx) * kBlk;
+    const int tid = threadIdx.x, seg = tid & 7, j = tid >> 3;
+    const int rows = b.h + R::H - oy + R::H;  // rows of the tile that outputs read
+    RowChunk k{};
+    if (2 * j < rows) {
+        row_load<REV, HI16, LL16>(b, ox, oy, j, seg, k);
+        row_lift<REV, HI16, LL16, LLF>(b, ox, j, seg, k, tile);
+    }
+    if (tid < 8 * (R::kPairs - 32) && 2 * (32 + j) < rows) {
+        row_load<REV, HI16, LL16>(b, ox, oy, 32 + j, seg, k);
+        row_lift<REV, HI16, LL16, LLF>(b, ox, 32 + j, seg, k, tile);
+    }
+    __syncthreads();
+    const int g = tid & 15, r = tid >> 4;
+    const int x = ox + 4 * g, y = oy + 4 * r;
+    if (x >= b.w || y >= b.h) return;
+    typename Sample<REV>::T v[4][4];
+    col_lift<REV>(tile, g, r, v);
+    // rows are padded to 16 elements: whole groups of four can be written
+    const uint32_t pitch = coef_pitch((uint32_t)b.w);
+    uint32_t *out = coef + lj->out + (uint32_t)y * pitch + (uint32_t)x;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        if (y + q < b.h)
+            *reinterpret_cast<uint4 *>(out + (uint32_t)q * pitch) = make_uint4(
+                __builtin_bit_cast(uint32_t, v[q][0]), __builtin_bit_cast(uint32_t, v[q][1]),
+                __builtin_bit_cast(uint32_t, v[q][2]), __builtin_bit_cast(uint32_t, v[q][3]));
+}
+
+// The levels of a launch whose jobs all fit (rows_level on the host).  What
+// bounds it: HBM.  The 256x256 levels of 192 tiles of 512x512 under 9/7 take 67 us
+// (80 in the general kernel), the 128x128 levels of 4096 tiles of 256x256 under
+// 5/3 287 (330; 1.3 GB, 4.5 TB/s).
+template <bool REV>
+__device__ __forceinline__ void level_rows_any(const LevelJob *lj, uint32_t local, uint32_t *coef) {
+    __shared__ __attribute__((aligned(16)))
+        typename Sample<REV>::T tile[RowTile<REV>::kRows * RowTile<REV>::kPitch];
+    const bool hi16 = (lj->narrow & 2u) != 0, ll16 = (lj->narrow & 1u) != 0;
+    const bool llf = !REV && (lj->float_in & 1u);
+    if (hi16) {
+        if (ll16)
+            level_rows<REV, true, true, false>(lj, local, coef, tile);
+        else if (REV || !llf)
+            level_rows<REV, true, false, false>(lj, local, coef, tile);
+        else
+            level_rows<REV, true, false, true>(lj, local, coef, tile);
+    } else if (ll16) {
+        level_rows<REV, false, true, false>(lj, local, coef, tile);
+    } else if (REV || !llf) {
+        level_rows<REV, false, false, false>(lj, local, coef, tile);
+    } else {
+        level_rows<REV, false, false, true>(lj, local, coef, tile);
+    }
+}
+template <bool REV>
+__device__ __forceinline__ void level_rows_body(const LevelJob *jobs, uint32_t njobs,
+                                                uint32_t block_offset, const uint32_t *block_job,
+                                                uint32_t *coef) {
+    const uint32_t blk = xcd_remap(blockIdx.x, gridDim.x) + block_offset;
+    const LevelJob *lj = job_of(jobs, njobs, block_job, blk);
+    level_rows_any<REV>(lj, blk - lj->block_base, coef);
+}
+extern "C" __global__ void __launch_bounds__(kIdwtThreads)
+sgn_idwt_rows_rev(const LevelJob *jobs, uint32_t njobs, uint32_t block_offset,
+                  const uint32_t *block_job, uint32_t *coef) {
+    level_rows_body<true>(jobs, njobs, block_offset, block_job, coef);
+}
+extern "C" __global__ void __launch_bounds__(kIdwtThreads)
+sgn_idwt_rows_irr(const LevelJob *jobs, uint32_t njobs, uint32_t block_offset,
+                  const uint32_t *block_job, uint32_t *coef) {
+    level_rows_body<false>(jobs, njobs, block_offset, block_job, coef);
+}
+
+// The lowest levels of tile-components, one block each, one after the other in
+// one work-group per component: job first[d] + blockIdx.x is its d-th, whose
+// low-pass band the one before wrote; bit d of `general`: some job of that depth
+// needs the general kernel.  A launch of its own takes a level of few components
+// about 5 us, most of it the launch and the loads' latency.
+struct LevelChain {
+    uint32_t first[8];
+    uint32_t levels, general;
+};
+template <bool REV>
+__device__ __forceinline__ void chain_body(const LevelJob *jobs, const LevelChain &c, uint32_t *coef) {
+    const uint32_t j = xcd_remap(blockIdx.x, gridDim.x);
+    for (uint32_t d = 0; d < c.levels; ++d) {
+        if ((c.general >> d) & 1u)
+            level_block<REV, Big>(jobs + c.first[d] + j, 0, coef);
+        else
+            level_rows_any<REV>(jobs + c.first[d] + j, 0, coef);
+        __syncthreads();  // the level's samples are the next one's low-pass band
+    }
+}
+extern "C" __global__ void __launch_bounds__(kIdwtThreads)
+sgn_idwt_chain_rev(const LevelJob *jobs, LevelChain c, uint32_t *coef) {
+    chain_body<true>(jobs, c, coef);
+}
+extern "C" __global__ void __launch_bounds__(kIdwtThreads)
+sgn_idwt_chain_irr(const LevelJob *jobs, LevelChain c, uint32_t *coef) {
+    chain_body<false>(jobs, c, coef);
+}
+
 // Rounds half away from zero and saturates to 8 bits, as `as u8` of a rounded
 // f32 does (NaN: 0).  From 0 up the largest f32 below a half, added before
 // truncation, rounds every f32 below 2^23 right.
