@@ -26,6 +26,7 @@
 #include <thread>
 #include <vector>
 
+#include "../host/host_images.hpp"
 #include "../host/parse.hpp"
 #include "../host/sgn_api.hpp"
 #include "ht_decode.hip"
@@ -2085,20 +2086,15 @@ Status decode_once(sgn_hip_session *s, const sgn_tile_req *reqs, size_t n, int m
     return status_check(*P, s->stat.p, mode, first_fail);
 }
 
-// An image in a call's device block (rows without gaps) and its host array.
-struct HostImage {
-    uint8_t *dst;
-    size_t stride, off, row, rows;
-};
-
 // Device images to host arrays.  The bytes travel in pinned chunks, one copied
 // by the DMA engine while the worker pool writes the previous one to its
 // arrays; a pitched copy straight to pageable memory took 1.6 ms for the 192 KB
-// of a 256x256 tile, this way takes about 25 us.
+// of a 256x256 tile, this way takes about 25 us.  Images that share bytes are
+// written one after the other: the last one's stay.
 class HostWriter {
   public:
     HostWriter(sgn_hip_session *s, const uint8_t *dev, std::vector<HostImage> images)
-        : s_(s), dev_(dev) {
+        : s_(s), dev_(dev), in_order_(images_overlap(images)) {
         // chunks of whole rows, consecutive in the device block
         for (const HostImage &im : images) {
             if (!im.row || !im.rows) continue;
@@ -2129,7 +2125,7 @@ class HostWriter {
             HIP_TRY(hipEventSynchronize(sl.done));
             sl.pending = false;
             const std::vector<HostImage> &ps = chunks_[k].pieces;
-            WorkerPool::get().run(ps.size(), [&](size_t i) {
+            auto copy = [&](size_t i) {
                 const HostImage &q = ps[i];
                 const uint8_t *src = sl.p + q.off;
                 if (q.stride == q.row) {
@@ -2138,7 +2134,11 @@ class HostWriter {
                     for (size_t y = 0; y < q.rows; ++y)
                         std::memcpy(q.dst + y * q.stride, src + y * q.row, q.row);
                 }
-            });
+            };
+            if (in_order_)
+                for (size_t i = 0; i < ps.size(); ++i) copy(i);
+            else
+                WorkerPool::get().run(ps.size(), copy);
         }
         return kOk;
     }
@@ -2162,6 +2162,7 @@ class HostWriter {
     }
     sgn_hip_session *s_;
     const uint8_t *dev_;
+    bool in_order_;
     std::vector<Chunk> chunks_;
 };
 

@@ -79,3 +79,23 @@ def test_small_array_and_failing_tile(session, tiles):
         ro.flags.writeable = False
         S.decode_tiles_into([(streams[0], ro, 768)], S.PixelFormat.RGB8, session=session)
     S.decode_tiles_into([], S.PixelFormat.RGB8, session=session)
+
+
+def test_arrays_that_share_bytes_and_one_canvas(session):
+    """Tiles decoded into one array: the last one stays.  Tiles of one canvas
+    (flat views that overlap in range only) land in their places."""
+    rng = np.random.default_rng(9)
+    imgs = [synth.texture_rgb(rng, 256, 256) for _ in range(64)]
+    streams = [S.encode_j2k_lossless(v, levels=2) for v in imgs]
+    for _ in range(3):
+        out = np.zeros(imgs[0].size, np.uint8)
+        S.decode_tiles_into([(c, out, 768) for c in streams], S.PixelFormat.RGB8, session=session)
+        assert np.array_equal(out.reshape(256, 256, 3), imgs[-1])
+    canvas = np.zeros((8 * 256, 8 * 256, 3), np.uint8)
+    flat = canvas.reshape(-1)
+    pitch = 8 * 768
+    S.decode_tiles_into([(c, flat[(k // 8) * 256 * pitch + (k % 8) * 768:], pitch)
+                         for k, c in enumerate(streams)], S.PixelFormat.RGB8, session=session)
+    for k, v in enumerate(imgs):
+        y, x = 256 * (k // 8), 256 * (k % 8)
+        assert np.array_equal(canvas[y:y + 256, x:x + 256], v), k
