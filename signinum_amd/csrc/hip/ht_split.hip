@@ -656,7 +656,9 @@ sgn_ht_magsgn(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restr
     HtHead hd{0, 0, 0, 0};
     const HtWork ws = ht_work(work, groups, valid ? i : 0);
     if (valid && !(j.flags & kCbZero)) hd = *reinterpret_cast<const HtHead *>(ws.head);
-    const bool on = hd.scup != 0;
+    // (the planner makes a block with zblk >= K a zero block; the 16-bit samples'
+    // windows rest on it)
+    const bool on = hd.scup != 0 && (sizeof(C) == 4 || j.zblk < 15u);
     const uint32_t nrows = (h + 1) >> 1;
     // pair q of a row: dword q % 8 of the row's chunk q / 8
     const uint32_t *sym = reinterpret_cast<const uint32_t *>(ws.sym) +
@@ -784,7 +786,8 @@ sgn_ht_magsgn(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restr
         };
         uint32_t bits[8];
         if constexpr (sizeof(C) == 2) {
-            // K <= 15: U_q is at most 17, two samples come from one window
+            // a coded block of K <= 15 has zblk <= 14 (`on`), so U_q is at most 16 and
+            // two samples come from one window
 #pragma unroll
             for (uint32_t k = 0; k < 8; k += 2) {
                 bits[k] = window(offset(k));

@@ -72,6 +72,7 @@ static int check(const LocalPlan &lp, size_t len, uint64_t capacity, const char 
     const uint64_t elems = 2 * lp.coef_elems;
     for (size_t i = 0; i < lp.cbs.size(); ++i) {
         const CbJob &j = lp.cbs[i];
+        if (!(j.flags & kCbZero) && j.zblk >= j.kmax) fail("zero bit-planes of a coded block", i);
         if (!(j.flags & kCbZero) && uint64_t(j.src) + j.lcup + j.lref > len)
             fail("code-block bytes past the codestream", i);
         if (j.w == 0 || j.h == 0 || uint32_t(j.w) * j.h > 4096 || j.stride < j.w) {
