@@ -283,6 +283,8 @@ int sgn_j2k_plan_decode_stage(sgn_hip_session *session, sgn_j2k_plan *plan, int 
  * as the cooperative one-block-per-wave kernel. */
 int sgn_ht_lane_variant_count(void);
 const char *sgn_ht_lane_variant_name(int variant);
+/* Also takes the former indexes up to 8: 6 is the cooperative kernel, the
+ * others past the count are the plan's own choice. */
 int sgn_j2k_plan_set_lane_variant(sgn_j2k_plan *plan, int variant);
 int sgn_j2k_plan_get_lane_variant(const sgn_j2k_plan *plan);
 /* Times every variant `reps` times on the plan's code-blocks (HIP events on

@@ -126,6 +126,10 @@ constexpr int kSplit64Variant = 0, kSplit32Variant = 1, kCoopVariant = 2;
 // 210 blocks 206 and 199 (16, 8, 4, 2 and 1 lanes are slower or within 2%
 // everywhere).
 constexpr size_t kSplit64Blocks = 131072;
+// Programs may hold an index of the nine variants there were before the split
+// kernels: past the present ones they stay accepted, the cooperative kernel's
+// as that, a lane kernel's shape as the plan's own choice.
+constexpr int kFormerVariantCount = 9, kFormerCoopVariant = 6;
 
 // The cooperative kernel: one code-block per wave, one wave per work-group.
 // refine: the list holds blocks with SigProp / MagRef passes
@@ -729,6 +733,10 @@ bool rgb8_final(const FinalJob &fj, const std::vector<LevelJob> &lv) {
     return true;
 }
 
+int default_variant(const sgn_j2k_plan &P) {
+    return P.cb_lane.size() >= kSplit64Blocks ? kSplit64Variant : kSplit32Variant;
+}
+
 // Merges the parsed tiles into the batch tables.  pool: fill the code-block
 // lists on the worker pool (false when another thread is parsing on it).
 Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
@@ -1017,7 +1025,7 @@ Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
             P.classic_begin[v + 1] = e;
         }
     }
-    P.lane_variant = P.cb_lane.size() >= kSplit64Blocks ? kSplit64Variant : kSplit32Variant;
+    P.lane_variant = default_variant(P);
     // synthesis levels grouped by (transform, depth), tiles in order: the
     // levels of each depth counted, then placed tile by tile
     const uint32_t D = P.depth_max;
@@ -2472,7 +2480,8 @@ const char *sgn_ht_lane_variant_name(int v) {
 }
 
 int sgn_j2k_plan_set_lane_variant(sgn_j2k_plan *P, int v) {
-    if (!P || v < 0 || v >= kRowsVariantCount) return SGN_E_ARG;
+    if (!P || v < 0 || v >= kFormerVariantCount) return SGN_E_ARG;
+    if (v >= kRowsVariantCount) v = v == kFormerCoopVariant ? kCoopVariant : default_variant(*P);
     if (P->lane_variant != v) drop_graph(*P);
     P->lane_variant = v;
     return SGN_OK;

@@ -107,3 +107,22 @@ def test_damaged_blocks_decode_as_the_oracle_does(session, oracle, variant):
             with pytest.raises((S.J2kError, S.TileBatchError)):
                 S.decode_tiles_to_device(session, [bad], S.PixelFormat.RGB8)
     assert same
+
+
+def test_former_variant_indexes(session):
+    """Indexes 0 to 8 are accepted and decode; 9 and -1 are refused."""
+    img = np.random.default_rng(4).integers(0, 256, (70, 90, 3), dtype=np.uint8)
+    plan = S.TilePlan(session, [S.encode_j2k_lossless(img)], S.PixelFormat.RGB8)
+    names, own = S.TilePlan.lane_variants(), plan.lane_variant
+    for v in range(9):
+        plan.lane_variant = v
+        want = v if v < len(names) else names.index("wave-coop") if v == 6 else own
+        assert plan.lane_variant == want
+        plan.surfaces[0].fill(0x5A)
+        plan.decode(S.MODE_GRAPH)
+        session.synchronize()
+        assert np.array_equal(plan.surfaces[0].to_numpy(), img), v
+    for v in (-1, 9):
+        with pytest.raises(S.J2kError):
+            plan.lane_variant = v
+    plan.close()
