@@ -330,6 +330,10 @@ typedef struct {
     uint64_t pruned_code_blocks;
 } sgn_j2k_plan_stats;
 int sgn_j2k_plan_get_stats(const sgn_j2k_plan *plan, sgn_j2k_plan_stats *stats);
+/* The kernels that a batched decode of the plan launches, one line each: stage,
+ * kernel and how many code-blocks, levels or 64x64 output blocks it takes.  Copies
+ * at most `capacity` bytes, with a closing zero; *length is the whole text's. */
+int sgn_j2k_plan_kernels(const sgn_j2k_plan *plan, char *out, size_t capacity, size_t *length);
 /* Output geometry of tile i: width, height, bytes per row (unpadded). */
 int sgn_j2k_plan_tile_dims(const sgn_j2k_plan *plan, size_t i, uint32_t *width,
                            uint32_t *height, size_t *row_bytes);

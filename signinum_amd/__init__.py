@@ -619,6 +619,17 @@ class TilePlan:
         _check(_lib.load().sgn_j2k_plan_get_stats(self.handle, ctypes.byref(st)))
         return {f: getattr(st, f) for f, _ in PlanStats._fields_}
 
+    def kernels(self):
+        """What a batched decode of the plan launches: (stage, kernel, count)
+        triples, counts in code-blocks, levels or 64x64 output blocks."""
+        L = _lib.load()
+        n = ctypes.c_size_t()
+        _check(L.sgn_j2k_plan_kernels(self.handle, None, 0, ctypes.byref(n)))
+        buf = ctypes.create_string_buffer(n.value + 1)
+        _check(L.sgn_j2k_plan_kernels(self.handle, buf, n.value + 1, None))
+        rows = (line.split() for line in buf.value.decode().splitlines())
+        return [(stage, kernel, int(count)) for stage, kernel, count in rows]
+
     def close(self):
         if getattr(self, "handle", None):
             _lib.load().sgn_j2k_plan_destroy(self.handle)

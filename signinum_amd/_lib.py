@@ -231,6 +231,8 @@ SIGNATURES = {
     "sgn_j2k_plan_decode": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int]),
     "sgn_j2k_plan_decode_stage": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int]),
     "sgn_j2k_plan_get_stats": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(PlanStats)]),
+    "sgn_j2k_plan_kernels": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_char_p, c_size_t,
+                                            ctypes.POINTER(c_size_t)]),
     "sgn_j2k_plan_tile_dims": (ctypes.c_int, [ctypes.c_void_p, c_size_t,
                                               ctypes.POINTER(ctypes.c_uint32),
                                               ctypes.POINTER(ctypes.c_uint32),

@@ -1626,20 +1626,29 @@ bool small_levels(const std::vector<LevelJob> &v, uint32_t a, uint32_t b) {
     return true;
 }
 
+// Kernel of the launch of levels [a, b).  Levels of at most 32x32 take the one-wave
+// kernel where the plan's shape says so (same block count: each is one block for
+// either kernel); the four-wave shapes lift in registers where every level of
+// the launch allows it.
+enum class LevelKind { kSmall, kRows, kGeneral };
+LevelKind level_kind(const sgn_j2k_plan &P, int rev, uint32_t a, uint32_t b) {
+    const DwtShape &g = kDwtShapes[P.dwt_shape];
+    if (g.small && small_levels(P.lv[rev], a, b)) return LevelKind::kSmall;
+    return g.threads == uint32_t(kIdwtThreads) && P.lv_general[rev][a] == P.lv_general[rev][b]
+               ? LevelKind::kRows
+               : LevelKind::kGeneral;
+}
+
 uint32_t launch_levels(sgn_hip_session *s, sgn_j2k_plan &P, int rev, uint32_t a, uint32_t b) {
     const uint32_t blocks = group_blocks(P.lv[rev], a, b);
     if (!blocks) return 0;
     const uint32_t off = P.lv[rev][a].block_base;
     const DwtShape &g = kDwtShapes[P.dwt_shape];
-    // levels of at most 32x32 take the one-wave kernel where the shape says
-    // so (same block count: each is one block for either kernel)
-    const bool small = g.small && small_levels(P.lv[rev], a, b);
-    // the four-wave shapes lift in registers where every level allows it
-    const bool rows = !small && g.threads == uint32_t(kIdwtThreads) &&
-                      P.lv_general[rev][a] == P.lv_general[rev][b];
-    const auto kernel = small  ? (rev ? sgn_idwt_level_rev_small : sgn_idwt_level_irr_small)
-                        : rows ? (rev ? sgn_idwt_rows_rev : sgn_idwt_rows_irr)
-                               : g.kernel[rev];
+    const LevelKind kind = level_kind(P, rev, a, b);
+    const bool small = kind == LevelKind::kSmall;
+    const auto kernel = small ? (rev ? sgn_idwt_level_rev_small : sgn_idwt_level_irr_small)
+                        : kind == LevelKind::kRows ? (rev ? sgn_idwt_rows_rev : sgn_idwt_rows_irr)
+                                                   : g.kernel[rev];
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(small ? Small::kThreads : g.threads), 0,
                        s->stream, P.d_lv[rev], uint32_t(P.lv[rev].size()), off,
                        P.d_lv_block_job[rev], P.d_coef);
@@ -2656,6 +2665,56 @@ int sgn_j2k_plan_get_stats(const sgn_j2k_plan *P, sgn_j2k_plan_stats *st) {
     st->host_copy_ms = float(P->t_copy);
     st->pruned_code_blocks = P->pruned_cbs;
     return SGN_OK;
+}
+
+int sgn_j2k_plan_kernels(const sgn_j2k_plan *P, char *out, size_t cap, size_t *len) {
+    API_GUARD_BEGIN
+    if (!P || (!out && cap)) return SGN_E_ARG;
+    std::string t;
+    auto line = [&](const char *stage, const std::string &kernel, size_t count) {
+        t += std::string(stage) + " " + kernel + " " + std::to_string(count) + "\n";
+    };
+    if (!P->cb_lane.empty())
+        line("blocks", kRowsVariants[P->d_work ? P->lane_variant : kCoopVariant].name,
+             P->cb_lane.size());
+    if (!P->cb_wave.empty()) line("blocks", "wave-coop-1024", P->cb_wave.size());
+    for (int v = 0; v < kClassicShapes; ++v) {
+        const size_t n = P->classic_begin[v + 1] - P->classic_begin[v];
+        static const char *const kShape[kClassicShapes] = {"small", "usual", "long", "usual-raw",
+                                                           "long-raw"};
+        if (!n) continue;
+        const int opt = P->classic_opt[v];
+        line("classic",
+             (opt < kClassicLaneOpts
+                  ? std::string(kShape[v]) + "-l" + std::to_string(classic_lanes(v, opt))
+                  : "rows-w" + std::to_string(kClassicRows[opt - kClassicLaneOpts].max_w)),
+             n);
+    }
+    for (int rev = 0; rev < 2; ++rev) {
+        const std::string w = rev ? "5/3-" : "9/7-";
+        const LevelChain &c = P->chain[rev];
+        for (uint32_t d = 0; d < P->depth_max; ++d) {
+            const uint32_t a = P->lv_group[rev][d], b = P->lv_group[rev][d + 1];
+            if (a == b) continue;
+            const char *kind = "general";
+            if (d < c.levels)
+                kind = (c.general >> d) & 1u ? "chain-general" : "chain-rows";
+            else if (level_kind(*P, rev, a, b) != LevelKind::kGeneral)
+                kind = level_kind(*P, rev, a, b) == LevelKind::kRows ? "rows" : "small";
+            line(("levels" + std::to_string(d + 1)).c_str(), w + kind, b - a);
+        }
+        if (!P->fin_rgb8[rev].empty())
+            line("final", rev ? "5/3-rgb8" : "9/7-rgb8", P->fin_rgb8[rev].size());
+        if (!P->fin_rest[rev].empty()) line("final", w + "general", P->fin_rest[rev].size());
+    }
+    if (len) *len = t.size();
+    if (cap) {
+        const size_t k = std::min(cap - 1, t.size());
+        std::memcpy(out, t.data(), k);
+        out[k] = 0;
+    }
+    return SGN_OK;
+    API_GUARD_END
 }
 
 int sgn_j2k_plan_tile_dims(const sgn_j2k_plan *P, size_t i, uint32_t *w, uint32_t *h,
