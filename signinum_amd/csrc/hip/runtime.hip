@@ -176,33 +176,39 @@ template <int LANES>
 using ClassicSmall = ClassicShape<32, 40, LANES, false>;
 template <int LANES, bool RAW>
 using ClassicUsual = ClassicShape<128, 144, LANES, RAW>;
-template <int LANES, bool RAW>
-using ClassicLong = ClassicShape<256, 384, LANES, RAW>;
+template <bool RAW>
+using ClassicLong = ClassicShape<256, 384, 1, RAW>;
 // Lanes per wave, and the most blocks per CU of a list that takes them: more
-// lanes decode more blocks at once, fewer wait less for each other.  32x32
-// blocks (210 a tile of 256x256): 16 tiles take 4.7, 5.3, 6.4 and 9.1 ms with
-// one, two, four and sixteen lanes, 64 tiles 9.1, 5.6, 6.2 and 9.0, 128 tiles
-// 17.7, 10.3, 6.5 and 9.1, 256 tiles 34.7, 20.1, 12.2 and 8.6.  64x64 blocks (75
-// a tile): up to 64 tiles 17.8 ms with one (the longest chain) and 22 with
-// three, 256 tiles 35.6 and 21.3.  Lists past the last line go to sgn_t1_rows,
-// whose header has the figures.
+// lanes decode more blocks at once, fewer wait less for each other; lists past
+// the last line go to sgn_t1_rows.  Each line is where the two kernels beside it
+// took the same time on lists of distinct tiles of 256x256 (neighbouring lanes
+// of a list that repeats a few tiles decode the same bits, which flatters the
+// kernels that walk in step):
+//   32x32 blocks (210 a tile), ms with 1, 2, 4 and 16 lanes and in rows: 32 tiles
+//   4.8, 5.25; 36 tiles 5.4, 5.2; 68 tiles -, 5.9, 6.2; 78 tiles -, 6.75, 6.1; 168
+//   tiles -, -, 8.6, 9.0; 180 tiles -, -, 9.25, 8.9; 544 tiles -, -, -, 21.0, 21.8;
+//   1024 tiles -, -, -, 40.6, 30.5.
+//   64x64 blocks (75 a tile), 1 and 3 lanes and in rows: up to 109 tiles 17 to 18
+//   (the longest chain), 23; 160 tiles 22.4, 22.4; 168 tiles 23.4, 22.3; 896 tiles
+//   -, 63.2, 68.9; 960 tiles -, 68.2, 68.0; 1024 tiles -, 72.2, 69.1.
+//   128x32 blocks (48 a tile without levels), 1 lane and in rows: 171 tiles 51, 61;
+//   213 tiles 57, 61; 256 tiles 71, 61.  Three lanes took 55, 68 and 75: their state
+//   leaves a CU too few waves.
 struct ClassicChoice {
     ClassicKernel kernel;
     uint32_t lanes, per_cu;
 };
 const ClassicChoice kClassicKernels[kClassicShapes][kClassicLaneOpts] = {
-    {{sgn_t1_classic<ClassicSmall<1>>, 1, 16},
-     {sgn_t1_classic<ClassicSmall<2>>, 2, 64},
-     {sgn_t1_classic<ClassicSmall<4>>, 4, 128},
-     {sgn_t1_classic<ClassicSmall<16>>, 16, 384}},
-    {{sgn_t1_classic<ClassicUsual<1, false>>, 1, 32},
-     {sgn_t1_classic<ClassicUsual<3, false>>, 3, 192}},
-    {{sgn_t1_classic<ClassicLong<1, false>>, 1, 32},
-     {sgn_t1_classic<ClassicLong<3, false>>, 3, 64}},
-    {{sgn_t1_classic<ClassicUsual<1, true>>, 1, 32},
-     {sgn_t1_classic<ClassicUsual<3, true>>, 3, 192}},
-    {{sgn_t1_classic<ClassicLong<1, true>>, 1, 32},
-     {sgn_t1_classic<ClassicLong<3, true>>, 3, 64}}};
+    {{sgn_t1_classic<ClassicSmall<1>>, 1, 28},
+     {sgn_t1_classic<ClassicSmall<2>>, 2, 58},
+     {sgn_t1_classic<ClassicSmall<4>>, 4, 142},
+     {sgn_t1_classic<ClassicSmall<16>>, 16, 450}},
+    {{sgn_t1_classic<ClassicUsual<1, false>>, 1, 46},
+     {sgn_t1_classic<ClassicUsual<3, false>>, 3, 280}},
+    {{sgn_t1_classic<ClassicLong<false>>, 1, 42}},
+    {{sgn_t1_classic<ClassicUsual<1, true>>, 1, 46},
+     {sgn_t1_classic<ClassicUsual<3, true>>, 3, 280}},
+    {{sgn_t1_classic<ClassicLong<true>>, 1, 42}}};
 // ... and of the row kernels by block width.
 using ClassicRowsKernel = void (*)(const ClassicJob *, uint32_t, const uint8_t *,
                                    const ClassicSeg *, int32_t *, uint32_t *);

@@ -8,9 +8,9 @@
 // needs 400 bytes of LDS where sgn_t1_classic keeps 1.2 to 10 KB, and many more
 // blocks are in flight.  Every turn costs more: the lanes wait at every sample
 // that any of them decides.  Lists of 64x64 blocks and smaller ones (75 a tile of
-// 256x256) take about 50 ms here up to 1024 tiles and 62 for 2048, where
-// sgn_t1_classic takes 33, 49, 66 and 136 for 512, 768, 1024 and 2048; 512 tiles
-// in 32x32 blocks (107,520) 17.3 and 18.1, 1024 tiles 26 and 35.  Magnitude bits go to the
+// 256x256, all tiles distinct) take 67, 69, 74 and 86 ms here for 512, 1024, 1536
+// and 2048 tiles, where sgn_t1_classic takes 37, 72, 108 and 144; 512 tiles in 32x32
+// blocks (107,520) 20.8 and 20.7, 1024 tiles 30 and 41.  Magnitude bits go to the
 // block's int32 coefficients in HBM by atomic OR; the block is zeroed first and
 // the signs are applied in a final sweep.
 #include <hip/hip_runtime.h>
