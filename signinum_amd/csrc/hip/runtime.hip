@@ -1226,7 +1226,8 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
     const uint64_t o_stl = take(P.cb_lane.size()), o_stw = take(P.cb_wave.size());
     const uint64_t o_ff = take(P.fin_block_job[1].size() * sizeof(uint32_t));
     // classic kernels by the length of each list (SGN_CLASSIC_LANES forces a
-    // lane count of the shape, or with 32 the row kernels)
+    // lane count that the shape has; else from 16 on the row kernels, as its
+    // former values 64, 32 and 16 did)
     uint64_t crows_bytes = 0;
     const char *lanes_env = std::getenv("SGN_CLASSIC_LANES");
     const uint32_t forced = lanes_env ? uint32_t(std::atoi(lanes_env)) : 0u;
@@ -1243,7 +1244,7 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
         int opt = 0;
         auto ends = [&](int o) { return o >= kClassicLaneOpts || !kClassicKernels[v][o].kernel; };
         while (!ends(opt) && n > kClassicKernels[v][opt].per_cu * session_cus(s)) ++opt;
-        bool by_rows = ends(opt) || forced == 32;
+        bool by_rows = ends(opt) || forced >= 16;
         for (int o = 0; !ends(o); ++o)
             if (kClassicKernels[v][o].lanes == forced) {
                 opt = o;

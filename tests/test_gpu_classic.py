@@ -96,8 +96,8 @@ def test_classic_styles_on_device(session, oracle):
 
 @pytest.mark.parametrize("lanes", ["64", "32", "16"])
 def test_classic_lanes_per_wave(session, oracle, monkeypatch, lanes):
-    """Every active-lane count of the classic kernels (64, 32 or 16 blocks
-    per wave) on blocks of every width class, against the oracle."""
+    """The row kernels (and, with 16, the sixteen-lane kernel of small blocks)
+    on blocks of every width class, against the oracle."""
     monkeypatch.setenv("SGN_CLASSIC_LANES", lanes)
     rng = np.random.default_rng(36)
     streams, want = [], []
@@ -111,6 +111,8 @@ def test_classic_lanes_per_wave(session, oracle, monkeypatch, lanes):
         streams += streams[:4]
         want += want[:4]
     plan = S.TilePlan(session, streams, S.PixelFormat.RGB8)
+    assert all(k.startswith("rows-") or (lanes == "16" and k == "small-l16")
+               for stage, k, _n in plan.kernels() if stage == "classic")
     plan.decode(S.MODE_GRAPH)
     session.synchronize()
     for k, s in enumerate(plan.surfaces):

@@ -59,3 +59,18 @@ def test_long_blocks(session, exps, style, kernel):
     assert _kernels(plan) == [kernel]
     _check(session, plan, imgs)
     plan.close()
+
+
+@pytest.mark.parametrize("lanes,usual,small,long", [
+    ("64", "rows-w64", "rows-w32", "rows-w256"), ("32", "rows-w64", "rows-w32", "rows-w256"),
+    ("16", "rows-w64", "small-l16", "rows-w256"), ("4", "usual-l1", "small-l4", "long-l1"),
+    ("3", "usual-l3", "small-l1", "long-l1"), ("1", "usual-l1", "small-l1", "long-l1"),
+    ("5", "usual-l1", "small-l1", "long-l1")])
+def test_forced_lanes(session, monkeypatch, lanes, usual, small, long):
+    """A forced count names a kernel of the shape, or the row kernels, or nothing."""
+    monkeypatch.setenv("SGN_CLASSIC_LANES", lanes)
+    for exps, kernel in (((6, 6), usual), ((5, 5), small), ((7, 5), long)):
+        plan, imgs = _plan(session, *exps, blocks=70, side=256)
+        assert _kernels(plan) == [kernel]
+        _check(session, plan, imgs)
+        plan.close()
