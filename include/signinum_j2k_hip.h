@@ -10,6 +10,11 @@
  * be used from one host thread at a time; separate sessions may be used
  * concurrently (crates/signinum-j2k-cuda/src/session.rs:11-49 has the same
  * rule for CudaSession).
+ *
+ * Device memory: a session keeps device blocks of finished calls for the next
+ * ones until it is destroyed: up to 4 GiB of plan and output blocks of
+ * synchronous decodes, and up to 16 GiB of chunk plans if pipelined batches ran.
+ * An allocation of the session that does not fit otherwise takes them back first.
  */
 #ifndef SIGNINUM_J2K_HIP_H
 #define SIGNINUM_J2K_HIP_H

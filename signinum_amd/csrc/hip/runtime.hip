@@ -26,6 +26,7 @@
 #include <thread>
 #include <vector>
 
+#include "../host/block_cache.hpp"
 #include "../host/host_images.hpp"
 #include "../host/parse.hpp"
 #include "../host/sgn_api.hpp"
@@ -51,7 +52,21 @@ using namespace sgn;
         }                                                                          \
     } while (0)
 
-class DeviceBlocks;
+// Device blocks kept for reuse: a serving loop and synchronous decodes allocate
+// and release plan and output blocks continuously, and hipFree waits for the
+// whole device, so a freed block would stall every batch in flight.
+struct HipMemory {
+    static int alloc(void **out, uint64_t bytes) {
+        const hipError_t e = hipMalloc(out, bytes);
+        if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch
+        return int(e);
+    }
+    static void free(void *p) { (void)hipFree(p); }
+};
+using DeviceBlocks = sgn::BlockCache<HipMemory>;
+// What a session keeps: chunks of pipelined batches, and the plan and output
+// blocks of other synchronous decodes (which hold no more than one call's).
+constexpr uint64_t kPipelineCache = uint64_t(16) << 30, kCallCache = uint64_t(4) << 30;
 
 // Device memory of sgn_j2k_decode_tiles_device_noalloc: every plan that
 // entry point decodes (codestream arena, job tables, status words, work
@@ -88,7 +103,8 @@ struct sgn_hip_session {
     hipStream_t aux_stream = nullptr;  // second decode stream: chunks alternate
     PinnedSlot slot[2];
     PinnedSlot down[2], stat;        // downloads to host arrays (two chunks), block status words
-    DeviceBlocks *blocks = nullptr;  // device blocks of the plans of one call, reused
+    DeviceBlocks *blocks = nullptr;       // device blocks of pipelined chunk plans, reused
+    DeviceBlocks *call_blocks = nullptr;  // of the other synchronous decodes
 };
 
 namespace {
@@ -318,57 +334,6 @@ struct sgn_cost_model {
         for (void *p : ptrs)
             if (p) (void)hipFree(p);
     }
-};
-
-// Device blocks kept for reuse instead of freed: a serving loop allocates
-// and releases plan and output blocks continuously, and hipFree waits for
-// the whole device, so a freed block would stall every batch in flight.
-// get() hands out a cached block of at least `bytes` (at most twice that,
-// plus 1 MiB) or allocates one; put() caches it, freeing the largest cached
-// blocks while more than `cap` bytes are cached.  Not thread-safe: one
-// owner (the server) drives it.
-class DeviceBlocks {
-  public:
-    explicit DeviceBlocks(uint64_t cap) : cap_(cap) {}
-    ~DeviceBlocks() { trim(0); }
-    DeviceBlocks(const DeviceBlocks &) = delete;
-    DeviceBlocks &operator=(const DeviceBlocks &) = delete;
-    hipError_t get(uint64_t bytes, void **out) {
-        bytes = std::max<uint64_t>(bytes, 256);
-        auto it = free_.lower_bound(bytes);
-        if (it != free_.end() && it->first <= 2 * bytes + (uint64_t(1) << 20)) {
-            *out = it->second;
-            size_[*out] = it->first;
-            cached_ -= it->first;
-            free_.erase(it);
-            return hipSuccess;
-        }
-        const hipError_t e = hipMalloc(out, bytes);
-        if (e == hipSuccess) size_[*out] = bytes;
-        return e;
-    }
-    void put(void *p) {
-        if (!p) return;
-        const auto it = size_.find(p);
-        if (it == size_.end()) return;
-        free_.emplace(it->second, p);
-        cached_ += it->second;
-        size_.erase(it);
-        trim(cap_);
-    }
-
-  private:
-    void trim(uint64_t keep) {
-        while (cached_ > keep && !free_.empty()) {
-            auto last = std::prev(free_.end());
-            (void)hipFree(last->second);
-            cached_ -= last->first;
-            free_.erase(last);
-        }
-    }
-    uint64_t cap_, cached_ = 0;
-    std::multimap<uint64_t, void *> free_;         // cached: size -> block
-    std::unordered_map<void *, uint64_t> size_;   // handed out: block -> size
 };
 
 struct sgn_j2k_plan {
@@ -1327,8 +1292,8 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
         P.t_stage = 0;
         P.t_copy = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() -
                                                               t0).count();
-    } else if ((P.blocks ? P.blocks->get(off, &P.d_block) : hipMalloc(&P.d_block, off)) !=
-               hipSuccess) {
+    } else if (P.blocks ? P.blocks->get(off, &P.d_block)
+                        : s->call_blocks->alloc(off, &P.d_block)) {
         P.d_block = nullptr;
         set_last_error("hipMalloc failed for the plan (" + std::to_string(off) + " bytes)");
         return kErrDevice;
@@ -2094,7 +2059,7 @@ Status decode_once(sgn_hip_session *s, const sgn_tile_req *reqs, size_t n, int m
                    size_t *first_fail, F after) {
     std::vector<int32_t> ts(n, 0);
     std::unique_ptr<sgn_j2k_plan> P;
-    Status st = make_plan(s, reqs, n, P, ts.data(), s->blocks, false);
+    Status st = make_plan(s, reqs, n, P, ts.data(), s->call_blocks, false);
     if (st) {
         if (first_fail)
             for (size_t i = 0; i < n; ++i)
@@ -2202,8 +2167,8 @@ Status decode_to_host(sgn_hip_session *s, const sgn_tile_req *reqs, size_t n,
         images[i].off = total;
         total = (total + images[i].row * images[i].rows + 255) & ~size_t(255);
     }
-    CachedBlock out{s->blocks};
-    if (s->blocks->get(std::max<size_t>(1, total), &out.p) != hipSuccess) {
+    CachedBlock out{s->call_blocks};
+    if (s->call_blocks->get(std::max<size_t>(1, total), &out.p)) {
         out.p = nullptr;
         set_last_error("hipMalloc failed for the output (" + std::to_string(total) + " bytes)");
         return kErrDevice;
@@ -2270,7 +2235,9 @@ int sgn_hip_session_create(int device, sgn_hip_session **out) {
     HIP_TRY(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
     HIP_TRY(hipStreamCreateWithFlags(&s->copy_stream, hipStreamNonBlocking));
     HIP_TRY(hipStreamCreateWithFlags(&s->aux_stream, hipStreamNonBlocking));
-    s->blocks = new DeviceBlocks(uint64_t(16) << 30);
+    s->blocks = new DeviceBlocks(kPipelineCache);
+    s->call_blocks = new DeviceBlocks(kCallCache, s->blocks);
+    s->blocks->set_sibling(s->call_blocks);
     const HtTables &T = ht_tables();
     std::vector<uint16_t> tab(2624);
     std::memcpy(tab.data(), T.vlc0, 2048);
@@ -2305,6 +2272,7 @@ void sgn_hip_session_destroy(sgn_hip_session *s) {
         if (sl->p) (void)hipHostFree(sl->p);
         if (sl->done) (void)hipEventDestroy(sl->done);
     }
+    delete s->call_blocks;
     delete s->blocks;
     if (s->d_tables) (void)hipFree(s->d_tables);
     if (s->d_split) (void)hipFree(s->d_split);
@@ -2322,11 +2290,17 @@ int sgn_hip_session_synchronize(sgn_hip_session *s) {
 uint64_t sgn_hip_session_dispatches(sgn_hip_session *s) { return s ? s->dispatches : 0; }
 
 int sgn_device_alloc(sgn_hip_session *s, size_t bytes, void **out) {
+    API_GUARD_BEGIN
     if (!s || !out) return SGN_E_ARG;
     *out = nullptr;
     HIP_TRY(hipSetDevice(s->device));
-    HIP_TRY(hipMalloc(out, bytes ? bytes : 1));
+    if (const int e = s->call_blocks->alloc(bytes ? bytes : 1, out)) {
+        *out = nullptr;
+        set_last_error(std::string("HIP: ") + hipGetErrorString(hipError_t(e)));
+        return SGN_E_DEVICE;
+    }
     return SGN_OK;
+    API_GUARD_END
 }
 
 void sgn_device_free(sgn_hip_session *s, void *p) {
@@ -3519,7 +3493,10 @@ int sgn_j2k_plan_order_code_blocks(sgn_hip_session *s, sgn_j2k_plan *P, int orde
     HIP_TRY(hipStreamSynchronize(s->stream));
     if (P->d_work && units > P->work_cap) {
         void *own = nullptr;
-        HIP_TRY(hipMalloc(&own, units * sizeof(uint4)));
+        if (s->call_blocks->alloc(units * sizeof(uint4), &own)) {
+            set_last_error("hipMalloc failed for the workspace");
+            return SGN_E_DEVICE;
+        }
         if (P->d_work_own) (void)hipFree(P->d_work_own);
         P->d_work_own = own;
         P->d_work = static_cast<uint4 *>(own);

@@ -205,7 +205,7 @@ Status launch_batch(sgn_server &S, bool force) {
             size_t total = 0;
             for (size_t t = 0; t < r.bytes.size(); ++t)
                 total += (std::max<size_t>(16, r.row_bytes[t] * r.height[t]) + 255) & ~size_t(255);
-            HIP_TRY(S.blocks->get(total, &r.out_block));
+            HIP_TRY(hipError_t(S.blocks->get(total, &r.out_block)));
             size_t o = 0;
             for (size_t t = 0; t < r.bytes.size(); ++t) {
                 r.out[t] = static_cast<uint8_t *>(r.out_block) + o;
