@@ -1141,58 +1141,13 @@ Status slot_reserve(PinnedSlot &sl, size_t bytes, uint8_t **out,
     return kOk;
 }
 
-// One device allocation per plan: codestream arena, job tables, status
-// words, work counter and coefficient arena, carved at 256-byte alignment.
-// Codestream runs of at least 64 KB in pinned host memory are copied
-// straight from the caller's memory; the other runs and the tables are
-// staged in the session's pinned slot `slot` and go up in as few copies as
-// the run layout allows.  Copies are enqueued on `copy`; the caller orders
-// the decode after them (same stream or an event).  With sync the call
-// returns after the copies completed.
-// With `fixed` (fixed_cap bytes of device memory the caller owns) nothing is
-// allocated: the plan is carved from it, every run and table is copied
-// straight from host memory (no pinned staging), and the call returns after
-// the copies completed.
 uint32_t classic_resident(sgn_hip_session *s, int v, int opt);
 uint32_t session_cus(sgn_hip_session *s);
 
-Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P,
-                   hipStream_t copy, int slot, bool sync, void *fixed = nullptr,
-                   uint64_t fixed_cap = 0) {
-    (void)jobs;
-    const auto t0 = std::chrono::steady_clock::now();
-    uint64_t off = 0;
-    auto take = [&](uint64_t bytes) {
-        const uint64_t o = off;
-        off = (off + bytes + 255) & ~uint64_t(255);
-        return o;
-    };
-    auto bytes_of = [](const auto &v) { return uint64_t(v.size()) * sizeof(v[0]); };
-    const uint64_t o_arena = take(P.arena_len);
-    const uint64_t o_tables = off;
-    const uint64_t o_lane = take(bytes_of(P.cb_lane)), o_plain = take(bytes_of(P.cb_lane_plain));
-    const uint64_t o_wave = take(bytes_of(P.cb_wave)), o_ref = take(bytes_of(P.cb_refine));
-    const uint64_t o_lv0 = take(bytes_of(P.lv[0])), o_lv1 = take(bytes_of(P.lv[1]));
-    const uint64_t o_fin0 = take(bytes_of(P.fin[0])), o_fin1 = take(bytes_of(P.fin[1]));
-    const uint64_t o_flv = take(bytes_of(P.final_lv));
-    const uint64_t o_lbj0 = take(bytes_of(P.lv_block_job[0])), o_lbj1 = take(bytes_of(P.lv_block_job[1]));
-    const uint64_t o_fbj0 = take(bytes_of(P.fin_block_job[0])), o_fbj1 = take(bytes_of(P.fin_block_job[1]));
-    const uint64_t o_cls = take(bytes_of(P.classic)), o_cseg = take(bytes_of(P.cseg));
-    const uint64_t o_sto = take(bytes_of(P.store)), o_sbj = take(bytes_of(P.store_block_job));
-    const uint64_t o_pkt = take(bytes_of(P.pk_tiles)), o_pkp = take(bytes_of(P.pk_parts));
-    const uint64_t o_pkk = take(bytes_of(P.pk_pkts)), o_pkb = take(bytes_of(P.pk_bands));
-    const uint64_t o_pkc = take(bytes_of(P.pk_cbs)), o_grp = take(bytes_of(P.groups));
-    const uint64_t o_frg[2] = {take(bytes_of(P.fin_rgb8[0])), take(bytes_of(P.fin_rgb8[1]))};
-    const uint64_t o_frs[2] = {take(bytes_of(P.fin_rest[0])), take(bytes_of(P.fin_rest[1]))};
-    const uint64_t o_rgr = take(bytes_of(P.ref_groups));
-    const uint64_t host_bytes = off;
-    const uint64_t o_pkn = take(P.pk_nodes * 2 * sizeof(uint32_t));
-    const uint64_t o_pkl = take(P.pk_cbs.size() * sizeof(uint32_t)), o_pks = take(P.pk_tiles.size());
-    const uint64_t o_stl = take(P.cb_lane.size()), o_stw = take(P.cb_wave.size());
-    const uint64_t o_ff = take(P.fin_block_job[1].size() * sizeof(uint32_t));
-    // classic kernels by the length of each list (SGN_CLASSIC_LANES forces a
-    // lane count that the shape has; else from 16 on the row kernels, as its
-    // former values 64, 32 and 16 did)
+// Chooses the classic kernels, by the length of each list (SGN_CLASSIC_LANES forces
+// a lane count that the shape has; else from 16 on the row kernels, as its former
+// values 64, 32 and 16 did).  Returns the bytes of their lanes' memory.
+uint64_t choose_classic(sgn_hip_session *s, sgn_j2k_plan &P, bool tight) {
     uint64_t crows_bytes = 0;
     const char *lanes_env = std::getenv("SGN_CLASSIC_LANES");
     const uint32_t forced = lanes_env ? uint32_t(std::atoi(lanes_env)) : 0u;
@@ -1215,10 +1170,14 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
                 opt = o;
                 by_rows = false;
             }
-        // in fixed memory the lanes' magnitude bits keep to 3 KB a block (a
-        // row store's size)
+        // tight: the lanes' magnitude bits keep to 3 KB a block (a row store's
+        // size), 16 blocks at least; one lane's 63 KB may be more than that
         const uint64_t budget = std::max<uint64_t>(n, 16) * rows::kStateDwords * 4;
-        if (fixed && !by_rows && uint64_t(classic_lanes(v, opt)) * mag * 4 > budget) opt = 0;
+        if (tight && !by_rows && uint64_t(classic_lanes(v, opt)) * mag * 4 > budget) {
+            opt = 0;
+            by_rows = uint64_t(mag) * 4 > budget;
+            if (by_rows) width = rows::W1024::kMaxW;
+        }
         if (by_rows) {
             opt = kClassicLaneOpts;
             while (kClassicRows[opt - kClassicLaneOpts].max_w < width) ++opt;
@@ -1227,21 +1186,101 @@ Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P
         const uint32_t lanes = classic_lanes(v, opt);
         const uint64_t group_bytes = uint64_t(lanes) * mag * 4;
         uint64_t grid = std::min((n + lanes - 1) / lanes, classic_resident(s, v, opt));
-        if (fixed && !by_rows && group_bytes)
+        if (tight && !by_rows && group_bytes)
             grid = std::min(grid, std::max<uint64_t>(budget / group_bytes, 1));
         P.classic_opt[v] = opt;
         P.classic_mag[v] = mag;
         P.classic_grid[v] = static_cast<uint32_t>(grid);
         crows_bytes = std::max(crows_bytes, grid * group_bytes);
     }
-    const uint64_t o_crows = take(crows_bytes);
-    const uint64_t o_queue = take(64), o_coef = take(P.coef_elems * sizeof(uint32_t));
-    // the workspaces last: a plan carved from fixed memory does without when
-    // they do not fit (the cooperative kernel needs none)
-    const uint64_t no_work = off, o_work = take(P.work_units * sizeof(uint4));
-    const uint64_t o_rwork = take(P.ref_units * sizeof(uint4));
-    const bool has_work = P.work_units != 0 && !(fixed && off > fixed_cap);
-    if (!has_work) off = no_work;
+    return crows_bytes;
+}
+
+// One device allocation per plan: codestream arena, job tables, status
+// words, work counter and coefficient arena, carved at 256-byte alignment.
+// Codestream runs of at least 64 KB in pinned host memory are copied
+// straight from the caller's memory; the other runs and the tables are
+// staged in the session's pinned slot `slot` and go up in as few copies as
+// the run layout allows.  Copies are enqueued on `copy`; the caller orders
+// the decode after them (same stream or an event).  With sync the call
+// returns after the copies completed.
+// With `fixed` (fixed_cap bytes of device memory the caller owns) nothing is
+// allocated: the plan is carved from it, every run and table is copied
+// straight from host memory (no pinned staging), and the call returns after
+// the copies completed.  A plan of more than `limit` bytes is laid out without
+// what only its faster kernels need; if it is larger all the same and too_big is
+// given, that is set and the call fails before any device work.
+Status upload_plan(sgn_hip_session *s, const sgn_tile_req *jobs, sgn_j2k_plan &P,
+                   hipStream_t copy, int slot, bool sync, void *fixed = nullptr,
+                   uint64_t fixed_cap = 0, uint64_t limit = UINT64_MAX, bool *too_big = nullptr) {
+    (void)jobs;
+    const auto t0 = std::chrono::steady_clock::now();
+    uint64_t off = 0;
+    auto take = [&](uint64_t bytes) {
+        const uint64_t o = off;
+        off = (off + bytes + 255) & ~uint64_t(255);
+        return o;
+    };
+    auto bytes_of = [](const auto &v) { return uint64_t(v.size()) * sizeof(v[0]); };
+    const uint64_t o_arena = take(P.arena_len);
+    const uint64_t o_tables = off;
+    const uint64_t o_lane = take(bytes_of(P.cb_lane)), o_plain = take(bytes_of(P.cb_lane_plain));
+    const uint64_t o_wave = take(bytes_of(P.cb_wave)), o_ref = take(bytes_of(P.cb_refine));
+    const uint64_t o_lv0 = take(bytes_of(P.lv[0])), o_lv1 = take(bytes_of(P.lv[1]));
+    const uint64_t o_fin0 = take(bytes_of(P.fin[0])), o_fin1 = take(bytes_of(P.fin[1]));
+    const uint64_t o_flv = take(bytes_of(P.final_lv));
+    const uint64_t o_lbj0 = take(bytes_of(P.lv_block_job[0])), o_lbj1 = take(bytes_of(P.lv_block_job[1]));
+    const uint64_t o_fbj0 = take(bytes_of(P.fin_block_job[0])), o_fbj1 = take(bytes_of(P.fin_block_job[1]));
+    const uint64_t o_cls = take(bytes_of(P.classic)), o_cseg = take(bytes_of(P.cseg));
+    const uint64_t o_sto = take(bytes_of(P.store)), o_sbj = take(bytes_of(P.store_block_job));
+    const uint64_t o_pkt = take(bytes_of(P.pk_tiles)), o_pkp = take(bytes_of(P.pk_parts));
+    const uint64_t o_pkk = take(bytes_of(P.pk_pkts)), o_pkb = take(bytes_of(P.pk_bands));
+    const uint64_t o_pkc = take(bytes_of(P.pk_cbs));
+    uint64_t o_grp = 0, o_frg[2] = {}, o_frs[2] = {}, o_rgr = 0, host_bytes = 0, o_pkn = 0, o_pkl = 0,
+             o_pks = 0, o_stl = 0, o_stw = 0, o_ff = 0, crows_bytes = 0, o_crows = 0, o_queue = 0,
+             o_coef = 0, o_work = 0, o_rwork = 0;
+    // What only the faster kernels need goes where the plan would not fit its
+    // memory with it: first the workspaces of the split kernels (the cooperative
+    // kernel needs none) and classic magnitude bits past a row store's size, then
+    // the lists of blocks by final kernel (the general one takes them all).
+    const uint64_t cap = fixed ? fixed_cap : limit, always = off;
+    for (int lean = 0; lean < 3; ++lean) {
+        off = always;
+        if (lean == 1) {
+            P.groups.clear();
+            P.ref_groups.clear();
+            P.work_units = P.ref_units = 0;
+        } else if (lean == 2) {
+            for (int r = 0; r < 2; ++r) {
+                P.fin_rgb8[r].clear();
+                P.fin_rest[r].clear();
+            }
+        }
+        o_grp = take(bytes_of(P.groups));
+        for (int r = 0; r < 2; ++r) o_frg[r] = take(bytes_of(P.fin_rgb8[r]));
+        for (int r = 0; r < 2; ++r) o_frs[r] = take(bytes_of(P.fin_rest[r]));
+        o_rgr = take(bytes_of(P.ref_groups));
+        host_bytes = off;
+        o_pkn = take(P.pk_nodes * 2 * sizeof(uint32_t));
+        o_pkl = take(P.pk_cbs.size() * sizeof(uint32_t));
+        o_pks = take(P.pk_tiles.size());
+        o_stl = take(P.cb_lane.size());
+        o_stw = take(P.cb_wave.size());
+        o_ff = take(P.fin_block_job[1].size() * sizeof(uint32_t));
+        crows_bytes = choose_classic(s, P, fixed || lean);
+        o_crows = take(crows_bytes);
+        o_queue = take(64);
+        o_coef = take(P.coef_elems * sizeof(uint32_t));
+        o_work = take(P.work_units * sizeof(uint4));
+        o_rwork = take(P.ref_units * sizeof(uint4));
+        if (off <= cap) break;
+    }
+    const bool has_work = P.work_units != 0;
+    if (too_big && off > limit) {
+        *too_big = true;
+        set_last_error("the plan needs " + std::to_string(off) + " bytes of device memory");
+        return kErrDevice;
+    }
     P.device_bytes = off;
     if (fixed) {
         if (off > fixed_cap) {
@@ -1852,7 +1891,8 @@ void drop_graph(sgn_j2k_plan &P) {
 
 Status make_plan(sgn_hip_session *s, const sgn_tile_req *jobs, size_t n,
                  std::unique_ptr<sgn_j2k_plan> &out, int32_t *tile_status,
-                 DeviceBlocks *blocks = nullptr, bool sync = true) {
+                 DeviceBlocks *blocks = nullptr, bool sync = true, uint64_t limit = UINT64_MAX,
+                 bool *too_big = nullptr) {
     if (!s || (!jobs && n)) {
         set_last_error("null session or jobs");
         return kErrArg;
@@ -1862,7 +1902,7 @@ Status make_plan(sgn_hip_session *s, const sgn_tile_req *jobs, size_t n,
     P->blocks = blocks;
     Status st = build_plan(jobs, n, *P, tile_status);
     if (st) return st;
-    st = upload_plan(s, jobs, *P, s->stream, 0, sync);
+    st = upload_plan(s, jobs, *P, s->stream, 0, sync, nullptr, 0, limit, too_big);
     if (st) {
         (void)hipStreamSynchronize(s->stream);  // before the block goes back
         return st;
@@ -3502,13 +3542,14 @@ int sgn_j2k_plan_order_code_blocks(sgn_hip_session *s, sgn_j2k_plan *P, int orde
         P->d_work = static_cast<uint4 *>(own);
         P->work_cap = units;
     }
-    P->work_units = units;
+    if (P->d_work) P->work_units = units;
     if (!v.empty()) {
         HIP_TRY(hipMemcpy(P->d_cb_lane, v.data(), v.size() * sizeof(CbJob), hipMemcpyHostToDevice));
-        HIP_TRY(hipMemcpy(P->d_groups, groups.data(), groups.size() * sizeof(HtGroup),
-                          hipMemcpyHostToDevice));
+        if (P->d_work)
+            HIP_TRY(hipMemcpy(P->d_groups, groups.data(), groups.size() * sizeof(HtGroup),
+                              hipMemcpyHostToDevice));
     }
-    P->groups.swap(groups);
+    if (P->d_work) P->groups.swap(groups);
     P->cb_lane.swap(v);
     drop_graph(*P);
     return SGN_OK;

@@ -87,3 +87,21 @@ def test_noalloc_rejects_batch_beyond_scratch(session):
     rc, _ = _decode(session, keep[:1], surfs[:1], fmt, True)
     assert rc == 0, _lib.last_error()
     assert np.array_equal(surfs[0].to_numpy(), img)
+
+
+@pytest.mark.parametrize("encode,opts,side,tiles", [
+    (S.encode_j2k_ht, {}, 16, 8015), (S.encode_j2k_ht, dict(ht_refine=2), 24, 5182),
+    (S.encode_j2k_ht, dict(reversible=0, base_step=1 / 64), 32, 4194),
+    (S.encode_j2k_classic, {}, 24, 4507)])
+def test_noalloc_largest_batches(session, encode, opts, side, tiles):
+    """Batches up to the scratch's limit: what only the faster kernels need is left
+    out of the plan rather than the batch refused."""
+    img = np.random.default_rng(1).integers(0, 256, (side, side, 3), dtype=np.uint8)
+    cs = encode(img, levels=1, use_mct=1, **opts)
+    keep = np.frombuffer(cs, np.uint8)
+    surf = S._alloc_surfaces(session, [(side, side)], [S.PixelFormat.RGB8])[0]
+    surf.fill(0)
+    rc, _ = _decode(session, [keep] * tiles, [surf] * tiles, S.PixelFormat.RGB8, True)
+    assert rc == 0, _lib.last_error()
+    if opts.get("reversible", 1) and not opts.get("ht_refine"):
+        assert np.array_equal(surf.to_numpy(), img)
