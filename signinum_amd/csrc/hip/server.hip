@@ -196,29 +196,53 @@ Status launch_batch(sgn_server &S, bool force) {
         ++taken;
     }
     if (!taken) return kOk;  // the oldest request waits for memory to free up
-    // outputs
-    size_t ti = 0;
-    for (uint64_t id : B->ids) {
-        ServeRequest &r = *S.reqs[id];
-        if (!r.out_block) {
-            // one allocation per request, surfaces at 256-byte alignment
-            size_t total = 0;
-            for (size_t t = 0; t < r.bytes.size(); ++t)
-                total += (std::max<size_t>(16, r.row_bytes[t] * r.height[t]) + 255) & ~size_t(255);
-            HIP_TRY(hipError_t(S.blocks->get(total, &r.out_block)));
-            size_t o = 0;
-            for (size_t t = 0; t < r.bytes.size(); ++t) {
-                r.out[t] = static_cast<uint8_t *>(r.out_block) + o;
-                o += (std::max<size_t>(16, r.row_bytes[t] * r.height[t]) + 255) & ~size_t(255);
-            }
-        }
-        for (size_t t = 0; t < r.bytes.size(); ++t, ++ti) tiles[ti].dst = r.out[t];
-        if (!r.out_counted) S.hbm_in_use += r.out_bytes;
-        r.out_counted = true;
-    }
-    std::vector<int32_t> ts(tiles.size(), 0);
+    std::vector<int32_t> ts;
     sgn_hip_session *sess = S.slots[size_t(slot)];
-    Status st = make_plan(sess, tiles.data(), tiles.size(), B->plan, ts.data(), S.blocks.get());
+    Status st = kOk;
+    for (;;) {
+        // outputs
+        size_t ti = 0;
+        for (uint64_t id : B->ids) {
+            ServeRequest &r = *S.reqs[id];
+            if (!r.out_block) {
+                // one allocation per request, surfaces at 256-byte alignment
+                size_t total = 0;
+                for (size_t t = 0; t < r.bytes.size(); ++t)
+                    total += (std::max<size_t>(16, r.row_bytes[t] * r.height[t]) + 255) & ~size_t(255);
+                HIP_TRY(hipError_t(S.blocks->get(total, &r.out_block)));
+                size_t o = 0;
+                for (size_t t = 0; t < r.bytes.size(); ++t) {
+                    r.out[t] = static_cast<uint8_t *>(r.out_block) + o;
+                    o += (std::max<size_t>(16, r.row_bytes[t] * r.height[t]) + 255) & ~size_t(255);
+                }
+            }
+            for (size_t t = 0; t < r.bytes.size(); ++t, ++ti) tiles[ti].dst = r.out[t];
+            if (!r.out_counted) S.hbm_in_use += r.out_bytes;
+            r.out_counted = true;
+        }
+        // The footprints above are estimates from the main headers (small
+        // code-blocks take more): the plan is held to what is left of the budget,
+        // by its layout or with half the requests, the oldest waiting for batches
+        // that run; with none, it is taken.
+        const uint64_t left =
+            S.cfg.hbm_budget > S.hbm_in_use ? S.cfg.hbm_budget - S.hbm_in_use : 0;
+        bool too_big = false;
+        ts.assign(tiles.size(), 0);
+        st = make_plan(sess, tiles.data(), tiles.size(), B->plan, ts.data(), S.blocks.get(), true,
+                       left, B->ids.size() > 1 || !S.running.empty() ? &too_big : nullptr);
+        if (!too_big) break;
+        for (const size_t keep = B->ids.size() / 2; B->ids.size() > keep;) {
+            ServeRequest &r = *S.reqs[B->ids.back()];
+            S.blocks->put(r.out_block);
+            r.out_block = nullptr;
+            S.hbm_in_use -= r.out_bytes;
+            r.out_counted = false;
+            tiles.resize(B->tile_base.back());
+            B->ids.pop_back();
+            B->tile_base.pop_back();
+        }
+        if (B->ids.empty()) return kOk;
+    }
     if (st) {
         // parse failures fail their own requests; the rest retry next pump
         size_t r = 0;

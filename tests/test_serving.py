@@ -100,6 +100,40 @@ def test_small_budget_splits_batches(oracle):
     srv.close()
 
 
+def test_budget_holds_for_small_code_blocks(oracle):
+    """Plans of 8x8 blocks take about twice what the main header lets expect: what
+    is in use stays within the budget all the same, and nothing is refused."""
+    rng = np.random.default_rng(4)
+    imgs = [rng.integers(0, 256, (256, 256, 3), dtype=np.uint8) for _ in range(3)]
+    tiles = [(S.encode_j2k_ht(v, cb_width_log2=3, cb_height_log2=3, ht_refine=2 * (k == 2)),
+              S.PixelFormat.RGB8, S.Downscale.NONE) for k, v in enumerate(imgs)]
+    budget = 10 << 20
+    srv = Server(window_us=0, max_inflight=3, hbm_budget=budget)
+    ids = [srv.submit([tiles[k % 3]]) for k in range(18)]
+    left, peak = set(ids), 0
+    for _ in range(100000):
+        srv.pump(flush=True)
+        peak = max(peak, srv.stats()["hbm_in_use"])
+        for rec in srv.poll():
+            assert rec["status"] == 0, rec
+            k = ids.index(rec["id"])
+            got = srv.download(rec["id"], 0, S.PixelFormat.RGB8)
+            assert np.array_equal(got, O.decode(tiles[k % 3][0], 1))
+            srv.release(rec["id"])
+            left.discard(rec["id"])
+        if not left:
+            break
+    assert not left
+    assert budget // 2 < peak <= budget, peak
+    # a request that the estimate admits, alone and larger than the budget
+    solo = Server(window_us=0, hbm_budget=1700 << 10)
+    rid = solo.submit([tiles[0]])
+    assert solo.wait([rid])[rid]["status"] == 0
+    assert np.array_equal(solo.download(rid, 0, S.PixelFormat.RGB8), imgs[0])
+    solo.close()
+    srv.close()
+
+
 def test_poisson_load_reports_latency(oracle):
     pool = [(cs, fmt, den, 0) for cs, fmt, den in _pool()]
     srv = Server(window_us=2000)
