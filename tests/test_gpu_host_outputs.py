@@ -99,3 +99,32 @@ def test_arrays_that_share_bytes_and_one_canvas(session):
     for k, v in enumerate(imgs):
         y, x = 256 * (k // 8), 256 * (k % 8)
         assert np.array_equal(canvas[y:y + 256, x:x + 256], v), k
+
+
+@pytest.mark.parametrize("pad", [0, 13])
+def test_page_locked_arrays(session, tiles, pad):
+    """Downloads and decodes into page-locked memory, tight and strided."""
+    import ctypes
+
+    from signinum_amd import _lib
+    imgs, streams = tiles
+    L = _lib.load()
+    p = ctypes.c_void_p()
+    size = max((v.shape[1] * 3 + pad) * v.shape[0] for v in imgs)
+    assert L.sgn_host_alloc(size, ctypes.byref(p)) == 0
+    try:
+        mem = np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_uint8)), (size,))
+        for v, c in zip(imgs, streams):
+            stride = v.shape[1] * 3 + pad
+            out = mem[:stride * v.shape[0]]
+            surf = S.J2kDecoder(c, session).submit_to_device(session, S.PixelFormat.RGB8)
+            for write in (lambda: surf.download_into(out, stride),
+                          lambda: S.decode_tiles_into([(c, out, stride)], S.PixelFormat.RGB8,
+                                                      session=session)):
+                out[:] = 0xEE
+                write()
+                rows = out.reshape(v.shape[0], stride)
+                assert np.array_equal(rows[:, :v.shape[1] * 3].reshape(v.shape), v)
+                assert (rows[:, v.shape[1] * 3:] == 0xEE).all()
+    finally:
+        L.sgn_host_free(p)
