@@ -1,12 +1,12 @@
 // HT cleanup decode in three kernels, each with the shape of its own work:
 //
-//   sgn_ht_clean    sixteen lanes per code-block: removes the bit stuffing of
+//   sgn_ht_clean    sixteen (or four) lanes per code-block: removes the bit stuffing of
 //                   the VLC stream, eight bytes a lane, into a plain bit string
 //                   in the block's workspace;
 //   sgn_ht_symbols  one block per lane (L of a wave's 64 lanes in use): the
 //                   serial MEL / VLC / UVLC chain, reading plain bits, writing
 //                   16 bits per quad into the workspace;
-//   sgn_ht_magsgn   sixteen lanes per block, a quad pair each: magnitudes and
+//   sgn_ht_magsgn   as many lanes per block, a quad pair each: magnitudes and
 //                   signs of a quad row at once, each quad's place in the
 //                   MagSgn stream a prefix sum of the quads' bit counts.
 //
@@ -95,11 +95,15 @@ inline void ht_split_tables(const uint16_t *vlc0, const uint16_t *vlc1, const ui
     for (uint32_t k = 0; k < 256; ++k) uentry(u1[k], 0, T.uother[k], T.uother[256 + k]);
 }
 
-// The clean and magnitude kernels give a block one DPP row (16 lanes), so that
-// neighbours, prefix sums and broadcasts inside a block are single VALU
-// operations that never cross into the next block.
-constexpr uint32_t kSplitLanes = 16;
-constexpr uint32_t kSplitBlocks = kSplitWaves * 64 / kSplitLanes;  // per work-group
+// The clean, magnitude and refinement kernels give a block one DPP row (16 lanes),
+// so that neighbours, prefix sums and broadcasts inside a block are single VALU
+// operations that never cross into the next block; or one quad (4 lanes) where all
+// blocks of the list are at most 16 wide and would leave the rest of a row idle.
+// Cleanup in us with rows, with quads, and in one kernel of a lane a block that
+// these replaced: 2.4 million 4x4 blocks 994, 431, 492; 614,400 8x8 blocks 354, 166,
+// 202; 310,800 16x16 blocks 320, 200, 244 (1.2 million 1190, 869, 725).
+constexpr uint32_t kSplitLanes = 16, kQuadLanes = 4, kQuadWidth = 16;
+constexpr uint32_t split_blocks(uint32_t lanes) { return kSplitWaves * 64 / lanes; }  // per work-group
 
 // Value of another lane of the row (CTRL), 0 past the row's ends.
 template <int CTRL>
@@ -107,17 +111,40 @@ __device__ __forceinline__ uint32_t row_dpp(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
 }
 
-// Inclusive prefix sum over each row.  Called by all lanes.
-__device__ __forceinline__ uint32_t row_scan(uint32_t v) {
-    v += row_dpp<0x111>(v);  // row_shr:1
-    v += row_dpp<0x112>(v);  // row_shr:2
-    v += row_dpp<0x114>(v);  // row_shr:4
-    v += row_dpp<0x118>(v);  // row_shr:8
-    return v;
-}
-
-// The value that the row's last lane holds (row_newbcast:15).
-__device__ __forceinline__ uint32_t row_last(uint32_t v) { return row_dpp<0x15F>(v); }
+// The L lanes of a block, this one being lane q.  Called by all lanes.
+template <uint32_t L>
+struct BlockLanes {
+    static_assert(L == 16 || L == 4, "a DPP row or quad");
+    uint32_t q;
+    // Value of the lane before (0 for the first) and after (0 for the last).
+    __device__ __forceinline__ uint32_t before(uint32_t v) const {
+        if constexpr (L == 16) return row_dpp<0x111>(v);  // row_shr:1
+        const uint32_t x = row_dpp<0x90>(v);              // quad_perm:[0,0,1,2]
+        return q ? x : 0u;
+    }
+    __device__ __forceinline__ uint32_t after(uint32_t v) const {
+        if constexpr (L == 16) return row_dpp<0x101>(v);  // row_shl:1
+        const uint32_t x = row_dpp<0xF9>(v);              // quad_perm:[1,2,3,3]
+        return q < 3 ? x : 0u;
+    }
+    // Inclusive prefix sum.
+    __device__ __forceinline__ uint32_t scan(uint32_t v) const {
+        v += before(v);
+        if constexpr (L == 16) {
+            v += row_dpp<0x112>(v);  // row_shr:2
+            v += row_dpp<0x114>(v);  // row_shr:4
+            v += row_dpp<0x118>(v);  // row_shr:8
+        } else {
+            const uint32_t x = row_dpp<0x40>(v);  // quad_perm:[0,0,0,1]
+            v += q >= 2 ? x : 0u;
+        }
+        return v;
+    }
+    // The last lane's value (row_newbcast:15, quad_perm:[3,3,3,3]).
+    __device__ __forceinline__ uint32_t last(uint32_t v) const {
+        return L == 16 ? row_dpp<0x15F>(v) : row_dpp<0xFF>(v);
+    }
+};
 
 // Orders the LDS accesses of one wave for the compiler; the LDS unit executes
 // a wave's instructions in order, so nothing is waited for.
@@ -128,31 +155,36 @@ __device__ __forceinline__ void wave_lds_fence() {
 
 // ---- stuffing removal ------------------------------------------------------
 
-constexpr uint32_t kCleanRing = 64;  // dwords of a block's ring: a partly filled unit and a round's 33
+// Dwords of a block's ring: a partly filled unit and a round's 2 L + 1.
+template <uint32_t L>
+constexpr uint32_t kCleanRing = 4 * L;
 
-// A plain bit string that a row of lanes writes to a block's interleaved
-// units, 128 bytes of stream a round, through a ring of words in LDS that whole
+// A plain bit string that a block's L lanes write to its interleaved
+// units, 8 L bytes of stream a round, through a ring of words in LDS that whole
 // units leave.  Every byte is ORed in at its place.
+template <uint32_t L>
 struct PlainString {
-    uint32_t *buf;  // kCleanRing words, 16-byte aligned
-    uint32_t q;     // lane of the row
-    uint4 *d;       // unit 0
+    static constexpr uint32_t kMask = kCleanRing<L> - 1;
+    uint32_t *buf;  // the ring, 16-byte aligned
+    BlockLanes<L> lanes;
+    uint32_t q;  // lane of the block
+    uint4 *d;    // unit 0
     uint32_t units, fill, done;
 
     __device__ __forceinline__ PlainString(uint32_t *b, uint32_t lane, uint4 *out, uint32_t n,
                                            uint32_t head, uint32_t bits)
-        : buf(b), q(lane), d(out), units(n), fill(bits), done(0) {
+        : buf(b), lanes{lane}, q(lane), d(out), units(n), fill(bits), done(0) {
         if (q < 4) buf[q] = q == 0 ? head : 0u;
     }
     // This lane's n0 and n1 next bits (25 to 32 each; a value may reach one bit
-    // past its count).  Called by all lanes; rows that are not `act` sit out.
+    // past its count).  Called by all lanes; blocks that are not `act` sit out.
     __device__ __forceinline__ void round(bool act, uint32_t v0, uint32_t n0, uint32_t v1,
                                           uint32_t n1) {
-        const uint32_t incl = row_scan(n0 + n1), tot = row_last(incl);
+        const uint32_t incl = lanes.scan(n0 + n1), tot = lanes.last(incl);
         if (act) {
             const uint32_t z = (fill >> 5) + 1 + q;
-            buf[z & (kCleanRing - 1)] = 0;
-            buf[(z + 16) & (kCleanRing - 1)] = 0;
+            buf[z & kMask] = 0;
+            buf[(z + L) & kMask] = 0;
         }
         wave_lds_fence();
         if (act) {
@@ -161,28 +193,28 @@ struct PlainString {
             const uint32_t pos = fill + incl - (n0 + n1), wi = pos >> 5, sh = pos & 31u;
             const uint64_t a = v << sh;
             const uint32_t x2 = sh ? (uint32_t)(v >> 32) >> (32u - sh) : 0u;
-            if ((uint32_t)a) atomicOr(&buf[wi & (kCleanRing - 1)], (uint32_t)a);
+            if ((uint32_t)a) atomicOr(&buf[wi & kMask], (uint32_t)a);
             if ((uint32_t)(a >> 32))
-                atomicOr(&buf[(wi + 1) & (kCleanRing - 1)], (uint32_t)(a >> 32));
-            if (x2) atomicOr(&buf[(wi + 2) & (kCleanRing - 1)], x2);
+                atomicOr(&buf[(wi + 1) & kMask], (uint32_t)(a >> 32));
+            if (x2) atomicOr(&buf[(wi + 2) & kMask], x2);
             fill += tot;
         }
         wave_lds_fence();
-        // whole units (at most 9 a round; the padding of the last round's
+        // whole units (at most 9 a round, 2 of a quad; the padding of the last round's
         // bytes may reach past the string's last unit)
         const uint32_t full = min(fill >> 7, units), u = done + q;
         if (act && u < full)
-            d[kHtGroup * u] = *reinterpret_cast<uint4 *>(&buf[4 * u & (kCleanRing - 1)]);
+            d[kHtGroup * u] = *reinterpret_cast<uint4 *>(&buf[4 * u & kMask]);
         done = act ? full : done;
     }
     // The partly filled unit, then zeros up to and with unit `units`
     // (seven-bit bytes leave the string short of it).
     __device__ __forceinline__ void finish() {
         const uint32_t last = fill >> 5;
-        for (uint32_t u = done + q; u <= units; u += kSplitLanes) {
+        for (uint32_t u = done + q; u <= units; u += L) {
             uint4 v = make_uint4(0, 0, 0, 0);
             if (u < units) {
-                const uint32_t *x = &buf[4 * u & (kCleanRing - 1)];
+                const uint32_t *x = &buf[4 * u & kMask];
                 v.x = 4 * u <= last ? x[0] : 0u;
                 v.y = 4 * u + 1 <= last ? x[1] : 0u;
                 v.z = 4 * u + 2 <= last ? x[2] : 0u;
@@ -215,22 +247,24 @@ __device__ __forceinline__ uint32_t bytes_7f(uint32_t d) {
     return ((d & 0x7F7F7F7Fu) + 0x01010101u) & 0x80808080u;
 }
 
-// The VLC string of one block per row: two zero bits, the 3 or 4 bits of the
+// The VLC string of one block per L lanes: two zero bits, the 3 or 4 bits of the
 // segment's second last byte, and from there it runs backward from the byte before; a byte
 // whose low 7 bits are ones after a byte > 0x8F carries 7 bits, and is ORed in
 // whole, as the byte-wise reader does (ht_block_decode.rs:931-999); zeros
 // follow it.  Two dependent trips to memory per block bound it (the first
-// bytes are asked for beside the length field); a round takes 128 bytes, eight
-// a lane, through a ring of words in LDS that whole 16-byte units leave.  *clear
+// bytes are asked for beside the length field); a round takes eight bytes a
+// lane, through a ring of words in LDS that whole 16-byte units leave.  *clear
 // (null: none) is a counter of a later launch, set to 0.
+template <uint32_t L>
 __global__ void __launch_bounds__(kSplitWaves * 64)
 sgn_ht_clean(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restrict__ arena,
              const HtGroup *__restrict__ groups, uint4 *__restrict__ work, uint32_t *clear) {
     if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
-    __shared__ __attribute__((aligned(16))) uint32_t s_buf[kSplitBlocks][kCleanRing];
-    const uint32_t row = threadIdx.x / kSplitLanes, q = threadIdx.x % kSplitLanes;
+    __shared__ __attribute__((aligned(16))) uint32_t s_buf[split_blocks(L)][kCleanRing<L>];
+    const uint32_t row = threadIdx.x / L, q = threadIdx.x % L;
+    const BlockLanes<L> lanes{q};
     uint32_t *buf = s_buf[row];
-    const uint32_t i = blockIdx.x * kSplitBlocks + row;
+    const uint32_t i = blockIdx.x * split_blocks(L) + row;
     const bool valid = i < n;
     CbJob j{};
     if (valid) j = jobs[i];
@@ -267,28 +301,28 @@ sgn_ht_clean(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restri
     if (!coded || bad) scup = 0;
     const HtWork w = ht_work(work, groups, valid ? i : 0);
     // the first MEL bytes, as they are
-    if (q < kHtMelUnits && scup > 16 * q) {
+    for (uint32_t u = q; u < kHtMelUnits && scup > 16 * u; u += L) {
         uint4 v;
-        __builtin_memcpy(&v, arena + (seg1 - scup) + 16 * q, 16);
-        w.mel[kHtGroup * q] = v;
+        __builtin_memcpy(&v, arena + (seg1 - scup) + 16 * u, 16);
+        w.mel[kHtGroup * u] = v;
     }
     const uint32_t len = scup ? scup - 2 : 0;
     const uint32_t units = (6 + 8 * len + 127) >> 7;  // 16-byte units that hold stream bits
     const uint32_t first = b0 >> 4;
     // two bits in front
-    PlainString str(buf, q, w.vlc, units, first << 2, 6u - ((first & 7u) == 7u ? 1u : 0u));
+    PlainString<L> str(buf, q, w.vlc, units, first << 2, 6u - ((first & 7u) == 7u ? 1u : 0u));
     uint32_t carry = b0 | 0x0Fu;  // the byte before this round's
 
-    for (uint32_t at = 0; __any(at < len); at += 128) {
+    for (uint32_t at = 0; __any(at < len); at += 8 * L) {
         const uint32_t k0 = at + 8 * q;
         uint32_t d0 = __builtin_bswap32(hi), d1 = __builtin_bswap32(lo);
         if (k0 + 4 > len) d0 &= k0 < len ? 0xFFFFFFFFu >> (8 * (4 - (len - k0))) : 0u;
         if (k0 + 8 > len) d1 &= k0 + 4 < len ? 0xFFFFFFFFu >> (8 * (8 - (len - k0))) : 0u;
-        fetch(k0 + 128, len);
+        fetch(k0 + 8 * L, len);
         const uint32_t g0 = bytes_above(d0), g1 = bytes_above(d1);
-        uint32_t pg = row_dpp<0x111>(g1);
+        uint32_t pg = lanes.before(g1);
         if (q == 0) pg = carry > 0x8Fu ? 0x80000000u : 0u;
-        carry = row_last(d1 >> 24);
+        carry = lanes.last(d1 >> 24);
         uint32_t n0, n1;
         const uint32_t v0 =
             close_up(d0, (bytes_7f(d0) & __builtin_amdgcn_alignbit(g0, pg, 24)) >> 7, n0);
@@ -613,23 +647,26 @@ sgn_ht_symbols(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__rest
 
 // ---- magnitudes and signs ------------------------------------------------------
 
-constexpr uint32_t kMagRing = 256;  // dwords of a block's unstuffed MagSgn ring (a power of two)
+// Dwords of a block's unstuffed MagSgn ring (a power of two).
+template <uint32_t L>
+constexpr uint32_t kMagRingOf = 16 * L;
 
 using s16x2 = int16_t __attribute__((ext_vector_type(2)));
 
-// One block per DPP row, a quad pair (eight samples) per lane.  A quad row
-// takes at most 32 quads * 4 samples * 31 bits = 496 bytes of the 1024-byte
-// ring, which is topped up 128 bytes at a time, eight bytes a lane, from words
-// loaded a round ahead.  Sample rows leave as whole 128-byte (int16) lines.
+// One block per L lanes, a quad pair (eight samples) per lane.  A quad row
+// takes at most 2 L quads * 4 samples * 31 bits = 31 L bytes of the ring's 64 L,
+// which is topped up eight bytes a lane at a time, from words loaded a round
+// ahead.  Sample rows leave as whole 128-byte (int16) lines.
 // Bound by VALU issue.
-template <typename C>
+template <typename C, uint32_t L>
 __global__ void __launch_bounds__(kSplitWaves * 64)
 sgn_ht_magsgn(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restrict__ arena,
               C *__restrict__ coef, const HtGroup *__restrict__ groups, uint4 *__restrict__ work,
               uint8_t *__restrict__ status) {
     // one dword more than the ring: a copy of the first, so that two adjacent
     // dwords can be read at any place
-    __shared__ uint32_t s_ring[kSplitBlocks][kMagRing + 1];
+    constexpr uint32_t kMagRing = kMagRingOf<L>;
+    __shared__ uint32_t s_ring[split_blocks(L)][kMagRing + 1];
     // per symbol code: byte s of .x is 0xFF where sample s is significant, of
     // .y 1 where its exponent is known, of .z that exponent bit
     __shared__ uint4 s_code[256];
@@ -646,9 +683,10 @@ sgn_ht_magsgn(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restr
         s_code[t] = make_uint4(sig, known, bit, 0);
     }
     __syncthreads();
-    const uint32_t row = threadIdx.x / kSplitLanes, q = threadIdx.x % kSplitLanes;
+    const uint32_t row = threadIdx.x / L, q = threadIdx.x % L;
+    const BlockLanes<L> lanes{q};
     uint32_t *ring = s_ring[row];
-    const uint32_t i = blockIdx.x * kSplitBlocks + row;
+    const uint32_t i = blockIdx.x * split_blocks(L) + row;
     const bool valid = i < n;
     CbJob j{};
     if (valid) j = jobs[i];
@@ -691,7 +729,7 @@ sgn_ht_magsgn(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restr
     uint32_t s_next = mask && nrows ? *sym : 0u;
     uint32_t rows_max = (uint32_t)__builtin_amdgcn_readlane((int)nrows, 0);
 #pragma unroll
-    for (int k = 16; k < 64; k += 16)
+    for (int k = L; k < 64; k += L)
         rows_max = max(rows_max, (uint32_t)__builtin_amdgcn_readlane((int)nrows, k));
     for (uint32_t r = 0; r < rows_max; ++r) {
         const bool live = r < nrows;
@@ -701,7 +739,7 @@ sgn_ht_magsgn(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restr
         if (r) {
             // exponent bound of the row above, over the quad and the samples
             // beside it, for quads with more than one significant sample
-            const uint32_t l = row_dpp<0x111>(e7), t = row_dpp<0x101>(e1);
+            const uint32_t l = lanes.before(e7), t = lanes.after(e1);
             const uint32_t mid = max(e3, e5);
             const uint32_t m0 = max(max(max(e1, mid), l), 1u), m1 = max(max(max(e7, mid), t), 1u);
             const uint32_t nz = (s | (s >> 1)) & 0x00550055u;
@@ -710,8 +748,8 @@ sgn_ht_magsgn(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restr
             uq1 += (z1 & (z1 - 1u)) ? m1 : 1u;
         }
         const bool over = live && ((mask && uq0 > mmsbp2) || ((mask >> 8) && uq1 > mmsbp2));
-        const uint64_t ov = __ballot(over) >> (threadIdx.x & 48u);
-        if ((uint32_t)ov & 0xFFFFu) bad = 1;
+        const uint64_t ov = __ballot(over) >> (threadIdx.x & (64u - L));
+        if ((uint32_t)ov & ((1u << L) - 1u)) bad = 1;
         const uint32_t code0 = live && !bad ? s & mask & 0xFFu : 0u;
         const uint32_t code1 = live && !bad ? (s >> 16) & (mask >> 8) : 0u;
         // bits per sample, a byte each: U_q, one less where the exponent is known
@@ -723,9 +761,9 @@ sgn_ht_magsgn(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restr
         a0 += a0 << 16;
         a1 += a1 << 16;
         const uint32_t t0 = a0 >> 24, tot = t0 + (a1 >> 24);
-        const uint32_t incl = row_scan(tot);
+        const uint32_t incl = lanes.scan(tot);
         const uint32_t at = pos + incl - tot;
-        pos += row_last(incl);
+        pos += lanes.last(incl);
         // every bit this row reads, and the sign bit that a sample without
         // magnitude bits takes from the position after the last one
         const uint32_t need = on ? pos + 1 : 0;
@@ -739,22 +777,22 @@ sgn_ht_magsgn(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restr
                     if (over8 > 4) d0 |= over8 >= 8 ? 0xFFFFFFFFu : 0xFFFFFFFFu << (64 - 8 * over8);
                 }
                 if (act) {
-                    next += 128;
+                    next += 8 * L;
                     if (next < end) __builtin_memcpy(&raw, arena + next, 8);
                 }
                 // bytes that are 0xFF, and those after one
                 const uint32_t f0 = bytes_ff(d0), f1 = bytes_ff(d1);
-                uint32_t pf = row_dpp<0x111>(f1);
+                uint32_t pf = lanes.before(f1);
                 if (q == 0) pf = prev;
                 uint32_t n0, n1;
                 const uint32_t v0 = close_up(d0, __builtin_amdgcn_alignbit(f0, pf, 24) >> 7, n0);
                 const uint32_t v1 = close_up(d1, __builtin_amdgcn_alignbit(f1, f0, 24) >> 7, n1);
-                const uint32_t sc = row_scan(n0 + n1), bits = row_last(sc), last = row_last(f1);
+                const uint32_t sc = lanes.scan(n0 + n1), bits = lanes.last(sc), last = lanes.last(f1);
                 const uint32_t wz = (fill >> 5) + 1 + q;
                 if (act) {
                     // the words past the partly filled one that this round reaches
                     ring[wz & (kMagRing - 1)] = 0;
-                    ring[(wz + 16) & (kMagRing - 1)] = 0;
+                    ring[(wz + L) & (kMagRing - 1)] = 0;
                 }
                 wave_lds_fence();
                 if (act) {
@@ -899,15 +937,16 @@ __device__ __forceinline__ bool ref_runs(const CbJob &j) {
 
 // Significance of the cleanup (16 bits per group of 4x4 samples, bit 4 column +
 // row; two groups a dword) and the plain SigProp bits: LSB-first, 7 bits after
-// 0xFF, zeros past the end.  One block per DPP row, a group a lane.
-template <typename C>
+// 0xFF, zeros past the end.  One block per L lanes, a group a lane.
+template <typename C, uint32_t L>
 __global__ void __launch_bounds__(kSplitWaves * 64)
 sgn_ht_refine_prep(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restrict__ arena,
                    const C *__restrict__ coef, const RefGroup *__restrict__ groups,
                    uint4 *__restrict__ work) {
-    __shared__ __attribute__((aligned(16))) uint32_t s_buf[kSplitBlocks][kCleanRing];
-    const uint32_t row = threadIdx.x / kSplitLanes, q = threadIdx.x % kSplitLanes;
-    const uint32_t i = blockIdx.x * kSplitBlocks + row;
+    __shared__ __attribute__((aligned(16))) uint32_t s_buf[split_blocks(L)][kCleanRing<L>];
+    const uint32_t row = threadIdx.x / L, q = threadIdx.x % L;
+    const BlockLanes<L> lanes{q};
+    const uint32_t i = blockIdx.x * split_blocks(L) + row;
     CbJob j{};
     if (i < n) j = jobs[i];
     const bool on = i < n && ref_runs(j);
@@ -915,9 +954,9 @@ sgn_ht_refine_prep(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__
     // SigProp bytes, eight a lane
     const uint32_t len = on ? min((uint32_t)j.lref, kRefSpBytes) : 0;
     const uint8_t *src = arena + j.src + j.lcup;
-    PlainString str(s_buf[row], q, w.sp, (8 * len + 127) >> 7, 0, 0);
+    PlainString<L> str(s_buf[row], q, w.sp, (8 * len + 127) >> 7, 0, 0);
     uint32_t prev = 0;
-    for (uint32_t at = 0; __any(at < len); at += 128) {
+    for (uint32_t at = 0; __any(at < len); at += 8 * L) {
         const uint32_t k = at + 8 * q;
         uint2 d = make_uint2(0, 0);
         if (k < len) {
@@ -927,9 +966,9 @@ sgn_ht_refine_prep(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__
             if (have < 4) d.x &= 0xFFFFFFFFu >> (8 * (4 - have));
         }
         const uint32_t f0 = bytes_ff(d.x), f1 = bytes_ff(d.y);
-        uint32_t pf = row_dpp<0x111>(f1);
+        uint32_t pf = lanes.before(f1);
         if (q == 0) pf = prev;
-        prev = row_last(f1);
+        prev = lanes.last(f1);
         uint32_t n0, n1;
         const uint32_t v0 = close_up(d.x, __builtin_amdgcn_alignbit(f0, pf, 24) >> 7, n0);
         const uint32_t v1 = close_up(d.y, __builtin_amdgcn_alignbit(f1, f0, 24) >> 7, n1);
@@ -947,6 +986,7 @@ sgn_ht_refine_prep(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__
         for (uint32_t r = 0; r < 4; ++r)
             refine_load<C>(v[r], out, 4 * s + r, 4 * q, j.w, j.h, j.stride, vec);
         cs[s * (kHtGroup * 16)] = (uint16_t)group_sig(v);
+        if constexpr (L < 8) cs[s * (kHtGroup * 16) + L] = 0;  // the group beside the last
     }
 }
 
@@ -1076,22 +1116,23 @@ sgn_ht_sigprop(const CbJob *__restrict__ jobs, uint32_t n, const RefGroup *__res
 }
 
 // What SigProp found and the MagRef bits (:1377-1432), applied to the samples:
-// one block per DPP row, a group a lane.  A sample that SigProp found gets the
+// one block per L lanes, a group a lane.  A sample that SigProp found gets the
 // word 3 << (p - 2); MagRef exchanges bit p - 1 of a sample that the cleanup
 // found for its bit and sets the midpoint 1 << (p - 2).  MagRef bits run
 // backward from the segment's last byte with the VLC stuffing rule, zeros past
 // its start, one per such sample in stripe-column order: a group's place is a
-// row scan of the groups' counts (a stripe takes at most 256 bits).
-template <typename C>
+// prefix sum of the groups' counts (a stripe takes at most 256 bits).
+template <typename C, uint32_t L>
 __global__ void __launch_bounds__(kSplitWaves * 64)
 sgn_ht_refine_apply(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *__restrict__ arena,
                     C *__restrict__ coef, const RefGroup *__restrict__ groups,
                     uint4 *__restrict__ work) {
-    constexpr uint32_t kRing = 64;  // dwords: a stripe's 256 bits and a round's 1024 (a power of two)
-    __shared__ uint32_t s_ring[kSplitBlocks][kRing + 1];  // and a copy of the first
-    const uint32_t row = threadIdx.x / kSplitLanes, q = threadIdx.x % kSplitLanes;
+    constexpr uint32_t kRing = 4 * L;  // dwords: a stripe's 16 L bits and a round's 64 L
+    __shared__ uint32_t s_ring[split_blocks(L)][kRing + 1];  // and a copy of the first
+    const uint32_t row = threadIdx.x / L, q = threadIdx.x % L;
+    const BlockLanes<L> lanes{q};
     uint32_t *ring = s_ring[row];
-    const uint32_t i = blockIdx.x * kSplitBlocks + row;
+    const uint32_t i = blockIdx.x * split_blocks(L) + row;
     CbJob j{};
     if (i < n) j = jobs[i];
     const bool on = i < n && ref_runs(j);
@@ -1147,27 +1188,27 @@ sgn_ht_refine_apply(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *_
         }
         const uint32_t cs = group_sig(v);
         const uint32_t cnt = mag ? (uint32_t)__builtin_popcount(cs) : 0u;
-        const uint32_t incl = row_scan(cnt);
+        const uint32_t incl = lanes.scan(cnt);
         const uint32_t at = pos + incl - cnt;
-        pos += row_last(incl);
+        pos += lanes.last(incl);
         while (__any(fill < pos)) {
             const bool act = fill < pos;
             const uint32_t g0 = bytes_above(raw.x), g1 = bytes_above(raw.y);
-            uint32_t pg = row_dpp<0x111>(g1);
+            uint32_t pg = lanes.before(g1);
             if (q == 0) pg = carry;
-            const uint32_t last = row_last(g1);
+            const uint32_t last = lanes.last(g1);
             uint32_t n0, n1;
             const uint32_t v0 =
                 close_up(raw.x, (bytes_7f(raw.x) & __builtin_amdgcn_alignbit(g0, pg, 24)) >> 7, n0);
             const uint32_t v1 =
                 close_up(raw.y, (bytes_7f(raw.y) & __builtin_amdgcn_alignbit(g1, g0, 24)) >> 7, n1);
-            const uint32_t sc = row_scan(n0 + n1), bits = row_last(sc);
+            const uint32_t sc = lanes.scan(n0 + n1), bits = lanes.last(sc);
             if (act) {
-                next += 128;
+                next += 8 * L;
                 fetch();
                 const uint32_t z = (fill >> 5) + 1 + q;
                 ring[z & (kRing - 1)] = 0;
-                ring[(z + 16) & (kRing - 1)] = 0;
+                ring[(z + L) & (kRing - 1)] = 0;
             }
             wave_lds_fence();
             if (act) {

@@ -446,6 +446,7 @@ struct sgn_j2k_plan {
     StoreJob *d_store = nullptr;
     uint32_t *d_store_block_job = nullptr;
     int lane_variant = kSplit64Variant;  // index into kRowsVariants
+    bool quads = false;  // every lane-list block is at most kQuadWidth wide
     int dwt_shape = 0;                       // index into kDwtShapes
     hipGraphExec_t graph_exec = nullptr;
     hipGraph_t graph = nullptr;
@@ -997,6 +998,8 @@ Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
         }
     }
     P.lane_variant = default_variant(P);
+    P.quads = true;
+    for (const CbJob &j : P.cb_lane) P.quads &= j.w <= kQuadWidth;
     // synthesis levels grouped by (transform, depth), tiles in order: the
     // levels of each depth counted, then placed tile by tile
     const uint32_t D = P.depth_max;
@@ -1517,18 +1520,42 @@ uint32_t classic_resident(sgn_hip_session *s, int v, int opt) {
 }
 
 // Refinement passes of the lane list's blocks, after their cleanup (three
-// launches).
-template <typename C>
+// launches; L lanes a block).
+template <typename C, uint32_t L>
 void launch_refine(sgn_hip_session *s, sgn_j2k_plan &P) {
     const uint32_t n = static_cast<uint32_t>(P.cb_refine.size());
     C *coef = reinterpret_cast<C *>(P.d_coef);
-    const dim3 g((n + kSplitBlocks - 1) / kSplitBlocks), b(kSplitWaves * 64);
-    hipLaunchKernelGGL(sgn_ht_refine_prep<C>, g, b, 0, s->stream, P.d_cb_refine, n, P.d_arena,
+    const dim3 g((n + split_blocks(L) - 1) / split_blocks(L)), b(kSplitWaves * 64);
+    hipLaunchKernelGGL((sgn_ht_refine_prep<C, L>), g, b, 0, s->stream, P.d_cb_refine, n, P.d_arena,
                        static_cast<const C *>(coef), P.d_ref_groups, P.d_ref_work);
     hipLaunchKernelGGL(sgn_ht_sigprop, dim3((n + 64 * kSplitWaves - 1) / (64 * kSplitWaves)), b, 0,
                        s->stream, P.d_cb_refine, n, P.d_ref_groups, P.d_ref_work);
-    hipLaunchKernelGGL(sgn_ht_refine_apply<C>, g, b, 0, s->stream, P.d_cb_refine, n, P.d_arena, coef,
-                       P.d_ref_groups, P.d_ref_work);
+    hipLaunchKernelGGL((sgn_ht_refine_apply<C, L>), g, b, 0, s->stream, P.d_cb_refine, n, P.d_arena,
+                       coef, P.d_ref_groups, P.d_ref_work);
+}
+
+// Every pass of the lane list in the split kernels (L lanes a block in all but
+// the two chains).  `clear`: set to 0 on the way, unless null.
+template <typename C, uint32_t L>
+uint32_t launch_split(sgn_hip_session *s, sgn_j2k_plan &P, SymbolsLaunch symbols, uint32_t *clear) {
+    const uint32_t n = static_cast<uint32_t>(P.cb_lane.size());
+    C *coef = reinterpret_cast<C *>(P.d_coef);
+    const dim3 g((n + split_blocks(L) - 1) / split_blocks(L)), b(kSplitWaves * 64);
+    hipLaunchKernelGGL(sgn_ht_clean<L>, g, b, 0, s->stream, P.d_cb_lane, n, P.d_arena, P.d_groups,
+                       P.d_work, clear);
+    symbols(s->stream, P.d_cb_lane, n, P.d_arena, P.d_groups, P.d_work, s->d_split);
+    hipLaunchKernelGGL((sgn_ht_magsgn<C, L>), g, b, 0, s->stream, P.d_cb_lane, n, P.d_arena, coef,
+                       P.d_groups, P.d_work, P.d_status_lane);
+    if (P.device_packets) {
+        // the pass counts are known on the device only: the kernel walks the
+        // whole lane list and skips the other blocks
+        hipLaunchKernelGGL(sgn_ht_refine<C>, dim3((n + 255) / 256), dim3(256), 0, s->stream,
+                           P.d_cb_lane, n, P.d_arena, coef);
+        return 4;
+    }
+    if (P.cb_refine.empty()) return 3;
+    launch_refine<C, L>(s, P);
+    return 6;
 }
 
 // Enqueue helpers; each returns the number of kernel launches issued.
@@ -1549,37 +1576,13 @@ uint32_t launch_lane_variant(sgn_hip_session *s, sgn_j2k_plan &P, int v, const C
                                  P.lane_refined);
         return 1;
     }
-    uint32_t k = 3;
-    const dim3 g((count + kSplitBlocks - 1) / kSplitBlocks), b(kSplitWaves * 64);
-    hipLaunchKernelGGL(sgn_ht_clean, g, b, 0, s->stream, d_jobs, count, P.d_arena, P.d_groups,
-                       P.d_work, clear ? *clear : nullptr);
+    uint32_t *const zero = clear ? *clear : nullptr;
     if (clear) *clear = nullptr;
-    symbols(s->stream, d_jobs, count, P.d_arena, P.d_groups, P.d_work, s->d_split);
-    if (P.narrow)
-        hipLaunchKernelGGL(sgn_ht_magsgn<int16_t>, g, b, 0, s->stream, d_jobs, count, P.d_arena,
-                           reinterpret_cast<int16_t *>(P.d_coef), P.d_groups, P.d_work, status);
-    else
-        hipLaunchKernelGGL(sgn_ht_magsgn<int32_t>, g, b, 0, s->stream, d_jobs, count, P.d_arena,
-                           reinterpret_cast<int32_t *>(P.d_coef), P.d_groups, P.d_work, status);
-    if (P.device_packets) {
-        // the pass counts are known on the device only: the kernel walks the
-        // whole lane list and skips the other blocks
-        const dim3 gr((count + 255) / 256), br(256);
-        if (P.narrow)
-            hipLaunchKernelGGL((sgn_ht_refine<int16_t>), gr, br, 0, s->stream, d_jobs, count,
-                               P.d_arena, reinterpret_cast<int16_t *>(P.d_coef));
-        else
-            hipLaunchKernelGGL((sgn_ht_refine<int32_t>), gr, br, 0, s->stream, d_jobs, count,
-                               P.d_arena, reinterpret_cast<int32_t *>(P.d_coef));
-        ++k;
-    } else if (!P.cb_refine.empty()) {
-        if (P.narrow)
-            launch_refine<int16_t>(s, P);
-        else
-            launch_refine<int32_t>(s, P);
-        k += 3;
-    }
-    return k;
+    if (P.quads)
+        return P.narrow ? launch_split<int16_t, kQuadLanes>(s, P, symbols, zero)
+                        : launch_split<int32_t, kQuadLanes>(s, P, symbols, zero);
+    return P.narrow ? launch_split<int16_t, kSplitLanes>(s, P, symbols, zero)
+                    : launch_split<int32_t, kSplitLanes>(s, P, symbols, zero);
 }
 
 uint32_t launch_lane(sgn_hip_session *s, sgn_j2k_plan &P, uint32_t **clear = nullptr) {
@@ -2698,7 +2701,9 @@ int sgn_j2k_plan_kernels(const sgn_j2k_plan *P, char *out, size_t cap, size_t *l
         t += std::string(stage) + " " + kernel + " " + std::to_string(count) + "\n";
     };
     if (!P->cb_lane.empty())
-        line("blocks", kRowsVariants[P->d_work ? P->lane_variant : kCoopVariant].name,
+        line("blocks",
+             std::string(kRowsVariants[P->d_work ? P->lane_variant : kCoopVariant].name) +
+                 (P->d_work && P->quads && kRowsVariants[P->lane_variant].symbols ? "-quads" : ""),
              P->cb_lane.size());
     if (!P->cb_wave.empty()) line("blocks", "wave-coop-1024", P->cb_wave.size());
     for (int v = 0; v < kClassicShapes; ++v) {
@@ -3450,7 +3455,8 @@ int sgn_j2k_plan_time_code_blocks(sgn_hip_session *s, sgn_j2k_plan *P, size_t st
         (st = dcyc.alloc(pick.size())))
         return st;
     const uint32_t n = uint32_t(pick.size());
-    hipLaunchKernelGGL(sgn_ht_clean, dim3((n + kSplitBlocks - 1) / kSplitBlocks),
+    hipLaunchKernelGGL(sgn_ht_clean<kSplitLanes>,
+                       dim3((n + split_blocks(kSplitLanes) - 1) / split_blocks(kSplitLanes)),
                        dim3(kSplitWaves * 64), 0, s->stream, djobs.p, n, P->d_arena, dgroups.p,
                        dwork.p, static_cast<uint32_t *>(nullptr));
     hipLaunchKernelGGL((sgn_ht_symbols<1, true>), dim3((n + kSplitWaves - 1) / kSplitWaves),
