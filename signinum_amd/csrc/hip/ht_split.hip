@@ -1247,10 +1247,10 @@ sgn_ht_refine_apply(const CbJob *__restrict__ jobs, uint32_t n, const uint8_t *_
     }
 }
 
-// The same of plans whose packet headers are parsed on the device (the host
-// knows neither which blocks are refined nor their lengths): all passes of the
-// code-blocks jobs[0 .. n), one block per lane, after the
-// cleanup kernels wrote their samples.  A block whose cleanup failed holds zeros or
+// The same of long lists whose packet headers are parsed on the device (the host
+// knows neither which blocks are refined nor their lengths, and reserves no
+// workspace for all): all passes of the code-blocks jobs[0 .. n), one block per
+// lane, after the cleanup kernels wrote their samples.  A block whose cleanup failed holds zeros or
 // partial samples; the passes keep to its rectangle and its refinement
 // segment whatever the samples, and its status already reports it.
 template <typename C>

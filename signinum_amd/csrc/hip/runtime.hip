@@ -147,6 +147,14 @@ constexpr size_t kSplit64Blocks = 131072;
 // as that, a lane kernel's shape as the plan's own choice.
 constexpr int kFormerVariantCount = 9, kFormerCoopVariant = 6;
 
+// With packet headers parsed on the device the host knows neither which blocks are
+// refined nor their lengths, so the refinement kernels' workspace has to be
+// reserved for all (up to 2.8 KB a block): up to this many blocks (180 MB); longer
+// lists take sgn_ht_refine, a lane per block without workspace.  One tile of
+// 256x256 with both passes takes 1196 us so and 2150 with a lane per block, 850 tiles
+// 2048 and 3092; without refined blocks the two launches more cost 10 us at most.
+constexpr size_t kPacketRefineBlocks = 65536;
+
 // The cooperative kernel: one code-block per wave, one wave per work-group.
 // refine: the list holds blocks with SigProp / MagRef passes
 template <typename C>
@@ -286,14 +294,14 @@ uint64_t layout_groups(const std::vector<CbJob> &list, bool unknown, std::vector
     return units;
 }
 
-// The same of the refined blocks' list.
-uint64_t layout_refine(const std::vector<CbJob> &list, std::vector<RefGroup> &groups) {
+// The same of a list of refined blocks.
+uint64_t layout_refine(const std::vector<CbJob> &list, bool unknown, std::vector<RefGroup> &groups) {
     uint64_t units = 0;
     groups.clear();
     for (size_t a = 0; a < list.size(); a += kHtGroup) {
         uint32_t sp = 0, ns = 0;
         for (size_t k = a; k < std::min(a + kHtGroup, list.size()); ++k) {
-            sp = std::max(sp, ref_sp_units(list[k].lref));
+            sp = std::max(sp, ref_sp_units(unknown ? kRefSpBytes : list[k].lref));
             ns = std::max(ns, (list[k].h + 3u) / 4u);
         }
         groups.push_back({static_cast<uint32_t>(units), ns, sp});
@@ -968,7 +976,10 @@ Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
     std::stable_sort(P.cb_refine.begin(), P.cb_refine.end(), [](const CbJob &a, const CbJob &b) {
         return uint32_t(a.lref) + a.lcup > uint32_t(b.lref) + b.lcup;
     });
-    P.ref_units = layout_refine(P.cb_refine, P.ref_groups);
+    P.ref_units = !P.device_packets ? layout_refine(P.cb_refine, false, P.ref_groups)
+                  : P.cb_lane.size() <= kPacketRefineBlocks
+                      ? layout_refine(P.cb_lane, true, P.ref_groups)
+                      : 0;
     if (P.ref_units >= (1ull << 32)) {
         set_last_error("batch too large for 32-bit plan offsets; split it");
         return kErrArg;
@@ -1520,18 +1531,21 @@ uint32_t classic_resident(sgn_hip_session *s, int v, int opt) {
 }
 
 // Refinement passes of the lane list's blocks, after their cleanup (three
-// launches; L lanes a block).
+// launches; L lanes a block).  With device packets the kernels walk the whole lane
+// list and skip the other blocks.
 template <typename C, uint32_t L>
 void launch_refine(sgn_hip_session *s, sgn_j2k_plan &P) {
-    const uint32_t n = static_cast<uint32_t>(P.cb_refine.size());
+    const CbJob *jobs = P.device_packets ? P.d_cb_lane : P.d_cb_refine;
+    const uint32_t n =
+        static_cast<uint32_t>(P.device_packets ? P.cb_lane.size() : P.cb_refine.size());
     C *coef = reinterpret_cast<C *>(P.d_coef);
     const dim3 g((n + split_blocks(L) - 1) / split_blocks(L)), b(kSplitWaves * 64);
-    hipLaunchKernelGGL((sgn_ht_refine_prep<C, L>), g, b, 0, s->stream, P.d_cb_refine, n, P.d_arena,
+    hipLaunchKernelGGL((sgn_ht_refine_prep<C, L>), g, b, 0, s->stream, jobs, n, P.d_arena,
                        static_cast<const C *>(coef), P.d_ref_groups, P.d_ref_work);
     hipLaunchKernelGGL(sgn_ht_sigprop, dim3((n + 64 * kSplitWaves - 1) / (64 * kSplitWaves)), b, 0,
-                       s->stream, P.d_cb_refine, n, P.d_ref_groups, P.d_ref_work);
-    hipLaunchKernelGGL((sgn_ht_refine_apply<C, L>), g, b, 0, s->stream, P.d_cb_refine, n, P.d_arena,
-                       coef, P.d_ref_groups, P.d_ref_work);
+                       s->stream, jobs, n, P.d_ref_groups, P.d_ref_work);
+    hipLaunchKernelGGL((sgn_ht_refine_apply<C, L>), g, b, 0, s->stream, jobs, n, P.d_arena, coef,
+                       P.d_ref_groups, P.d_ref_work);
 }
 
 // Every pass of the lane list in the split kernels (L lanes a block in all but
@@ -1546,16 +1560,14 @@ uint32_t launch_split(sgn_hip_session *s, sgn_j2k_plan &P, SymbolsLaunch symbols
     symbols(s->stream, P.d_cb_lane, n, P.d_arena, P.d_groups, P.d_work, s->d_split);
     hipLaunchKernelGGL((sgn_ht_magsgn<C, L>), g, b, 0, s->stream, P.d_cb_lane, n, P.d_arena, coef,
                        P.d_groups, P.d_work, P.d_status_lane);
-    if (P.device_packets) {
-        // the pass counts are known on the device only: the kernel walks the
-        // whole lane list and skips the other blocks
-        hipLaunchKernelGGL(sgn_ht_refine<C>, dim3((n + 255) / 256), dim3(256), 0, s->stream,
-                           P.d_cb_lane, n, P.d_arena, coef);
-        return 4;
+    if (P.ref_units) {
+        launch_refine<C, L>(s, P);
+        return 6;
     }
-    if (P.cb_refine.empty()) return 3;
-    launch_refine<C, L>(s, P);
-    return 6;
+    if (!P.device_packets) return 3;
+    hipLaunchKernelGGL(sgn_ht_refine<C>, dim3((n + 255) / 256), dim3(256), 0, s->stream,
+                       P.d_cb_lane, n, P.d_arena, coef);
+    return 4;
 }
 
 // Enqueue helpers; each returns the number of kernel launches issued.
@@ -2705,6 +2717,9 @@ int sgn_j2k_plan_kernels(const sgn_j2k_plan *P, char *out, size_t cap, size_t *l
              std::string(kRowsVariants[P->d_work ? P->lane_variant : kCoopVariant].name) +
                  (P->d_work && P->quads && kRowsVariants[P->lane_variant].symbols ? "-quads" : ""),
              P->cb_lane.size());
+    if (P->d_work && kRowsVariants[P->lane_variant].symbols && (P->ref_units || P->device_packets))
+        line("refine", P->ref_units ? "split" : "lane",
+             P->device_packets ? P->cb_lane.size() : P->cb_refine.size());
     if (!P->cb_wave.empty()) line("blocks", "wave-coop-1024", P->cb_wave.size());
     for (int v = 0; v < kClassicShapes; ++v) {
         const size_t n = P->classic_begin[v + 1] - P->classic_begin[v];

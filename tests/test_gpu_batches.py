@@ -220,3 +220,29 @@ def test_device_packet_headers_pipelined_and_region(session, oracle, small_chunk
     cs = S.encode_j2k_ht(img, tile_width=128, tile_height=96, progression=2, precinct_log2=5)
     got = S.J2kDecoder(cs, session).decode_region_to_numpy(S.PixelFormat.RGB8, (70, 33, 150, 90))
     assert np.array_equal(got, img[33:123, 70:220])
+
+
+@pytest.mark.parametrize("tiles,kernel", [(3, "split"), (27, "lane")])
+@pytest.mark.parametrize("refine", [1, 2])
+def test_device_packet_headers_refined(session, oracle, monkeypatch, tiles, kernel, refine):
+    """Refinement passes that only the device knows of: in the split kernels up to
+    65,536 code-blocks, a lane per block past that, refined blocks beside others."""
+    monkeypatch.setenv("SGN_DEVICE_PACKETS", "1")
+    rng = np.random.default_rng(refine)
+    img = rng.integers(0, 256, (256, 256), dtype=np.uint8)
+    opts = dict(use_mct=0, levels=1, cb_width_log2=2, cb_height_log2=2)
+    streams = [S.encode_j2k_ht(img, ht_refine=refine, **opts), S.encode_j2k_ht(img, **opts),
+               S.encode_j2k_ht(img[:77, :130], use_mct=0, levels=2, ht_refine=refine)]
+    want = [O.decode(cs, int(S.PixelFormat.GRAY8)) for cs in streams]
+    plan = S.TilePlan(session, (streams * tiles)[:tiles], S.PixelFormat.GRAY8)
+    blocks = sum(n for stage, _k, n in plan.kernels() if stage == "blocks")
+    assert [(k, n) for stage, k, n in plan.kernels() if stage == "refine"] == [(kernel, blocks)]
+    assert (blocks > 65536) == (kernel == "lane")
+    for mode in (S.MODE_GRAPH, S.MODE_GRAPH, S.MODE_PLAIN):
+        for s in plan.surfaces:
+            s.fill(0)
+        plan.decode(mode)
+        session.synchronize()
+        for k, s in enumerate(plan.surfaces):
+            assert np.array_equal(s.to_numpy(), want[k % 3]), (mode, k)
+    plan.close()
