@@ -96,7 +96,7 @@ struct sgn_hip_session {
     HtSplitTables *d_split = nullptr;
     uint64_t dispatches = 0;
     int cus = 0;                    // compute units of the device
-    uint32_t classic_resident[5][8] = {};  // resident work-groups per classic kernel (shape, lanes)
+    uint32_t classic_resident[6][10] = {};  // resident work-groups per classic kernel (shape, lanes)
     // pipelined batch decode: host-to-device copies run on copy_stream
     // while the previous chunk decodes on `stream`; two staging slots
     hipStream_t copy_stream = nullptr;
@@ -194,56 +194,71 @@ constexpr int kDwtShapeCount = int(sizeof(kDwtShapes) / sizeof(kDwtShapes[0]));
 // style has raw segments, and by lanes per wave.
 using ClassicKernel = void (*)(const ClassicJob *, uint32_t, const uint8_t *, const ClassicSeg *,
                                int32_t *, uint32_t *, uint32_t, uint32_t *);
-constexpr int kClassicShapes = 5;
+constexpr int kClassicShapes = 6;
 constexpr int kClassicLaneOpts = 4;
-template <int LANES>
-using ClassicSmall = ClassicShape<32, 40, LANES, false>;
+template <int LANES, bool RAW>
+using ClassicSmall = ClassicShape<32, 40, LANES, RAW>;
 template <int LANES, bool RAW>
 using ClassicUsual = ClassicShape<128, 144, LANES, RAW>;
 template <bool RAW>
 using ClassicLong = ClassicShape<256, 384, 1, RAW>;
-// Lanes per wave, and the most blocks per CU of a list that takes them: more
-// lanes decode more blocks at once, fewer wait less for each other; lists past
-// the last line go to sgn_t1_rows.  Each line is where the two kernels beside it
-// took the same time on lists of distinct tiles of 256x256 (neighbouring lanes
-// of a list that repeats a few tiles decode the same bits, which flatters the
-// kernels that walk in step):
-//   32x32 blocks (210 a tile), ms with 1, 2, 4 and 16 lanes and in rows: 32 tiles
-//   4.8, 5.25; 36 tiles 5.4, 5.2; 68 tiles -, 5.9, 6.2; 78 tiles -, 6.75, 6.1; 168
-//   tiles -, -, 8.6, 9.0; 180 tiles -, -, 9.25, 8.9; 544 tiles -, -, -, 21.0, 21.8;
-//   1024 tiles -, -, -, 40.6, 30.5.
-//   64x64 blocks (75 a tile), 1 and 3 lanes and in rows: up to 109 tiles 17 to 18
-//   (the longest chain), 23; 160 tiles 22.4, 22.4; 168 tiles 23.4, 22.3; 896 tiles
-//   -, 63.2, 68.9; 960 tiles -, 68.2, 68.0; 1024 tiles -, 72.2, 69.1.
-//   128x32 blocks (48 a tile without levels), 1 lane and in rows: 171 tiles 51, 61;
-//   213 tiles 57, 61; 256 tiles 71, 61.  Three lanes took 55, 68 and 75: their state
-//   leaves a CU too few waves.
+// A list takes about as long as its costliest block, or as all its blocks at the
+// rate of a full device, whichever is longer (the row kernels a fifth of the
+// shorter on top).  A block's cost is its samples times its coding passes, and 256
+// for its start.  More lanes decode more blocks at once, fewer wait less for each
+// other.  The figures are fitted to 1300 timed lists: 16 to 900 distinct tiles of
+// 256x256 (slides, tissue, near-white), blocks from 8x8 to 64x64, 4x1024 and 1024x4,
+// with and without raw segments; the kernel with the shortest estimate was 1.2%
+// slower than the fastest one in the mean.  Some of them, ms with one, three lanes
+// and in rows: 64 tiles of a slide in 64x64 blocks 17.8, 23.0, 64; 300 tiles 40,
+// 22.8, 65; 1024 tiles -, 72, 69; 900 tiles of tissue 64, 34.6, 28.4.  With one, two,
+// four, sixteen lanes and in rows of 16, 32 and 64: 160 tiles in 32x32 blocks 21.8,
+// 12.6, 8.2, 9.0, 15.5, 16.8, 19.4; 900 tiles -, 69, 42, 35, 28.6, 25.1, 27.8.
+// (Lists that repeat a few tiles flatter the kernels that walk in step: lanes
+// beside each other decode the same bits.)
+struct ClassicTime {
+    float chain;  // ns a unit of the costliest block's cost
+    float flow;   // ps a unit of the list's cost on 256 CUs
+};
+constexpr uint64_t kClassicStart = 256;
 struct ClassicChoice {
     ClassicKernel kernel;
-    uint32_t lanes, per_cu;
+    uint32_t lanes;
+    ClassicTime time;
 };
+// (Long blocks with three lanes lose to one lane at every length: their state
+// leaves a CU too few waves.)
 const ClassicChoice kClassicKernels[kClassicShapes][kClassicLaneOpts] = {
-    {{sgn_t1_classic<ClassicSmall<1>>, 1, 28},
-     {sgn_t1_classic<ClassicSmall<2>>, 2, 58},
-     {sgn_t1_classic<ClassicSmall<4>>, 4, 142},
-     {sgn_t1_classic<ClassicSmall<16>>, 16, 450}},
-    {{sgn_t1_classic<ClassicUsual<1, false>>, 1, 46},
-     {sgn_t1_classic<ClassicUsual<3, false>>, 3, 280}},
-    {{sgn_t1_classic<ClassicLong<false>>, 1, 42}},
-    {{sgn_t1_classic<ClassicUsual<1, true>>, 1, 46},
-     {sgn_t1_classic<ClassicUsual<3, true>>, 3, 280}},
-    {{sgn_t1_classic<ClassicLong<true>>, 1, 42}}};
+    {{sgn_t1_classic<ClassicSmall<1, false>>, 1, {163, 69.4f}},
+     {sgn_t1_classic<ClassicSmall<2, false>>, 2, {166, 40.1f}},
+     {sgn_t1_classic<ClassicSmall<4, false>>, 4, {210, 25.3f}},
+     {sgn_t1_classic<ClassicSmall<16, false>>, 16, {335, 21.3f}}},
+    {{sgn_t1_classic<ClassicUsual<1, false>>, 1, {160, 72.4f}},
+     {sgn_t1_classic<ClassicUsual<3, false>>, 3, {202, 40.1f}}},
+    {{sgn_t1_classic<ClassicLong<false>>, 1, {165, 78}}},
+    {{sgn_t1_classic<ClassicSmall<1, true>>, 1, {160, 78.8f}},
+     {sgn_t1_classic<ClassicSmall<2, true>>, 2, {187, 47.5f}},
+     {sgn_t1_classic<ClassicSmall<4, true>>, 4, {227, 28.7f}},
+     {sgn_t1_classic<ClassicSmall<16, true>>, 16, {335, 22.3f}}},
+    {{sgn_t1_classic<ClassicUsual<1, true>>, 1, {166, 78.8f}},
+     {sgn_t1_classic<ClassicUsual<3, true>>, 3, {210, 41.9f}}},
+    {{sgn_t1_classic<ClassicLong<true>>, 1, {170, 83}}}};
 // ... and of the row kernels by block width.
 using ClassicRowsKernel = void (*)(const ClassicJob *, uint32_t, const uint8_t *,
                                    const ClassicSeg *, int32_t *, uint32_t *);
 struct ClassicRowsChoice {
     ClassicRowsKernel kernel;
     uint32_t lanes, max_w;
+    ClassicTime time;
 };
-const ClassicRowsChoice kClassicRows[4] = {{rows::sgn_t1_rows<rows::W32>, 64, 32},
-                                           {rows::sgn_t1_rows<rows::W64>, 32, 64},
-                                           {rows::sgn_t1_rows<rows::W256>, 32, 256},
-                                           {rows::sgn_t1_rows<rows::W1024>, 16, 1024}};
+constexpr int kClassicRowsOpts = 6;
+const ClassicRowsChoice kClassicRows[kClassicRowsOpts] = {
+    {rows::sgn_t1_rows<rows::W32<64>>, 64, 32, {732, 14.6f}},
+    {rows::sgn_t1_rows<rows::W32<32>>, 32, 32, {626, 16.6f}},
+    {rows::sgn_t1_rows<rows::W32<16>>, 16, 32, {557, 20.5f}},
+    {rows::sgn_t1_rows<rows::W64>, 32, 64, {626, 23.2f}},
+    {rows::sgn_t1_rows<rows::W256>, 32, 256, {704, 40.1f}},
+    {rows::sgn_t1_rows<rows::W1024>, 16, 1024, {740, 180}}};
 // Kernel options of a list: kClassicLaneOpts of its shape, then the row kernels.
 const void *classic_kernel(int v, int opt) {
     return opt < kClassicLaneOpts
@@ -257,9 +272,9 @@ uint32_t classic_lanes(int v, int opt) {
 // `small`: small blocks have a list of their own.
 int classic_shape(const ClassicJob &j, bool small) {
     const uint32_t g = classic_groups(j.w, j.h), p = classic_padded(j.w, j.h);
-    const bool raw = (j.style & kCbsBypass) != 0;
-    if (g <= 32 && p <= 40 && !raw && small) return 0;
-    return (g <= 128 && p <= 144 ? 1 : 2) + (raw ? 2 : 0);
+    const int raw = (j.style & kCbsBypass) != 0 ? 3 : 0;
+    if (g <= 32 && p <= 40 && small) return raw;
+    return (g <= 128 && p <= 144 ? 1 : 2) + raw;
 }
 }  // namespace
 
@@ -437,10 +452,10 @@ struct sgn_j2k_plan {
     // [classic_begin[v], classic_begin[v + 1])), costliest first; their
     // segment table; bytes of blocks joined from several packets
     std::vector<ClassicJob> classic;
-    uint32_t classic_begin[6] = {};
-    uint32_t classic_grid[5] = {};  // work-groups launched per shape
-    int classic_opt[5] = {};        // kernel option per shape (classic_kernel)
-    uint32_t classic_mag[5] = {};   // dwords of a lane's magnitude bits or row store
+    uint32_t classic_begin[7] = {};
+    uint32_t classic_grid[6] = {};  // work-groups launched per shape
+    int classic_opt[6] = {};        // kernel option per shape (classic_kernel)
+    uint32_t classic_mag[6] = {};   // dwords of a lane's magnitude bits or row store
     uint32_t *d_crows = nullptr;              // the lanes' magnitude bits or row stores
     std::vector<ClassicSeg> cseg;
     std::vector<uint8_t> joined;
@@ -991,8 +1006,8 @@ Status merge_batch(ParsedBatch &B, sgn_j2k_plan &P, bool pool) {
         size_t n_small = 0, n_usual = 0;
         for (const ClassicJob &j : P.classic) {
             const int v = classic_shape(j, true);
-            n_small += v == 0;
-            n_usual += v == 1;
+            n_small += v % 3 == 0;
+            n_usual += v % 3 == 1;
         }
         const bool small = n_small > 4 * n_usual;
         auto shape = [&](const ClassicJob &j) { return classic_shape(j, small); };
@@ -1158,45 +1173,66 @@ Status slot_reserve(PinnedSlot &sl, size_t bytes, uint8_t **out,
 uint32_t classic_resident(sgn_hip_session *s, int v, int opt);
 uint32_t session_cus(sgn_hip_session *s);
 
-// Chooses the classic kernels, by the length of each list (SGN_CLASSIC_LANES forces
-// a lane count that the shape has; else from 16 on the row kernels, as its former
-// values 64, 32 and 16 did).  Returns the bytes of their lanes' memory.
+// Chooses the kernel of each classic list by its estimated time (ClassicTime).
+// SGN_CLASSIC_LANES forces a lane count that the shape has; else from 16 on the
+// row kernel of the blocks' width with most lanes, as its former values 64, 32
+// and 16 did; "rN" the row kernel with N lanes where there is one.  Returns the
+// bytes of the lanes' memory.
 uint64_t choose_classic(sgn_hip_session *s, sgn_j2k_plan &P, bool tight) {
     uint64_t crows_bytes = 0;
-    const char *lanes_env = std::getenv("SGN_CLASSIC_LANES");
-    const uint32_t forced = lanes_env ? uint32_t(std::atoi(lanes_env)) : 0u;
+    const char *env = std::getenv("SGN_CLASSIC_LANES");
+    const uint32_t forced = env ? uint32_t(std::atoi(env + (env[0] == 'r'))) : 0u;
+    const bool force_rows = env && env[0] == 'r';
     for (int v = 0; v < kClassicShapes; ++v) {
         const uint32_t n = P.classic_begin[v + 1] - P.classic_begin[v];
         P.classic_grid[v] = 0;
         if (!n) continue;
         uint32_t mag = 0, width = 0;
+        uint64_t most = 0, all = 0;
         for (uint32_t k = P.classic_begin[v]; k < P.classic_begin[v + 1]; ++k) {
             const ClassicJob &j = P.classic[k];
             mag = std::max(mag, classic_mag_dwords(j.planes, classic_groups(j.w, j.h)));
             width = std::max<uint32_t>(width, j.w);
+            const uint64_t cost =
+                (j.planes ? uint64_t(j.w) * j.h * j.passes : 0) + kClassicStart;
+            most = std::max(most, cost);
+            all += cost;
         }
-        int opt = 0;
-        auto ends = [&](int o) { return o >= kClassicLaneOpts || !kClassicKernels[v][o].kernel; };
-        while (!ends(opt) && n > kClassicKernels[v][opt].per_cu * session_cus(s)) ++opt;
-        bool by_rows = ends(opt) || forced >= 16;
-        for (int o = 0; !ends(o); ++o)
-            if (kClassicKernels[v][o].lanes == forced) {
-                opt = o;
-                by_rows = false;
-            }
         // tight: the lanes' magnitude bits keep to 3 KB a block (a row store's
         // size), 16 blocks at least; one lane's 63 KB may be more than that
         const uint64_t budget = std::max<uint64_t>(n, 16) * rows::kStateDwords * 4;
-        if (tight && !by_rows && uint64_t(classic_lanes(v, opt)) * mag * 4 > budget) {
-            opt = 0;
-            by_rows = uint64_t(mag) * 4 > budget;
-            if (by_rows) width = rows::W1024::kMaxW;
+        int opt = -1;
+        bool named = false;
+        float best = 0;
+        auto offer = [&](int o, const ClassicTime &t, bool rows, bool force) {
+            const float a = t.chain * 1e-3f * float(most),
+                        b = t.flow * 1e-6f * float(all) * 256.0f / float(session_cus(s));
+            const float us = std::max(a, b) + (rows ? 0.2f * std::min(a, b) : 0.0f);
+            if (!named && (opt < 0 || force || us < best)) {
+                opt = o;
+                best = us;
+            }
+            named |= force;
+        };
+        for (int o = 0; o < kClassicLaneOpts && kClassicKernels[v][o].kernel; ++o) {
+            const ClassicChoice &c = kClassicKernels[v][o];
+            if (!tight || uint64_t(c.lanes) * mag * 4 <= budget)
+                offer(o, c.time, false, !force_rows && c.lanes == forced);
         }
-        if (by_rows) {
-            opt = kClassicLaneOpts;
-            while (kClassicRows[opt - kClassicLaneOpts].max_w < width) ++opt;
-            mag = rows::kStateDwords;
+        if (tight && opt < 0) width = rows::W1024::kMaxW;
+        if (!tight || opt < 0 || forced >= 16) {
+            uint32_t w = 0;
+            for (int o = 0; o < kClassicRowsOpts; ++o) {
+                const ClassicRowsChoice &c = kClassicRows[o];
+                if (c.max_w < width || (w && c.max_w != w)) continue;
+                const bool most_lanes = !w;
+                w = c.max_w;
+                offer(kClassicLaneOpts + o, c.time, true,
+                      force_rows ? c.lanes == forced : forced >= 16 && most_lanes);
+            }
         }
+        const bool by_rows = opt >= kClassicLaneOpts;
+        if (by_rows) mag = rows::kStateDwords;
         const uint32_t lanes = classic_lanes(v, opt);
         const uint64_t group_bytes = uint64_t(lanes) * mag * 4;
         uint64_t grid = std::min((n + lanes - 1) / lanes, classic_resident(s, v, opt));
@@ -2723,14 +2759,15 @@ int sgn_j2k_plan_kernels(const sgn_j2k_plan *P, char *out, size_t cap, size_t *l
     if (!P->cb_wave.empty()) line("blocks", "wave-coop-1024", P->cb_wave.size());
     for (int v = 0; v < kClassicShapes; ++v) {
         const size_t n = P->classic_begin[v + 1] - P->classic_begin[v];
-        static const char *const kShape[kClassicShapes] = {"small", "usual", "long", "usual-raw",
-                                                           "long-raw"};
+        static const char *const kShape[kClassicShapes] = {"small",     "usual",     "long",
+                                                           "small-raw", "usual-raw", "long-raw"};
         if (!n) continue;
         const int opt = P->classic_opt[v];
         line("classic",
              (opt < kClassicLaneOpts
                   ? std::string(kShape[v]) + "-l" + std::to_string(classic_lanes(v, opt))
-                  : "rows-w" + std::to_string(kClassicRows[opt - kClassicLaneOpts].max_w)),
+                  : "rows-w" + std::to_string(kClassicRows[opt - kClassicLaneOpts].max_w) + "-l" +
+                        std::to_string(classic_lanes(v, opt))),
              n);
     }
     for (int rev = 0; rev < 2; ++rev) {

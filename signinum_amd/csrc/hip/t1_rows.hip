@@ -1,5 +1,5 @@
-// Classic (EBCOT) code-blocks of very long lists: one block per lane, 64 lanes of
-// a wave (32 for blocks over 32 wide, 16 over 256) walking the samples in step.
+// Classic (EBCOT) code-blocks of long lists: one block per lane, 64, 32 or 16 lanes
+// of a wave (32 for blocks over 32 wide, 16 over 256) walking the samples in step.
 //
 // The state is one 16-bit word per stripe column (4 samples: significance, sign,
 // visited-in-this-bit-plane and refined-before bits) in a row store in HBM (one
@@ -7,12 +7,12 @@
 // LDS at a time (the stripe above, this one, the one below: a ring), so a lane
 // needs 400 bytes of LDS where sgn_t1_classic keeps 1.2 to 10 KB, and many more
 // blocks are in flight.  Every turn costs more: the lanes wait at every sample
-// that any of them decides.  Lists of 64x64 blocks and smaller ones (75 a tile of
-// 256x256, all tiles distinct) take 67, 69, 74 and 86 ms here for 512, 1024, 1536
-// and 2048 tiles, where sgn_t1_classic takes 37, 72, 108 and 144; 512 tiles in 32x32
-// blocks (107,520) 20.8 and 20.7, 1024 tiles 30 and 41.  Magnitude bits go to the
-// block's int32 coefficients in HBM by atomic OR; the block is zeroed first and
-// the signs are applied in a final sweep.
+// that any of them decides.  Distinct tiles of 256x256 in 64x64 blocks (75 a tile)
+// take 67, 69, 74 and 86 ms here for 512, 1024, 1536 and 2048 tiles, where
+// sgn_t1_classic takes 37, 72, 108 and 144; in 32x32 blocks 600 tiles take 20.4,
+// 19.6 and 21.7 with 16, 32 and 64 lanes and 23.6 there, 900 tiles 28.6, 25.1, 27.8
+// and 35.  Magnitude bits go to the block's int32 coefficients in HBM by atomic
+// OR; the block is zeroed first and the signs are applied in a final sweep.
 #include <hip/hip_runtime.h>
 
 #include "../host/plan_types.h"
@@ -36,7 +36,8 @@ template <int ROWDW, int LANES, int MAXW>
 struct Shape {
     static constexpr int kRowDw = ROWDW, kLanes = LANES, kMaxW = MAXW;
 };
-using W32 = Shape<17, 64, 32>;
+template <int LANES>
+using W32 = Shape<17, LANES, 32>;
 using W64 = Shape<33, 32, 64>;
 using W256 = Shape<129, 32, 256>;
 using W1024 = Shape<513, 16, 1024>;

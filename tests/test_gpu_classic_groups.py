@@ -16,7 +16,7 @@ SHAPES = [(1, 1, 2, 2), (7, 3, 3, 2), (8, 4, 3, 2), (9, 5, 4, 3), (97, 75, 6, 6)
           (5, 90, 2, 8), (260, 4, 10, 2), (3, 300, 2, 10), (64, 64, 6, 6)]
 
 
-@pytest.mark.parametrize("lanes", ["16", "3", "1", "32"])
+@pytest.mark.parametrize("lanes", ["16", "4", "3", "2", "1", "32", "r32", "r16"])
 @pytest.mark.parametrize("style", [0, 1, 2 | 4, 8, 1 | 2 | 4 | 8 | 0x20])
 def test_blocks_of_every_shape(session, oracle, monkeypatch, style, lanes):
     monkeypatch.setenv("SGN_CLASSIC_LANES", lanes)

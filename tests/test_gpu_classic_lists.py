@@ -1,4 +1,4 @@
-"""Which classic kernel a list takes (block shape and blocks per CU), and that
+"""Which classic kernel a list takes (block shape, costs and blocks per CU), and that
 each one decodes full-size blocks: 64x64, 32x32, and the long shapes (more than
 128 groups of 8x4 samples) with and without raw segments, against the source."""
 import numpy as np
@@ -37,14 +37,16 @@ def _check(session, plan, imgs):
         assert np.array_equal(plan.surfaces[k].to_numpy(), imgs[k % 2]), k
 
 
-@pytest.mark.parametrize("exps,per_cu,kernel", [
-    ((6, 6), 1, "usual-l1"), ((6, 6), 45, "usual-l1"), ((6, 6), 48, "usual-l3"),
-    ((6, 6), 270, "usual-l3"), ((6, 6), 290, "rows-w64"),
-    ((5, 5), 20, "small-l1"), ((5, 5), 40, "small-l2"), ((5, 5), 100, "small-l4"),
-    ((5, 5), 300, "small-l16"), ((5, 5), 470, "rows-w32"),
-    ((7, 5), 1, "long-l1"), ((7, 5), 40, "long-l1"), ((7, 5), 50, "rows-w256")])
-def test_kernel_of_a_list(session, exps, per_cu, kernel):
-    plan, imgs = _plan(session, *exps, blocks=per_cu * CUS)
+@pytest.mark.parametrize("exps,style,per_cu,kernel", [
+    ((6, 6), 0, 1, "usual-l1"), ((6, 6), 0, 16, "usual-l3"), ((6, 6), 0, 130, "rows-w64-l32"),
+    ((5, 5), 0, 1, "small-l1"), ((5, 5), 0, 15, "small-l2"), ((5, 5), 0, 30, "small-l4"),
+    ((5, 5), 0, 90, "small-l16"), ((5, 5), 0, 150, "rows-w32-l32"), ((5, 5), 0, 600, "rows-w32-l64"),
+    ((7, 5), 0, 1, "long-l1"), ((7, 5), 0, 80, "rows-w256-l32"),
+    ((6, 6), 1, 1, "usual-raw-l1"), ((6, 6), 1, 16, "usual-raw-l3"), ((6, 6), 1, 130, "rows-w64-l32"),
+    ((5, 5), 1, 1, "small-raw-l1"), ((5, 5), 1, 16, "small-raw-l2"), ((5, 5), 1, 30, "small-raw-l4"),
+    ((5, 5), 1, 90, "small-raw-l16"), ((5, 5), 1, 600, "rows-w32-l64"), ((7, 5), 1, 1, "long-raw-l1")])
+def test_kernel_of_a_list(session, exps, style, per_cu, kernel):
+    plan, imgs = _plan(session, *exps, blocks=per_cu * CUS, style=style)
     assert _kernels(plan) == [kernel]
     _check(session, plan, imgs)
     plan.close()
@@ -62,8 +64,11 @@ def test_long_blocks(session, exps, style, kernel):
 
 
 @pytest.mark.parametrize("lanes,usual,small,long", [
-    ("64", "rows-w64", "rows-w32", "rows-w256"), ("32", "rows-w64", "rows-w32", "rows-w256"),
-    ("16", "rows-w64", "small-l16", "rows-w256"), ("4", "usual-l1", "small-l4", "long-l1"),
+    ("64", "rows-w64-l32", "rows-w32-l64", "rows-w256-l32"),
+    ("32", "rows-w64-l32", "rows-w32-l64", "rows-w256-l32"),
+    ("16", "rows-w64-l32", "small-l16", "rows-w256-l32"),
+    ("r32", "rows-w64-l32", "rows-w32-l32", "rows-w256-l32"),
+    ("r16", "usual-l1", "rows-w32-l16", "long-l1"), ("4", "usual-l1", "small-l4", "long-l1"),
     ("3", "usual-l3", "small-l1", "long-l1"), ("1", "usual-l1", "small-l1", "long-l1"),
     ("5", "usual-l1", "small-l1", "long-l1")])
 def test_forced_lanes(session, monkeypatch, lanes, usual, small, long):
@@ -74,3 +79,13 @@ def test_forced_lanes(session, monkeypatch, lanes, usual, small, long):
         assert _kernels(plan) == [kernel]
         _check(session, plan, imgs)
         plan.close()
+
+
+@pytest.mark.parametrize("style", [0, 1])
+def test_widest_rows(session, monkeypatch, style):
+    """The row kernel of blocks over 256 wide, at full size."""
+    monkeypatch.setenv("SGN_CLASSIC_LANES", "32")
+    plan, imgs = _plan(session, 10, 2, blocks=40, style=style, side=64)
+    assert _kernels(plan) == ["rows-w1024-l16"]
+    _check(session, plan, imgs)
+    plan.close()
