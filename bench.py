@@ -437,23 +437,29 @@ def main():
     achieved = alg / (stage_ms[dom] * 1e-3) / 1e9
     samples = pixels * 3
     es = 2 if st["narrow_samples"] else 4
+    # blocks: coded bytes, samples, and the quads' symbols (16 bits each) written and read
     stage_bytes = {
-        "blocks": st["coded_bytes"] + es * samples,
+        "blocks": st["coded_bytes"] + es * samples + 2 * (2 * samples // 4),
         "levels": es * samples // 4 + 4 * samples // 16,
         "final": 4 * samples // 4 + es * 3 * samples // 4 + samples,
     }
-    kernel_name = {"blocks": "sgn_ht_magsgn", "levels": "sgn_idwt_level", "final": "sgn_final"}[dom]
+    # bytes that the stage's kernels moved on the whole batch, from the tracked counters
+    kernels = {"blocks": ("sgn_ht_clean", "sgn_ht_symbols", "sgn_ht_magsgn"),
+               "levels": ("sgn_idwt_rows_rev",), "final": ("sgn_final_rgb8",)}[dom]
     traffic = None
     tpath = os.path.join(ROOT, "profiles", "hbm_traffic_4096x256_rgb8.json")
     if args.tiles == 4096 and os.path.exists(tpath):
         with open(tpath) as fh:
             tj = json.load(fh)
         lane = S.TilePlan.lane_variants()[plan.lane_variant]
-        cands = [k for k in tj["kernels"].values() if k["kernel"].startswith(kernel_name) and
-                 (dom != "blocks" or k.get("variant") == lane)]
-        if cands:
-            k = max(cands, key=lambda k: k["read_bytes"] + k["write_bytes"])
-            traffic = int(k["read_bytes"] + k["write_bytes"])
+        moved = []
+        for name in kernels:
+            cands = [k["read_bytes"] + k["write_bytes"] for k in tj["kernels"].values()
+                     if k["kernel"].split("<")[0] == name and k.get("variant") in (None, lane)]
+            if cands:
+                moved.append(max(cands))
+        if len(moved) == len(kernels):
+            traffic = int(sum(moved))
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                 "kernel": dom, "kernel_ms": round(stage_ms[dom], 4),
