@@ -26,6 +26,7 @@ def test_sizes(session, w, h, levels):
     img = np.random.default_rng(w * 7 + h).integers(0, 256, (h, w, 3), dtype=np.uint8)
     cs = S.encode_j2k_lossless(img, levels=levels)
     plan = S.TilePlan(session, [cs], S.PixelFormat.RGB8)
+    assert [k for stage, k, _n in plan.kernels() if stage == "final"] == ["5/3-rgb8"]
     for mode in (S.MODE_GRAPH, S.MODE_PLAIN):
         plan.surfaces[0].fill(0x5A)
         plan.decode(mode)
@@ -56,6 +57,7 @@ def test_offsets_pitches_and_neighbouring_kernels(session, offset, pitch_extra):
         bases.append(base)
         surfs.append(_Surface(base, offset, pitch, h))
     plan = S.TilePlan(session, streams, [s[2] for s in shapes], surfaces=surfs)
+    assert [k for stage, k, _n in plan.kernels() if stage == "final"] == ["5/3-rgb8", "5/3-general"]
     plan.decode(S.MODE_GRAPH)
     session.synchronize()
     for (w, h, fmt, _o), img, base in zip(shapes, imgs, bases):

@@ -10,14 +10,20 @@ from signinum_amd import synth
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("tiles,levels", [(1, (5,)), (3, (6, 3)), (7, (2,)), (4, (5, 5, 1)), (171, (4,))])
+@pytest.mark.parametrize("tiles,levels,size,chained", [
+    (1, (5,), 70, 4), (3, (6, 3), 70, 2), (7, (2,), 70, 0), (4, (5, 5, 1), 70, 4), (171, (4,), 70, 0),
+    (2, (3,), 80, 2), (24, (2, 4), 200, 0)])
 @pytest.mark.parametrize("reversible", [1, 0])
-def test_replays_equal_the_per_tile_path(session, tiles, levels, reversible):
+def test_replays_equal_the_per_tile_path(session, tiles, levels, size, chained, reversible):
     rng = np.random.default_rng(tiles)
-    imgs = [synth.tissue_rgb(rng, 90 + 13 * (k % 3), 70 + 5 * (k % 4)) for k in range(12)]
+    imgs = [synth.tissue_rgb(rng, size + 20 + 13 * (k % 3), size + 5 * (k % 4)) for k in range(12)]
     streams = [S.encode_j2k_ht(imgs[k % 12], levels=levels[k % len(levels)], reversible=reversible,
                                use_mct=1) for k in range(tiles)]
     plan = S.TilePlan(session, streams, S.PixelFormat.RGB8)
+    kernels = [k for stage, k, _n in plan.kernels() if stage.startswith("levels")]
+    assert sum("chain" in k for k in kernels) == chained, kernels
+    # levels of at least 8x8 lift in registers, also inside a chain
+    assert size != 80 or set(kernels) == {("5/3" if reversible else "9/7") + "-chain-rows"}
     plan.decode(S.MODE_PLAIN)
     session.synchronize()
     want = [s.to_numpy() for s in plan.surfaces]
